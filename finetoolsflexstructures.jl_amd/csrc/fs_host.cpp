@@ -63,6 +63,15 @@ hipError_t launch_mass(int nen, int64_t N, int E, int composite, const double *g
                        const int32_t *elem_group, const double *x, const double *y, const double *z,
                        const int32_t *conn, const int32_t *ne_ptr, const int32_t *ne_list, const int64_t *node_dof,
                        int64_t nrows, double *diag, hipStream_t st);
+hipError_t launch_cd_mass(int64_t nv, int64_t n, const int64_t *map, const double *mdiag, double dt, double cdamp,
+                          const int32_t *row_group, const double *group_dt, const double *group_cdamp, double *Cd,
+                          double *invMC, hipStream_t st);
+hipError_t launch_cd_place(int64_t nv, int64_t n, const int64_t *map, const double *src, double *dst, hipStream_t st);
+hipError_t launch_cd_place(int64_t nv, int64_t n, const int64_t *map, const int32_t *src, int32_t *dst, hipStream_t st);
+hipError_t launch_cd_probe(int64_t nv, const int64_t *map, int nprobes, const int64_t *plist, int32_t *slot,
+                           hipStream_t st);
+hipError_t launch_cd_collect(int64_t nv, int64_t n, const int64_t *map, const double *src, double *dst,
+                             hipStream_t st);
 hipError_t launch_cd_init(int64_t n, double dt, double g0, const double *invMC, const double *Fmag, const double *U0,
                           const double *V, double *A, double *U1, const int32_t *row_group, const double *group_dt,
                           const double *gtab, hipStream_t st);
@@ -286,7 +295,7 @@ struct MixedStore {
 // uploads its initial state into the same buffers and replays the graph,
 // instead of capturing and instantiating its nsteps launches again.
 struct StepCache {
-    DevBuf dU[2], dV, dA, dF, dInv, dC, dSlot, dProbe, dRG, dGdt, dG;
+    DevBuf dU[2], dV, dA, dF, dInv, dC, dSlot, dProbe, dRG, dGdt, dGcd, dG, dPlist;
     std::vector<uint64_t> key;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -2246,58 +2255,60 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
     // State vectors: the free dofs themselves (FP64 CSR path), or node-major
     // dof positions 6 i + c (mixed path; fixed positions stay zero).
     const int64_t nv = mixed ? 6 * m->N : n;
-    std::vector<int64_t> pos(n);
-    if (mixed) {
-        for (int64_t I = 0; I < m->N; ++I)
-            for (int cc = 0; cc < 6; ++cc) {
-                const int64_t d = m->dof[I * 6 + cc];
-                if (d < n) pos[d] = 6 * I + cc;
-            }
-    } else {
-        for (int64_t d = 0; d < n; ++d) pos[d] = d;
-    }
-    std::vector<double> M(n), U0v(nv, 0.0), V0v(nv, 0.0), Fv(nv, 0.0), Cd(nv, 0.0), invMC(nv, 0.0);
-    std::vector<int32_t> rgv(batch ? nv : 0, 0);
-    if ((s = d2h(c, M.data(), B.mdiag.p, n * 8))) return s;
-    for (int64_t i = 0; i < n; ++i) {
-        const double dt = batch ? p->group_dt[p->row_group[i]] : (p->dt_mass > 0.0 ? p->dt_mass : p->dt);
-        const double cd = batch ? p->group_cdamp[p->row_group[i]] : p->cdamp;
-        const int64_t q = pos[i];
-        Cd[q] = cd * M[i];
-        invMC[q] = 1.0 / (M[i] + (dt / 2) * Cd[q]);  // plate_expl_examples.jl:68-71, before the dt adjustment
-        U0v[q] = U0[i];
-        V0v[q] = V0[i];
-        Fv[q] = Fmag[i];
-        if (batch) rgv[q] = p->row_group[i];
-    }
+    const int64_t *map = mixed ? m->node_dof.as<int64_t>() : nullptr;  // dof at each position
     bool damped = false;
     for (int gi = 0; gi < ng; ++gi) damped |= (batch ? p->group_cdamp[gi] : p->cdamp) != 0.0;
     StepCache &sc = m->step;
     DevBuf(&dU)[2] = sc.dU;
     DevBuf &dV = sc.dV, &dA = sc.dA, &dF = sc.dF, &dInv = sc.dInv, &dC = sc.dC, &dSlot = sc.dSlot,
            &dProbe = sc.dProbe, &dRG = sc.dRG, &dGdt = sc.dGdt, &dG = sc.dG;
-    if ((s = put(c, dU[0], U0v.data(), nv)) || (s = ensure(c, dU[1], nv * 8)) || (s = put(c, dV, V0v.data(), nv)) ||
-        (s = ensure(c, dA, nv * 8)) || (s = put(c, dF, Fv.data(), nv)) || (s = put(c, dInv, invMC.data(), nv)) ||
-        (s = put(c, dC, Cd.data(), nv))) {
+    const int64_t nrec = p->nsteps / stride + 1;
+    std::vector<int64_t> probe_list;  // read by a copy that the loop does not wait for
+    // the caller's vectors into the state buffers; the mixed path's positions
+    // are filled on the device from the free-dof order (through dA, which the
+    // first step's acceleration overwrites afterwards)
+    auto set_up = [&]() -> int {
+        int e;
+        for (DevBuf *b : {&dU[0], &dU[1], &dV, &dA, &dF, &dInv, &dC})
+            if ((e = ensure(c, *b, nv * 8))) return e;
+        const struct {
+            const double *src;
+            double *dst;
+        } vec[3] = {{U0, dU[0].as<double>()}, {V0, dV.as<double>()}, {Fmag, dF.as<double>()}};
+        for (const auto &v : vec) {
+            FS_HIP(c, hipMemcpyAsync(mixed ? dA.as<double>() : v.dst, v.src, n * 8, hipMemcpyHostToDevice, c->stream));
+            if (mixed) FS_HIP(c, fs::launch_cd_place(nv, n, map, dA.as<double>(), v.dst, c->stream));
+        }
+        if (batch) {
+            if ((e = ensure(c, dRG, nv * 4)) || (e = put(c, dGdt, p->group_dt, ng)) ||
+                (e = put(c, sc.dGcd, p->group_cdamp, ng)) || (e = put(c, dG, g, (size_t)(p->nsteps + 1) * ng)))
+                return e;
+            FS_HIP(c, hipMemcpyAsync(mixed ? dA.p : dRG.p, p->row_group, n * 4, hipMemcpyHostToDevice, c->stream));
+            if (mixed)
+                FS_HIP(c, fs::launch_cd_place(nv, n, map, dA.as<int32_t>(), dRG.as<int32_t>(), c->stream));
+        }
+        FS_HIP(c, fs::launch_cd_mass(nv, n, map, B.mdiag.as<double>(), p->dt_mass > 0.0 ? p->dt_mass : p->dt, p->cdamp,
+                                     batch ? dRG.as<int32_t>() : nullptr, dGdt.as<double>(), sc.dGcd.as<double>(),
+                                     dC.as<double>(), dInv.as<double>(), c->stream));
+        if (nprobes > 0) {
+            // the probes sorted by dof (of two probes of one dof the later one
+            // counts): dofs, then their slots, in one buffer
+            std::map<int64_t, int64_t> by_dof;
+            for (int k = 0; k < nprobes; ++k) by_dof[probe_dofs[k]] = k;
+            for (const auto &kv : by_dof) probe_list.push_back(kv.first);
+            for (const auto &kv : by_dof) probe_list.push_back(kv.second);
+            if ((e = ensure(c, dSlot, nv * 4)) || (e = put(c, sc.dPlist, probe_list.data(), probe_list.size())) ||
+                (e = ensure(c, dProbe, (size_t)nrec * nprobes * 8)))
+                return e;
+            FS_HIP(c, fs::launch_cd_probe(nv, map, (int)by_dof.size(), sc.dPlist.as<int64_t>(), dSlot.as<int32_t>(),
+                                          c->stream));
+            for (int k = 0; k < nprobes; ++k) probe_out[k] = U0[probe_dofs[k]];  // peek(0, U0)
+        }
+        return FS_OK;
+    };
+    if ((s = set_up())) {
         sc.drop_graph();
         return s;
-    }
-    if (batch) {
-        if ((s = put(c, dRG, rgv.data(), nv)) || (s = put(c, dGdt, p->group_dt, ng)) ||
-            (s = put(c, dG, g, (size_t)(p->nsteps + 1) * ng))) {
-            sc.drop_graph();
-            return s;
-        }
-    }
-    const int64_t nrec = p->nsteps / stride + 1;
-    if (nprobes > 0) {
-        std::vector<int32_t> slot(nv, -1);
-        for (int k = 0; k < nprobes; ++k) slot[pos[probe_dofs[k]]] = k;
-        if ((s = put(c, dSlot, slot.data(), nv)) || (s = ensure(c, dProbe, (size_t)nrec * nprobes * 8))) {
-            sc.drop_graph();
-            return s;
-        }
-        for (int k = 0; k < nprobes; ++k) probe_out[k] = U0[probe_dofs[k]];  // peek(0, U0)
     }
     // steps whose load factor is zero for every model skip the Fmag read (mixed path)
     std::vector<uint8_t> forced(p->nsteps + 1, 0);
@@ -2407,14 +2418,15 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
     m->timing[4] = build_ms;
     // after the last step the buffer not indexed by the loop's final `cur` holds U_nsteps
     const int fin = (p->nsteps % 2 == 1) ? 1 : 0;
-    if (U_out || V_out) {
-        std::vector<double> Uv(nv), Vv(nv);
-        if ((s = d2h(c, Uv.data(), dU[p->nsteps == 0 ? 0 : fin].p, nv * 8)) || (s = d2h(c, Vv.data(), dV.p, nv * 8)))
-            return s;
-        for (int64_t i = 0; i < n; ++i) {
-            if (U_out) U_out[i] = Uv[pos[i]];
-            if (V_out) V_out[i] = Vv[pos[i]];
-        }
+    const double *Ufin = dU[p->nsteps == 0 ? 0 : fin].as<double>();
+    const struct {
+        const double *src;
+        double *out;
+    } res[2] = {{Ufin, U_out}, {dV.as<double>(), V_out}};
+    for (const auto &r : res) {
+        if (!r.out) continue;
+        if (mixed) FS_HIP(c, fs::launch_cd_collect(nv, n, map, r.src, dA.as<double>(), c->stream));
+        if ((s = d2h(c, r.out, mixed ? dA.p : r.src, n * 8))) return s;
     }
     if (nprobes > 0 && nrec > 1 &&
         (s = d2h(c, probe_out + nprobes, dProbe.as<double>() + nprobes, (size_t)(nrec - 1) * nprobes * 8)))
