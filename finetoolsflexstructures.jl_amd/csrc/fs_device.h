@@ -210,4 +210,42 @@ struct NodeRows {
     const int32_t *info;
 };
 
+// Symmetric form of the free-free stiffness for the time loop, by patches: up
+// to PATCH_NODES nodes that lie together, all of one connected component.
+// Node slot s = p PATCH_NODES + li holds local node li of patch p, and the
+// state vectors of the loop are in slot order, position q = 6 s + c (unused
+// slots and fixed dofs carry zeros).  A block K_IJ (6 x 6, zero rows and
+// columns at fixed dofs) is stored once where I and J lie in one patch
+// (an inner entry, li < lj), and in both patches otherwise (an outer entry of
+// each, with the row node local).
+//   rec[p]    {first block (a multiple of 8), entries, -, -}; the inner entries
+//             come first
+//   ent       entry e of patch p: x = li << 26 | slot of J; y = partial slot of
+//             I | partial slot of J << 16 (0xffff: an outer entry).  The first
+//             PATCH_WG entries are at p PATCH_WG + e, so that their loads wait on
+//             nothing; the others at over + first block + e.
+//   entk      neighbour slot of J in I's list (ScatterPlan), indexed as ent
+//   pnode[s]  node of slot s, -1 if unused
+//   nptr[p (PATCH_NODES + 1) + li]  partial slots of local node li: one per
+//             neighbour, in the order of its list
+//   k2        blocks of patch p from 18 first block on, two values a unit: unit
+//             v of entry e (rows in order, three units a row) at v nep + e,
+//             nep = entries rounded up to 8
+//   dg        diagonal blocks, 21 upper values (row by row) per slot
+constexpr int PATCH_NODES = 42;
+constexpr int PATCH_WG = 6 * PATCH_NODES;  // lanes of a patch: a dof each, or an entry each
+constexpr int PATCH_TRI = 21;
+struct PatchOp {
+    int32_t npatch;
+    int32_t slots;            // partial slots of the largest patch
+    int64_t over;
+    const int4 *rec;
+    const uint2 *ent;
+    const int32_t *entk;
+    const int32_t *pnode;
+    const uint16_t *nptr;
+    double2 *k2;
+    double *dg;
+};
+
 }  // namespace fs

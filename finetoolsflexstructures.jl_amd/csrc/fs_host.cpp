@@ -88,6 +88,16 @@ hipError_t launch_cd_node_step(int nl, int pj, const NodeRows &nrw, const int2 *
                                const double *Cd, const double *Fmag, double gstep, double dt, int damped,
                                const int32_t *probe_slot, double *probe_dst, const int32_t *row_group,
                                const double *group_dt, const double *gtab, hipStream_t st);
+hipError_t launch_patch_map(const PatchOp &op, const int64_t *node_dof, int64_t *map, hipStream_t st);
+hipError_t launch_patch_build(const PatchOp &op, const ScatterPlan &sp, const double *kval, hipStream_t st);
+hipError_t launch_patch_init(const PatchOp &op, double dt, double g0, const double *invMC, const double *Fmag,
+                             const double *U0, double *W, double *U1, const int32_t *row_group,
+                             const double *group_dt, const double *gtab, hipStream_t st);
+size_t patch_smem(int slots);
+hipError_t launch_cd_patch_step(const PatchOp &op, const double *Ucur, double *Unext, double *W, const double *invMC,
+                                const double *Cd, const double *Fmag, double gstep, double dt, int damped, int forced,
+                                int last, const int32_t *probe_slot, double *probe_dst,
+                                const int32_t *row_group, const double *group_dt, const double *gtab, hipStream_t st);
 hipError_t launch_dot(int64_t n, int mode, const double *x, const double *y, const double *d, double *part,
                       double *out, hipStream_t st);
 hipError_t launch_scale(int64_t n, const double *ss, const double *d, const double *x, double *y, hipStream_t st);
@@ -214,6 +224,25 @@ struct TileStore {
     }
 };
 
+// Patch form of the free-free stiffness (fs::PatchOp): the plan, built on
+// the first loop that takes it, and the values it holds.
+struct PatchStore {
+    bool planned = false, usable = false;
+    int64_t npatch = 0, nent = 0;
+    int slots = 0;
+    uint64_t vgen = 0;  // generation of the values it was filled from
+    std::vector<int32_t> pnode;  // host copy: the node of each slot
+    DevBuf rec, ent, entk, dpnode, nptr, map, k2, dg;
+    void reset() {
+        planned = usable = false;
+        npatch = nent = 0;
+        slots = 0;
+        vgen = 0;
+        pnode.clear();
+        for (DevBuf *b : {&rec, &ent, &entk, &dpnode, &nptr, &map, &k2, &dg}) b->release();
+    }
+};
+
 struct Block {
     bool built = false;
     int64_t nrows = 0;
@@ -242,6 +271,8 @@ struct Block {
     int64_t nrownodes = 0;
     int32_t max_rowlen = 0;
     bool k_ready = false, m_ready = false;
+    uint64_t vgen = 0;  // raised before each launch that writes kval
+    PatchStore patch;
     // host copies for the fused-assembly planner: neighbour slot -> (pair <<
     // 1 | side), pair nodes and slots, contributions per pair (counts)
     std::vector<int32_t> h_nb_pair, h_pnode, h_pslot, h_cptr;
@@ -258,6 +289,7 @@ struct Block {
         h_node_rec.clear();
         h_nb_off.clear();
         tiles.reset();
+        patch.reset();
         nrows = nnz = npairs = nrownodes = 0;
         max_rowlen = 0;
         rowptr.clear();
@@ -890,6 +922,271 @@ fs::TilePlan tileplan_of(const Block &B) {
     tp.bp_ptr = B.tiles.bp_ptr.as<int32_t>();
     tp.partial = B.tiles.partial.as<double>();
     return tp;
+}
+
+fs::PatchOp patchop_of(const PatchStore &P) {
+    fs::PatchOp op;
+    op.npatch = (int32_t)P.npatch;
+    op.slots = P.slots;
+    op.over = P.npatch * fs::PATCH_WG;
+    op.rec = P.rec.as<int4>();
+    op.ent = P.ent.as<uint2>();
+    op.entk = P.entk.as<int32_t>();
+    op.pnode = P.dpnode.as<int32_t>();
+    op.nptr = P.nptr.as<uint16_t>();
+    op.k2 = P.k2.as<double2>();
+    op.dg = P.dg.as<double>();
+    return op;
+}
+
+// Partial slots a patch may have: 6 doubles each in LDS (48 KB), so that two
+// workgroups fit a CU.
+constexpr int PATCH_MAX_SLOTS = 1024;
+
+// Patch plan of the free-free block (fs::PatchOp).  The nodes with free dofs
+// are grouped by connected component, and each component is cut by
+// recursive coordinate bisection into patches of at most PATCH_NODES nodes of
+// nearly equal size: a set that needs k patches is cut across its longest
+// extent, ties by node number, into shares of floor(k/2) and the rest.  The
+// cuts depend on a component's own nodes only, so a model has the same
+// patches alone and in a batch.  A mesh with a node of more neighbours than a
+// patch may have partial slots keeps the row forms (usable false).
+int build_patches(fs_model *m) {
+    fs_ctx *c = m->ctx;
+    Block &B = m->blk[FS_BLOCK_FF];
+    PatchStore &P = B.patch;
+    P.reset();
+    P.planned = true;
+    const int64_t N = m->N;
+    constexpr int PN = fs::PATCH_NODES;
+    if (N >= (int64_t(1) << 24)) return FS_OK;  // slots are 26-bit numbers
+    auto active = [&](int64_t I) { return B.h_node_rec[4 * I] >= 0; };  // node with free dofs
+    auto degree = [&](int64_t I) { return m->nbr_ptr[I + 1] - m->nbr_ptr[I]; };
+    for (int64_t I = 0; I < N; ++I)
+        if (active(I) && degree(I) > PATCH_MAX_SLOTS) return FS_OK;
+    // components: union-find, the smaller number of two roots stays one
+    std::vector<int32_t> par(N);
+    for (int64_t i = 0; i < N; ++i) par[i] = (int32_t)i;
+    auto find = [&](int32_t x) {
+        for (;;) {
+            const int32_t px = __atomic_load_n(&par[x], __ATOMIC_RELAXED);
+            if (px == x) return x;
+            const int32_t g = __atomic_load_n(&par[px], __ATOMIC_RELAXED);
+            if (g != px) __atomic_store_n(&par[x], g, __ATOMIC_RELAXED);
+            x = g;
+        }
+    };
+    parallel_chunks(N, [&](int64_t I0, int64_t I1) {
+        for (int64_t I = I0; I < I1; ++I)
+            for (int k = m->nbr_ptr[I]; k < m->nbr_ptr[I + 1] && m->nbr_list[k] < I; ++k) {
+                int32_t a = (int32_t)I, b = m->nbr_list[k];
+                for (;;) {
+                    a = find(a);
+                    b = find(b);
+                    if (a == b) break;
+                    if (a < b) std::swap(a, b);
+                    int32_t want = a;
+                    if (__atomic_compare_exchange_n(&par[a], &want, b, false, __ATOMIC_RELAXED, __ATOMIC_RELAXED)) break;
+                }
+            }
+    }, 16384);
+    // active nodes by component (components by their smallest node)
+    struct Pt {
+        double x[3];
+        int64_t id;
+    };
+    std::vector<int32_t> cid(N, -1);
+    std::vector<int64_t> cptr(1, 0);
+    for (int64_t I = 0; I < N; ++I) {
+        const int32_t r = find((int32_t)I);
+        if (cid[r] < 0) {
+            cid[r] = (int32_t)cptr.size() - 1;
+            cptr.push_back(0);
+        }
+        cid[I] = cid[r];
+        if (active(I)) ++cptr[cid[I] + 1];
+    }
+    const int64_t nc = (int64_t)cptr.size() - 1;
+    for (int64_t k = 0; k < nc; ++k) cptr[k + 1] += cptr[k];
+    std::vector<double> xyz(3 * N);
+    FS_HIP(c, hipMemcpyAsync(xyz.data(), m->x.p, N * 8, hipMemcpyDeviceToHost, c->stream));
+    FS_HIP(c, hipMemcpyAsync(xyz.data() + N, m->y.p, N * 8, hipMemcpyDeviceToHost, c->stream));
+    FS_HIP(c, hipMemcpyAsync(xyz.data() + 2 * N, m->z.p, N * 8, hipMemcpyDeviceToHost, c->stream));
+    FS_HIP(c, hipStreamSynchronize(c->stream));
+    std::vector<Pt> pt(cptr[nc]);
+    {
+        std::vector<int64_t> fill(cptr.begin(), cptr.end() - 1);
+        auto num = [](double v) { return std::isfinite(v) ? v : 0.0; };  // an order needs numbers
+        for (int64_t I = 0; I < N; ++I)
+            if (active(I)) pt[fill[cid[I]]++] = Pt{{num(xyz[I]), num(xyz[N + I]), num(xyz[2 * N + I])}, I};
+    }
+    std::vector<uint8_t> head(pt.size() + 1, 0);  // 1 where a patch begins
+    std::function<void(int64_t, int64_t)> bisect = [&](int64_t b, int64_t n) {
+        Pt *q = pt.data() + b;
+        int64_t k = (n + PN - 1) / PN;
+        if (k == 1) {
+            int64_t slots = 0;
+            for (int64_t i = 0; i < n; ++i) slots += degree(q[i].id);
+            if (slots <= PATCH_MAX_SLOTS) {
+                head[b] = 1;
+                return;
+            }
+            k = 2;
+        }
+        const int64_t n1 = n * (k / 2) / k;
+        double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+        for (int64_t i = 0; i < n; ++i)
+            for (int d = 0; d < 3; ++d) {
+                lo[d] = std::min(lo[d], q[i].x[d]);
+                hi[d] = std::max(hi[d], q[i].x[d]);
+            }
+        int ax = 0;
+        for (int d = 1; d < 3; ++d)
+            if (hi[d] - lo[d] > hi[ax] - lo[ax]) ax = d;
+        std::nth_element(q, q + n1, q + n, [ax](const Pt &u, const Pt &v) {
+            return u.x[ax] != v.x[ax] ? u.x[ax] < v.x[ax] : u.id < v.id;
+        });
+        if (n > 8192) {
+            std::thread th(bisect, b + n1, n - n1);
+            bisect(b, n1);
+            th.join();
+        } else {
+            bisect(b, n1);
+            bisect(b + n1, n - n1);
+        }
+    };
+    parallel_chunks(nc, [&](int64_t k0, int64_t k1) {
+        for (int64_t k = k0; k < k1; ++k)
+            if (cptr[k + 1] > cptr[k]) bisect(cptr[k], cptr[k + 1] - cptr[k]);
+    }, 4);
+    std::vector<int64_t> pstart;
+    for (int64_t i = 0; i < (int64_t)pt.size(); ++i)
+        if (head[i]) pstart.push_back(i);
+    const int64_t np = (int64_t)pstart.size();
+    pstart.push_back((int64_t)pt.size());
+    if (np * PN >= (int64_t(1) << 26)) return FS_OK;
+    P.pnode.assign(np * PN, -1);
+    std::vector<int32_t> slot(N, -1);
+    std::vector<int32_t> rec(4 * np, 0);
+    parallel_chunks(np, [&](int64_t p0, int64_t p1) {
+        for (int64_t p = p0; p < p1; ++p) {
+            std::sort(pt.begin() + pstart[p], pt.begin() + pstart[p + 1], [](const Pt &u, const Pt &v) { return u.id < v.id; });
+            for (int64_t i = pstart[p]; i < pstart[p + 1]; ++i) {
+                P.pnode[p * PN + i - pstart[p]] = (int32_t)pt[i].id;
+                slot[pt[i].id] = (int32_t)(p * PN + i - pstart[p]);
+            }
+        }
+    }, 512);
+    // entries of each patch: counts, then the lists
+    std::vector<int32_t> ninner(np, 0);
+    parallel_chunks(np, [&](int64_t p0, int64_t p1) {
+        for (int64_t p = p0; p < p1; ++p) {
+            int inner = 0, outer = 0;
+            for (int64_t i = pstart[p]; i < pstart[p + 1]; ++i) {
+                const int64_t I = pt[i].id;
+                for (int k = m->nbr_ptr[I]; k < m->nbr_ptr[I + 1]; ++k) {
+                    const int32_t sj = slot[m->nbr_list[k]];
+                    if (sj < 0) continue;
+                    if (sj / PN != p) ++outer;
+                    else if (sj > slot[I]) ++inner;
+                }
+            }
+            ninner[p] = inner;
+            rec[4 * p + 1] = inner + outer;
+        }
+    }, 512);
+    int64_t nent = 0, nover = 0;  // blocks, and the reach of the entries past PATCH_WG
+    for (int64_t p = 0; p < np; ++p) {
+        rec[4 * p] = (int32_t)nent;
+        if (rec[4 * p + 1] > fs::PATCH_WG) nover = nent + rec[4 * p + 1];
+        nent += (rec[4 * p + 1] + 7) & ~7;
+    }
+    if (nent >= (int64_t(1) << 30)) return FS_OK;
+    const int64_t over = np * fs::PATCH_WG, ntab = over + nover;
+    std::vector<uint32_t> ent(2 * ntab, 0);
+    std::vector<int32_t> entk(ntab, 0);
+    std::vector<uint16_t> nptr(np * (PN + 1), 0);
+    std::atomic<int> most{0};
+    parallel_chunks(np, [&](int64_t p0, int64_t p1) {
+        std::vector<int32_t> by(PN * PN);  // place of the inner entry of (li, lj)
+        for (int64_t p = p0; p < p1; ++p) {
+            int ei = 0, eo = ninner[p];
+            auto place = [&](int e) { return e < fs::PATCH_WG ? p * fs::PATCH_WG + e : over + rec[4 * p] + e; };
+            const int n = (int)(pstart[p + 1] - pstart[p]);
+            int sl = 0;  // partial slots: one per active neighbour, in list order
+            for (int li = 0; li < n; ++li) {
+                const int64_t I = pt[pstart[p] + li].id;
+                nptr[p * (PN + 1) + li] = (uint16_t)sl;
+                for (int k = m->nbr_ptr[I]; k < m->nbr_ptr[I + 1]; ++k) {
+                    const int32_t sj = slot[m->nbr_list[k]];
+                    if (sj < 0 || m->nbr_list[k] == I) continue;
+                    const int lj = (int)(sj - p * PN);
+                    if (sj / PN == p && lj < li) {
+                        const int64_t at = by[lj * PN + li];
+                        ent[2 * at + 1] = (ent[2 * at + 1] & 0xffffu) | (uint32_t)sl << 16;
+                    } else {
+                        const bool inner = sj / PN == p;
+                        const int64_t at = place(inner ? ei++ : eo++);
+                        if (inner) by[li * PN + lj] = (int32_t)at;
+                        ent[2 * at] = (uint32_t)li << 26 | (uint32_t)sj;
+                        ent[2 * at + 1] = (uint32_t)sl | 0xffff0000u;
+                        entk[at] = k;
+                    }
+                    ++sl;
+                }
+            }
+            for (int li = n; li <= PN; ++li) nptr[p * (PN + 1) + li] = (uint16_t)sl;
+            int cur = most.load();
+            while (cur < sl && !most.compare_exchange_weak(cur, sl)) {
+            }
+        }
+    }, 512);
+    int s;
+    if ((s = upload(c, P.rec, rec.data(), rec.size())) || (s = upload(c, P.ent, ent.data(), ent.size())) ||
+        (s = upload(c, P.entk, entk.data(), entk.size())) || (s = upload(c, P.dpnode, P.pnode.data(), P.pnode.size())) ||
+        (s = upload(c, P.nptr, nptr.data(), nptr.size())) || (s = dalloc(c, P.map, (size_t)np * PN * 6 * 8)) ||
+        (s = dalloc(c, P.k2, (size_t)nent * 288)) || (s = dalloc(c, P.dg, (size_t)np * PN * fs::PATCH_TRI * 8)))
+        return s;
+    P.npatch = np;
+    P.nent = nent;
+    P.slots = most;
+    P.usable = true;
+    fs::PatchOp op = patchop_of(P);
+    FS_HIP(c, fs::launch_patch_map(op, m->node_dof.as<int64_t>(), P.map.as<int64_t>(), c->stream));
+    FS_HIP(c, hipStreamSynchronize(c->stream));  // the host lists end here
+    return FS_OK;
+}
+
+// Steps from which an FP64 loop takes the patch form.  Its plan costs a model's
+// first such loop about 47 ns per node once (12 ms on the 512 x 512 Q4 panel, 26
+// ms on the 1024 x 512 T3 plate, 16 host threads), and a step then saves 0.2 ns
+// per node (63 and 103 us): from 100 steps on the second loop has paid for it.
+constexpr int64_t PATCH_MIN_STEPS = 100;
+
+// The patch form with the resident values of K: its plan, if there is none
+// yet, and its blocks, if K was computed again since.  *use becomes false
+// where the form does not take the mesh, or there is no memory for it.
+int prepare_patches(fs_model *m, bool *use) {
+    fs_ctx *c = m->ctx;
+    Block &B = m->blk[FS_BLOCK_FF];
+    PatchStore &P = B.patch;
+    if (!P.planned) {
+        const int s = build_patches(m);
+        if (s == FS_ERR_NOMEM) {
+            P.reset();
+            P.planned = true;  // not tried again for this block
+            c->err.clear();
+        } else if (s) {
+            P.reset();
+            return s;
+        }
+    }
+    *use = P.usable;
+    if (P.usable && P.vgen != B.vgen) {
+        FS_HIP(c, fs::launch_patch_build(patchop_of(P), plan_of(B), B.kval.as<double>(), c->stream));
+        P.vgen = B.vgen;
+    }
+    return FS_OK;
 }
 
 // 3 x 21-bit Morton code of a point scaled into [0, 1)^3.
@@ -1945,6 +2242,7 @@ int fs_model_stiffness(fs_model *m, const fs_shell_params *p, int block, double 
         FS_HIP(c, hipEventCreate(&t1));
         FS_HIP(c, hipEventCreate(&t2));
         FS_HIP(c, hipEventRecord(t0, c->stream));
+        ++B.vgen;
         FS_HIP(c, fs::launch_element_fused(ep, m->x.as<double>(), m->y.as<double>(), m->z.as<double>(),
                                            m->dconn.as<int32_t>(), m->nx.as<double>(), m->ny.as<double>(),
                                            m->nz.as<double>(), m->valid.as<uint8_t>(), m->status.as<int>(), sp, tp,
@@ -1999,6 +2297,7 @@ int fs_model_stiffness(fs_model *m, const fs_shell_params *p, int block, double 
     FS_HIP(c, hipEventCreate(&t2));
     FS_HIP(c, hipEventRecord(t0, c->stream));
     fs::ScatterPlan sp = plan_of(B);
+    ++B.vgen;
     int64_t pdone = 0;
     for (int64_t k = 0; k < nranges; ++k) {
         ep.ebegin = (int32_t)(k * per);
@@ -2252,10 +2551,21 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
             build_ms = m->mixed.build_ms;
         }
     }
-    // State vectors: the free dofs themselves (FP64 CSR path), or node-major
-    // dof positions 6 i + c (mixed path; fixed positions stay zero).
-    const int64_t nv = mixed ? 6 * m->N : n;
-    const int64_t *map = mixed ? m->node_dof.as<int64_t>() : nullptr;  // dof at each position
+    // FP64 loops of PATCH_MIN_STEPS steps or more run on the patch form of K
+    // unless the row products were chosen (fs_ctx_set_cd_lanes); a rule on the
+    // call's step count alone, so that a model takes the same form alone and
+    // in a batch.
+    PatchStore &P = B.patch;
+    bool patch = !mixed && c->cd_lanes == 8 && c->cd_pj == 0 && p->nsteps >= PATCH_MIN_STEPS;
+    if (patch && (s = prepare_patches(m, &patch))) return s;
+    const fs::PatchOp pop = patchop_of(P);
+    // State vectors: the free dofs themselves (row products), node-major dof
+    // positions 6 i + c (mixed path), or the patches' slot positions; fixed
+    // dofs stay zero in the last two.
+    const bool placed = mixed || patch;
+    const int64_t nv = mixed ? 6 * m->N : patch ? P.npatch * 6 * fs::PATCH_NODES : n;
+    // dof at each position
+    const int64_t *map = mixed ? m->node_dof.as<int64_t>() : patch ? P.map.as<int64_t>() : nullptr;
     bool damped = false;
     for (int gi = 0; gi < ng; ++gi) damped |= (batch ? p->group_cdamp[gi] : p->cdamp) != 0.0;
     StepCache &sc = m->step;
@@ -2264,27 +2574,27 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
            &dProbe = sc.dProbe, &dRG = sc.dRG, &dGdt = sc.dGdt, &dG = sc.dG;
     const int64_t nrec = p->nsteps / stride + 1;
     std::vector<int64_t> probe_list;  // read by a copy that the loop does not wait for
-    // the caller's vectors into the state buffers; the mixed path's positions
-    // are filled on the device from the free-dof order (through dA, which the
-    // first step's acceleration overwrites afterwards)
+    // the caller's vectors into the state buffers; placed positions are filled
+    // on the device from the free-dof order (through dA, which is free until
+    // the loop starts)
     auto set_up = [&]() -> int {
         int e;
         for (DevBuf *b : {&dU[0], &dU[1], &dV, &dA, &dF, &dInv, &dC})
-            if ((e = ensure(c, *b, nv * 8))) return e;
+            if ((e = ensure(c, *b, std::max(nv, n) * 8))) return e;
         const struct {
             const double *src;
             double *dst;
         } vec[3] = {{U0, dU[0].as<double>()}, {V0, dV.as<double>()}, {Fmag, dF.as<double>()}};
         for (const auto &v : vec) {
-            FS_HIP(c, hipMemcpyAsync(mixed ? dA.as<double>() : v.dst, v.src, n * 8, hipMemcpyHostToDevice, c->stream));
-            if (mixed) FS_HIP(c, fs::launch_cd_place(nv, n, map, dA.as<double>(), v.dst, c->stream));
+            FS_HIP(c, hipMemcpyAsync(placed ? dA.as<double>() : v.dst, v.src, n * 8, hipMemcpyHostToDevice, c->stream));
+            if (placed) FS_HIP(c, fs::launch_cd_place(nv, n, map, dA.as<double>(), v.dst, c->stream));
         }
         if (batch) {
             if ((e = ensure(c, dRG, nv * 4)) || (e = put(c, dGdt, p->group_dt, ng)) ||
                 (e = put(c, sc.dGcd, p->group_cdamp, ng)) || (e = put(c, dG, g, (size_t)(p->nsteps + 1) * ng)))
                 return e;
-            FS_HIP(c, hipMemcpyAsync(mixed ? dA.p : dRG.p, p->row_group, n * 4, hipMemcpyHostToDevice, c->stream));
-            if (mixed)
+            FS_HIP(c, hipMemcpyAsync(placed ? dA.p : dRG.p, p->row_group, n * 4, hipMemcpyHostToDevice, c->stream));
+            if (placed)
                 FS_HIP(c, fs::launch_cd_place(nv, n, map, dA.as<int32_t>(), dRG.as<int32_t>(), c->stream));
         }
         FS_HIP(c, fs::launch_cd_mass(nv, n, map, B.mdiag.as<double>(), p->dt_mass > 0.0 ? p->dt_mass : p->dt, p->cdamp,
@@ -2323,7 +2633,10 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
     const double *gdt = batch ? dGdt.as<double>() : nullptr;
     const fs::MixedOp op = mixed ? mixed_op(m) : fs::MixedOp{};
     auto enqueue = [&](hipStream_t st) -> hipError_t {
-        hipError_t e = fs::launch_cd_init(nv, p->dt, batch ? 0.0 : g[0], dInv.as<double>(), dF.as<double>(),
+        hipError_t e = patch ? fs::launch_patch_init(pop, p->dt, batch ? 0.0 : g[0], dInv.as<double>(), dF.as<double>(),
+                                                     dU[0].as<double>(), dV.as<double>(), dU[1].as<double>(), rg, gdt,
+                                                     batch ? dG.as<double>() : nullptr, st)
+                             : fs::launch_cd_init(nv, p->dt, batch ? 0.0 : g[0], dInv.as<double>(), dF.as<double>(),
                                           dU[0].as<double>(), dV.as<double>(), dA.as<double>(), dU[1].as<double>(),
                                           rg, gdt, batch ? dG.as<double>() : nullptr, st);
         if (e != hipSuccess) return e;
@@ -2338,6 +2651,11 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
                                              dU[1 - cur].as<double>(), dV.as<double>(), dA.as<double>(),
                                              dInv.as<double>(), dC.as<double>(), dF.as<double>(),
                                              batch ? 0.0 : g[step], p->dt, damped ? 1 : 0, forced[step] ? 1 : 0,
+                                             slot, pdst, rg, gdt, gt, st);
+            else if (patch)
+                e = fs::launch_cd_patch_step(pop, dU[cur].as<double>(), dU[1 - cur].as<double>(), dV.as<double>(),
+                                             dInv.as<double>(), dC.as<double>(), dF.as<double>(), batch ? 0.0 : g[step],
+                                             p->dt, damped ? 1 : 0, forced[step] ? 1 : 0, step == p->nsteps ? 1 : 0,
                                              slot, pdst, rg, gdt, gt, st);
             else if (c->cd_lanes > 0)
                 e = fs::launch_cd_node_step(c->cd_lanes, cd_pj, noderows_of(B), B.slotrec.as<int2>(), B.kval.as<double>(),
@@ -2364,7 +2682,7 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
         key.reserve(64 + (size_t)p->nsteps + 1);
         for (const int64_t v : {nv, n, (int64_t)p->nsteps, (int64_t)p->precision, (int64_t)stride, (int64_t)nprobes,
                                 (int64_t)ng, (int64_t)batch, (int64_t)damped, (int64_t)c->cd_lanes, (int64_t)cd_pj,
-                                (int64_t)tpr, (int64_t)m->nen, (int64_t)m->mixed.nsr})
+                                (int64_t)tpr, (int64_t)m->nen, (int64_t)m->mixed.nsr, (int64_t)patch})
             key_add(key, v);
         key_add(key, p->dt);
         for (const DevBuf *b : {&dU[0], &dU[1], &dV, &dA, &dF, &dInv, &dC, &dSlot, &dProbe, &dRG, &dGdt, &dG})
@@ -2372,6 +2690,7 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
         key_add(key, B.kval.p);
         key_add(key, B.slotrec.p);
         if (mixed) key_add(key, op);
+        else if (patch) key_add(key, pop);
         else if (c->cd_lanes > 0) key_add(key, noderows_of(B));
         else key_add(key, runrows_of(B));
         for (int64_t step = 0; step <= p->nsteps; ++step) {
@@ -2425,8 +2744,8 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
     } res[2] = {{Ufin, U_out}, {dV.as<double>(), V_out}};
     for (const auto &r : res) {
         if (!r.out) continue;
-        if (mixed) FS_HIP(c, fs::launch_cd_collect(nv, n, map, r.src, dA.as<double>(), c->stream));
-        if ((s = d2h(c, r.out, mixed ? dA.p : r.src, n * 8))) return s;
+        if (placed) FS_HIP(c, fs::launch_cd_collect(nv, n, map, r.src, dA.as<double>(), c->stream));
+        if ((s = d2h(c, r.out, placed ? dA.p : r.src, n * 8))) return s;
     }
     if (nprobes > 0 && nrec > 1 &&
         (s = d2h(c, probe_out + nprobes, dProbe.as<double>() + nprobes, (size_t)(nrec - 1) * nprobes * 8)))

@@ -2504,6 +2504,220 @@ __global__ __launch_bounds__(CDN_WG) void cd_node_step_kernel(NodeRows nrw, cons
 }
 
 // ---------------------------------------------------------------------------
+// Step on the symmetric patch form of K (PatchOp)
+// ---------------------------------------------------------------------------
+//
+// The step is HBM-bound, and the row forms above read every block of K twice
+// (as K_IJ and as K_JI) and 72 B of state per dof.  Here a workgroup takes a
+// patch of nodes: a lane loads one stored block, and multiplies it with x_J
+// and, where J is in the patch too, its transpose with x_I; the products go
+// to LDS and six lanes per node add them in the order of the node's neighbour
+// list, so the sums are deterministic and the same alone and in a batch.
+// With 42 nodes a patch, a Q4 interior node reads 5.8 of its nine blocks and a
+// T3 node 4.6 of its seven.
+// The state is U and the half-step velocity W_n = V_n + dt/2 A_n, from which
+// U_{n+1} = U_n + dt W_n; no A, and Fmag only at steps with a load: 40 B per
+// dof.  The last step leaves V in W.
+// Layout: the blocks are stored unit by unit over the patch's entries, so a
+// wave loads 1 KB stretches, all 18 of a lane in flight at once; x, the
+// diagonals and the partial products take 27 KB of LDS (Q4), so four
+// workgroups fit a CU, as many as the registers allow.
+// Measured, us per step, node-grouped rows -> patches: 512 x 512 Q4 160 -> 97
+// (315 B per dof, 5.2 TB/s), 1024 x 512 T3 255 -> 152 (5.6 TB/s), 48 T3 plates
+// of 8 to 64 squares 32 -> 22, 97 x 61 Q4 5.7 -> 4.5, 32 x 32 T3 4.3 -> 4.2 (the
+// last two wait on loads, not on bandwidth).  Nodes per patch 21, 32, 42, 53,
+// 64: 105, 98, 96, 99, 97 us on the first mesh, 162, 154, 152, 153, 149 on the
+// second, 22.8, 22.7, 22.0, 25.7, 23.9 on the batch, where large patches leave
+// a half-empty last round of workgroups.
+
+// Positions to dofs: map[q] = dof of position q, or past every free dof.
+__global__ __launch_bounds__(256) void patch_map_kernel(int64_t nv, const int32_t *__restrict__ pnode,
+                                                        const int64_t *__restrict__ node_dof,
+                                                        int64_t *__restrict__ map) {
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= nv) return;
+    const int32_t node = pnode[q / 6];
+    map[q] = node < 0 ? INT64_MAX : node_dof[6 * (int64_t)node + q % 6];
+}
+
+// Place of entry e of patch p in the entry lists.
+__device__ __forceinline__ int64_t patch_entry(const PatchOp &op, const int4 &rec, int p, int e) {
+    return e < PATCH_WG ? (int64_t)p * PATCH_WG + e : op.over + rec.x + e;
+}
+
+// Stored blocks from the CSR values: workgroup per patch, thread per (entry,
+// row) for the blocks and per (slot, row) for the diagonals.
+__global__ __launch_bounds__(256) void patch_build_kernel(PatchOp op, ScatterPlan sp,
+                                                          const double *__restrict__ kval) {
+    const int p = (int)xcd_block(blockIdx.x, gridDim.x);
+    const int4 rec = op.rec[p];
+    const int ne = rec.y, nep = (ne + 7) & ~7;
+    const int32_t *pn = op.pnode + (int64_t)p * PATCH_NODES;
+    double2 *kb = op.k2 + (int64_t)rec.x * 18;
+    for (int i = threadIdx.x; i < 6 * nep; i += 256) {
+        const int r = i / nep, e = i % nep;
+        double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+        if (e < ne) {
+            const int64_t at = patch_entry(op, rec, p, e);
+            const int I = pn[op.ent[at].x >> 26];
+            const int k = op.entk[at];
+            const int J = sp.nbr_node[k], rs = sp.node_rowstart[6 * I + r], off = sp.nbr_off[2 * k];
+            if (rs >= 0 && off >= 0)
+                for (int c = 0; c < 6; ++c) {
+                    const int code = sp.node_code[6 * J + c];
+                    if (code >= 0) v[c] = kval[rs + off + code];
+                }
+        }
+        for (int c2 = 0; c2 < 3; ++c2) kb[(int64_t)(3 * r + c2) * nep + e] = make_double2(v[2 * c2], v[2 * c2 + 1]);
+    }
+    for (int i = threadIdx.x; i < 6 * PATCH_NODES; i += 256) {
+        const int li = i / 6, r = i % 6, I = pn[li];
+        double *dg = op.dg + ((int64_t)p * PATCH_NODES + li) * PATCH_TRI + r * (11 - r) / 2;
+        const int rs = I < 0 ? -1 : sp.node_rowstart[6 * I + r];
+        int off = -1;
+        if (I >= 0)
+            for (int k = sp.nbr_ptr[I]; k < sp.nbr_ptr[I + 1]; ++k)
+                if (sp.nbr_node[k] == I) off = sp.nbr_off[2 * k];
+        for (int c = r; c < 6; ++c) {
+            const int code = I < 0 ? -1 : sp.node_code[6 * I + c];
+            dg[c] = (rs >= 0 && off >= 0 && code >= 0) ? kval[rs + off + code] : 0.0;
+        }
+    }
+}
+
+// W_0 = V_0 + dt/2 A_0 with A_0 = invMC g_0 Fmag (in place of V_0), and
+// U_1 = U_0 + dt W_0.
+__global__ __launch_bounds__(256) void patch_init_kernel(int64_t nv, double dt, double g0,
+                                                         const double *__restrict__ invMC,
+                                                         const double *__restrict__ Fmag,
+                                                         const double *__restrict__ U0, double *__restrict__ W,
+                                                         double *__restrict__ U1, const int32_t *__restrict__ row_group,
+                                                         const double *__restrict__ group_dt,
+                                                         const double *__restrict__ gtab) {
+    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= nv) return;
+    if (row_group) {
+        const int gi = row_group[q];
+        dt = group_dt[gi];
+        g0 = gtab[gi];
+    }
+    const double w = W[q] + (dt / 2) * (invMC[q] * (g0 * Fmag[q]));
+    W[q] = w;
+    U1[q] = U0[q] + dt * w;
+}
+
+__global__ __launch_bounds__(PATCH_WG) __attribute__((amdgpu_waves_per_eu(3))) void cd_patch_step_kernel(
+    PatchOp op, const double *__restrict__ Ucur, double *__restrict__ Unext, double *__restrict__ W,
+    const double *__restrict__ invMC, const double *__restrict__ Cd, const double *__restrict__ Fmag, double gstep,
+    double dt, int damped, int forced, int last, const int32_t *__restrict__ probe_slot,
+    double *__restrict__ probe_dst, const int32_t *__restrict__ row_group, const double *__restrict__ group_dt,
+    const double *__restrict__ gtab) {
+    extern __shared__ double smem[];
+    double *xs = smem;                                   // x of the patch's nodes
+    double *dg = xs + 6 * PATCH_NODES;                   // diagonal blocks
+    double *part = dg + PATCH_TRI * PATCH_NODES;         // partial products
+    const int p = (int)xcd_block(blockIdx.x, gridDim.x);
+    const int tid = threadIdx.x;
+    const int64_t q = (int64_t)p * PATCH_WG + tid;
+    const double u = Ucur[q];
+    uint2 en = op.ent[q];  // the lane's first entry
+    const int4 rec = op.rec[p];
+    const int ne = rec.y, nep = (ne + 7) & ~7;
+    const double2 *kb = op.k2 + (int64_t)rec.x * 18;
+    const double *dgp = op.dg + (int64_t)p * (PATCH_TRI * PATCH_NODES);
+    constexpr int ND = PATCH_TRI * PATCH_NODES;
+    double dv[(ND + PATCH_WG - 1) / PATCH_WG];
+#pragma unroll
+    for (int i = 0; i < (ND + PATCH_WG - 1) / PATCH_WG; ++i)
+        dv[i] = tid + i * PATCH_WG < ND ? dgp[tid + i * PATCH_WG] : 0.0;
+    const int li = tid / 6, r = tid % 6;
+    const uint16_t *np = op.nptr + p * (PATCH_NODES + 1) + li;
+    const int s0 = np[0], s1 = np[1];
+    int e = tid;
+    double2 k2[18];
+    if (e < ne) {
+#pragma unroll
+        for (int v = 0; v < 18; ++v) k2[v] = kb[v * nep + e];
+    }
+    const double w = W[q], im = invMC[q];
+    const int gi = row_group ? row_group[q] : 0;
+    xs[tid] = u;
+#pragma unroll
+    for (int i = 0; i < (ND + PATCH_WG - 1) / PATCH_WG; ++i)
+        if (tid + i * PATCH_WG < ND) dg[tid + i * PATCH_WG] = dv[i];
+    __syncthreads();
+    while (e < ne) {
+        const bool inner = (en.y >> 16) != 0xffffu;
+        const int64_t sj = en.x & 0x3ffffff;
+        double2 xj[3];
+        const double2 *x2 = inner ? reinterpret_cast<const double2 *>(xs + 6 * (int)(sj - (int64_t)p * PATCH_NODES))
+                                  : reinterpret_cast<const double2 *>(Ucur + 6 * sj);
+        if (inner) {
+            for (int c = 0; c < 3; ++c) xj[c] = x2[c];
+        } else {
+            for (int c = 0; c < 3; ++c) xj[c] = x2[c];
+        }
+        double *pi = part + 6 * (en.y & 0xffff);
+#pragma unroll
+        for (int rr = 0; rr < 6; ++rr)
+            pi[rr] = k2[3 * rr].x * xj[0].x + k2[3 * rr].y * xj[0].y + k2[3 * rr + 1].x * xj[1].x +
+                     k2[3 * rr + 1].y * xj[1].y + k2[3 * rr + 2].x * xj[2].x + k2[3 * rr + 2].y * xj[2].y;
+        if (inner) {
+            const double *xi = xs + 6 * (en.x >> 26);
+            double *pj = part + 6 * (en.y >> 16);
+            double2 y[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                y[c].x = k2[c].x * xi[0];
+                y[c].y = k2[c].y * xi[0];
+            }
+#pragma unroll
+            for (int rr = 1; rr < 6; ++rr)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    y[c].x += k2[3 * rr + c].x * xi[rr];
+                    y[c].y += k2[3 * rr + c].y * xi[rr];
+                }
+            for (int c = 0; c < 3; ++c) {
+                pj[2 * c] = y[c].x;
+                pj[2 * c + 1] = y[c].y;
+            }
+        }
+        e += PATCH_WG;
+        if (e < ne) {
+            en = op.ent[op.over + rec.x + e];
+#pragma unroll
+            for (int v = 0; v < 18; ++v) k2[v] = kb[v * nep + e];
+        }
+    }
+    __syncthreads();
+    double f = 0.0;
+    {
+        const double *xi = xs + 6 * li, *di = dg + PATCH_TRI * li;
+#pragma unroll
+        for (int c = 0; c < 6; ++c) {
+            const int a = min(r, c), b = max(r, c);
+            f += di[a * (11 - a) / 2 + b] * xi[c];
+        }
+    }
+    for (int s = s0; s < s1; ++s) f += part[6 * s + r];
+    if (row_group) {  // batch: the row's model has its own dt and load history
+        dt = group_dt[gi];
+        gstep = gtab[gi];
+    }
+    f = forced ? gstep * Fmag[q] - f : -f;
+    if (damped) f -= Cd[q] * w;
+    const double a = im * f;
+    const double wn = w + dt * a;
+    W[q] = last ? w + (dt / 2) * a : wn;
+    Unext[q] = u + dt * wn;
+    if (probe_slot) {
+        const int ps = probe_slot[q];
+        if (ps >= 0) probe_dst[ps] = u;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Mixed-precision explicit step (FP32 membrane + bending, FP64 elsewhere)
 // ---------------------------------------------------------------------------
 //
@@ -3388,6 +3602,45 @@ hipError_t launch_coo_reduce(int64_t nnz, const int64_t *cptr, const int64_t *cl
     if (nnz == 0) return hipSuccess;
     const unsigned blocks = (unsigned)((nnz + 255) / 256);
     hipLaunchKernelGGL(coo_reduce_kernel, dim3(blocks), dim3(256), 0, st, nnz, cptr, clist, mats, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_patch_map(const PatchOp &op, const int64_t *node_dof, int64_t *map, hipStream_t st) {
+    if (op.npatch == 0) return hipSuccess;
+    const int64_t nv = (int64_t)op.npatch * PATCH_WG;
+    hipLaunchKernelGGL(patch_map_kernel, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, st, nv, op.pnode, node_dof,
+                       map);
+    return hipGetLastError();
+}
+
+hipError_t launch_patch_build(const PatchOp &op, const ScatterPlan &sp, const double *kval, hipStream_t st) {
+    if (op.npatch == 0) return hipSuccess;
+    hipLaunchKernelGGL(patch_build_kernel, dim3((unsigned)op.npatch), dim3(256), 0, st, op, sp, kval);
+    return hipGetLastError();
+}
+
+hipError_t launch_patch_init(const PatchOp &op, double dt, double g0, const double *invMC, const double *Fmag,
+                             const double *U0, double *W, double *U1, const int32_t *row_group,
+                             const double *group_dt, const double *gtab, hipStream_t st) {
+    if (op.npatch == 0) return hipSuccess;
+    const int64_t nv = (int64_t)op.npatch * PATCH_WG;
+    hipLaunchKernelGGL(patch_init_kernel, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, st, nv, dt, g0, invMC, Fmag,
+                       U0, W, U1, row_group, group_dt, gtab);
+    return hipGetLastError();
+}
+
+size_t patch_smem(int slots) {
+    return sizeof(double) * (size_t)(6 * PATCH_NODES + PATCH_TRI * PATCH_NODES + 6 * slots);
+}
+
+hipError_t launch_cd_patch_step(const PatchOp &op, const double *Ucur, double *Unext, double *W, const double *invMC,
+                                const double *Cd, const double *Fmag, double gstep, double dt, int damped, int forced,
+                                int last, const int32_t *probe_slot, double *probe_dst,
+                                const int32_t *row_group, const double *group_dt, const double *gtab, hipStream_t st) {
+    if (op.npatch == 0) return hipSuccess;
+    hipLaunchKernelGGL(cd_patch_step_kernel, dim3((unsigned)op.npatch), dim3(PATCH_WG), patch_smem(op.slots), st, op,
+                       Ucur, Unext, W, invMC, Cd, Fmag, gstep, dt, damped, forced, last, probe_slot, probe_dst, row_group,
+                       group_dt, gtab);
     return hipGetLastError();
 }
 

@@ -42,7 +42,8 @@ def footprint_bytes(nen, nelem, nnodes, nrows, kind):
     blocks = nelem * nblk * (36 * 8 + 4)
     csr = nnz * 12 + nrows * 16
     vec = nrows * 8 * (11 if kind == EXPLICIT else 1)
-    return int(1.25 * (mesh + blocks + csr + vec)) + (4 << 20)
+    patch = nnz * 6 if kind == EXPLICIT else 0  # 0.67 of the values, entry tables
+    return int(1.25 * (mesh + blocks + csr + vec + patch)) + (4 << 20)
 
 
 class Request:

@@ -454,7 +454,9 @@ int fs_ctx_set_assembly(fs_ctx *ctx, int mode);
  * 16 lanes: 2..4; 0 = chosen from the block's longest row).  All forms give
  * the same sums up to their order of addition; every setting is bitwise
  * reproducible and gives a model bitwise the same result alone and in a
- * batch.  Default 8 lanes per node, positions chosen. */
+ * batch.  Default 8 lanes per node, positions chosen; with that setting,
+ * explicit loops of 100 steps or more run on a symmetric copy of K cut into
+ * node patches (each block read once per patch), which the model keeps. */
 int fs_ctx_set_cd_lanes(fs_ctx *ctx, int lanes_per_node, int positions_per_lane);
 
 /* Storage of the mixed-precision operator built by the last FS_PREC_MIXED /

@@ -1,0 +1,111 @@
+"""The explicit step on the patch form of K (the default of loops of 100
+steps or more) against the row products and the oracle.
+
+Both forms add the same products in different orders: 1e-12 relative between
+them over 120 steps at 0.8 of the stable dt (the bound of the row forms among
+themselves), 1e-10 against the oracle's loop.  Meshes at the edges of the
+plan: one node with free dofs, one and two patches (42 and 43 nodes), a hub
+whose patch has more blocks than the workgroup has lanes, a hub of more
+neighbours than a patch takes (row products throughout), two components,
+partly fixed nodes, a permuted numbering."""
+import numpy as np
+import pytest
+
+from flexshell import _lib, explicit, fe, femm as FM
+from flexshell.material import MatDeforElastIso
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _grid(nen, nx, ny, clamp="left", perm=False):
+    xy, conn = (fe.T3block if nen == 3 else fe.Q4block)(0.1 * nx, 0.1 * ny, nx, ny)
+    xyz = fe.xyz3(xy)
+    xyz[:, 2] = 0.05 * np.sin(2.0 * xyz[:, 0])
+    d = fe.DofField(xyz.shape[0])
+    left = xy[:, 0] < 1e-9
+    if clamp == "left":
+        d.setebc(np.nonzero(left)[0], [1, 2, 3, 4, 5, 6])
+    elif clamp == "partial":
+        d.setebc(np.nonzero(left)[0], [1, 2, 3])
+        d.setebc(np.nonzero(xy[:, 1] < 1e-9)[0], [3, 5])
+    else:
+        d.setebc(np.arange(1, xyz.shape[0]), [1, 2, 3, 4, 5, 6])
+    d.numberdofs(perm=np.random.default_rng(5).permutation(xyz.shape[0]) if perm else None)
+    return nen, xyz, conn, d
+
+
+def _fan(m):
+    a = 2 * np.pi * np.arange(m) / m
+    xyz = np.vstack([[0.0, 0.0, 0.0], np.column_stack([np.cos(a), np.sin(a), 0 * a])])
+    conn = np.column_stack([np.zeros(m, dtype=np.int64), 1 + np.arange(m), 1 + (np.arange(m) + 1) % m])
+    d = fe.DofField(m + 1)
+    d.setebc([1, 2, 3], [1, 2, 3, 4, 5, 6])
+    d.numberdofs()
+    return 3, xyz, conn, d
+
+
+def _two():
+    _, x1, c1, _ = _grid(4, 7, 6)
+    _, x2, c2, _ = _grid(4, 3, 11)
+    xyz = np.vstack([x1, x2 + [5.0, 0.0, 0.0]])
+    conn = np.vstack([c1, c2 + len(x1)])
+    d = fe.DofField(len(xyz))
+    d.setebc([0, 1, 2, len(x1), len(x1) + 1], [1, 2, 3, 4, 5, 6])
+    d.numberdofs()
+    return 4, xyz, conn, d
+
+
+MESHES = {
+    "one_node": lambda: _grid(4, 3, 3, "all_but_one"),
+    "q4_42": lambda: _grid(4, 6, 6),               # 42 of 49 nodes have free dofs
+    "q4_43": lambda: _grid(4, 1, 42),
+    "t3_43": lambda: _grid(3, 1, 42),
+    "t3_perm": lambda: _grid(3, 17, 13, perm=True),
+    "q4_partial": lambda: _grid(4, 23, 9, "partial"),
+    "hub_300": lambda: _fan(300),
+    "hub_1100": lambda: _fan(1100),
+    "two": _two,
+}
+
+
+@pytest.mark.parametrize("name", list(MESHES))
+@pytest.mark.parametrize("cdamp", [0.0, 50.0], ids=["undamped", "damped"])
+def test_patch_step(ctx, name, cdamp):
+    print(f"[gpu] patch step {name} {cdamp}", flush=True)
+    nen, xyz, conn, d = MESHES[name]()
+    f = FM.make(conn, MatDeforElastIso(70e9, 0.33, 2700.0), thickness=0.02, ctx=ctx)
+    f.associategeometry(xyz)
+    nf = d.nfreedofs
+    K = f.stiffness(FM.SysmatAssemblerFFBlock(nf), xyz, None, None, d)
+    M = f.mass(FM.SysmatAssemblerFFBlock(FM.SysmatAssemblerSparseDiag(), nf, nf), xyz, d).diagonal()
+    rng = np.random.default_rng(7)
+    U0, V0, F = rng.normal(0, 1e-6, nf), rng.normal(0, 1e-3, nf), rng.normal(0, 1.0, nf)
+    dt = 0.8 * explicit.stable_dt(O.pwr(K, M, rng.standard_normal(nf), 200))
+    nsteps = 120
+    g = np.where(np.arange(nsteps + 1) < 40, np.cos(0.1 * np.arange(nsteps + 1)), 0.0)
+    probes = np.array([nf - 1, 0, nf // 2])
+    Uo, Vo, po = O.cd_loop(K, M, cdamp, dt, nsteps, F, g, U0, V0, probes)
+    r = explicit.run(f._model, cdamp, U0, V0, dt, nsteps, F, g, probes, 7)
+    again = explicit.run(f._model, cdamp, U0, V0, dt, nsteps, F, g, probes, 7, use_graph=True)
+    try:
+        ctx.set_cd_lanes(0)
+        rows = explicit.run(f._model, cdamp, U0, V0, dt, nsteps, F, g, probes, 7)
+    finally:
+        ctx.set_cd_lanes(8)
+    for key, ref in (("U", Uo), ("V", Vo)):
+        assert np.array_equal(r[key], again[key])
+        assert np.linalg.norm(r[key] - rows[key]) <= 1e-12 * np.linalg.norm(rows[key]), key
+        assert np.linalg.norm(r[key] - ref) <= 1e-10 * np.linalg.norm(ref), key
+    assert np.linalg.norm(r["probes"] - po[::7]) <= 1e-10 * np.linalg.norm(po)
+    # new values behind the same plan
+    f.thickness = 0.03
+    f.stiffness(FM.SysmatAssemblerHIP(_lib.FS_BLOCK_FF), xyz, None, None, d)
+    a = explicit.run(f._model, cdamp, U0, V0, 0.5 * dt, nsteps, F, g)
+    try:
+        ctx.set_cd_lanes(0)
+        b = explicit.run(f._model, cdamp, U0, V0, 0.5 * dt, nsteps, F, g)
+    finally:
+        ctx.set_cd_lanes(8)
+    assert np.linalg.norm(a["U"] - b["U"]) <= 1e-12 * np.linalg.norm(b["U"])
+    f._model.close()
