@@ -98,10 +98,13 @@ hipError_t launch_cd_patch_step(const PatchOp &op, const double *Ucur, double *U
                                 const double *Cd, const double *Fmag, double gstep, double dt, int damped, int forced,
                                 int last, const int32_t *probe_slot, double *probe_dst,
                                 const int32_t *row_group, const double *group_dt, const double *gtab, hipStream_t st);
-hipError_t launch_dot(int64_t n, int mode, const double *x, const double *y, const double *d, double *part,
-                      double *out, hipStream_t st);
-hipError_t launch_scale(int64_t n, const double *ss, const double *d, const double *x, double *y, hipStream_t st);
-hipError_t launch_pwr_init(int64_t n, const double *mdiag, double *inv, double *ss, hipStream_t st);
+hipError_t launch_dot(int64_t n, const double *x, const double *y, const double *d, double *part, double *out,
+                      hipStream_t st);
+hipError_t launch_pwr(const RunRows &rows, const double *kval, const double *x, double *y, const double *mdiag,
+                      const double *scale, double *part, double *ss, hipStream_t st);
+hipError_t launch_pwr_node(int nl, int pj, const NodeRows &nrw, const int2 *slotrec, const double *kval,
+                           const double *x, double *y, const double *mdiag, const double *scale, double *part,
+                           double *ss, hipStream_t st);
 hipError_t noalloc_workspace(int device, double **out);
 hipError_t launch_mixed_build(const ScatterPlan &sp, const double *Kb, const int64_t *goff, float2 *kmb, short2 *kml,
                               hipStream_t st);
@@ -2757,34 +2760,34 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
 
 namespace {
 // Power iteration of pwr (clamp_cyl_transient_examples.jl:45-60) on the
-// resident FF-block K and M, from v (device, overwritten): w, inv (n each),
-// part (512) and ss (4) are device work arrays.
-int power_iteration(fs_model *m, double *v, double *w, double *inv, double *part, double *ss, int32_t maxit,
+// resident FF-block K and M, from v (device, overwritten): w (n), sums (n +
+// 64: the waves' partial norms), part (512) and ss (4) are device work arrays.
+// The vectors are taken in turn as an iteration's start and end; the last one
+// keeps its length, which the quotient does not see.
+int power_iteration(fs_model *m, double *v, double *w, double *sums, double *part, double *ss, int32_t maxit,
                     double *omega_max) {
     fs_ctx *c = m->ctx;
     Block &B = m->blk[FS_BLOCK_FF];
     const int64_t n = B.nrows;
     const fs::RunRows rows = runrows_of(B);
     const fs::NodeRows nrw = noderows_of(B);
-    const double *kv = B.kval.as<double>();
+    const double *kv = B.kval.as<double>(), *md = B.mdiag.as<double>();
     const int pj = node_pj(c, B);
-    // w = K v in the step's form (node-grouped unless the row form is set)
-    auto spmv = [&]() {
-        return c->cd_lanes > 0 ? fs::launch_spmv_node(c->cd_lanes, pj, nrw, B.slotrec.as<int2>(), kv, v, w, c->stream)
-                               : fs::launch_spmv(rows, kv, v, w, c->stream);
-    };
-    FS_HIP(c, fs::launch_pwr_init(n, B.mdiag.as<double>(), inv, ss, c->stream));  // invM, scale factors 1
+    // the step's form of the product (node-grouped unless the row form is set)
     for (int it = 0; it < maxit; ++it) {
-        FS_HIP(c, spmv());                                                            // w = K v
-        FS_HIP(c, fs::launch_dot(n, 0, w, nullptr, nullptr, part, ss, c->stream));
-        FS_HIP(c, fs::launch_scale(n, ss, nullptr, w, w, c->stream));                 // w /= |w|
-        FS_HIP(c, fs::launch_scale(n, ss + 3, inv, w, v, c->stream));                 // v = invM .* w
-        FS_HIP(c, fs::launch_dot(n, 0, v, nullptr, nullptr, part, ss + 1, c->stream));
-        FS_HIP(c, fs::launch_scale(n, ss + 1, nullptr, v, v, c->stream));             // v /= |v|
+        // the length is taken after even iterations, divided out in odd ones
+        const double *scale = it % 2 ? ss : nullptr;
+        double *norms = it % 2 ? nullptr : sums;
+        FS_HIP(c, c->cd_lanes > 0 ? fs::launch_pwr_node(c->cd_lanes, pj, nrw, B.slotrec.as<int2>(), kv, v, w, md, scale,
+                                                        norms, ss, c->stream)
+                                  : fs::launch_pwr(rows, kv, v, w, md, scale, norms, ss, c->stream));
+        std::swap(v, w);
     }
-    FS_HIP(c, spmv());
-    FS_HIP(c, fs::launch_dot(n, 1, w, v, nullptr, part, ss, c->stream));
-    FS_HIP(c, fs::launch_dot(n, 2, v, nullptr, B.mdiag.as<double>(), part, ss + 1, c->stream));
+    FS_HIP(c, c->cd_lanes > 0
+                  ? fs::launch_spmv_node(c->cd_lanes, pj, nrw, B.slotrec.as<int2>(), kv, v, w, c->stream)
+                  : fs::launch_spmv(rows, kv, v, w, c->stream));
+    FS_HIP(c, fs::launch_dot(n, w, v, nullptr, part, ss, c->stream));
+    FS_HIP(c, fs::launch_dot(n, v, nullptr, md, part, ss + 1, c->stream));
     double h[2];
     FS_HIP(c, hipMemcpyAsync(h, ss, 16, hipMemcpyDeviceToHost, c->stream));
     FS_HIP(c, hipStreamSynchronize(c->stream));
@@ -2803,12 +2806,12 @@ int fs_model_omega_max(fs_model *m, const double *v0, int32_t maxit, double *ome
     if (!B.k_ready || !B.m_ready) return fail(c, FS_ERR_STATE, "omega_max: FF-block K and M must be computed first");
     FS_HIP(c, hipSetDevice(c->device));
     const int64_t n = B.nrows;
-    DevBuf dv, dw, dinv, dpart, dss;
+    DevBuf dv, dw, dsums, dpart, dss;
     int s;
-    if ((s = upload(c, dv, v0, n)) || (s = dalloc(c, dw, n * 8)) || (s = dalloc(c, dinv, n * 8)) ||
+    if ((s = upload(c, dv, v0, n)) || (s = dalloc(c, dw, n * 8)) || (s = dalloc(c, dsums, (n + 64) * 8)) ||
         (s = dalloc(c, dpart, 512 * 8)) || (s = dalloc(c, dss, 4 * 8)))
         return s;
-    return power_iteration(m, dv.as<double>(), dw.as<double>(), dinv.as<double>(), dpart.as<double>(),
+    return power_iteration(m, dv.as<double>(), dw.as<double>(), dsums.as<double>(), dpart.as<double>(),
                            dss.as<double>(), maxit, omega_max);
 }
 
@@ -2827,10 +2830,10 @@ int fs_model_omega_max_noalloc(fs_model *m, const double *v0, int32_t maxit, dou
         return fail(c, FS_ERR_DEVICE, "omega_max without allocation: no workspace on device %d (%s)", c->device,
                     hipGetErrorString(c->scratch_status));
     FS_HIP(c, hipSetDevice(c->device));
-    double *v = c->scratch, *w = v + fs::NOALLOC_MAX_ROWS, *inv = w + fs::NOALLOC_MAX_ROWS;
-    double *part = inv + fs::NOALLOC_MAX_ROWS, *ss = part + 512;
+    double *v = c->scratch, *w = v + fs::NOALLOC_MAX_ROWS, *sums = w + fs::NOALLOC_MAX_ROWS;
+    double *part = sums + fs::NOALLOC_MAX_ROWS, *ss = part + 512;
     if (n) FS_HIP(c, hipMemcpyAsync(v, v0, (size_t)n * 8, hipMemcpyHostToDevice, c->stream));
-    return power_iteration(m, v, w, inv, part, ss, maxit, omega_max);
+    return power_iteration(m, v, w, sums, part, ss, maxit, omega_max);
 }
 
 int fs_ctx_tuning(const fs_ctx *ctx, int nen, int formulation, int32_t *shape) {

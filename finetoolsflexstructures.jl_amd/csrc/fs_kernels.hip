@@ -2976,25 +2976,56 @@ __global__ void gather_kernel(int n, const int64_t *__restrict__ idx, const doub
     if (k < n) out[k] = U[idx[k]];
 }
 
-// y = K x (power iteration)
-template <int TPR>
+// Products of the power iteration.  PWR false: y = K x.  PWR true, one
+// iteration of pwr: y = invM .* (K x), with ss given divided by sqrt(ss[0]),
+// and with part given, part[g] = the sum of y^2 over the rows of wave g, which
+// pwr_norm_kernel adds into ss[0].  The quotient at the end does not see the
+// length of the vector, so of the reference's two scalings per iteration one
+// in two iterations is left: the length is taken after the first, third, ...
+// iteration and divided out by the next, so a vector grows by two iterations
+// at most (the fourth power of omega_max) before its squares are summed.
+// 300 x 211 layered T3 mesh, 100 iterations: 4.5 -> 2.5 ms of kernels (the
+// product 22 us), against a product, two norms and three scalings in eight
+// launches an iteration; with the length taken every time 2.7 ms.
+template <bool PWR>
+__device__ __forceinline__ double pwr_row(double e, int64_t row, const double *__restrict__ ss,
+                                          const double *__restrict__ mdiag, double *__restrict__ y) {
+    if constexpr (PWR) e = (ss ? e * (1.0 / sqrt(ss[0])) : e) / mdiag[row];
+    y[row] = e;
+    return e * e;
+}
+
+template <bool PWR>
+__device__ __forceinline__ void pwr_wave(double sq, double *__restrict__ part) {
+    if (PWR && part) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) sq += __shfl_xor(sq, off, 64);
+        if ((threadIdx.x & 63) == 0) part[(blockIdx.x * blockDim.x + threadIdx.x) >> 6] = sq;
+    }
+}
+
+template <int TPR, bool PWR>
 __global__ __launch_bounds__(256) void spmv_kernel(RunRows rows, const double *__restrict__ kval,
-                                                   const double *__restrict__ x, double *__restrict__ y) {
+                                                   const double *__restrict__ x, double *__restrict__ y,
+                                                   const double *__restrict__ ss, const double *__restrict__ mdiag,
+                                                   double *__restrict__ part) {
     const int64_t gt = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     const int64_t row = gt / TPR;
     const int lane = (int)(gt % TPR);
-    double e = 0.0;
+    double e = 0.0, sq = 0.0;
     if (row < rows.n) e = run_row_dot<TPR>(rows.rowrec[row], lane, rows.slotrec, kval, x);
 #pragma unroll
     for (int off = TPR / 2; off > 0; off >>= 1) e += __shfl_xor(e, off, TPR);
-    if (row < rows.n && lane == 0) y[row] = e;
+    if (row < rows.n && lane == 0) sq = pwr_row<PWR>(e, row, ss, mdiag, y);
+    pwr_wave<PWR>(sq, part);
 }
 
-// y = K x in the node-grouped form of cd_node_step_kernel (same row sums).
-template <int NL, int PJ>
+// The same in the node-grouped form of cd_node_step_kernel (same row sums).
+template <int NL, int PJ, bool PWR>
 __global__ __launch_bounds__(CDN_WG) void spmv_node_kernel(NodeRows nrw, const int2 *__restrict__ slotrec,
                                                         const double *__restrict__ kval, const double *__restrict__ x,
-                                                        double *__restrict__ y) {
+                                                        double *__restrict__ y, const double *__restrict__ ss,
+                                                        const double *__restrict__ mdiag, double *__restrict__ part) {
     const int64_t gt = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     const int64_t node = gt / NL;
     const int lane = (int)(gt % NL);
@@ -3012,26 +3043,46 @@ __global__ __launch_bounds__(CDN_WG) void spmv_node_kernel(NodeRows nrw, const i
     for (int off = NL / 2; off > 0; off >>= 1)
 #pragma unroll
         for (int r = 0; r < 6; ++r) acc[r] += __shfl_xor(acc[r], off, NL);
+    double sq = 0.0;
     if (active && lane < nr) {
         double e = acc[0];
 #pragma unroll
         for (int r = 1; r < 6; ++r)
             if (lane == r) e = acc[r];
-        y[(int64_t)d0 + lane] = e;
+        sq = pwr_row<PWR>(e, (int64_t)d0 + lane, ss, mdiag, y);
+    }
+    pwr_wave<PWR>(sq, part);
+}
+
+// ss[0] = sum of the n wave sums, in a fixed order.
+__global__ __launch_bounds__(1024) void pwr_norm_kernel(int64_t n, const double *__restrict__ part,
+                                                        double *__restrict__ ss) {
+    __shared__ double sh[16];
+    double s = 0.0;
+#pragma unroll 8
+    for (int64_t i = threadIdx.x; i < n; i += 1024) s += part[i];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        s = sh[0];
+        for (int i = 1; i < 16; ++i) s += sh[i];
+        ss[0] = s;
     }
 }
 
-// Deterministic reductions for the power iteration: fixed tree per block,
-// then one block sums the block partials in index order.
-// mode 0: sum x*x; mode 1: sum x*y; mode 2: sum x*(d*x)
-__global__ __launch_bounds__(256) void dot_partial_kernel(int64_t n, int mode, const double *__restrict__ x,
+// Dot products at the end of the power iteration: fixed tree per block, then
+// one block sums the block partials in index order.  d null: sum x*y; else
+// sum x*(d*x).
+__global__ __launch_bounds__(256) void dot_partial_kernel(int64_t n, const double *__restrict__ x,
                                                           const double *__restrict__ y,
                                                           const double *__restrict__ d, double *__restrict__ part) {
     __shared__ double sh[256];
     double s = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
         const double xv = x[i];
-        s += mode == 0 ? xv * xv : (mode == 1 ? xv * y[i] : xv * (d[i] * xv));
+        s += d ? xv * (d[i] * xv) : xv * y[i];
     }
     sh[threadIdx.x] = s;
     __syncthreads();
@@ -3054,26 +3105,6 @@ __global__ __launch_bounds__(256) void dot_final_kernel(int nb, const double *__
         __syncthreads();
     }
     if (threadIdx.x == 0) out[0] = sh[0];
-}
-
-// Start of the power iteration: inv[i] = 1 / mdiag[i] (the invM of pwr,
-// clamp_cyl_transient_examples.jl:47) and the four scale factors set to one
-// (a fill kernel rather than a memset, so that the sequence can be captured).
-__global__ __launch_bounds__(256) void pwr_init_kernel(int64_t n, const double *__restrict__ mdiag,
-                                                       double *__restrict__ inv, double *__restrict__ ss) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < 4) ss[i] = 1.0;
-    if (i < n) inv[i] = 1.0 / mdiag[i];
-}
-
-// y = (d ? d : 1) * x / sqrt(ss[0])  (normalisation steps of pwr)
-__global__ __launch_bounds__(256) void scale_kernel(int64_t n, const double *__restrict__ ss,
-                                                    const double *__restrict__ d, const double *__restrict__ x,
-                                                    double *__restrict__ y) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double f = 1.0 / sqrt(ss[0]);
-    y[i] = d ? d[i] * (x[i] * f) : x[i] * f;
 }
 
 // ---------------------------------------------------------------------------
@@ -3495,20 +3526,40 @@ hipError_t launch_gather(int n, const int64_t *idx, const double *U, double *out
     return hipGetLastError();
 }
 
+// Waves of one product (the partial sums pwr_norm_kernel adds).
+static int64_t spmv_row_blocks(const RunRows &rows) { return (rows.n * 4 + 255) / 256; }
+static int64_t spmv_node_blocks(int nl, const NodeRows &nrw) { return (nrw.n * nl + CDN_WG - 1) / CDN_WG; }
+
 hipError_t launch_spmv(const RunRows &rows, const double *kval, const double *x, double *y, hipStream_t st) {
     if (rows.n == 0) return hipSuccess;
-    const int64_t threads = rows.n * 4;
-    hipLaunchKernelGGL(spmv_kernel<4>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, rows, kval, x, y);
+    hipLaunchKernelGGL((spmv_kernel<4, false>), dim3((unsigned)spmv_row_blocks(rows)), dim3(256), 0, st, rows, kval, x, y,
+                       nullptr, nullptr, nullptr);
     return hipGetLastError();
 }
 
-hipError_t launch_spmv_node(int nl, int pj, const NodeRows &nrw, const int2 *slotrec, const double *kval,
-                            const double *x, double *y, hipStream_t st) {
-    if (nrw.n == 0) return hipSuccess;
-    const unsigned blocks = (unsigned)((nrw.n * nl + CDN_WG - 1) / CDN_WG);
+static hipError_t launch_norm(int64_t n, const double *part, double *ss, hipStream_t st) {
+    hipLaunchKernelGGL(pwr_norm_kernel, dim3(1), dim3(1024), 0, st, n, part, ss);
+    return hipGetLastError();
+}
+
+hipError_t launch_pwr(const RunRows &rows, const double *kval, const double *x, double *y, const double *mdiag,
+                      const double *scale, double *part, double *ss, hipStream_t st) {
+    if (rows.n == 0) return hipSuccess;
+    const int64_t blocks = spmv_row_blocks(rows);
+    hipLaunchKernelGGL((spmv_kernel<4, true>), dim3((unsigned)blocks), dim3(256), 0, st, rows, kval, x, y, scale,
+                       mdiag, part);
+    return part ? launch_norm(blocks * 4, part, ss, st) : hipGetLastError();
+}
+
+template <bool PWR>
+static hipError_t launch_node_product(int nl, int pj, const NodeRows &nrw, const int2 *slotrec, const double *kval,
+                                      const double *x, double *y, const double *ss, const double *mdiag, double *part,
+                                      hipStream_t st) {
+    const unsigned blocks = (unsigned)spmv_node_blocks(nl, nrw);
 #define FS_SPN_CASE(T, P)                                                                                         \
     if (nl == T && pj == P) {                                                                                     \
-        hipLaunchKernelGGL((spmv_node_kernel<T, P>), dim3(blocks), dim3(CDN_WG), 0, st, nrw, slotrec, kval, x, y);   \
+        hipLaunchKernelGGL((spmv_node_kernel<T, P, PWR>), dim3(blocks), dim3(CDN_WG), 0, st, nrw, slotrec, kval, x, y, \
+                           ss, mdiag, part);                                                                      \
         return hipGetLastError();                                                                                 \
     }
     FS_SPN_CASE(8, 4)
@@ -3523,18 +3574,26 @@ hipError_t launch_spmv_node(int nl, int pj, const NodeRows &nrw, const int2 *slo
     return hipErrorInvalidValue;
 }
 
-static constexpr int kDotBlocks = 512;
-
-hipError_t launch_dot(int64_t n, int mode, const double *x, const double *y, const double *d, double *part,
-                      double *out, hipStream_t st) {
-    hipLaunchKernelGGL(dot_partial_kernel, dim3(kDotBlocks), dim3(256), 0, st, n, mode, x, y, d, part);
-    hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(256), 0, st, kDotBlocks, part, out);
-    return hipGetLastError();
+hipError_t launch_spmv_node(int nl, int pj, const NodeRows &nrw, const int2 *slotrec, const double *kval,
+                            const double *x, double *y, hipStream_t st) {
+    if (nrw.n == 0) return hipSuccess;
+    return launch_node_product<false>(nl, pj, nrw, slotrec, kval, x, y, nullptr, nullptr, nullptr, st);
 }
 
-hipError_t launch_pwr_init(int64_t n, const double *mdiag, double *inv, double *ss, hipStream_t st) {
-    const int64_t m = n > 4 ? n : 4;
-    hipLaunchKernelGGL(pwr_init_kernel, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, st, n, mdiag, inv, ss);
+hipError_t launch_pwr_node(int nl, int pj, const NodeRows &nrw, const int2 *slotrec, const double *kval,
+                           const double *x, double *y, const double *mdiag, const double *scale, double *part,
+                           double *ss, hipStream_t st) {
+    if (nrw.n == 0) return hipSuccess;
+    const hipError_t e = launch_node_product<true>(nl, pj, nrw, slotrec, kval, x, y, scale, mdiag, part, st);
+    return e != hipSuccess || !part ? e : launch_norm(spmv_node_blocks(nl, nrw), part, ss, st);
+}
+
+static constexpr int kDotBlocks = 512;
+
+hipError_t launch_dot(int64_t n, const double *x, const double *y, const double *d, double *part,
+                      double *out, hipStream_t st) {
+    hipLaunchKernelGGL(dot_partial_kernel, dim3(kDotBlocks), dim3(256), 0, st, n, x, y, d, part);
+    hipLaunchKernelGGL(dot_final_kernel, dim3(1), dim3(256), 0, st, kDotBlocks, part, out);
     return hipGetLastError();
 }
 
@@ -3569,12 +3628,6 @@ hipError_t noalloc_workspace(int device, double **out) {
     }
     *out = g_scratch_ptr[device];
     return hipSuccess;
-}
-
-hipError_t launch_scale(int64_t n, const double *ss, const double *d, const double *x, double *y, hipStream_t st) {
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(scale_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, n, ss, d, x, y);
-    return hipGetLastError();
 }
 
 hipError_t launch_mixed_build(const ScatterPlan &sp, const double *Kb, const int64_t *goff, float2 *kmb,
