@@ -231,6 +231,8 @@ struct NodeRows {
 //   k2        blocks of patch p from 18 first block on, two values a unit: unit
 //             v of entry e (rows in order, three units a row) at v nep + e,
 //             nep = entries rounded up to 8
+//   kh, kl    in k2's place for FS_PREC_MIXED_F32: the values as FP32 and int16
+//             residual (MixedOp), four a unit: unit v of entry e at v nep + e
 //   dg        diagonal blocks, 21 upper values (row by row) per slot
 constexpr int PATCH_NODES = 42;
 constexpr int PATCH_WG = 6 * PATCH_NODES;  // lanes of a patch: a dof each, or an entry each
@@ -245,6 +247,8 @@ struct PatchOp {
     const int32_t *pnode;
     const uint16_t *nptr;
     double2 *k2;
+    float4 *kh;
+    short4 *kl;
     double *dg;
 };
 

@@ -89,12 +89,13 @@ hipError_t launch_cd_node_step(int nl, int pj, const NodeRows &nrw, const int2 *
                                const int32_t *probe_slot, double *probe_dst, const int32_t *row_group,
                                const double *group_dt, const double *gtab, hipStream_t st);
 hipError_t launch_patch_map(const PatchOp &op, const int64_t *node_dof, int64_t *map, hipStream_t st);
-hipError_t launch_patch_build(const PatchOp &op, const ScatterPlan &sp, const double *kval, hipStream_t st);
+hipError_t launch_patch_build(const PatchOp &op, int kind, const ScatterPlan &sp, const double *kval,
+                              const MixedOp &mixed, const int32_t *conn, int nen, int nsr, hipStream_t st);
 hipError_t launch_patch_init(const PatchOp &op, double dt, double g0, const double *invMC, const double *Fmag,
                              const double *U0, double *W, double *U1, const int32_t *row_group,
                              const double *group_dt, const double *gtab, hipStream_t st);
 size_t patch_smem(int slots);
-hipError_t launch_cd_patch_step(const PatchOp &op, const double *Ucur, double *Unext, double *W, const double *invMC,
+hipError_t launch_cd_patch_step(const PatchOp &op, int f32, const double *Ucur, double *Unext, double *W, const double *invMC,
                                 const double *Cd, const double *Fmag, double gstep, double dt, int damped, int forced,
                                 int last, const int32_t *probe_slot, double *probe_dst,
                                 const int32_t *row_group, const double *group_dt, const double *gtab, hipStream_t st);
@@ -233,16 +234,19 @@ struct PatchStore {
     bool planned = false, usable = false;
     int64_t npatch = 0, nent = 0;
     int slots = 0;
-    uint64_t vgen = 0;  // generation of the values it was filled from
+    // what it is filled with (FS_PREC_*, -1 nothing) and the generations of the
+    // values (Block::vgen, MixedStore::kgen) that came from
+    int kind = -1;
+    uint64_t vgen = 0, kgen = 0;
     std::vector<int32_t> pnode;  // host copy: the node of each slot
-    DevBuf rec, ent, entk, dpnode, nptr, map, k2, dg;
+    DevBuf rec, ent, entk, dpnode, nptr, map, k2, kh, kl, dg;
     void reset() {
         planned = usable = false;
         npatch = nent = 0;
         slots = 0;
-        vgen = 0;
+        kind = -1;
         pnode.clear();
-        for (DevBuf *b : {&rec, &ent, &entk, &dpnode, &nptr, &map, &k2, &dg}) b->release();
+        for (DevBuf *b : {&rec, &ent, &entk, &dpnode, &nptr, &map, &k2, &kh, &kl, &dg}) b->release();
     }
 };
 
@@ -938,6 +942,8 @@ fs::PatchOp patchop_of(const PatchStore &P) {
     op.pnode = P.dpnode.as<int32_t>();
     op.nptr = P.nptr.as<uint16_t>();
     op.k2 = P.k2.as<double2>();
+    op.kh = P.kh.as<float4>();
+    op.kl = P.kl.as<short4>();
     op.dg = P.dg.as<double>();
     return op;
 }
@@ -1148,7 +1154,7 @@ int build_patches(fs_model *m) {
     if ((s = upload(c, P.rec, rec.data(), rec.size())) || (s = upload(c, P.ent, ent.data(), ent.size())) ||
         (s = upload(c, P.entk, entk.data(), entk.size())) || (s = upload(c, P.dpnode, P.pnode.data(), P.pnode.size())) ||
         (s = upload(c, P.nptr, nptr.data(), nptr.size())) || (s = dalloc(c, P.map, (size_t)np * PN * 6 * 8)) ||
-        (s = dalloc(c, P.k2, (size_t)nent * 288)) || (s = dalloc(c, P.dg, (size_t)np * PN * fs::PATCH_TRI * 8)))
+        (s = dalloc(c, P.dg, (size_t)np * PN * fs::PATCH_TRI * 8)))
         return s;
     P.npatch = np;
     P.nent = nent;
@@ -1165,32 +1171,6 @@ int build_patches(fs_model *m) {
 // ms on the 1024 x 512 T3 plate, 16 host threads), and a step then saves 0.2 ns
 // per node (63 and 103 us): from 100 steps on the second loop has paid for it.
 constexpr int64_t PATCH_MIN_STEPS = 100;
-
-// The patch form with the resident values of K: its plan, if there is none
-// yet, and its blocks, if K was computed again since.  *use becomes false
-// where the form does not take the mesh, or there is no memory for it.
-int prepare_patches(fs_model *m, bool *use) {
-    fs_ctx *c = m->ctx;
-    Block &B = m->blk[FS_BLOCK_FF];
-    PatchStore &P = B.patch;
-    if (!P.planned) {
-        const int s = build_patches(m);
-        if (s == FS_ERR_NOMEM) {
-            P.reset();
-            P.planned = true;  // not tried again for this block
-            c->err.clear();
-        } else if (s) {
-            P.reset();
-            return s;
-        }
-    }
-    *use = P.usable;
-    if (P.usable && P.vgen != B.vgen) {
-        FS_HIP(c, fs::launch_patch_build(patchop_of(P), plan_of(B), B.kval.as<double>(), c->stream));
-        P.vgen = B.vgen;
-    }
-    return FS_OK;
-}
 
 // 3 x 21-bit Morton code of a point scaled into [0, 1)^3.
 uint64_t morton3(double x, double y, double z) {
@@ -1764,6 +1744,42 @@ fs::MixedOp mixed_op(const fs_model *m) {
     op.ne_pack = m->mixed.ne_pack.as<int32_t>();
     op.cs = m->mixed.cs.as<double>();
     return op;
+}
+
+// The patch form of a precision's operator (the mixed ones built already): its
+// plan, if there is none yet, and its blocks, if they are of another precision
+// or other values.  *use becomes false where the form does not take the mesh,
+// or there is no memory for it.
+int prepare_patches(fs_model *m, int precision, bool *use) {
+    fs_ctx *c = m->ctx;
+    Block &B = m->blk[FS_BLOCK_FF];
+    PatchStore &P = B.patch;
+    auto without = [&](int s) {  // no memory: the other forms, for this block
+        P.reset();
+        if (s != FS_ERR_NOMEM) return s;
+        P.planned = true;
+        *use = false;
+        c->err.clear();
+        return FS_OK;
+    };
+    int s;
+    if (!P.planned && (s = build_patches(m))) return without(s);
+    *use = P.usable;
+    const uint64_t kgen = precision == FS_PREC_FP64 ? 0 : m->mixed.kgen;
+    if (!P.usable || (P.kind == precision && P.vgen == B.vgen && P.kgen == kgen)) return FS_OK;
+    P.kind = -1;
+    const bool f32 = precision == FS_PREC_MIXED_F32;
+    if (f32 ? (s = ensure(c, P.kh, (size_t)P.nent * 144)) || (s = ensure(c, P.kl, (size_t)P.nent * 72))
+            : (s = ensure(c, P.k2, (size_t)P.nent * 288)))
+        return without(s);
+    FS_HIP(c, fs::launch_patch_build(patchop_of(P), precision == FS_PREC_FP64 ? 0 : f32 ? 2 : 1, plan_of(B),
+                                     B.kval.as<double>(), precision == FS_PREC_FP64 ? fs::MixedOp{} : mixed_op(m),
+                                     m->dconn.as<int32_t>(), m->nen, precision == FS_PREC_FP64 ? 0 : m->mixed.nsr,
+                                     c->stream));
+    P.kind = precision;
+    P.vgen = B.vgen;
+    P.kgen = kgen;
+    return FS_OK;
 }
 
 }  // namespace
@@ -2554,21 +2570,21 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
             build_ms = m->mixed.build_ms;
         }
     }
-    // FP64 loops of PATCH_MIN_STEPS steps or more run on the patch form of K
-    // unless the row products were chosen (fs_ctx_set_cd_lanes); a rule on the
-    // call's step count alone, so that a model takes the same form alone and
-    // in a batch.
+    // Loops of PATCH_MIN_STEPS steps or more run on the patch form of K, FP64
+    // loops unless the row products were chosen (fs_ctx_set_cd_lanes); a rule
+    // on the call's step count alone, so that a model takes the same form
+    // alone and in a batch.
     PatchStore &P = B.patch;
-    bool patch = !mixed && c->cd_lanes == 8 && c->cd_pj == 0 && p->nsteps >= PATCH_MIN_STEPS;
-    if (patch && (s = prepare_patches(m, &patch))) return s;
+    bool patch = (mixed || (c->cd_lanes == 8 && c->cd_pj == 0)) && p->nsteps >= PATCH_MIN_STEPS;
+    if (patch && (s = prepare_patches(m, p->precision, &patch))) return s;
     const fs::PatchOp pop = patchop_of(P);
     // State vectors: the free dofs themselves (row products), node-major dof
     // positions 6 i + c (mixed path), or the patches' slot positions; fixed
     // dofs stay zero in the last two.
     const bool placed = mixed || patch;
-    const int64_t nv = mixed ? 6 * m->N : patch ? P.npatch * 6 * fs::PATCH_NODES : n;
+    const int64_t nv = patch ? P.npatch * fs::PATCH_WG : mixed ? 6 * m->N : n;
     // dof at each position
-    const int64_t *map = mixed ? m->node_dof.as<int64_t>() : patch ? P.map.as<int64_t>() : nullptr;
+    const int64_t *map = patch ? P.map.as<int64_t>() : mixed ? m->node_dof.as<int64_t>() : nullptr;
     bool damped = false;
     for (int gi = 0; gi < ng; ++gi) damped |= (batch ? p->group_cdamp[gi] : p->cdamp) != 0.0;
     StepCache &sc = m->step;
@@ -2649,16 +2665,17 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
             int32_t *slot = rec ? dSlot.as<int32_t>() : nullptr;
             double *pdst = rec ? dProbe.as<double>() + (step / stride) * nprobes : nullptr;
             const double *gt = batch ? dG.as<double>() + step * ng : nullptr;
-            if (mixed)
+            if (patch)
+                e = fs::launch_cd_patch_step(pop, p->precision == FS_PREC_MIXED_F32, dU[cur].as<double>(),
+                                             dU[1 - cur].as<double>(), dV.as<double>(), dInv.as<double>(),
+                                             dC.as<double>(), dF.as<double>(), batch ? 0.0 : g[step], p->dt,
+                                             damped ? 1 : 0, forced[step] ? 1 : 0, step == p->nsteps ? 1 : 0, slot, pdst,
+                                             rg, gdt, gt, st);
+            else if (mixed)
                 e = fs::launch_cd_mixed_step(m->nen, m->mixed.nsr, op, dU[cur].as<double>(),
                                              dU[1 - cur].as<double>(), dV.as<double>(), dA.as<double>(),
                                              dInv.as<double>(), dC.as<double>(), dF.as<double>(),
                                              batch ? 0.0 : g[step], p->dt, damped ? 1 : 0, forced[step] ? 1 : 0,
-                                             slot, pdst, rg, gdt, gt, st);
-            else if (patch)
-                e = fs::launch_cd_patch_step(pop, dU[cur].as<double>(), dU[1 - cur].as<double>(), dV.as<double>(),
-                                             dInv.as<double>(), dC.as<double>(), dF.as<double>(), batch ? 0.0 : g[step],
-                                             p->dt, damped ? 1 : 0, forced[step] ? 1 : 0, step == p->nsteps ? 1 : 0,
                                              slot, pdst, rg, gdt, gt, st);
             else if (c->cd_lanes > 0)
                 e = fs::launch_cd_node_step(c->cd_lanes, cd_pj, noderows_of(B), B.slotrec.as<int2>(), B.kval.as<double>(),
@@ -2692,8 +2709,8 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
             key_add(key, b->p);
         key_add(key, B.kval.p);
         key_add(key, B.slotrec.p);
-        if (mixed) key_add(key, op);
-        else if (patch) key_add(key, pop);
+        if (patch) key_add(key, pop);
+        else if (mixed) key_add(key, op);
         else if (c->cd_lanes > 0) key_add(key, noderows_of(B));
         else key_add(key, runrows_of(B));
         for (int64_t step = 0; step <= p->nsteps; ++step) {

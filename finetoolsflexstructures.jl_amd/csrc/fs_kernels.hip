@@ -2503,6 +2503,23 @@ __global__ __launch_bounds__(CDN_WG) void cd_node_step_kernel(NodeRows nrw, cons
     }
 }
 
+// Split of an FP64 value into FP32 hi and an int16 residual lo in units of
+// 2^-15 of hi's ulp: v = hi + lo 2^(e - 165) (e = biased exponent of hi)
+// to within 2^(e - 166), a relative 2^-39.  |v - hi| <= ulp(hi) / 2 bounds
+// |lo| by 2^14.
+__device__ __forceinline__ double mx_scale(float hi) {
+    const unsigned e = (__float_as_uint(hi) >> 23) & 0xffu;
+    return e ? __longlong_as_double((long long)(e + 858u) << 52) : 0.0;
+}
+
+__device__ __forceinline__ void mx_split(double v, float &hi, short &lo) {
+    hi = (float)v;
+    const double s = mx_scale(hi);
+    lo = s != 0.0 ? (short)rint((v - (double)hi) / s) : (short)0;
+}
+
+__device__ __forceinline__ double mx_value(float hi, short lo) { return (double)hi + (double)lo * mx_scale(hi); }
+
 // ---------------------------------------------------------------------------
 // Step on the symmetric patch form of K (PatchOp)
 // ---------------------------------------------------------------------------
@@ -2545,43 +2562,112 @@ __device__ __forceinline__ int64_t patch_entry(const PatchOp &op, const int4 &re
     return e < PATCH_WG ? (int64_t)p * PATCH_WG + e : op.over + rec.x + e;
 }
 
-// Stored blocks from the CSR values: workgroup per patch, thread per (entry,
-// row) for the blocks and per (slot, row) for the diagonals.
-__global__ __launch_bounds__(256) void patch_build_kernel(PatchOp op, ScatterPlan sp,
-                                                          const double *__restrict__ kval) {
+// Where the blocks of a patch form come from.
+//   PATCH_FP64   the CSR values
+//   PATCH_MIXED  the mixed operator's parts (MixedOp): the slices' rounded
+//                membrane and bending values, the shear factor rows (nsr > 0),
+//                the drilling blocks, summed in FP64
+//   PATCH_F32    the slices' values as they are stored (shear among them), the
+//                diagonal blocks as PATCH_MIXED
+enum { PATCH_FP64 = 0, PATCH_MIXED = 1, PATCH_F32 = 2 };
+struct PatchSource {
+    ScatterPlan sp;
+    const double *kval;
+    MixedOp op;
+    const int32_t *conn;
+    int nen, nsr;
+};
+
+// Row r of block (I, J), J the neighbour at slot k of I's list.
+template <int KIND>
+__device__ __forceinline__ void patch_block_row(const PatchSource &src, int I, int k, int r, double v[6]) {
+    const ScatterPlan &sp = src.sp;
+    for (int c = 0; c < 6; ++c) v[c] = 0.0;
+    const int J = sp.nbr_node[k];
+    if constexpr (KIND == PATCH_FP64) {
+        const int rs = sp.node_rowstart[6 * I + r], off = sp.nbr_off[2 * k];
+        if (rs >= 0 && off >= 0)
+            for (int c = 0; c < 6; ++c) {
+                const int code = sp.node_code[6 * J + c];
+                if (code >= 0) v[c] = src.kval[rs + off + code];
+            }
+    } else {
+        const MixedOp &op = src.op;
+        const int64_t at = op.goff[I / 10] + 6 * (I % 10) + r + (int64_t)(3 * (k - sp.nbr_ptr[I])) * 60;
+        for (int c2 = 0; c2 < 3; ++c2) {
+            const float2 h = op.kmb[at + 60 * c2];
+            const short2 l = op.kml[at + 60 * c2];
+            v[2 * c2] = mx_value(h.x, l.x);
+            v[2 * c2 + 1] = mx_value(h.y, l.y);
+        }
+        if (src.nsr > 0) {
+            const int nen = src.nen, K = 6 * nen, nblk = nen * (nen + 1) / 2;
+            const int pr = sp.nbr_pair[k] >> 1;
+            for (int q = sp.contrib_ptr[pr]; q < sp.contrib_ptr[pr + 1]; ++q) {
+                const int e = (sp.contrib[q] >> 1) / nblk;
+                int a = 0, b = 0;
+                for (int n = 0; n < nen; ++n) {
+                    const int node = src.conn[(int64_t)n * op.nelem + e];
+                    if (node == I) a = n;
+                    if (node == J) b = n;
+                }
+                const double *C = op.cs + (int64_t)e * src.nsr * K;
+                for (int s = 0; s < src.nsr; ++s)
+                    for (int c = 0; c < 6; ++c) v[c] += C[s * K + 6 * a + r] * C[s * K + 6 * b + c];
+            }
+        }
+        if (I == J && r >= 3) {
+            const double *d = op.dr + 6 * (int64_t)I;
+            for (int c = 3; c < 6; ++c) {
+                const int x = min(r, c) - 3, y = max(r, c) - 3;
+                v[c] += d[x * (5 - x) / 2 + y];
+            }
+        }
+    }
+}
+
+// Stored blocks: workgroup per patch, thread per (entry, row) for the blocks
+// and per (slot, row) for the diagonals.
+template <int KIND>
+__global__ __launch_bounds__(256) void patch_build_kernel(PatchOp op, PatchSource src) {
     const int p = (int)xcd_block(blockIdx.x, gridDim.x);
     const int4 rec = op.rec[p];
     const int ne = rec.y, nep = (ne + 7) & ~7;
     const int32_t *pn = op.pnode + (int64_t)p * PATCH_NODES;
-    double2 *kb = op.k2 + (int64_t)rec.x * 18;
-    for (int i = threadIdx.x; i < 6 * nep; i += 256) {
-        const int r = i / nep, e = i % nep;
-        double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        if (e < ne) {
-            const int64_t at = patch_entry(op, rec, p, e);
-            const int I = pn[op.ent[at].x >> 26];
-            const int k = op.entk[at];
-            const int J = sp.nbr_node[k], rs = sp.node_rowstart[6 * I + r], off = sp.nbr_off[2 * k];
-            if (rs >= 0 && off >= 0)
-                for (int c = 0; c < 6; ++c) {
-                    const int code = sp.node_code[6 * J + c];
-                    if (code >= 0) v[c] = kval[rs + off + code];
-                }
+    for (int i = threadIdx.x; i < 6 * ne; i += 256) {
+        const int r = i / ne, e = i % ne;
+        const int64_t at = patch_entry(op, rec, p, e);
+        const int I = pn[op.ent[at].x >> 26], k = op.entk[at];
+        if constexpr (KIND == PATCH_F32) {
+            const MixedOp &mo = src.op;
+            const int64_t m = mo.goff[I / 10] + 6 * (I % 10) + r + (int64_t)(3 * (k - src.sp.nbr_ptr[I])) * 60;
+            float *kh = reinterpret_cast<float *>(op.kh + (int64_t)rec.x * 9);
+            short *kl = reinterpret_cast<short *>(op.kl + (int64_t)rec.x * 9);
+            for (int c = 0; c < 6; ++c) {
+                const int w = 6 * r + c;
+                const float2 h = mo.kmb[m + 60 * (c / 2)];
+                const short2 l = mo.kml[m + 60 * (c / 2)];
+                const int64_t to = 4 * ((int64_t)(w / 4) * nep + e) + w % 4;
+                kh[to] = c % 2 ? h.y : h.x;
+                kl[to] = c % 2 ? l.y : l.x;
+            }
+        } else {
+            double v[6];
+            patch_block_row<KIND>(src, I, k, r, v);
+            double2 *kb = op.k2 + (int64_t)rec.x * 18;
+            for (int c2 = 0; c2 < 3; ++c2) kb[(int64_t)(3 * r + c2) * nep + e] = make_double2(v[2 * c2], v[2 * c2 + 1]);
         }
-        for (int c2 = 0; c2 < 3; ++c2) kb[(int64_t)(3 * r + c2) * nep + e] = make_double2(v[2 * c2], v[2 * c2 + 1]);
     }
     for (int i = threadIdx.x; i < 6 * PATCH_NODES; i += 256) {
         const int li = i / 6, r = i % 6, I = pn[li];
         double *dg = op.dg + ((int64_t)p * PATCH_NODES + li) * PATCH_TRI + r * (11 - r) / 2;
-        const int rs = I < 0 ? -1 : sp.node_rowstart[6 * I + r];
-        int off = -1;
-        if (I >= 0)
-            for (int k = sp.nbr_ptr[I]; k < sp.nbr_ptr[I + 1]; ++k)
-                if (sp.nbr_node[k] == I) off = sp.nbr_off[2 * k];
-        for (int c = r; c < 6; ++c) {
-            const int code = I < 0 ? -1 : sp.node_code[6 * I + c];
-            dg[c] = (rs >= 0 && off >= 0 && code >= 0) ? kval[rs + off + code] : 0.0;
+        double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+        if (I >= 0) {
+            int k = src.sp.nbr_ptr[I];
+            while (src.sp.nbr_node[k] != I) ++k;  // a node is in its own list
+            patch_block_row<KIND>(src, I, k, r, v);
         }
+        for (int c = r; c < 6; ++c) dg[c] = v[c];
     }
 }
 
@@ -2606,6 +2692,41 @@ __global__ __launch_bounds__(256) void patch_init_kernel(int64_t nv, double dt, 
     U1[q] = U0[q] + dt * w;
 }
 
+// The lane's stored block: 36 FP64 values, or FP32 values with their residuals.
+template <bool F32>
+struct PatchBlock;
+template <>
+struct PatchBlock<false> {
+    double2 u[18];
+    __device__ __forceinline__ void load(const PatchOp &op, int first, int nep, int e) {
+        const double2 *kb = op.k2 + (int64_t)first * 18 + e;
+#pragma unroll
+        for (int v = 0; v < 18; ++v) u[v] = kb[v * nep];
+    }
+    __device__ __forceinline__ double at(int i) const { return i % 2 ? u[i / 2].y : u[i / 2].x; }
+};
+template <>
+struct PatchBlock<true> {
+    float4 h[9];
+    short4 l[9];
+    __device__ __forceinline__ void load(const PatchOp &op, int first, int nep, int e) {
+        const float4 *kh = op.kh + (int64_t)first * 9 + e;
+        const short4 *kl = op.kl + (int64_t)first * 9 + e;
+#pragma unroll
+        for (int v = 0; v < 9; ++v) {
+            h[v] = kh[v * nep];
+            l[v] = kl[v * nep];
+        }
+    }
+    __device__ __forceinline__ double at(int i) const {
+        const float4 a = h[i / 4];
+        const short4 b = l[i / 4];
+        return i % 4 == 0 ? mx_value(a.x, b.x) : i % 4 == 1 ? mx_value(a.y, b.y) : i % 4 == 2 ? mx_value(a.z, b.z)
+                                                                                 : mx_value(a.w, b.w);
+    }
+};
+
+template <bool F32>
 __global__ __launch_bounds__(PATCH_WG) __attribute__((amdgpu_waves_per_eu(3))) void cd_patch_step_kernel(
     PatchOp op, const double *__restrict__ Ucur, double *__restrict__ Unext, double *__restrict__ W,
     const double *__restrict__ invMC, const double *__restrict__ Cd, const double *__restrict__ Fmag, double gstep,
@@ -2623,7 +2744,6 @@ __global__ __launch_bounds__(PATCH_WG) __attribute__((amdgpu_waves_per_eu(3))) v
     uint2 en = op.ent[q];  // the lane's first entry
     const int4 rec = op.rec[p];
     const int ne = rec.y, nep = (ne + 7) & ~7;
-    const double2 *kb = op.k2 + (int64_t)rec.x * 18;
     const double *dgp = op.dg + (int64_t)p * (PATCH_TRI * PATCH_NODES);
     constexpr int ND = PATCH_TRI * PATCH_NODES;
     double dv[(ND + PATCH_WG - 1) / PATCH_WG];
@@ -2634,11 +2754,8 @@ __global__ __launch_bounds__(PATCH_WG) __attribute__((amdgpu_waves_per_eu(3))) v
     const uint16_t *np = op.nptr + p * (PATCH_NODES + 1) + li;
     const int s0 = np[0], s1 = np[1];
     int e = tid;
-    double2 k2[18];
-    if (e < ne) {
-#pragma unroll
-        for (int v = 0; v < 18; ++v) k2[v] = kb[v * nep + e];
-    }
+    PatchBlock<F32> kb;
+    if (e < ne) kb.load(op, rec.x, nep, e);
     const double w = W[q], im = invMC[q];
     const int gi = row_group ? row_group[q] : 0;
     xs[tid] = u;
@@ -2658,36 +2775,28 @@ __global__ __launch_bounds__(PATCH_WG) __attribute__((amdgpu_waves_per_eu(3))) v
             for (int c = 0; c < 3; ++c) xj[c] = x2[c];
         }
         double *pi = part + 6 * (en.y & 0xffff);
+        const double xa[6] = {xj[0].x, xj[0].y, xj[1].x, xj[1].y, xj[2].x, xj[2].y};
+        const double *xi = xs + 6 * (en.x >> 26);
+        double *pj = part + 6 * (en.y >> 16);
+        double y[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int rr = 0; rr < 6; ++rr)
-            pi[rr] = k2[3 * rr].x * xj[0].x + k2[3 * rr].y * xj[0].y + k2[3 * rr + 1].x * xj[1].x +
-                     k2[3 * rr + 1].y * xj[1].y + k2[3 * rr + 2].x * xj[2].x + k2[3 * rr + 2].y * xj[2].y;
-        if (inner) {
-            const double *xi = xs + 6 * (en.x >> 26);
-            double *pj = part + 6 * (en.y >> 16);
-            double2 y[3];
+        for (int rr = 0; rr < 6; ++rr) {
+            const double xr = xi[rr];
+            double f = 0.0;
 #pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                y[c].x = k2[c].x * xi[0];
-                y[c].y = k2[c].y * xi[0];
+            for (int c = 0; c < 6; ++c) {
+                const double v = kb.at(6 * rr + c);
+                f += v * xa[c];
+                y[c] += v * xr;
             }
-#pragma unroll
-            for (int rr = 1; rr < 6; ++rr)
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    y[c].x += k2[3 * rr + c].x * xi[rr];
-                    y[c].y += k2[3 * rr + c].y * xi[rr];
-                }
-            for (int c = 0; c < 3; ++c) {
-                pj[2 * c] = y[c].x;
-                pj[2 * c + 1] = y[c].y;
-            }
+            pi[rr] = f;
         }
+        if (inner)
+            for (int c = 0; c < 6; ++c) pj[c] = y[c];
         e += PATCH_WG;
         if (e < ne) {
             en = op.ent[op.over + rec.x + e];
-#pragma unroll
-            for (int v = 0; v < 18; ++v) k2[v] = kb[v * nep + e];
+            kb.load(op, rec.x, nep, e);
         }
     }
     __syncthreads();
@@ -2735,23 +2844,6 @@ __global__ __launch_bounds__(PATCH_WG) __attribute__((amdgpu_waves_per_eu(3))) v
 
 // K_mb slices from the split element blocks: thread per (node, row, neighbour
 // slot); the sum over the pair's contributions follows scatter_pair_kernel.
-// Split of an FP64 value into FP32 hi and an int16 residual lo in units of
-// 2^-15 of hi's ulp: v = hi + lo 2^(e - 165) (e = biased exponent of hi)
-// to within 2^(e - 166), a relative 2^-39.  |v - hi| <= ulp(hi) / 2 bounds
-// |lo| by 2^14.
-__device__ __forceinline__ double mx_scale(float hi) {
-    const unsigned e = (__float_as_uint(hi) >> 23) & 0xffu;
-    return e ? __longlong_as_double((long long)(e + 858u) << 52) : 0.0;
-}
-
-__device__ __forceinline__ void mx_split(double v, float &hi, short &lo) {
-    hi = (float)v;
-    const double s = mx_scale(hi);
-    lo = s != 0.0 ? (short)rint((v - (double)hi) / s) : (short)0;
-}
-
-__device__ __forceinline__ double mx_value(float hi, short lo) { return (double)hi + (double)lo * mx_scale(hi); }
-
 __global__ __launch_bounds__(256) void mixed_build_kernel(ScatterPlan sp, const double *__restrict__ Kb,
                                                           const int64_t *__restrict__ goff, float2 *__restrict__ kmb,
                                                           short2 *__restrict__ kml) {
@@ -3666,9 +3758,25 @@ hipError_t launch_patch_map(const PatchOp &op, const int64_t *node_dof, int64_t 
     return hipGetLastError();
 }
 
-hipError_t launch_patch_build(const PatchOp &op, const ScatterPlan &sp, const double *kval, hipStream_t st) {
+// kind: 0 the CSR values, 1 the mixed operator in FP64 blocks, 2 in FP32 with
+// residuals (op, conn, nen and nsr describe the mixed operator).
+hipError_t launch_patch_build(const PatchOp &op, int kind, const ScatterPlan &sp, const double *kval,
+                              const MixedOp &mixed, const int32_t *conn, int nen, int nsr, hipStream_t st) {
     if (op.npatch == 0) return hipSuccess;
-    hipLaunchKernelGGL(patch_build_kernel, dim3((unsigned)op.npatch), dim3(256), 0, st, op, sp, kval);
+    PatchSource src;
+    src.sp = sp;
+    src.kval = kval;
+    src.op = mixed;
+    src.conn = conn;
+    src.nen = nen;
+    src.nsr = nsr;
+    const dim3 grid((unsigned)op.npatch), wg(256);
+    if (kind == PATCH_FP64)
+        hipLaunchKernelGGL(patch_build_kernel<PATCH_FP64>, grid, wg, 0, st, op, src);
+    else if (kind == PATCH_MIXED)
+        hipLaunchKernelGGL(patch_build_kernel<PATCH_MIXED>, grid, wg, 0, st, op, src);
+    else
+        hipLaunchKernelGGL(patch_build_kernel<PATCH_F32>, grid, wg, 0, st, op, src);
     return hipGetLastError();
 }
 
@@ -3686,14 +3794,19 @@ size_t patch_smem(int slots) {
     return sizeof(double) * (size_t)(6 * PATCH_NODES + PATCH_TRI * PATCH_NODES + 6 * slots);
 }
 
-hipError_t launch_cd_patch_step(const PatchOp &op, const double *Ucur, double *Unext, double *W, const double *invMC,
+hipError_t launch_cd_patch_step(const PatchOp &op, int f32, const double *Ucur, double *Unext, double *W, const double *invMC,
                                 const double *Cd, const double *Fmag, double gstep, double dt, int damped, int forced,
                                 int last, const int32_t *probe_slot, double *probe_dst,
                                 const int32_t *row_group, const double *group_dt, const double *gtab, hipStream_t st) {
     if (op.npatch == 0) return hipSuccess;
-    hipLaunchKernelGGL(cd_patch_step_kernel, dim3((unsigned)op.npatch), dim3(PATCH_WG), patch_smem(op.slots), st, op,
-                       Ucur, Unext, W, invMC, Cd, Fmag, gstep, dt, damped, forced, last, probe_slot, probe_dst, row_group,
-                       group_dt, gtab);
+    const dim3 grid((unsigned)op.npatch), wg(PATCH_WG);
+    const size_t smem = patch_smem(op.slots);
+    if (f32)
+        hipLaunchKernelGGL(cd_patch_step_kernel<true>, grid, wg, smem, st, op, Ucur, Unext, W, invMC, Cd, Fmag, gstep, dt,
+                           damped, forced, last, probe_slot, probe_dst, row_group, group_dt, gtab);
+    else
+        hipLaunchKernelGGL(cd_patch_step_kernel<false>, grid, wg, smem, st, op, Ucur, Unext, W, invMC, Cd, Fmag, gstep, dt,
+                           damped, forced, last, probe_slot, probe_dst, row_group, group_dt, gtab);
     return hipGetLastError();
 }
 

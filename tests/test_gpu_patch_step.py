@@ -3,7 +3,9 @@ steps or more) against the row products and the oracle.
 
 Both forms add the same products in different orders: 1e-12 relative between
 them over 120 steps at 0.8 of the stable dt (the bound of the row forms among
-themselves), 1e-10 against the oracle's loop.  Meshes at the edges of the
+themselves), 1e-10 against the oracle's loop.  The mixed precisions hold
+values to a relative 2^-39: over n steps at omega dt <= 2 a phase error of 2 n
+2^-39, 4.4e-10 for 120 steps, bounded by 1e-9 against the oracle.  Meshes at the edges of the
 plan: one node with free dofs, one and two patches (42 and 43 nodes), a hub
 whose patch has more blocks than the workgroup has lanes, a hub of more
 neighbours than a patch takes (row products throughout), two components,
@@ -70,11 +72,12 @@ MESHES = {
 
 
 @pytest.mark.parametrize("name", list(MESHES))
-@pytest.mark.parametrize("cdamp", [0.0, 50.0], ids=["undamped", "damped"])
-def test_patch_step(ctx, name, cdamp):
+@pytest.mark.parametrize("cdamp,form", [(0.0, 0), (50.0, 1)], ids=["undamped", "damped_average_k"])
+def test_patch_step(ctx, name, cdamp, form):
     print(f"[gpu] patch step {name} {cdamp}", flush=True)
     nen, xyz, conn, d = MESHES[name]()
     f = FM.make(conn, MatDeforElastIso(70e9, 0.33, 2700.0), thickness=0.02, ctx=ctx)
+    f.transv_shear_formulation = form if nen == 3 else 0
     f.associategeometry(xyz)
     nf = d.nfreedofs
     K = f.stiffness(FM.SysmatAssemblerFFBlock(nf), xyz, None, None, d)
@@ -98,6 +101,13 @@ def test_patch_step(ctx, name, cdamp):
         assert np.linalg.norm(r[key] - rows[key]) <= 1e-12 * np.linalg.norm(rows[key]), key
         assert np.linalg.norm(r[key] - ref) <= 1e-10 * np.linalg.norm(ref), key
     assert np.linalg.norm(r["probes"] - po[::7]) <= 1e-10 * np.linalg.norm(po)
+    # the mixed precisions on the same plan, also after one another
+    for prec in (_lib.FS_PREC_MIXED, _lib.FS_PREC_MIXED_F32, _lib.FS_PREC_MIXED):
+        q = explicit.run(f._model, cdamp, U0, V0, dt, nsteps, F, g, probes, 7, precision=prec)
+        for key, ref in (("U", Uo), ("V", Vo)):
+            assert np.linalg.norm(q[key] - ref) <= 1e-9 * np.linalg.norm(ref), (prec, key)
+    back = explicit.run(f._model, cdamp, U0, V0, dt, nsteps, F, g, probes, 7)
+    assert np.array_equal(r["U"], back["U"]) and np.array_equal(r["V"], back["V"])
     # new values behind the same plan
     f.thickness = 0.03
     f.stiffness(FM.SysmatAssemblerHIP(_lib.FS_BLOCK_FF), xyz, None, None, d)
