@@ -17,6 +17,7 @@
 #include <cstdlib>
 #include <functional>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <cstdarg>
 #include <cstdio>
@@ -401,6 +402,15 @@ int64_t host_threads() {
         return n;
     }();
     return nt;
+}
+
+// Host array whose elements are not initialised: for large arrays that
+// threads fill, so that one thread does not touch all their pages first.
+template <class T>
+using HostArray = std::unique_ptr<T[]>;
+template <class T>
+HostArray<T> host_array(int64_t n) {
+    return HostArray<T>(new T[(size_t)std::max<int64_t>(n, 1)]);
 }
 
 // Runs fn(begin, end) over [0, n) in up to host_threads() chunks of at
@@ -971,10 +981,13 @@ int build_patches(fs_model *m) {
     if (N >= (int64_t(1) << 24)) return FS_OK;  // slots are 26-bit numbers
     auto active = [&](int64_t I) { return B.h_node_rec[4 * I] >= 0; };  // node with free dofs
     auto degree = [&](int64_t I) { return m->nbr_ptr[I + 1] - m->nbr_ptr[I]; };
-    for (int64_t I = 0; I < N; ++I)
-        if (active(I) && degree(I) > PATCH_MAX_SLOTS) return FS_OK;
+    // coordinates, copied while the components are found
+    HostArray<double> xyz = host_array<double>(3 * N);
+    FS_HIP(c, hipMemcpyAsync(xyz.get(), m->x.p, N * 8, hipMemcpyDeviceToHost, c->stream));
+    FS_HIP(c, hipMemcpyAsync(xyz.get() + N, m->y.p, N * 8, hipMemcpyDeviceToHost, c->stream));
+    FS_HIP(c, hipMemcpyAsync(xyz.get() + 2 * N, m->z.p, N * 8, hipMemcpyDeviceToHost, c->stream));
     // components: union-find, the smaller number of two roots stays one
-    std::vector<int32_t> par(N);
+    HostArray<int32_t> par = host_array<int32_t>(N);
     for (int64_t i = 0; i < N; ++i) par[i] = (int32_t)i;
     auto find = [&](int32_t x) {
         for (;;) {
@@ -999,39 +1012,63 @@ int build_patches(fs_model *m) {
                 }
             }
     }, 16384);
-    // active nodes by component (components by their smallest node)
+    // active nodes by component (components by their smallest node), in node
+    // order within one; a mesh of one component is laid out in parallel
     struct Pt {
         double x[3];
         int64_t id;
     };
-    std::vector<int32_t> cid(N, -1);
-    std::vector<int64_t> cptr(1, 0);
-    for (int64_t I = 0; I < N; ++I) {
-        const int32_t r = find((int32_t)I);
-        if (cid[r] < 0) {
-            cid[r] = (int32_t)cptr.size() - 1;
-            cptr.push_back(0);
+    FS_HIP(c, hipStreamSynchronize(c->stream));
+    auto num = [](double v) { return std::isfinite(v) ? v : 0.0; };  // an order needs numbers
+    auto point = [&](int64_t I) { return Pt{{num(xyz[I]), num(xyz[N + I]), num(xyz[2 * N + I])}, I}; };
+    std::atomic<int64_t> roots{0};
+    std::atomic<bool> hub{false};
+    constexpr int64_t CH = 8192;  // nodes counted together
+    const int64_t nch = (N + CH - 1) / CH;
+    std::vector<int64_t> at(nch + 1, 0);
+    parallel_chunks(nch, [&](int64_t k0, int64_t k1) {
+        int64_t nr = 0;
+        for (int64_t k = k0; k < k1; ++k)
+            for (int64_t I = k * CH; I < std::min(N, (k + 1) * CH); ++I) {
+                nr += find((int32_t)I) == I;
+                at[k + 1] += active(I);
+                if (active(I) && degree(I) > PATCH_MAX_SLOTS) hub = true;
+            }
+        roots += nr;
+    }, 4);
+    if (hub) return FS_OK;
+    for (int64_t k = 0; k < nch; ++k) at[k + 1] += at[k];
+    const int64_t npt = at[nch];
+    HostArray<Pt> pt = host_array<Pt>(npt);
+    std::vector<int64_t> cptr(2, 0);
+    if (roots == 1) {
+        cptr[1] = npt;
+        parallel_chunks(nch, [&](int64_t k0, int64_t k1) {
+            int64_t to = at[k0];
+            for (int64_t I = k0 * CH; I < std::min(N, k1 * CH); ++I)
+                if (active(I)) pt[to++] = point(I);
+        }, 4);
+    } else {
+        cptr.assign(1, 0);
+        std::vector<int32_t> cid(N, -1);
+        for (int64_t I = 0; I < N; ++I) {
+            const int32_t r = find((int32_t)I);
+            if (cid[r] < 0) {
+                cid[r] = (int32_t)cptr.size() - 1;
+                cptr.push_back(0);
+            }
+            cid[I] = cid[r];
+            if (active(I)) ++cptr[cid[I] + 1];
         }
-        cid[I] = cid[r];
-        if (active(I)) ++cptr[cid[I] + 1];
+        for (size_t k = 0; k + 1 < cptr.size(); ++k) cptr[k + 1] += cptr[k];
+        std::vector<int64_t> fill(cptr.begin(), cptr.end() - 1);
+        for (int64_t I = 0; I < N; ++I)
+            if (active(I)) pt[fill[cid[I]]++] = point(I);
     }
     const int64_t nc = (int64_t)cptr.size() - 1;
-    for (int64_t k = 0; k < nc; ++k) cptr[k + 1] += cptr[k];
-    std::vector<double> xyz(3 * N);
-    FS_HIP(c, hipMemcpyAsync(xyz.data(), m->x.p, N * 8, hipMemcpyDeviceToHost, c->stream));
-    FS_HIP(c, hipMemcpyAsync(xyz.data() + N, m->y.p, N * 8, hipMemcpyDeviceToHost, c->stream));
-    FS_HIP(c, hipMemcpyAsync(xyz.data() + 2 * N, m->z.p, N * 8, hipMemcpyDeviceToHost, c->stream));
-    FS_HIP(c, hipStreamSynchronize(c->stream));
-    std::vector<Pt> pt(cptr[nc]);
-    {
-        std::vector<int64_t> fill(cptr.begin(), cptr.end() - 1);
-        auto num = [](double v) { return std::isfinite(v) ? v : 0.0; };  // an order needs numbers
-        for (int64_t I = 0; I < N; ++I)
-            if (active(I)) pt[fill[cid[I]]++] = Pt{{num(xyz[I]), num(xyz[N + I]), num(xyz[2 * N + I])}, I};
-    }
-    std::vector<uint8_t> head(pt.size() + 1, 0);  // 1 where a patch begins
+    std::vector<uint8_t> head(npt + 1, 0);  // 1 where a patch begins
     std::function<void(int64_t, int64_t)> bisect = [&](int64_t b, int64_t n) {
-        Pt *q = pt.data() + b;
+        Pt *q = pt.get() + b;
         int64_t k = (n + PN - 1) / PN;
         if (k == 1) {
             int64_t slots = 0;
@@ -1069,17 +1106,17 @@ int build_patches(fs_model *m) {
             if (cptr[k + 1] > cptr[k]) bisect(cptr[k], cptr[k + 1] - cptr[k]);
     }, 4);
     std::vector<int64_t> pstart;
-    for (int64_t i = 0; i < (int64_t)pt.size(); ++i)
+    for (int64_t i = 0; i < npt; ++i)
         if (head[i]) pstart.push_back(i);
     const int64_t np = (int64_t)pstart.size();
-    pstart.push_back((int64_t)pt.size());
+    pstart.push_back(npt);
     if (np * PN >= (int64_t(1) << 26)) return FS_OK;
     P.pnode.assign(np * PN, -1);
     std::vector<int32_t> slot(N, -1);
     std::vector<int32_t> rec(4 * np, 0);
     parallel_chunks(np, [&](int64_t p0, int64_t p1) {
         for (int64_t p = p0; p < p1; ++p) {
-            std::sort(pt.begin() + pstart[p], pt.begin() + pstart[p + 1], [](const Pt &u, const Pt &v) { return u.id < v.id; });
+            std::sort(pt.get() + pstart[p], pt.get() + pstart[p + 1], [](const Pt &u, const Pt &v) { return u.id < v.id; });
             for (int64_t i = pstart[p]; i < pstart[p + 1]; ++i) {
                 P.pnode[p * PN + i - pstart[p]] = (int32_t)pt[i].id;
                 slot[pt[i].id] = (int32_t)(p * PN + i - pstart[p]);
@@ -1112,9 +1149,11 @@ int build_patches(fs_model *m) {
     }
     if (nent >= (int64_t(1) << 30)) return FS_OK;
     const int64_t over = np * fs::PATCH_WG, ntab = over + nover;
-    std::vector<uint32_t> ent(2 * ntab, 0);
-    std::vector<int32_t> entk(ntab, 0);
-    std::vector<uint16_t> nptr(np * (PN + 1), 0);
+    HostArray<uint32_t> ent = host_array<uint32_t>(2 * ntab);
+    HostArray<int32_t> entk = host_array<int32_t>(ntab);
+    HostArray<uint16_t> nptr = host_array<uint16_t>(np * (PN + 1));
+    std::fill(ent.get() + 2 * over, ent.get() + 2 * ntab, 0u);
+    std::fill(entk.get() + over, entk.get() + ntab, 0);
     std::atomic<int> most{0};
     parallel_chunks(np, [&](int64_t p0, int64_t p1) {
         std::vector<int32_t> by(PN * PN);  // place of the inner entry of (li, lj)
@@ -1145,15 +1184,19 @@ int build_patches(fs_model *m) {
                 }
             }
             for (int li = n; li <= PN; ++li) nptr[p * (PN + 1) + li] = (uint16_t)sl;
+            for (int64_t e = rec[4 * p + 1]; e < fs::PATCH_WG; ++e) {  // lanes without an entry
+                ent[2 * (p * fs::PATCH_WG + e)] = ent[2 * (p * fs::PATCH_WG + e) + 1] = 0;
+                entk[p * fs::PATCH_WG + e] = 0;
+            }
             int cur = most.load();
             while (cur < sl && !most.compare_exchange_weak(cur, sl)) {
             }
         }
     }, 512);
     int s;
-    if ((s = upload(c, P.rec, rec.data(), rec.size())) || (s = upload(c, P.ent, ent.data(), ent.size())) ||
-        (s = upload(c, P.entk, entk.data(), entk.size())) || (s = upload(c, P.dpnode, P.pnode.data(), P.pnode.size())) ||
-        (s = upload(c, P.nptr, nptr.data(), nptr.size())) || (s = dalloc(c, P.map, (size_t)np * PN * 6 * 8)) ||
+    if ((s = upload(c, P.rec, rec.data(), rec.size())) || (s = upload(c, P.ent, ent.get(), 2 * ntab)) ||
+        (s = upload(c, P.entk, entk.get(), ntab)) || (s = upload(c, P.dpnode, P.pnode.data(), P.pnode.size())) ||
+        (s = upload(c, P.nptr, nptr.get(), np * (PN + 1))) || (s = dalloc(c, P.map, (size_t)np * PN * 6 * 8)) ||
         (s = dalloc(c, P.dg, (size_t)np * PN * fs::PATCH_TRI * 8)))
         return s;
     P.npatch = np;
