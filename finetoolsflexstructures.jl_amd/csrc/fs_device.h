@@ -218,13 +218,17 @@ struct NodeRows {
 // columns at fixed dofs) is stored once where I and J lie in one patch
 // (an inner entry, li < lj), and in both patches otherwise (an outer entry of
 // each, with the row node local).
-//   rec[p]    {first block (a multiple of 8), entries, -, -}; the inner entries
-//             come first
+//   rec[p]    {first block (a multiple of 8), entries, inner entries, partial
+//             slots}; the inner entries come first
 //   ent       entry e of patch p: x = li << 26 | slot of J; y = partial slot of
 //             I | partial slot of J << 16 (0xffff: an outer entry).  The first
 //             PATCH_WG entries are at p PATCH_WG + e, so that their loads wait on
 //             nothing; the others at over + first block + e.
 //   entk      neighbour slot of J in I's list (ScatterPlan), indexed as ent
+//   hpos      for the one-launch loop (nullptr where it does not take the mesh):
+//             the patch's halo, the nodes of other patches that its outer
+//             entries take x from: at p PATCH_HALO + t the position of component
+//             t % 6 of halo node t / 6, -1 past the last
 //   pnode[s]  node of slot s, -1 if unused
 //   nptr[p (PATCH_NODES + 1) + li]  partial slots of local node li: one per
 //             neighbour, in the order of its list
@@ -236,6 +240,7 @@ struct NodeRows {
 //   dg        diagonal blocks, 21 upper values (row by row) per slot
 constexpr int PATCH_NODES = 42;
 constexpr int PATCH_WG = 6 * PATCH_NODES;  // lanes of a patch: a dof each, or an entry each
+constexpr int PATCH_HALO = 2 * PATCH_WG;   // halo dofs the one-launch loop takes, two a lane
 constexpr int PATCH_TRI = 21;
 struct PatchOp {
     int32_t npatch;
@@ -244,12 +249,33 @@ struct PatchOp {
     const int4 *rec;
     const uint2 *ent;
     const int32_t *entk;
+    const int32_t *hpos;
     const int32_t *pnode;
     const uint16_t *nptr;
     double2 *k2;
     float4 *kh;
     short4 *kl;
     double *dg;
+};
+
+// One launch of the whole loop on the patch form (cd_patch_loop_kernel).
+struct PatchLoop {
+    PatchOp op;
+    const double *U1;            // U of the first step, in slot positions
+    double *U;                   // out: U of the last step
+    double *W;                   // half-step velocity in, V of the last step out
+    const double *invMC, *Cd, *Fmag;
+    const double *gtab;          // (nsteps + 1) x ng load factors
+    const uint8_t *forced;       // nsteps + 1: a model has a load at this step
+    const int32_t *row_group;    // batch: the row's model, or nullptr
+    const double *group_dt;
+    const int32_t *probe_slot;   // or nullptr
+    double *probe_dst;
+    unsigned long long *pub;     // published displacements, 4 words per position
+    int *stop;                   // host memory: set where a wait ran out
+    double dt;
+    int32_t nsteps, ng, damped, stride, nprobes;
+    uint32_t polls;              // longest wait, in polls
 };
 
 }  // namespace fs

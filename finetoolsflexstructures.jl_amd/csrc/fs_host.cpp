@@ -89,13 +89,20 @@ hipError_t launch_cd_node_step(int nl, int pj, const NodeRows &nrw, const int2 *
                                const double *Cd, const double *Fmag, double gstep, double dt, int damped,
                                const int32_t *probe_slot, double *probe_dst, const int32_t *row_group,
                                const double *group_dt, const double *gtab, hipStream_t st);
+hipError_t launch_patch_count(int64_t np, const int32_t *order, const int32_t *pstart, const int32_t *nbr_ptr,
+                              const int32_t *nbr_node, int32_t *pnode, int32_t *slot, int4 *rec, uint16_t *nptr,
+                              int64_t *tot, hipStream_t st);
+hipError_t launch_patch_fill(int64_t np, const int32_t *nbr_ptr, const int32_t *nbr_node, const int32_t *pnode,
+                             const int32_t *slot, const int4 *rec, const uint16_t *nptr, int64_t over, uint2 *ent,
+                             int32_t *entk, int32_t *hpos, int64_t *tot, hipStream_t st);
 hipError_t launch_patch_map(const PatchOp &op, const int64_t *node_dof, int64_t *map, hipStream_t st);
 hipError_t launch_patch_build(const PatchOp &op, int kind, const ScatterPlan &sp, const double *kval,
                               const MixedOp &mixed, const int32_t *conn, int nen, int nsr, hipStream_t st);
 hipError_t launch_patch_init(const PatchOp &op, double dt, double g0, const double *invMC, const double *Fmag,
                              const double *U0, double *W, double *U1, const int32_t *row_group,
-                             const double *group_dt, const double *gtab, hipStream_t st);
-size_t patch_smem(int slots);
+                             const double *group_dt, const double *gtab, unsigned long long *pub, hipStream_t st);
+hipError_t patch_loop_occupancy(const PatchOp &op, int f32, int *per_cu);
+hipError_t launch_cd_patch_loop(const PatchLoop &a, int f32, hipStream_t st);
 hipError_t launch_cd_patch_step(const PatchOp &op, int f32, const double *Ucur, double *Unext, double *W, const double *invMC,
                                 const double *Cd, const double *Fmag, double gstep, double dt, int damped, int forced,
                                 int last, const int32_t *probe_slot, double *probe_dst,
@@ -172,6 +179,12 @@ struct fs_ctx {
     // status of that lookup
     double *scratch = nullptr;
     hipError_t scratch_status = hipSuccess;
+    // one-launch loop: longest wait of a lane in polls (0: the default, negative:
+    // the loop runs step by step), the word its waits run out into (pinned
+    // host memory, allocated on first use), and whether one has
+    int64_t loop_polls = 0;
+    int *loop_stop = nullptr;
+    bool loop_gave_up = false;
     // stiffness assembly: 1 = fused element tiles (element kernel writes the
     // CSR values of the pairs it completes, boundary pairs finalised after);
     // 0 = element blocks to HBM, then the pair scatter
@@ -235,19 +248,21 @@ struct PatchStore {
     bool planned = false, usable = false;
     int64_t npatch = 0, nent = 0;
     int slots = 0;
+    bool loops = false;        // the one-launch loop takes the plan (hpos is there)
+    int loop_per_cu[2] = {0, 0};  // its workgroups per CU, FP64 and F32 (0: not asked yet)
     // what it is filled with (FS_PREC_*, -1 nothing) and the generations of the
     // values (Block::vgen, MixedStore::kgen) that came from
     int kind = -1;
     uint64_t vgen = 0, kgen = 0;
-    std::vector<int32_t> pnode;  // host copy: the node of each slot
-    DevBuf rec, ent, entk, dpnode, nptr, map, k2, kh, kl, dg;
+    DevBuf rec, ent, entk, hpos, dpnode, nptr, map, k2, kh, kl, dg;
     void reset() {
         planned = usable = false;
         npatch = nent = 0;
         slots = 0;
+        loops = false;
+        loop_per_cu[0] = loop_per_cu[1] = 0;
         kind = -1;
-        pnode.clear();
-        for (DevBuf *b : {&rec, &ent, &entk, &dpnode, &nptr, &map, &k2, &kh, &kl, &dg}) b->release();
+        for (DevBuf *b : {&rec, &ent, &entk, &hpos, &dpnode, &nptr, &map, &k2, &kh, &kl, &dg}) b->release();
     }
 };
 
@@ -335,6 +350,7 @@ struct MixedStore {
 // uploads its initial state into the same buffers and replays the graph,
 // instead of capturing and instantiating its nsteps launches again.
 struct StepCache {
+    DevBuf dPub, dForced;  // one-launch loop
     DevBuf dU[2], dV, dA, dF, dInv, dC, dSlot, dProbe, dRG, dGdt, dGcd, dG, dPlist;
     std::vector<uint64_t> key;
     hipGraph_t graph = nullptr;
@@ -949,6 +965,7 @@ fs::PatchOp patchop_of(const PatchStore &P) {
     op.rec = P.rec.as<int4>();
     op.ent = P.ent.as<uint2>();
     op.entk = P.entk.as<int32_t>();
+    op.hpos = P.hpos.as<int32_t>();
     op.pnode = P.dpnode.as<int32_t>();
     op.nptr = P.nptr.as<uint16_t>();
     op.k2 = P.k2.as<double2>();
@@ -957,6 +974,9 @@ fs::PatchOp patchop_of(const PatchStore &P) {
     op.dg = P.dg.as<double>();
     return op;
 }
+
+// Patches from which the one-launch loop is not tried: two a CU of 256 CUs.
+constexpr int64_t PATCH_LOOP_MAX = 512;
 
 // Partial slots a patch may have: 6 doubles each in LDS (48 KB), so that two
 // workgroups fit a CU.
@@ -978,7 +998,7 @@ int build_patches(fs_model *m) {
     P.planned = true;
     const int64_t N = m->N;
     constexpr int PN = fs::PATCH_NODES;
-    if (N >= (int64_t(1) << 24)) return FS_OK;  // slots are 26-bit numbers
+    if (N >= (int64_t(1) << 27)) return FS_OK;
     auto active = [&](int64_t I) { return B.h_node_rec[4 * I] >= 0; };  // node with free dofs
     auto degree = [&](int64_t I) { return m->nbr_ptr[I + 1] - m->nbr_ptr[I]; };
     // coordinates, copied while the components are found
@@ -1011,16 +1031,22 @@ int build_patches(fs_model *m) {
                     if (__atomic_compare_exchange_n(&par[a], &want, b, false, __ATOMIC_RELAXED, __ATOMIC_RELAXED)) break;
                 }
             }
-    }, 16384);
+    }, 65536);
     // active nodes by component (components by their smallest node), in node
     // order within one; a mesh of one component is laid out in parallel
     struct Pt {
-        double x[3];
-        int64_t id;
+        float x[3];  // from the component's first node
+        int32_t id;
     };
     FS_HIP(c, hipStreamSynchronize(c->stream));
-    auto num = [](double v) { return std::isfinite(v) ? v : 0.0; };  // an order needs numbers
-    auto point = [&](int64_t I) { return Pt{{num(xyz[I]), num(xyz[N + I]), num(xyz[2 * N + I])}, I}; };
+    auto point = [&](int64_t I, int64_t I0) {
+        Pt q{{0.f, 0.f, 0.f}, (int32_t)I};
+        for (int d = 0; d < 3; ++d) {
+            const float v = (float)(xyz[d * N + I] - xyz[d * N + I0]);
+            if (std::isfinite(v)) q.x[d] = v;  // an order needs numbers
+        }
+        return q;
+    };
     std::atomic<int64_t> roots{0};
     std::atomic<bool> hub{false};
     constexpr int64_t CH = 8192;  // nodes counted together
@@ -1035,10 +1061,10 @@ int build_patches(fs_model *m) {
                 if (active(I) && degree(I) > PATCH_MAX_SLOTS) hub = true;
             }
         roots += nr;
-    }, 4);
-    if (hub) return FS_OK;
+    }, 16);
     for (int64_t k = 0; k < nch; ++k) at[k + 1] += at[k];
     const int64_t npt = at[nch];
+    if (hub || npt == 0) return FS_OK;
     HostArray<Pt> pt = host_array<Pt>(npt);
     std::vector<int64_t> cptr(2, 0);
     if (roots == 1) {
@@ -1046,16 +1072,17 @@ int build_patches(fs_model *m) {
         parallel_chunks(nch, [&](int64_t k0, int64_t k1) {
             int64_t to = at[k0];
             for (int64_t I = k0 * CH; I < std::min(N, k1 * CH); ++I)
-                if (active(I)) pt[to++] = point(I);
-        }, 4);
+                if (active(I)) pt[to++] = point(I, 0);
+        }, 16);
     } else {
         cptr.assign(1, 0);
-        std::vector<int32_t> cid(N, -1);
+        std::vector<int32_t> cid(N, -1), cfirst;
         for (int64_t I = 0; I < N; ++I) {
-            const int32_t r = find((int32_t)I);
+            const int32_t r = find((int32_t)I);  // the component's first node
             if (cid[r] < 0) {
                 cid[r] = (int32_t)cptr.size() - 1;
                 cptr.push_back(0);
+                cfirst.push_back(r);
             }
             cid[I] = cid[r];
             if (active(I)) ++cptr[cid[I] + 1];
@@ -1063,7 +1090,7 @@ int build_patches(fs_model *m) {
         for (size_t k = 0; k + 1 < cptr.size(); ++k) cptr[k + 1] += cptr[k];
         std::vector<int64_t> fill(cptr.begin(), cptr.end() - 1);
         for (int64_t I = 0; I < N; ++I)
-            if (active(I)) pt[fill[cid[I]]++] = point(I);
+            if (active(I)) pt[fill[cid[I]]++] = point(I, cfirst[cid[I]]);
     }
     const int64_t nc = (int64_t)cptr.size() - 1;
     std::vector<uint8_t> head(npt + 1, 0);  // 1 where a patch begins
@@ -1080,7 +1107,7 @@ int build_patches(fs_model *m) {
             k = 2;
         }
         const int64_t n1 = n * (k / 2) / k;
-        double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+        float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
         for (int64_t i = 0; i < n; ++i)
             for (int d = 0; d < 3; ++d) {
                 lo[d] = std::min(lo[d], q[i].x[d]);
@@ -1092,7 +1119,7 @@ int build_patches(fs_model *m) {
         std::nth_element(q, q + n1, q + n, [ax](const Pt &u, const Pt &v) {
             return u.x[ax] != v.x[ax] ? u.x[ax] < v.x[ax] : u.id < v.id;
         });
-        if (n > 8192) {
+        if (n > 65536) {  // creating a thread can take as long as cutting 50,000 nodes (3 ms)
             std::thread th(bisect, b + n1, n - n1);
             bisect(b, n1);
             th.join();
@@ -1104,115 +1131,55 @@ int build_patches(fs_model *m) {
     parallel_chunks(nc, [&](int64_t k0, int64_t k1) {
         for (int64_t k = k0; k < k1; ++k)
             if (cptr[k + 1] > cptr[k]) bisect(cptr[k], cptr[k + 1] - cptr[k]);
-    }, 4);
-    std::vector<int64_t> pstart;
+    }, 16);
+    std::vector<int32_t> pstart;
     for (int64_t i = 0; i < npt; ++i)
-        if (head[i]) pstart.push_back(i);
+        if (head[i]) pstart.push_back((int32_t)i);
     const int64_t np = (int64_t)pstart.size();
-    pstart.push_back(npt);
-    if (np * PN >= (int64_t(1) << 26)) return FS_OK;
-    P.pnode.assign(np * PN, -1);
-    std::vector<int32_t> slot(N, -1);
-    std::vector<int32_t> rec(4 * np, 0);
-    parallel_chunks(np, [&](int64_t p0, int64_t p1) {
-        for (int64_t p = p0; p < p1; ++p) {
-            std::sort(pt.get() + pstart[p], pt.get() + pstart[p + 1], [](const Pt &u, const Pt &v) { return u.id < v.id; });
-            for (int64_t i = pstart[p]; i < pstart[p + 1]; ++i) {
-                P.pnode[p * PN + i - pstart[p]] = (int32_t)pt[i].id;
-                slot[pt[i].id] = (int32_t)(p * PN + i - pstart[p]);
-            }
-        }
-    }, 512);
-    // entries of each patch: counts, then the lists
-    std::vector<int32_t> ninner(np, 0);
-    parallel_chunks(np, [&](int64_t p0, int64_t p1) {
-        for (int64_t p = p0; p < p1; ++p) {
-            int inner = 0, outer = 0;
-            for (int64_t i = pstart[p]; i < pstart[p + 1]; ++i) {
-                const int64_t I = pt[i].id;
-                for (int k = m->nbr_ptr[I]; k < m->nbr_ptr[I + 1]; ++k) {
-                    const int32_t sj = slot[m->nbr_list[k]];
-                    if (sj < 0) continue;
-                    if (sj / PN != p) ++outer;
-                    else if (sj > slot[I]) ++inner;
-                }
-            }
-            ninner[p] = inner;
-            rec[4 * p + 1] = inner + outer;
-        }
-    }, 512);
-    int64_t nent = 0, nover = 0;  // blocks, and the reach of the entries past PATCH_WG
-    for (int64_t p = 0; p < np; ++p) {
-        rec[4 * p] = (int32_t)nent;
-        if (rec[4 * p + 1] > fs::PATCH_WG) nover = nent + rec[4 * p + 1];
-        nent += (rec[4 * p + 1] + 7) & ~7;
-    }
-    if (nent >= (int64_t(1) << 30)) return FS_OK;
-    const int64_t over = np * fs::PATCH_WG, ntab = over + nover;
-    HostArray<uint32_t> ent = host_array<uint32_t>(2 * ntab);
-    HostArray<int32_t> entk = host_array<int32_t>(ntab);
-    HostArray<uint16_t> nptr = host_array<uint16_t>(np * (PN + 1));
-    std::fill(ent.get() + 2 * over, ent.get() + 2 * ntab, 0u);
-    std::fill(entk.get() + over, entk.get() + ntab, 0);
-    std::atomic<int> most{0};
-    parallel_chunks(np, [&](int64_t p0, int64_t p1) {
-        std::vector<int32_t> by(PN * PN);  // place of the inner entry of (li, lj)
-        for (int64_t p = p0; p < p1; ++p) {
-            int ei = 0, eo = ninner[p];
-            auto place = [&](int e) { return e < fs::PATCH_WG ? p * fs::PATCH_WG + e : over + rec[4 * p] + e; };
-            const int n = (int)(pstart[p + 1] - pstart[p]);
-            int sl = 0;  // partial slots: one per active neighbour, in list order
-            for (int li = 0; li < n; ++li) {
-                const int64_t I = pt[pstart[p] + li].id;
-                nptr[p * (PN + 1) + li] = (uint16_t)sl;
-                for (int k = m->nbr_ptr[I]; k < m->nbr_ptr[I + 1]; ++k) {
-                    const int32_t sj = slot[m->nbr_list[k]];
-                    if (sj < 0 || m->nbr_list[k] == I) continue;
-                    const int lj = (int)(sj - p * PN);
-                    if (sj / PN == p && lj < li) {
-                        const int64_t at = by[lj * PN + li];
-                        ent[2 * at + 1] = (ent[2 * at + 1] & 0xffffu) | (uint32_t)sl << 16;
-                    } else {
-                        const bool inner = sj / PN == p;
-                        const int64_t at = place(inner ? ei++ : eo++);
-                        if (inner) by[li * PN + lj] = (int32_t)at;
-                        ent[2 * at] = (uint32_t)li << 26 | (uint32_t)sj;
-                        ent[2 * at + 1] = (uint32_t)sl | 0xffff0000u;
-                        entk[at] = k;
-                    }
-                    ++sl;
-                }
-            }
-            for (int li = n; li <= PN; ++li) nptr[p * (PN + 1) + li] = (uint16_t)sl;
-            for (int64_t e = rec[4 * p + 1]; e < fs::PATCH_WG; ++e) {  // lanes without an entry
-                ent[2 * (p * fs::PATCH_WG + e)] = ent[2 * (p * fs::PATCH_WG + e) + 1] = 0;
-                entk[p * fs::PATCH_WG + e] = 0;
-            }
-            int cur = most.load();
-            while (cur < sl && !most.compare_exchange_weak(cur, sl)) {
-            }
-        }
-    }, 512);
+    pstart.push_back((int32_t)npt);
+    if (np * PN >= (int64_t(1) << 26) || npt >= INT32_MAX) return FS_OK;  // slots are 26-bit numbers
+    HostArray<int32_t> order = host_array<int32_t>(npt);
+    for (int64_t i = 0; i < npt; ++i) order[i] = pt[i].id;
+    // the lists on the device; halos for the one-launch loop where it may take
+    // so many patches
     int s;
-    if ((s = upload(c, P.rec, rec.data(), rec.size())) || (s = upload(c, P.ent, ent.get(), 2 * ntab)) ||
-        (s = upload(c, P.entk, entk.get(), ntab)) || (s = upload(c, P.dpnode, P.pnode.data(), P.pnode.size())) ||
-        (s = upload(c, P.nptr, nptr.get(), np * (PN + 1))) || (s = dalloc(c, P.map, (size_t)np * PN * 6 * 8)) ||
-        (s = dalloc(c, P.dg, (size_t)np * PN * fs::PATCH_TRI * 8)))
+    DevBuf dorder, dstart, dslot, dtot;
+    const int32_t *nbp = B.nbr_ptr.as<int32_t>(), *nbn = B.nbr_node.as<int32_t>();
+    if ((s = upload(c, dorder, order.get(), npt)) || (s = upload(c, dstart, pstart.data(), pstart.size())) ||
+        (s = dalloc(c, dslot, N * 4)) || (s = dalloc(c, dtot, 32)) || (s = dalloc(c, P.dpnode, (size_t)np * PN * 4)) ||
+        (s = dalloc(c, P.rec, (size_t)np * 16)) || (s = dalloc(c, P.nptr, (size_t)np * (PN + 1) * 2)))
         return s;
+    FS_HIP(c, hipMemsetAsync(dslot.p, 0xff, N * 4, c->stream));
+    FS_HIP(c, fs::launch_patch_count(np, dorder.as<int32_t>(), dstart.as<int32_t>(), nbp, nbn, P.dpnode.as<int32_t>(),
+                                     dslot.as<int32_t>(), P.rec.as<int4>(), P.nptr.as<uint16_t>(),
+                                     dtot.as<int64_t>(), c->stream));
+    int64_t tot[4];
+    if ((s = d2h(c, tot, dtot.p, 32))) return s;
+    const int64_t nent = tot[0], over = np * fs::PATCH_WG, ntab = over + tot[2];
+    if (nent >= (int64_t(1) << 30)) return FS_OK;
+    const bool halos = np <= PATCH_LOOP_MAX;
+    if ((s = dalloc(c, P.ent, (size_t)ntab * 8)) || (s = dalloc(c, P.entk, (size_t)ntab * 4)) ||
+        (halos && (s = dalloc(c, P.hpos, (size_t)np * fs::PATCH_HALO * 4))) ||
+        (s = dalloc(c, P.map, (size_t)np * PN * 6 * 8)) || (s = dalloc(c, P.dg, (size_t)np * PN * fs::PATCH_TRI * 8)))
+        return s;
+    FS_HIP(c, fs::launch_patch_fill(np, nbp, nbn, P.dpnode.as<int32_t>(), dslot.as<int32_t>(), P.rec.as<int4>(),
+                                    P.nptr.as<uint16_t>(), over, P.ent.as<uint2>(), P.entk.as<int32_t>(),
+                                    halos ? P.hpos.as<int32_t>() : nullptr, dtot.as<int64_t>(), c->stream));
     P.npatch = np;
     P.nent = nent;
-    P.slots = most;
+    P.slots = (int)tot[1];
+    FS_HIP(c, fs::launch_patch_map(patchop_of(P), m->node_dof.as<int64_t>(), P.map.as<int64_t>(), c->stream));
+    if ((s = d2h(c, tot, dtot.p, 32))) return s;  // and the host lists end here
+    P.loops = halos && tot[3] != 0;
     P.usable = true;
-    fs::PatchOp op = patchop_of(P);
-    FS_HIP(c, fs::launch_patch_map(op, m->node_dof.as<int64_t>(), P.map.as<int64_t>(), c->stream));
-    FS_HIP(c, hipStreamSynchronize(c->stream));  // the host lists end here
     return FS_OK;
 }
 
-// Steps from which an FP64 loop takes the patch form.  Its plan costs a model's
-// first such loop about 47 ns per node once (12 ms on the 512 x 512 Q4 panel, 26
-// ms on the 1024 x 512 T3 plate, 16 host threads), and a step then saves 0.2 ns
-// per node (63 and 103 us): from 100 steps on the second loop has paid for it.
+// Steps from which a loop takes the patch form.  Its plan costs a model's first
+// such loop once about 60 ns per node (0.4 ms for 6,076 nodes, 2.7 for 36,381; 12 ms
+// for the 1024 x 512 plate's 525,825 on 16 threads), and a step then saves 0.2 to 0.5
+// ns per node: from 100 to 200 steps on the first loop has paid for it, from 100
+// on the second.
 constexpr int64_t PATCH_MIN_STEPS = 100;
 
 // 3 x 21-bit Morton code of a point scaled into [0, 1)^3.
@@ -1789,6 +1756,63 @@ fs::MixedOp mixed_op(const fs_model *m) {
     return op;
 }
 
+// Places of the one-launch loops on each device: a loop's workgroups wait for
+// one another, so all loops in flight have to fit the device together.  A loop
+// takes as many places as it has patches and gives them back when it has
+// ended; there are two per CU, of the three and more workgroups that a CU holds.
+class LoopPlaces {
+  public:
+    ~LoopPlaces() {
+        if (n_ == 0) return;
+        std::lock_guard<std::mutex> lk(mu());
+        used(dev_) -= n_;
+    }
+    bool take(int dev, int64_t n) {
+        static std::array<int64_t, 64> cus{};
+        if (dev < 0 || dev >= 64) return false;
+        std::lock_guard<std::mutex> lk(mu());
+        if (cus[dev] == 0) {
+            int v = 0;
+            if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return false;
+            cus[dev] = v;
+        }
+        if (used(dev) + n > 2 * cus[dev]) return false;
+        used(dev) += n;
+        dev_ = dev;
+        n_ = n;
+        return true;
+    }
+
+  private:
+    static std::mutex &mu() {
+        static std::mutex m;
+        return m;
+    }
+    static int64_t &used(int dev) {
+        static std::array<int64_t, 64> u{};
+        return u[dev];
+    }
+    int dev_ = 0;
+    int64_t n_ = 0;
+};
+
+// Polls after which a lane of the one-launch loop gives up: about two seconds.
+constexpr uint32_t LOOP_POLLS = 1u << 21;
+
+// Whether the one-launch loop takes a plan at this precision.
+int patch_loops(fs_model *m, int precision, bool *yes) {
+    fs_ctx *c = m->ctx;
+    PatchStore &P = m->blk[FS_BLOCK_FF].patch;
+    *yes = false;
+    if (!P.loops || c->loop_polls < 0 || c->loop_gave_up) return FS_OK;
+    const int f32 = precision == FS_PREC_MIXED_F32;
+    if (P.loop_per_cu[f32] == 0) FS_HIP(c, fs::patch_loop_occupancy(patchop_of(P), f32, &P.loop_per_cu[f32]));
+    if (P.loop_per_cu[f32] < 3) return FS_OK;  // LoopPlaces counts on it
+    if (!c->loop_stop) FS_HIP(c, hipHostMalloc((void **)&c->loop_stop, 64, hipHostMallocDefault));
+    *yes = true;
+    return FS_OK;
+}
+
 // The patch form of a precision's operator (the mixed ones built already): its
 // plan, if there is none yet, and its blocks, if they are of another precision
 // or other values.  *use becomes false where the form does not take the mesh,
@@ -1875,6 +1899,7 @@ void ctx_release(fs_ctx *ctx) {
         if (ctx->stage[i]) (void)hipHostFree(ctx->stage[i]);
         if (ctx->stage_ev[i]) (void)hipEventDestroy(ctx->stage_ev[i]);
     }
+    if (ctx->loop_stop) (void)hipHostFree(ctx->loop_stop);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -2621,6 +2646,12 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
     bool patch = (mixed || (c->cd_lanes == 8 && c->cd_pj == 0)) && p->nsteps >= PATCH_MIN_STEPS;
     if (patch && (s = prepare_patches(m, p->precision, &patch))) return s;
     const fs::PatchOp pop = patchop_of(P);
+    // in one launch where the mesh is small enough and there is room
+    bool loop = false;
+    if (patch && p->nsteps < INT32_MAX && (s = patch_loops(m, p->precision, &loop))) return s;
+    const bool loop_form = loop;
+    LoopPlaces places;
+    if (loop) loop = places.take(c->device, P.npatch);
     // State vectors: the free dofs themselves (row products), node-major dof
     // positions 6 i + c (mixed path), or the patches' slot positions; fixed
     // dofs stay zero in the last two.
@@ -2678,14 +2709,16 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
         }
         return FS_OK;
     };
-    if ((s = set_up())) {
-        sc.drop_graph();
-        return s;
-    }
-    // steps whose load factor is zero for every model skip the Fmag read (mixed path)
+    // steps whose load factor is zero for every model skip the Fmag read
     std::vector<uint8_t> forced(p->nsteps + 1, 0);
     for (int64_t step = 0; step <= p->nsteps; ++step)
         for (int gi = 0; gi < ng && !forced[step]; ++gi) forced[step] = g[step * ng + gi] != 0.0;
+    if ((s = set_up()) ||
+        (loop && ((s = ensure(c, sc.dPub, nv * 32)) || (s = put(c, sc.dForced, forced.data(), forced.size())) ||
+                  (!batch && (s = put(c, dG, g, (size_t)p->nsteps + 1)))))) {
+        sc.drop_graph();
+        return s;
+    }
     // rows of the shell stencils hold 7 (T3) to 9 (Q4) neighbour runs: 4 lanes
     // per row, up to three runs per lane loaded together (measured fastest
     // of 2, 4, 8 and 16 lanes per row on both families)
@@ -2697,11 +2730,38 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
     auto enqueue = [&](hipStream_t st) -> hipError_t {
         hipError_t e = patch ? fs::launch_patch_init(pop, p->dt, batch ? 0.0 : g[0], dInv.as<double>(), dF.as<double>(),
                                                      dU[0].as<double>(), dV.as<double>(), dU[1].as<double>(), rg, gdt,
-                                                     batch ? dG.as<double>() : nullptr, st)
+                                                     batch ? dG.as<double>() : nullptr,
+                                                     loop ? sc.dPub.as<unsigned long long>() : nullptr, st)
                              : fs::launch_cd_init(nv, p->dt, batch ? 0.0 : g[0], dInv.as<double>(), dF.as<double>(),
                                           dU[0].as<double>(), dV.as<double>(), dA.as<double>(), dU[1].as<double>(),
                                           rg, gdt, batch ? dG.as<double>() : nullptr, st);
         if (e != hipSuccess) return e;
+        if (loop) {
+            fs::PatchLoop lp{};
+            lp.op = pop;
+            lp.U1 = dU[1].as<double>();
+            lp.U = dU[p->nsteps % 2].as<double>();
+            lp.W = dV.as<double>();
+            lp.invMC = dInv.as<double>();
+            lp.Cd = dC.as<double>();
+            lp.Fmag = dF.as<double>();
+            lp.gtab = dG.as<double>();
+            lp.forced = sc.dForced.as<uint8_t>();
+            lp.row_group = rg;
+            lp.group_dt = gdt;
+            lp.probe_slot = nprobes > 0 ? dSlot.as<int32_t>() : nullptr;
+            lp.probe_dst = dProbe.as<double>();
+            lp.pub = sc.dPub.as<unsigned long long>();
+            lp.stop = c->loop_stop;
+            lp.dt = p->dt;
+            lp.nsteps = (int32_t)p->nsteps;
+            lp.ng = ng;
+            lp.damped = damped ? 1 : 0;
+            lp.stride = stride;
+            lp.nprobes = nprobes;
+            lp.polls = c->loop_polls > 0 ? (uint32_t)std::min<int64_t>(c->loop_polls, LOOP_POLLS) : LOOP_POLLS;
+            return fs::launch_cd_patch_loop(lp, p->precision == FS_PREC_MIXED_F32, st);
+        }
         int cur = 1;
         for (int64_t step = 1; step <= p->nsteps; ++step) {
             const bool rec = nprobes > 0 && (step % stride == 0);
@@ -2739,19 +2799,24 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
     FS_HIP(c, hipEventCreate(&e0));
     FS_HIP(c, hipEventCreate(&e1));
     m->timing[6] = 0.0;
-    if (p->use_graph) {
+    if (loop) __atomic_store_n(c->loop_stop, 0, __ATOMIC_SEQ_CST);
+    // a small mesh without room for its loop now runs step by step, beside a
+    // graph that it may have of the loop
+    if (p->use_graph && loop == loop_form) {
         // everything the captured launches take as arguments
         std::vector<uint64_t> key;
         key.reserve(64 + (size_t)p->nsteps + 1);
         for (const int64_t v : {nv, n, (int64_t)p->nsteps, (int64_t)p->precision, (int64_t)stride, (int64_t)nprobes,
                                 (int64_t)ng, (int64_t)batch, (int64_t)damped, (int64_t)c->cd_lanes, (int64_t)cd_pj,
-                                (int64_t)tpr, (int64_t)m->nen, (int64_t)m->mixed.nsr, (int64_t)patch})
+                                (int64_t)tpr, (int64_t)m->nen, (int64_t)m->mixed.nsr, (int64_t)patch, (int64_t)loop, c->loop_polls})
             key_add(key, v);
         key_add(key, p->dt);
         for (const DevBuf *b : {&dU[0], &dU[1], &dV, &dA, &dF, &dInv, &dC, &dSlot, &dProbe, &dRG, &dGdt, &dG})
             key_add(key, b->p);
         key_add(key, B.kval.p);
         key_add(key, B.slotrec.p);
+        key_add(key, sc.dPub.p);
+        key_add(key, sc.dForced.p);
         if (patch) key_add(key, pop);
         else if (mixed) key_add(key, op);
         else if (c->cd_lanes > 0) key_add(key, noderows_of(B));
@@ -2788,6 +2853,20 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
         FS_HIP(c, hipStreamSynchronize(c->stream));
     } else {
         FS_HIP(c, hipEventRecord(e0, c->stream));
+        FS_HIP(c, enqueue(c->stream));
+        FS_HIP(c, hipEventRecord(e1, c->stream));
+        FS_HIP(c, hipStreamSynchronize(c->stream));
+    }
+    if (loop && __atomic_load_n(c->loop_stop, __ATOMIC_SEQ_CST) != 0) {
+        // a wait ran out: from the start again, step by step, and no such loop
+        // on this context any more
+        c->loop_gave_up = true;
+        loop = false;
+        probe_list.clear();
+        if ((s = set_up())) {
+            sc.drop_graph();
+            return s;
+        }
         FS_HIP(c, enqueue(c->stream));
         FS_HIP(c, hipEventRecord(e1, c->stream));
         FS_HIP(c, hipStreamSynchronize(c->stream));
@@ -2945,6 +3024,13 @@ int fs_ctx_set_cd_lanes(fs_ctx *ctx, int lanes_per_node, int positions_per_lane)
     if (!ok) return fail(ctx, FS_ERR_ARG, "cd lanes: %d lanes per node with %d positions per lane", lanes_per_node, pj);
     ctx->cd_lanes = lanes_per_node;
     ctx->cd_pj = lanes_per_node ? pj : 0;
+    return FS_OK;
+}
+
+int fs_ctx_set_cd_loop(fs_ctx *ctx, int64_t polls) {
+    if (!ctx) return FS_ERR_ARG;
+    ctx->loop_polls = polls;
+    ctx->loop_gave_up = false;
     return FS_OK;
 }
 

@@ -2547,6 +2547,195 @@ __device__ __forceinline__ double mx_value(float hi, short lo) { return (double)
 // second, 22.8, 22.7, 22.0, 25.7, 23.9 on the batch, where large patches leave
 // a half-empty last round of workgroups.
 
+// Plan of the patch form, from the nodes of each patch (the host's cuts): four
+// small kernels, a workgroup per patch, the scan one workgroup.  (On the host,
+// with 16 threads, the same lists took 1.3 ms of a plan of 3.2 ms for 12,221
+// nodes, and as much again to create the threads.)
+
+// Nodes of a patch by their numbers: pnode and slot.
+__global__ __launch_bounds__(64) void patch_rank_kernel(const int32_t *__restrict__ order,
+                                                        const int32_t *__restrict__ pstart,
+                                                        int32_t *__restrict__ pnode, int32_t *__restrict__ slot) {
+    __shared__ int32_t id[PATCH_NODES];
+    const int p = blockIdx.x, t = threadIdx.x;
+    const int b = pstart[p], n = pstart[p + 1] - b;
+    if (t < n) id[t] = order[b + t];
+    __syncthreads();
+    if (t >= PATCH_NODES) return;
+    if (t < n) {
+        int rank = 0;
+        for (int j = 0; j < n; ++j) rank += id[j] < id[t];
+        pnode[p * PATCH_NODES + rank] = id[t];
+        slot[id[t]] = p * PATCH_NODES + rank;
+    } else {
+        pnode[p * PATCH_NODES + t] = -1;
+    }
+}
+
+// Neighbours of local node li that have a slot, itself left out: all, those in
+// the patch with a larger number, those of other patches.
+struct PatchDegree {
+    int all = 0, inner = 0, outer = 0;
+    __device__ __forceinline__ PatchDegree(int p, int li, int I, const int32_t *__restrict__ nbr_ptr,
+                                           const int32_t *__restrict__ nbr_node, const int32_t *__restrict__ slot) {
+        if (I < 0) return;
+        for (int k = nbr_ptr[I]; k < nbr_ptr[I + 1]; ++k) {
+            const int sj = slot[nbr_node[k]];
+            if (sj < 0 || nbr_node[k] == I) continue;
+            ++all;
+            if (sj / PATCH_NODES != p)
+                ++outer;
+            else if (sj - p * PATCH_NODES > li)
+                ++inner;
+        }
+    }
+};
+
+// Entries and partial slots of a patch: rec = {-, entries, inner entries, partial
+// slots}, nptr.
+__global__ __launch_bounds__(64) void patch_count_kernel(const int32_t *__restrict__ nbr_ptr,
+                                                         const int32_t *__restrict__ nbr_node,
+                                                         const int32_t *__restrict__ pnode,
+                                                         const int32_t *__restrict__ slot, int4 *__restrict__ rec,
+                                                         uint16_t *__restrict__ nptr) {
+    __shared__ int all[PATCH_NODES], in[PATCH_NODES], out[PATCH_NODES];
+    const int p = blockIdx.x, li = threadIdx.x;
+    if (li < PATCH_NODES) {
+        const PatchDegree d(p, li, pnode[p * PATCH_NODES + li], nbr_ptr, nbr_node, slot);
+        all[li] = d.all;
+        in[li] = d.inner;
+        out[li] = d.outer;
+    }
+    __syncthreads();
+    if (li > PATCH_NODES) return;
+    int before = 0, ni = 0, no = 0;
+    for (int j = 0; j < PATCH_NODES; ++j) {
+        if (j < li) before += all[j];
+        ni += in[j];
+        no += out[j];
+    }
+    nptr[p * (PATCH_NODES + 1) + li] = (uint16_t)before;
+    if (li == PATCH_NODES) rec[p] = make_int4(0, ni + no, ni, before);
+}
+
+// First block of each patch (multiples of 8), and in tot: blocks, partial slots
+// of the largest patch, reach of the entries past PATCH_WG, 1.
+__global__ __launch_bounds__(1024) void patch_scan_kernel(int np, int4 *__restrict__ rec, int64_t *__restrict__ tot) {
+    __shared__ int64_t sum[1024];
+    __shared__ int slots;
+    __shared__ unsigned long long reach;
+    const int t = threadIdx.x;
+    if (t == 0) {
+        slots = 0;
+        reach = 0;
+    }
+    int64_t base = 0;
+    for (int p0 = 0; p0 < np; p0 += 1024) {
+        const int p = p0 + t;
+        const int4 r = p < np ? rec[p] : make_int4(0, 0, 0, 0);
+        const int64_t len = (r.y + 7) & ~7;
+        sum[t] = len;
+        __syncthreads();
+        for (int w = 1; w < 1024; w <<= 1) {
+            const int64_t v = t >= w ? sum[t - w] : 0;
+            __syncthreads();
+            sum[t] += v;
+            __syncthreads();
+        }
+        const int64_t first = base + sum[t] - len;
+        if (p < np) {
+            rec[p].x = (int)first;
+            atomicMax(&slots, r.w);
+            if (r.y > PATCH_WG) atomicMax(&reach, (unsigned long long)(first + r.y));
+        }
+        base += sum[1023];
+        __syncthreads();
+    }
+    if (t == 0) {
+        tot[0] = base;
+        tot[1] = slots;
+        tot[2] = (int64_t)reach;
+        tot[3] = 1;
+    }
+}
+
+// Entry lists, and with hpos the halos (tot[3] = 0 where one is too large for the
+// one-launch loop).  Entries are in the order of their nodes and of the nodes'
+// lists, a halo in the order of its slots.
+__global__ __launch_bounds__(PATCH_WG) void patch_fill_kernel(const int32_t *__restrict__ nbr_ptr,
+                                                              const int32_t *__restrict__ nbr_node,
+                                                              const int32_t *__restrict__ pnode,
+                                                              const int32_t *__restrict__ slot,
+                                                              const int4 *__restrict__ rec,
+                                                              const uint16_t *__restrict__ nptr, int64_t over,
+                                                              uint2 *__restrict__ ent, int32_t *__restrict__ entk,
+                                                              int32_t *__restrict__ hpos, int64_t *__restrict__ tot) {
+    __shared__ int in[PATCH_NODES], out[PATCH_NODES], far[PATCH_WG], uniq[PATCH_WG], count;
+    const int p = blockIdx.x, t = threadIdx.x;
+    const int4 r = rec[p];
+    const int ne = r.y, ni = r.z, no = ne - ni;
+    const int I = t < PATCH_NODES ? pnode[p * PATCH_NODES + t] : -1;
+    if (t == 0) count = 0;
+    if (t < PATCH_NODES) {
+        const PatchDegree d(p, t, I, nbr_ptr, nbr_node, slot);
+        in[t] = d.inner;
+        out[t] = d.outer;
+    }
+    if (t >= ne) {  // lanes without an entry
+        ent[(int64_t)p * PATCH_WG + t] = make_uint2(0, 0);
+        entk[(int64_t)p * PATCH_WG + t] = 0;
+    }
+    __syncthreads();
+    if (I >= 0) {
+        int ei = 0, eo = ni, sl = nptr[p * (PATCH_NODES + 1) + t];
+        for (int j = 0; j < t; ++j) {
+            ei += in[j];
+            eo += out[j];
+        }
+        for (int k = nbr_ptr[I]; k < nbr_ptr[I + 1]; ++k) {
+            const int J = nbr_node[k], sj = slot[J];
+            if (sj < 0 || J == I) continue;
+            const int lj = sj - p * PATCH_NODES;
+            const bool inner = sj / PATCH_NODES == p;
+            if (!inner || lj > t) {
+                const int e = inner ? ei++ : eo++;
+                unsigned back = 0xffffu;
+                if (inner) {  // place of I among J's neighbours
+                    back = nptr[p * (PATCH_NODES + 1) + lj];
+                    for (int m = nbr_ptr[J]; m < nbr_ptr[J + 1] && nbr_node[m] != I; ++m)
+                        back += nbr_node[m] != J && slot[nbr_node[m]] >= 0;
+                } else if (e - ni < PATCH_WG) {
+                    far[e - ni] = sj;
+                }
+                const int64_t at = e < PATCH_WG ? (int64_t)p * PATCH_WG + e : over + r.x + e;
+                ent[at] = make_uint2((unsigned)t << 26 | (unsigned)sj, (unsigned)sl | back << 16);
+                entk[at] = k;
+            }
+            ++sl;
+        }
+    }
+    if (!hpos) return;
+    __syncthreads();
+    // one-launch loop: the outer entries' nodes, each once
+    bool first = t < no && ne <= PATCH_WG;
+    const int mine = first ? far[t] : 0;
+    for (int j = 0; first && j < t; ++j) first = far[j] != mine;
+    if (t < no) uniq[t] = first;
+    if (first) atomicAdd(&count, 1);
+    __syncthreads();
+    if (ne > PATCH_WG || 6 * count > PATCH_HALO) {
+        if (t == 0) tot[3] = 0;
+        return;
+    }
+    int32_t *to = hpos + (int64_t)p * PATCH_HALO;
+    for (int i = 6 * count + t; i < PATCH_HALO; i += PATCH_WG) to[i] = -1;
+    if (first) {
+        int rank = 0;
+        for (int j = 0; j < no; ++j) rank += uniq[j] && far[j] < mine;
+        for (int c = 0; c < 6; ++c) to[6 * rank + c] = 6 * mine + c;
+    }
+}
+
 // Positions to dofs: map[q] = dof of position q, or past every free dof.
 __global__ __launch_bounds__(256) void patch_map_kernel(int64_t nv, const int32_t *__restrict__ pnode,
                                                         const int64_t *__restrict__ node_dof,
@@ -2672,16 +2861,18 @@ __global__ __launch_bounds__(256) void patch_build_kernel(PatchOp op, PatchSourc
 }
 
 // W_0 = V_0 + dt/2 A_0 with A_0 = invMC g_0 Fmag (in place of V_0), and
-// U_1 = U_0 + dt W_0.
+// U_1 = U_0 + dt W_0; pub is cleared for the one-launch loop.
 __global__ __launch_bounds__(256) void patch_init_kernel(int64_t nv, double dt, double g0,
                                                          const double *__restrict__ invMC,
                                                          const double *__restrict__ Fmag,
                                                          const double *__restrict__ U0, double *__restrict__ W,
                                                          double *__restrict__ U1, const int32_t *__restrict__ row_group,
                                                          const double *__restrict__ group_dt,
-                                                         const double *__restrict__ gtab) {
+                                                         const double *__restrict__ gtab,
+                                                         ulonglong2 *__restrict__ pub) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= nv) return;
+    if (pub) pub[q] = pub[nv + q] = make_ulonglong2(0, 0);  // no step published yet
     if (row_group) {
         const int gi = row_group[q];
         dt = group_dt[gi];
@@ -2726,6 +2917,76 @@ struct PatchBlock<true> {
     }
 };
 
+// The patch's diagonal blocks on their way from memory to LDS.
+struct PatchDiag {
+    static constexpr int ND = PATCH_TRI * PATCH_NODES, NL = (ND + PATCH_WG - 1) / PATCH_WG;
+    double v[NL];
+    __device__ __forceinline__ void load(const PatchOp &op, int p) {
+        const double *dgp = op.dg + (int64_t)p * ND;
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const int t = (int)threadIdx.x + i * PATCH_WG;
+            v[i] = t < ND ? dgp[t] : 0.0;
+        }
+    }
+    __device__ __forceinline__ void store(double *dg) const {
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            const int t = (int)threadIdx.x + i * PATCH_WG;
+            if (t < ND) dg[t] = v[i];
+        }
+    }
+};
+
+// Products of the lane's entry: K_IJ x_J, and K_IJ' x_I if J is in the patch.
+template <bool F32>
+__device__ __forceinline__ void patch_products(const PatchBlock<F32> &kb, uint2 en, const double2 xj[3],
+                                               const double *xs, double *part) {
+    const double xa[6] = {xj[0].x, xj[0].y, xj[1].x, xj[1].y, xj[2].x, xj[2].y};
+    const double *xi = xs + 6 * (en.x >> 26);
+    double *pi = part + 6 * (en.y & 0xffff);
+    double y[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int rr = 0; rr < 6; ++rr) {
+        const double xr = xi[rr];
+        double f = 0.0;
+#pragma unroll
+        for (int c = 0; c < 6; ++c) {
+            const double v = kb.at(6 * rr + c);
+            f += v * xa[c];
+            y[c] += v * xr;
+        }
+        pi[rr] = f;
+    }
+    if ((en.y >> 16) != 0xffffu) {
+        double *pj = part + 6 * (en.y >> 16);
+        for (int c = 0; c < 6; ++c) pj[c] = y[c];
+    }
+}
+
+// Row r of local node li: its diagonal block, then the products in the order of
+// the node's neighbour list.
+__device__ __forceinline__ double patch_row(const double *xs, const double *dg, const double *part, int li, int r,
+                                            int s0, int s1) {
+    const double *xi = xs + 6 * li, *di = dg + PATCH_TRI * li;
+    double f = 0.0;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
+        const int a = min(r, c), b = max(r, c);
+        f += di[a * (11 - a) / 2 + b] * xi[c];
+    }
+    for (int s = s0; s < s1; ++s) f += part[6 * s + r];
+    return f;
+}
+
+// Acceleration of a row: f its row of K U, w its half-step velocity.
+__device__ __forceinline__ double patch_accel(double f, double im, double w, bool forced, double gstep, double fm,
+                                              bool damped, double cd) {
+    f = forced ? gstep * fm - f : -f;
+    if (damped) f -= cd * w;
+    return im * f;
+}
+
 template <bool F32>
 __global__ __launch_bounds__(PATCH_WG) __attribute__((amdgpu_waves_per_eu(3))) void cd_patch_step_kernel(
     PatchOp op, const double *__restrict__ Ucur, double *__restrict__ Unext, double *__restrict__ W,
@@ -2744,12 +3005,8 @@ __global__ __launch_bounds__(PATCH_WG) __attribute__((amdgpu_waves_per_eu(3))) v
     uint2 en = op.ent[q];  // the lane's first entry
     const int4 rec = op.rec[p];
     const int ne = rec.y, nep = (ne + 7) & ~7;
-    const double *dgp = op.dg + (int64_t)p * (PATCH_TRI * PATCH_NODES);
-    constexpr int ND = PATCH_TRI * PATCH_NODES;
-    double dv[(ND + PATCH_WG - 1) / PATCH_WG];
-#pragma unroll
-    for (int i = 0; i < (ND + PATCH_WG - 1) / PATCH_WG; ++i)
-        dv[i] = tid + i * PATCH_WG < ND ? dgp[tid + i * PATCH_WG] : 0.0;
+    PatchDiag pd;
+    pd.load(op, p);
     const int li = tid / 6, r = tid % 6;
     const uint16_t *np = op.nptr + p * (PATCH_NODES + 1) + li;
     const int s0 = np[0], s1 = np[1];
@@ -2759,40 +3016,19 @@ __global__ __launch_bounds__(PATCH_WG) __attribute__((amdgpu_waves_per_eu(3))) v
     const double w = W[q], im = invMC[q];
     const int gi = row_group ? row_group[q] : 0;
     xs[tid] = u;
-#pragma unroll
-    for (int i = 0; i < (ND + PATCH_WG - 1) / PATCH_WG; ++i)
-        if (tid + i * PATCH_WG < ND) dg[tid + i * PATCH_WG] = dv[i];
+    pd.store(dg);
     __syncthreads();
     while (e < ne) {
-        const bool inner = (en.y >> 16) != 0xffffu;
         const int64_t sj = en.x & 0x3ffffff;
         double2 xj[3];
-        const double2 *x2 = inner ? reinterpret_cast<const double2 *>(xs + 6 * (int)(sj - (int64_t)p * PATCH_NODES))
-                                  : reinterpret_cast<const double2 *>(Ucur + 6 * sj);
-        if (inner) {
+        if ((en.y >> 16) != 0xffffu) {
+            const double2 *x2 = reinterpret_cast<const double2 *>(xs + 6 * (int)(sj - (int64_t)p * PATCH_NODES));
             for (int c = 0; c < 3; ++c) xj[c] = x2[c];
-        } else {
+        } else {  // a node of another patch
+            const double2 *x2 = reinterpret_cast<const double2 *>(Ucur + 6 * sj);
             for (int c = 0; c < 3; ++c) xj[c] = x2[c];
         }
-        double *pi = part + 6 * (en.y & 0xffff);
-        const double xa[6] = {xj[0].x, xj[0].y, xj[1].x, xj[1].y, xj[2].x, xj[2].y};
-        const double *xi = xs + 6 * (en.x >> 26);
-        double *pj = part + 6 * (en.y >> 16);
-        double y[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int rr = 0; rr < 6; ++rr) {
-            const double xr = xi[rr];
-            double f = 0.0;
-#pragma unroll
-            for (int c = 0; c < 6; ++c) {
-                const double v = kb.at(6 * rr + c);
-                f += v * xa[c];
-                y[c] += v * xr;
-            }
-            pi[rr] = f;
-        }
-        if (inner)
-            for (int c = 0; c < 6; ++c) pj[c] = y[c];
+        patch_products(kb, en, xj, xs, part);
         e += PATCH_WG;
         if (e < ne) {
             en = op.ent[op.over + rec.x + e];
@@ -2800,23 +3036,12 @@ __global__ __launch_bounds__(PATCH_WG) __attribute__((amdgpu_waves_per_eu(3))) v
         }
     }
     __syncthreads();
-    double f = 0.0;
-    {
-        const double *xi = xs + 6 * li, *di = dg + PATCH_TRI * li;
-#pragma unroll
-        for (int c = 0; c < 6; ++c) {
-            const int a = min(r, c), b = max(r, c);
-            f += di[a * (11 - a) / 2 + b] * xi[c];
-        }
-    }
-    for (int s = s0; s < s1; ++s) f += part[6 * s + r];
+    double f = patch_row(xs, dg, part, li, r, s0, s1);
     if (row_group) {  // batch: the row's model has its own dt and load history
         dt = group_dt[gi];
         gstep = gtab[gi];
     }
-    f = forced ? gstep * Fmag[q] - f : -f;
-    if (damped) f -= Cd[q] * w;
-    const double a = im * f;
+    const double a = patch_accel(f, im, w, forced, gstep, forced ? Fmag[q] : 0.0, damped, damped ? Cd[q] : 0.0);
     const double wn = w + dt * a;
     W[q] = last ? w + (dt / 2) * a : wn;
     Unext[q] = u + dt * wn;
@@ -2824,6 +3049,137 @@ __global__ __launch_bounds__(PATCH_WG) __attribute__((amdgpu_waves_per_eu(3))) v
         const int ps = probe_slot[q];
         if (ps >= 0) probe_dst[ps] = u;
     }
+}
+
+// The whole loop in one launch, for meshes whose patches all fit on the GPU at
+// once.  A step of such a mesh waits on latencies: 4.4 us for 32 x 32 or 97 x 61
+// elements, a kernel boundary and three dependent loads.  Here a workgroup
+// keeps its patch's blocks, state and factors in registers and LDS for all
+// steps, and takes from memory only the displacements of its halo.
+// A lane publishes its new U in two words, each half of the value with the
+// step's number in its low half, and a reader polls until both words carry the
+// step it is at: no flag, no fence, and nothing is read before it is whole.
+// Two sets of words in turn are enough: a patch overwrites the set of step n
+// with step n + 2 after it has read its neighbours' step n + 1, which they publish
+// after they have read step n.  The words are read and written as relaxed
+// atomics of device scope, past the caches that are not shared.
+// Every wait is bounded: a lane that has polled `polls` times, or sees that
+// another patch gave up, sets *stop, and its workgroup leaves; the host then
+// runs the loop step by step (the arithmetic is the same, statement by
+// statement, so the results are too).
+// Measured, us per step, step by step -> one launch: 80 nodes T3 3.6 -> 1.7,
+// 1,089 T3 4.3 -> 2.0, 6,076 Q4 4.3 -> 2.3, 12,221 Q4 5.2 -> 3.2, 21,009 Q4 7.7 ->
+// 3.9 (512 patches, the most that LoopPlaces lets run, two a CU; 146
+// registers allow three).
+template <bool F32>
+__global__ __launch_bounds__(PATCH_WG) __attribute__((amdgpu_waves_per_eu(2))) void cd_patch_loop_kernel(PatchLoop a) {
+    extern __shared__ double smem[];
+    constexpr int XS = PATCH_WG + PATCH_HALO;  // x of the patch's nodes and of its halo
+    constexpr int HN = PATCH_HALO / 6;         // halo nodes at most
+    double *dg = smem + 2 * XS;
+    double *part = dg + PATCH_TRI * PATCH_NODES;
+    __shared__ int leave;
+    __shared__ int hslot[HN], edge[PATCH_NODES];
+    const PatchOp &op = a.op;
+    const int p = (int)xcd_block(blockIdx.x, gridDim.x);
+    const int tid = threadIdx.x;
+    const int64_t q = (int64_t)p * PATCH_WG + tid, nv = (int64_t)op.npatch * PATCH_WG;
+    const int hq0 = op.hpos[2 * (int64_t)p * PATCH_WG + tid], hq1 = op.hpos[(2 * (int64_t)p + 1) * PATCH_WG + tid];
+    uint2 en = op.ent[q];
+    const int4 rec = op.rec[p];
+    const bool has = tid < rec.y, inner = (en.y >> 16) != 0xffffu;
+    PatchDiag pd;
+    pd.load(op, p);
+    PatchBlock<F32> kb;
+    if (has) kb.load(op, rec.x, (rec.y + 7) & ~7, tid);
+    const int li = tid / 6, r = tid % 6;
+    const uint16_t *np = op.nptr + p * (PATCH_NODES + 1) + li;
+    const int s0 = np[0], s1 = np[1];
+    const int gi = a.row_group ? a.row_group[q] : 0;
+    const double dt = a.row_group ? a.group_dt[gi] : a.dt;
+    double u = a.U1[q], w = a.W[q];
+    const double im = a.invMC[q], cd = a.damped ? a.Cd[q] : 0.0, fm = a.Fmag[q];
+    const int ps = a.probe_slot ? a.probe_slot[q] : -1;
+    if (tid == 0) leave = 0;
+    if (tid < PATCH_NODES) edge[tid] = 0;
+    if (r == 0) {
+        hslot[li] = hq0 >= 0 ? hq0 / 6 : -1;
+        hslot[PATCH_NODES + li] = hq1 >= 0 ? hq1 / 6 : -1;
+    }
+    pd.store(dg);
+    __syncthreads();
+    // x of the entry's J in LDS; nodes with an outer entry are some other patch's halo
+    int lj = 0;
+    if (has) {
+        const int sj = (int)(en.x & 0x3ffffff);
+        if (inner) {
+            lj = sj - p * PATCH_NODES;
+        } else {
+            edge[en.x >> 26] = 1;
+            while (lj < HN - 1 && hslot[lj] != sj) ++lj;  // the halo holds every outer entry's node
+            lj += PATCH_NODES;
+        }
+    }
+    __syncthreads();
+    const bool shared = edge[li] != 0;
+    auto publish = [&](uint32_t step) {
+        if (!shared) return;
+        const unsigned long long b = (unsigned long long)__double_as_longlong(u);
+        unsigned long long *to = a.pub + 2 * ((int64_t)(step & 1) * nv + q);
+        __hip_atomic_store(to, b << 32 | step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(to + 1, (b & 0xffffffff00000000ull) | step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    publish(1);
+    smem[XS + tid] = u;
+    double v = 0.0;
+    for (uint32_t n = 1; n <= (uint32_t)a.nsteps; ++n) {
+        double *xs = smem + (n & 1) * XS;
+        const bool forced = a.forced[n] != 0;
+        const double gstep = forced ? a.gtab[(int64_t)n * a.ng + gi] : 0.0;
+        if (hq0 >= 0) {
+            // a lane's second dof, where it has one, is polled with the first
+            unsigned long long *at = a.pub + 2 * (int64_t)(n & 1) * nv;
+            unsigned long long *f0 = at + 2 * (int64_t)hq0, *f1 = at + 2 * (int64_t)(hq1 >= 0 ? hq1 : hq0);
+            unsigned long long x0, x1, y0, y1;
+            for (uint32_t k = 1;; ++k) {
+                x0 = __hip_atomic_load(f0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                x1 = __hip_atomic_load(f0 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                y0 = __hip_atomic_load(f1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                y1 = __hip_atomic_load(f1 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if ((uint32_t)x0 == n && (uint32_t)x1 == n && (uint32_t)y0 == n && (uint32_t)y1 == n) break;
+                if (k >= a.polls ||
+                    ((k & 255) == 0 && __hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) != 0)) {
+                    __hip_atomic_store(a.stop, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    leave = 1;
+                    break;
+                }
+            }
+            xs[PATCH_WG + tid] = __longlong_as_double((long long)(x0 >> 32 | (x1 & 0xffffffff00000000ull)));
+            xs[2 * PATCH_WG + tid] = __longlong_as_double((long long)(y0 >> 32 | (y1 & 0xffffffff00000000ull)));
+        }
+        __syncthreads();
+        if (leave) return;  // set before the barrier only, so the same for all lanes
+        if (has) {
+            const double2 *x2 = reinterpret_cast<const double2 *>(xs + 6 * lj);
+            const double2 xj[3] = {x2[0], x2[1], x2[2]};
+            patch_products(kb, en, xj, xs, part);
+        }
+        __syncthreads();
+        const double f = patch_row(xs, dg, part, li, r, s0, s1);
+        const double acc = patch_accel(f, im, w, forced, gstep, fm, a.damped, cd);
+        const double wn = w + dt * acc;
+        if (ps >= 0 && n % (uint32_t)a.stride == 0) a.probe_dst[(int64_t)(n / (uint32_t)a.stride) * a.nprobes + ps] = u;
+        if (n == (uint32_t)a.nsteps) {
+            v = w + (dt / 2) * acc;
+            break;
+        }
+        w = wn;
+        u = u + dt * wn;
+        publish(n + 1);
+        smem[((n + 1) & 1) * XS + tid] = u;
+    }
+    a.U[q] = u;
+    a.W[q] = v;
 }
 
 // ---------------------------------------------------------------------------
@@ -3750,6 +4106,24 @@ hipError_t launch_coo_reduce(int64_t nnz, const int64_t *cptr, const int64_t *cl
     return hipGetLastError();
 }
 
+hipError_t launch_patch_count(int64_t np, const int32_t *order, const int32_t *pstart, const int32_t *nbr_ptr,
+                              const int32_t *nbr_node, int32_t *pnode, int32_t *slot, int4 *rec, uint16_t *nptr,
+                              int64_t *tot, hipStream_t st) {
+    const dim3 grid((unsigned)np);
+    hipLaunchKernelGGL(patch_rank_kernel, grid, dim3(64), 0, st, order, pstart, pnode, slot);
+    hipLaunchKernelGGL(patch_count_kernel, grid, dim3(64), 0, st, nbr_ptr, nbr_node, pnode, slot, rec, nptr);
+    hipLaunchKernelGGL(patch_scan_kernel, dim3(1), dim3(1024), 0, st, (int)np, rec, tot);
+    return hipGetLastError();
+}
+
+hipError_t launch_patch_fill(int64_t np, const int32_t *nbr_ptr, const int32_t *nbr_node, const int32_t *pnode,
+                             const int32_t *slot, const int4 *rec, const uint16_t *nptr, int64_t over, uint2 *ent,
+                             int32_t *entk, int32_t *hpos, int64_t *tot, hipStream_t st) {
+    hipLaunchKernelGGL(patch_fill_kernel, dim3((unsigned)np), dim3(PATCH_WG), 0, st, nbr_ptr, nbr_node, pnode, slot, rec,
+                       nptr, over, ent, entk, hpos, tot);
+    return hipGetLastError();
+}
+
 hipError_t launch_patch_map(const PatchOp &op, const int64_t *node_dof, int64_t *map, hipStream_t st) {
     if (op.npatch == 0) return hipSuccess;
     const int64_t nv = (int64_t)op.npatch * PATCH_WG;
@@ -3782,11 +4156,11 @@ hipError_t launch_patch_build(const PatchOp &op, int kind, const ScatterPlan &sp
 
 hipError_t launch_patch_init(const PatchOp &op, double dt, double g0, const double *invMC, const double *Fmag,
                              const double *U0, double *W, double *U1, const int32_t *row_group,
-                             const double *group_dt, const double *gtab, hipStream_t st) {
+                             const double *group_dt, const double *gtab, unsigned long long *pub, hipStream_t st) {
     if (op.npatch == 0) return hipSuccess;
     const int64_t nv = (int64_t)op.npatch * PATCH_WG;
     hipLaunchKernelGGL(patch_init_kernel, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, st, nv, dt, g0, invMC, Fmag,
-                       U0, W, U1, row_group, group_dt, gtab);
+                       U0, W, U1, row_group, group_dt, gtab, reinterpret_cast<ulonglong2 *>(pub));
     return hipGetLastError();
 }
 
@@ -3807,6 +4181,28 @@ hipError_t launch_cd_patch_step(const PatchOp &op, int f32, const double *Ucur, 
     else
         hipLaunchKernelGGL(cd_patch_step_kernel<false>, grid, wg, smem, st, op, Ucur, Unext, W, invMC, Cd, Fmag, gstep, dt,
                            damped, forced, last, probe_slot, probe_dst, row_group, group_dt, gtab);
+    return hipGetLastError();
+}
+
+static size_t patch_loop_smem(const PatchOp &op) {
+    return sizeof(double) * (size_t)(2 * (PATCH_WG + PATCH_HALO) + PATCH_TRI * PATCH_NODES + 6 * op.slots);
+}
+
+// Workgroups of the one-launch loop that a CU holds at once.
+hipError_t patch_loop_occupancy(const PatchOp &op, int f32, int *per_cu) {
+    return f32 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, cd_patch_loop_kernel<true>, PATCH_WG,
+                                                              patch_loop_smem(op))
+               : hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, cd_patch_loop_kernel<false>, PATCH_WG,
+                                                              patch_loop_smem(op));
+}
+
+hipError_t launch_cd_patch_loop(const PatchLoop &a, int f32, hipStream_t st) {
+    if (a.op.npatch == 0) return hipSuccess;
+    const dim3 grid((unsigned)a.op.npatch), wg(PATCH_WG);
+    if (f32)
+        hipLaunchKernelGGL(cd_patch_loop_kernel<true>, grid, wg, patch_loop_smem(a.op), st, a);
+    else
+        hipLaunchKernelGGL(cd_patch_loop_kernel<false>, grid, wg, patch_loop_smem(a.op), st, a);
     return hipGetLastError();
 }
 

@@ -125,6 +125,7 @@ SIGNATURES = {
     "fs_ctx_set_pipeline": (C.c_int, [C.c_void_p, C.c_int]),
     "fs_ctx_set_assembly": (C.c_int, [C.c_void_p, C.c_int]),
     "fs_ctx_set_cd_lanes": (C.c_int, [C.c_void_p, C.c_int, C.c_int]),
+    "fs_ctx_set_cd_loop": (C.c_int, [C.c_void_p, C.c_int64]),
     "fs_coo_create": (C.c_int, [C.c_void_p, C.c_int64, C.c_int64, C.c_int32, C.c_int32, C.c_int64, _i64p, _i64p,
                                 C.c_int, C.POINTER(C.c_void_p)]),
     "fs_coo_pattern": (C.c_int, [C.c_void_p, _i64p]),
@@ -212,6 +213,11 @@ class Context:
         the longest row)."""
         self.check(self.lib.fs_ctx_set_cd_lanes(self.h, int(lanes_per_node), int(positions_per_lane)),
                    "fs_ctx_set_cd_lanes")
+
+    def set_cd_loop(self, polls=0):
+        """Explicit loops of small meshes in one launch: longest wait of a lane
+        in polls (0: the default), negative: always step by step."""
+        self.check(self.lib.fs_ctx_set_cd_loop(self.h, int(polls)), "fs_ctx_set_cd_loop")
 
     def close(self):
         if self.h:

@@ -459,6 +459,15 @@ int fs_ctx_set_assembly(fs_ctx *ctx, int mode);
  * node patches (each block read once per patch), which the model keeps. */
 int fs_ctx_set_cd_lanes(fs_ctx *ctx, int lanes_per_node, int positions_per_lane);
 
+/* Explicit loops of 100 steps or more on small meshes (no counterpart in the
+ * reference) run in one launch whose workgroups wait for one another's
+ * displacements, where there is room for all of them on the device, else
+ * step by step with bitwise the same results.  polls: the longest wait of a
+ * lane in polls (at most 2^21, about two seconds; 0 = that default), after
+ * which the call starts again step by step, as do later calls on the context;
+ * negative: always step by step. */
+int fs_ctx_set_cd_loop(fs_ctx *ctx, int64_t polls);
+
 /* Storage of the mixed-precision operator built by the last FS_PREC_MIXED /
  * FS_PREC_MIXED_F32 loop (no counterpart in the reference, whose loop runs on
  * the FP64 CSR matrix only): info[0] FP32 value pairs of the slices

@@ -10,6 +10,8 @@ plan: one node with free dofs, one and two patches (42 and 43 nodes), a hub
 whose patch has more blocks than the workgroup has lanes, a hub of more
 neighbours than a patch takes (row products throughout), two components,
 partly fixed nodes, a permuted numbering."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -69,6 +71,73 @@ MESHES = {
     "hub_1100": lambda: _fan(1100),
     "two": _two,
 }
+
+
+@pytest.mark.parametrize("nen,nx,ny", [(4, 3, 2), (3, 9, 7), (4, 97, 61), (3, 140, 70)],
+                         ids=["one_patch", "t3", "q4_146_patches", "t3_245_patches"])
+@pytest.mark.parametrize("prec", [_lib.FS_PREC_FP64, _lib.FS_PREC_MIXED_F32], ids=["fp64", "f32"])
+def test_loop_in_one_launch(ctx, nen, nx, ny, prec):
+    """The one-launch loop gives bitwise what the same steps give one by one,
+    in a graph too, with odd and even step counts, and where its waits run out
+    (a limit of one poll), in which case the call runs step by step."""
+    print(f"[gpu] loop in one launch {nen} {nx}x{ny} precision {prec}", flush=True)
+    _, xyz, conn, d = _grid(nen, nx, ny, "partial")
+    f = FM.make(conn, MatDeforElastIso(70e9, 0.33, 2700.0), thickness=0.02, ctx=ctx)
+    f.associategeometry(xyz)
+    nf = d.nfreedofs
+    f.stiffness(FM.SysmatAssemblerHIP(), xyz, None, None, d)
+    f.mass(FM.SysmatAssemblerHIP(), xyz, d)
+    rng = np.random.default_rng(3)
+    dt = 0.8 * explicit.stable_dt(explicit.omega_max(f, rng.standard_normal(nf), 200))
+    U0, V0, F = rng.normal(0, 1e-6, nf), rng.normal(0, 1e-3, nf), rng.normal(0, 1.0, nf)
+    probes = rng.choice(nf, 5, replace=False)
+
+    def run(polls, nsteps, cdamp, graph=False):
+        ctx.set_cd_loop(polls)
+        try:
+            g = np.where(np.arange(nsteps + 1) % 50 < 20, np.cos(0.1 * np.arange(nsteps + 1)), 0.0)
+            return explicit.run(f._model, cdamp, U0, V0, dt, nsteps, F, g, probes, 7, prec, use_graph=graph)
+        finally:
+            ctx.set_cd_loop(0)
+
+    for nsteps, cdamp in ((100, 0.0), (301, 40.0)):
+        ref = run(-1, nsteps, cdamp)
+        for polls, graph in ((0, False), (0, True), (0, True), (1, False), (0, False)):
+            r = run(polls, nsteps, cdamp, graph)
+            for key in ("U", "V", "probes"):
+                assert np.array_equal(r[key], ref[key]), (nsteps, polls, graph, key)
+    f._model.close()
+
+
+def test_loops_at_the_same_time(ctx):
+    """Contexts whose loops together have more patches than the device has
+    places for: some run step by step meanwhile, all give what they give alone."""
+    print("[gpu] loops of four contexts", flush=True)
+    jobs = []
+    for k in range(4):
+        c = _lib.Context(ctx.device)
+        _, xyz, conn, d = _grid(3, 140, 70 - k)
+        f = FM.make(conn, MatDeforElastIso(70e9, 0.33, 2700.0), thickness=0.02, ctx=c)
+        f.associategeometry(xyz)
+        f.stiffness(FM.SysmatAssemblerHIP(), xyz, None, None, d)
+        f.mass(FM.SysmatAssemblerHIP(), xyz, d)
+        nf = d.nfreedofs
+        dt = 0.8 * explicit.stable_dt(explicit.omega_max(f, np.random.default_rng(k).standard_normal(nf), 200))
+        V0, z = np.random.default_rng(k).normal(0, 1e-3, nf), np.zeros(nf)
+        jobs.append((f, lambda m=f._model, z=z, V0=V0, dt=dt: explicit.run(m, 0.0, z, V0, dt, 2000, z, np.zeros(2001))))
+    alone = [run() for _, run in jobs]
+    got = [[] for _ in jobs]
+    threads = [threading.Thread(target=lambda k=k: got[k].extend(jobs[k][1]() for _ in range(5))) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for a, rs in zip(alone, got):
+        assert len(rs) == 5
+        for r in rs:
+            assert np.array_equal(a["U"], r["U"]) and np.array_equal(a["V"], r["V"])
+    for f, _ in jobs:
+        f._model.close()
 
 
 @pytest.mark.parametrize("name", list(MESHES))
