@@ -258,9 +258,11 @@ struct PatchOp {
     double *dg;
 };
 
-// One launch of the whole loop on the patch form (cd_patch_loop_kernel).
+// One launch of the whole loop on the patches first .. first + count - 1, whole
+// components (cd_patch_loop_kernel).
 struct PatchLoop {
     PatchOp op;
+    int32_t first, count;
     const double *U1;            // U of the first step, in slot positions
     double *U;                   // out: U of the last step
     double *W;                   // half-step velocity in, V of the last step out

@@ -249,6 +249,9 @@ struct PatchStore {
     int64_t npatch = 0, nent = 0;
     int slots = 0;
     bool loops = false;        // the one-launch loop takes the plan (hpos is there)
+    // its launches: bounds of sets of whole components, and the largest set
+    std::vector<int32_t> sets;
+    int32_t largest_set = 0;
     int loop_per_cu[2] = {0, 0};  // its workgroups per CU, FP64 and F32 (0: not asked yet)
     // what it is filled with (FS_PREC_*, -1 nothing) and the generations of the
     // values (Block::vgen, MixedStore::kgen) that came from
@@ -260,6 +263,8 @@ struct PatchStore {
         npatch = nent = 0;
         slots = 0;
         loops = false;
+        sets.clear();
+        largest_set = 0;
         loop_per_cu[0] = loop_per_cu[1] = 0;
         kind = -1;
         for (DevBuf *b : {&rec, &ent, &entk, &hpos, &dpnode, &nptr, &map, &k2, &kh, &kl, &dg}) b->release();
@@ -975,7 +980,8 @@ fs::PatchOp patchop_of(const PatchStore &P) {
     return op;
 }
 
-// Patches from which the one-launch loop is not tried: two a CU of 256 CUs.
+// Patches of one launch of the one-launch loop at most, so of one component too:
+// two a CU of 256 CUs.
 constexpr int64_t PATCH_LOOP_MAX = 512;
 
 // Partial slots a patch may have: 6 doubles each in LDS (48 KB), so that two
@@ -1031,7 +1037,7 @@ int build_patches(fs_model *m) {
                     if (__atomic_compare_exchange_n(&par[a], &want, b, false, __ATOMIC_RELAXED, __ATOMIC_RELAXED)) break;
                 }
             }
-    }, 65536);
+    }, 262144);
     // active nodes by component (components by their smallest node), in node
     // order within one; a mesh of one component is laid out in parallel
     struct Pt {
@@ -1140,8 +1146,19 @@ int build_patches(fs_model *m) {
     if (np * PN >= (int64_t(1) << 26) || npt >= INT32_MAX) return FS_OK;  // slots are 26-bit numbers
     HostArray<int32_t> order = host_array<int32_t>(npt);
     for (int64_t i = 0; i < npt; ++i) order[i] = pt[i].id;
-    // the lists on the device; halos for the one-launch loop where it may take
-    // so many patches
+    // sets of consecutive components for the one-launch loop (a component begins
+    // a patch, and is a set of its own unless it fits the current one)
+    P.sets.assign(1, 0);
+    bool halos = true;
+    for (int64_t k = 0; k < nc && halos; ++k) {
+        auto patch_at = [&](int64_t i) { return (int32_t)(std::lower_bound(pstart.begin(), pstart.end(), (int32_t)i) - pstart.begin()); };
+        const int32_t b = patch_at(cptr[k]), e = patch_at(cptr[k + 1]);
+        halos = e - b <= PATCH_LOOP_MAX;
+        if (e - P.sets.back() > PATCH_LOOP_MAX) P.sets.push_back(b);
+    }
+    P.sets.push_back((int32_t)np);
+    for (size_t k = 0; k + 1 < P.sets.size(); ++k) P.largest_set = std::max(P.largest_set, P.sets[k + 1] - P.sets[k]);
+    // the lists on the device
     int s;
     DevBuf dorder, dstart, dslot, dtot;
     const int32_t *nbp = B.nbr_ptr.as<int32_t>(), *nbn = B.nbr_node.as<int32_t>();
@@ -1157,7 +1174,6 @@ int build_patches(fs_model *m) {
     if ((s = d2h(c, tot, dtot.p, 32))) return s;
     const int64_t nent = tot[0], over = np * fs::PATCH_WG, ntab = over + tot[2];
     if (nent >= (int64_t(1) << 30)) return FS_OK;
-    const bool halos = np <= PATCH_LOOP_MAX;
     if ((s = dalloc(c, P.ent, (size_t)ntab * 8)) || (s = dalloc(c, P.entk, (size_t)ntab * 4)) ||
         (halos && (s = dalloc(c, P.hpos, (size_t)np * fs::PATCH_HALO * 4))) ||
         (s = dalloc(c, P.map, (size_t)np * PN * 6 * 8)) || (s = dalloc(c, P.dg, (size_t)np * PN * fs::PATCH_TRI * 8)))
@@ -2651,7 +2667,7 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
     if (patch && p->nsteps < INT32_MAX && (s = patch_loops(m, p->precision, &loop))) return s;
     const bool loop_form = loop;
     LoopPlaces places;
-    if (loop) loop = places.take(c->device, P.npatch);
+    if (loop) loop = places.take(c->device, P.largest_set);
     // State vectors: the free dofs themselves (row products), node-major dof
     // positions 6 i + c (mixed path), or the patches' slot positions; fixed
     // dofs stay zero in the last two.
@@ -2760,7 +2776,12 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
             lp.stride = stride;
             lp.nprobes = nprobes;
             lp.polls = c->loop_polls > 0 ? (uint32_t)std::min<int64_t>(c->loop_polls, LOOP_POLLS) : LOOP_POLLS;
-            return fs::launch_cd_patch_loop(lp, p->precision == FS_PREC_MIXED_F32, st);
+            for (size_t k = 0; k + 1 < P.sets.size() && e == hipSuccess; ++k) {
+                lp.first = P.sets[k];
+                lp.count = P.sets[k + 1] - P.sets[k];
+                e = fs::launch_cd_patch_loop(lp, p->precision == FS_PREC_MIXED_F32, st);
+            }
+            return e;
         }
         int cur = 1;
         for (int64_t step = 1; step <= p->nsteps; ++step) {

@@ -3051,11 +3051,13 @@ __global__ __launch_bounds__(PATCH_WG) __attribute__((amdgpu_waves_per_eu(3))) v
     }
 }
 
-// The whole loop in one launch, for meshes whose patches all fit on the GPU at
-// once.  A step of such a mesh waits on latencies: 4.4 us for 32 x 32 or 97 x 61
-// elements, a kernel boundary and three dependent loads.  Here a workgroup
-// keeps its patch's blocks, state and factors in registers and LDS for all
-// steps, and takes from memory only the displacements of its halo.
+// The whole loop in one launch, for patches that all fit on the GPU at once: a
+// small mesh, or as many whole components of a batch.  A step of a small mesh
+// waits on latencies: 4.4 us for 32 x 32 or 97 x 61 elements, a kernel boundary
+// and three dependent loads.  Here a workgroup keeps its patch's blocks, state
+// and factors in registers and LDS for all steps, and takes from memory only
+// the displacements of its halo.  Components do not wait for one another, so a
+// batch runs all steps of one set of components before the next set.
 // A lane publishes its new U in two words, each half of the value with the
 // step's number in its low half, and a reader polls until both words carry the
 // step it is at: no flag, no fence, and nothing is read before it is whole.
@@ -3081,7 +3083,7 @@ __global__ __launch_bounds__(PATCH_WG) __attribute__((amdgpu_waves_per_eu(2))) v
     __shared__ int leave;
     __shared__ int hslot[HN], edge[PATCH_NODES];
     const PatchOp &op = a.op;
-    const int p = (int)xcd_block(blockIdx.x, gridDim.x);
+    const int p = a.first + (int)xcd_block(blockIdx.x, gridDim.x);
     const int tid = threadIdx.x;
     const int64_t q = (int64_t)p * PATCH_WG + tid, nv = (int64_t)op.npatch * PATCH_WG;
     const int hq0 = op.hpos[2 * (int64_t)p * PATCH_WG + tid], hq1 = op.hpos[(2 * (int64_t)p + 1) * PATCH_WG + tid];
@@ -4197,8 +4199,8 @@ hipError_t patch_loop_occupancy(const PatchOp &op, int f32, int *per_cu) {
 }
 
 hipError_t launch_cd_patch_loop(const PatchLoop &a, int f32, hipStream_t st) {
-    if (a.op.npatch == 0) return hipSuccess;
-    const dim3 grid((unsigned)a.op.npatch), wg(PATCH_WG);
+    if (a.count == 0) return hipSuccess;
+    const dim3 grid((unsigned)a.count), wg(PATCH_WG);
     if (f32)
         hipLaunchKernelGGL(cd_patch_loop_kernel<true>, grid, wg, patch_loop_smem(a.op), st, a);
     else
