@@ -24,6 +24,7 @@
 #include <cstring>
 #include <new>
 #include <string>
+#include <system_error>
 #include <thread>
 #include <type_traits>
 #include <vector>
@@ -38,6 +39,8 @@ hipError_t launch_element_blocks(const ElemParams &p, const double *x, const dou
 int element_variants(int nen);
 void element_variant_shape(int nen, int variant, int *ne, int *wg);
 hipError_t launch_scatter(const ScatterPlan &sp, const double *Kb, double *vals, hipStream_t st);
+hipError_t launch_pattern_cols(const ScatterPlan &sp, const int64_t *node_dof, int base, int64_t w0, int64_t w1,
+                               int64_t *col, hipStream_t st);
 int fused_tile_elems(int nen);
 hipError_t launch_element_fused(const ElemParams &p, const double *x, const double *y, const double *z,
                                 const int32_t *conn, const double *nx, const double *ny, const double *nz,
@@ -145,6 +148,9 @@ struct BufCache {
 };
 }  // namespace
 
+// Slots and threads of a device-to-host copy (d2h).
+constexpr int STAGE_SLOTS = 16, STAGE_THREADS = 8;
+
 struct fs_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -165,10 +171,11 @@ struct fs_ctx {
     hipStream_t stream2 = nullptr;
     int asm_chunks = 1;
     std::vector<hipEvent_t> ev;  // ordering events of the pipeline (no timing)
-    // pinned staging buffers of the large device-to-host copies (allocated
-    // on first use, FS_STAGE_BYTES each) and their completion events
-    void *stage[2] = {nullptr, nullptr};
-    hipEvent_t stage_ev[2] = {nullptr, nullptr};
+    // pinned staging slots of the device-to-host copies (64 MB at most, grown
+    // by the copies that use them) and their completion events
+    char *stage = nullptr;
+    size_t stage_bytes = 0;
+    hipEvent_t stage_ev[STAGE_SLOTS] = {};
     // row products of the FP64 explicit step: 0 = lanes per row
     // (cd_step_kernel), 8/16 = lanes per node (cd_node_step_kernel) with
     // cd_pj positions per lane (0: from the block's longest row)
@@ -277,12 +284,6 @@ struct Block {
     int64_t nnz = 0;
     int64_t nnodes = 0;
     std::vector<int64_t> rowptr;   // nrows + 1
-    // column lists, kept as per-node structure and expanded on request
-    // (fs_model_pattern_get): code[J*6+c] offset of comp c within J's free
-    // (0..5) or fixed (8..13) run, -1 not in the block; off_free[k] /
-    // off_fix[k] offset of neighbour slot k's free / fixed run in the row
-    std::vector<int8_t> code;
-    std::vector<int32_t> off_free, off_fix;
     // scatter plan (device)
     int64_t npairs = 0;
     // running maximum over the pairs, in pair order, of the last element
@@ -321,9 +322,6 @@ struct Block {
         nrows = nnz = npairs = nrownodes = 0;
         max_rowlen = 0;
         rowptr.clear();
-        code.clear();
-        off_free.clear();
-        off_fix.clear();
         pair_emax.clear();
         for (DevBuf *b : {&nbr_ptr, &nbr_node, &nbr_pair, &nbr_off, &node_code, &node_rowstart, &contrib_ptr,
                           &contrib, &pair_node, &pair_slot, &rowrec, &slotrec, &kval, &mdiag, &noderec, &nodeinfo})
@@ -550,42 +548,85 @@ void key_add(std::vector<uint64_t> &k, const T &v) {
     k.insert(k.end(), w, w + (sizeof(T) + 7) / 8);
 }
 
-constexpr size_t FS_STAGE_BYTES = size_t(32) << 20;
-
 // Device-to-host copy ordered on the context's own stream, so that contexts
-// sharing a device never serialise on the null stream.  Copies of more than
-// two staging buffers go through the context's pinned buffers in chunks: the
-// DMA of chunk i+1 runs while host threads copy chunk i into `dst` (which
-// also spreads the first-touch page faults of a fresh destination over the
-// threads).
+// sharing a device never serialise on the null stream.  The bytes go through
+// pinned chunks: while the DMA of later chunks runs, up to STAGE_THREADS
+// threads copy the arrived ones into `dst`, which spreads the first-touch page
+// faults of a fresh destination over them.  A thread that has emptied a chunk's
+// slot queues the copy that uses the slot next.  Into fresh pages, direct copy
+// (pinned by the runtime) against this: 2 MB 1.2 -> 0.4 ms, 28 MB 2.8 -> 0.9,
+// 100 MB 10 -> 2.6, 680 MB 68 -> 15.5 (18 through two 32 MB chunks in turn); into
+// touched pages 256 KB 120 -> 25 us, 1 MB 440 -> 74, 28 MB 1.7 -> 0.9 ms.  More
+// threads than 8, or more slots than 16, gain nothing; chunks of 1 MB cost 30 %
+// on the largest copies, of 4 MB idle threads on those below 64 MB.
 int d2h(fs_ctx *c, void *dst, const void *src, size_t bytes) {
     if (bytes == 0) return FS_OK;
-    if (bytes <= 2 * FS_STAGE_BYTES) {
-        FS_HIP(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
+    const size_t MB = size_t(1) << 20;
+    const size_t ch = bytes <= 4 * MB ? MB : bytes <= 64 * MB ? 2 * MB : 4 * MB;
+    const size_t n = (bytes + ch - 1) / ch, ns = std::min(n, (size_t)STAGE_SLOTS);
+    if (c->stage_bytes < std::min(bytes, ns * ch)) {
+        if (c->stage) (void)hipHostFree(c->stage);
+        c->stage = nullptr;
+        c->stage_bytes = 0;
+        size_t want = MB;
+        while (want < std::min(bytes, ns * ch)) want *= 2;
+        if (hipHostMalloc((void **)&c->stage, want, hipHostMallocDefault) == hipSuccess) {
+            c->stage_bytes = want;
+        } else {  // no pinned memory to be had: the direct copy
+            (void)hipGetLastError();
+            c->stage = nullptr;
+            FS_HIP(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
+            FS_HIP(c, hipStreamSynchronize(c->stream));
+            return FS_OK;
+        }
+    }
+    if (n == 1) {
+        FS_HIP(c, hipMemcpyAsync(c->stage, src, bytes, hipMemcpyDeviceToHost, c->stream));
         FS_HIP(c, hipStreamSynchronize(c->stream));
+        std::memcpy(dst, c->stage, bytes);
         return FS_OK;
     }
-    for (int i = 0; i < 2; ++i) {
-        if (!c->stage[i]) FS_HIP(c, hipHostMalloc(&c->stage[i], FS_STAGE_BYTES, hipHostMallocDefault));
+    for (size_t i = 0; i < ns; ++i)
         if (!c->stage_ev[i]) FS_HIP(c, hipEventCreateWithFlags(&c->stage_ev[i], hipEventDisableTiming));
-    }
-    const size_t nch = (bytes + FS_STAGE_BYTES - 1) / FS_STAGE_BYTES;
-    auto chunk = [&](size_t i) { return std::min(FS_STAGE_BYTES, bytes - i * FS_STAGE_BYTES); };
-    auto enqueue = [&](size_t i) -> hipError_t {
-        hipError_t e = hipMemcpyAsync(c->stage[i % 2], (const char *)src + i * FS_STAGE_BYTES, chunk(i),
+    std::atomic<size_t> queued[STAGE_SLOTS], next{0};  // queued[i % ns]: chunk i + 1 once i is on its way
+    std::atomic<int> err{hipSuccess};
+    for (auto &q : queued) q = 0;
+    auto enqueue = [&](size_t i) {
+        hipError_t e = hipMemcpyAsync(c->stage + (i % ns) * ch, (const char *)src + i * ch, std::min(ch, bytes - i * ch),
                                       hipMemcpyDeviceToHost, c->stream);
-        return e != hipSuccess ? e : hipEventRecord(c->stage_ev[i % 2], c->stream);
+        if (e == hipSuccess) e = hipEventRecord(c->stage_ev[i % ns], c->stream);
+        if (e != hipSuccess) err = e;
+        queued[i % ns].store(i + 1, std::memory_order_release);
     };
-    FS_HIP(c, enqueue(0));
-    for (size_t i = 0; i < nch; ++i) {
-        // buffer (i+1) % 2 was last read by the host copy of chunk i-1, which has returned
-        if (i + 1 < nch) FS_HIP(c, enqueue(i + 1));
-        FS_HIP(c, hipEventSynchronize(c->stage_ev[i % 2]));
-        const char *from = (const char *)c->stage[i % 2];
-        char *to = (char *)dst + i * FS_STAGE_BYTES;
-        parallel_chunks((int64_t)chunk(i), [&](int64_t b0, int64_t b1) { std::memcpy(to + b0, from + b0, b1 - b0); },
-                        int64_t(1) << 20);
+    for (size_t i = 0; i < ns; ++i) enqueue(i);
+    auto work = [&] {
+        hipError_t e = hipSetDevice(c->device);
+        if (e != hipSuccess) err = e;
+        for (size_t i; err == hipSuccess && (i = next++) < n;) {
+            // chunk i is queued by the thread that empties its slot of chunk i - ns
+            while (queued[i % ns].load(std::memory_order_acquire) != i + 1) {
+                if (err != hipSuccess) return;
+                std::this_thread::yield();
+            }
+            if ((e = hipEventSynchronize(c->stage_ev[i % ns])) != hipSuccess) {
+                err = e;
+                return;
+            }
+            std::memcpy((char *)dst + i * ch, c->stage + (i % ns) * ch, std::min(ch, bytes - i * ch));
+            if (i + ns < n) enqueue(i + ns);
+        }
+    };
+    std::thread th[STAGE_THREADS - 1];
+    const size_t nt = std::min({(size_t)host_threads(), (size_t)STAGE_THREADS, bytes / (2 * MB) + 1});
+    try {
+        for (size_t t = 0; t + 1 < nt; ++t) th[t] = std::thread(work);
+    } catch (const std::system_error &) {
+        // no more threads to be had: those there, and this one, do the copy
     }
+    work();
+    for (auto &t : th)
+        if (t.joinable()) t.join();
+    FS_HIP(c, (hipError_t)err.load());
     return FS_OK;
 }
 
@@ -622,8 +663,7 @@ int build_block(fs_model *m, int which) {
     const int64_t nrows = which == FS_BLOCK_FF ? m->nfree : m->nall;
     const int64_t nfree = m->nfree;
     // per-node codes: offset of each comp within the node's free / fixed run
-    std::vector<int8_t> &code = B.code;
-    code.assign(N * 6, -1);
+    std::vector<int8_t> code(N * 6, -1);
     std::vector<int8_t> nfr(N, 0), nfx(N, 0);
     std::vector<int64_t> minfr(N, INT64_MAX), minfx(N, INT64_MAX);
     // lowest node (2 I + 0: free, 2 I + 1: fixed) whose dofs are not consecutive
@@ -676,9 +716,7 @@ int build_block(fs_model *m, int which) {
     // (runs are contiguous integer ranges, so sorting runs sorts the columns)
     const size_t nnb = m->nbr_list.size();
     std::vector<int32_t> rowlen(N, 0);
-    std::vector<int32_t> &nb_offfree = B.off_free, &nb_offfix = B.off_fix;
-    nb_offfree.assign(nnb, -1);
-    nb_offfix.assign(nnb, -1);
+    std::vector<int32_t> nb_offfree(nnb, -1), nb_offfix(nnb, -1);
     parallel_chunks(N, [&](int64_t I0, int64_t I1) {
         std::vector<std::pair<int64_t, int64_t>> runs;  // (first dof, nbr slot*2 + kind)
         for (int64_t I = I0; I < I1; ++I) {
@@ -1911,10 +1949,9 @@ void ctx_release(fs_ctx *ctx) {
         (void)hipStreamDestroy(ctx->stream2);
     }
     for (hipEvent_t ev : ctx->ev) (void)hipEventDestroy(ev);
-    for (int i = 0; i < 2; ++i) {
-        if (ctx->stage[i]) (void)hipHostFree(ctx->stage[i]);
-        if (ctx->stage_ev[i]) (void)hipEventDestroy(ctx->stage_ev[i]);
-    }
+    if (ctx->stage) (void)hipHostFree(ctx->stage);
+    for (hipEvent_t ev : ctx->stage_ev)
+        if (ev) (void)hipEventDestroy(ev);
     if (ctx->loop_stop) (void)hipHostFree(ctx->loop_stop);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -2260,6 +2297,9 @@ int fs_model_pattern(fs_model *m, int block, int64_t *nrows, int64_t *nnz) {
     return FS_OK;
 }
 
+// Column entries that fs_model_pattern_get holds on the device at a time (64 MB).
+static constexpr int64_t PATTERN_WINDOW = int64_t(1) << 23;
+
 int fs_model_pattern_get(fs_model *m, int block, int64_t *rowptr, int64_t *colval, int index_base) {
     if (!m) return FS_ERR_ARG;
     int s = fs_model_pattern(m, block, nullptr, nullptr);
@@ -2269,33 +2309,22 @@ int fs_model_pattern_get(fs_model *m, int block, int64_t *rowptr, int64_t *colva
         parallel_chunks(B.nrows + 1, [&](int64_t i0, int64_t i1) {
             for (int64_t i = i0; i < i1; ++i) rowptr[i] = B.rowptr[i] + index_base;
         });
-    if (colval) {
-        // every row of node I holds the same columns: the runs of I's
-        // neighbours, each at its offset within the row
-        const int64_t nrows = B.nrows;
-        parallel_chunks(m->N, [&](int64_t I0, int64_t I1) {
-            std::vector<int64_t> cols;
-            for (int64_t I = I0; I < I1; ++I) {
-                int64_t r0 = -1;
-                for (int cc = 0; cc < 6 && r0 < 0; ++cc)
-                    if (m->dof[I * 6 + cc] < nrows) r0 = m->dof[I * 6 + cc];
-                if (r0 < 0) continue;  // no row of this node in the block
-                cols.assign(B.rowptr[r0 + 1] - B.rowptr[r0], 0);
-                for (int k = m->nbr_ptr[I]; k < m->nbr_ptr[I + 1]; ++k) {
-                    const int J = m->nbr_list[k];
-                    for (int cc = 0; cc < 6; ++cc) {
-                        const int cd = B.code[(int64_t)J * 6 + cc];
-                        if (cd < 0) continue;
-                        const int pos = cd < 8 ? B.off_free[k] + cd : B.off_fix[k] + cd - 8;
-                        cols[pos] = m->dof[(int64_t)J * 6 + cc] + index_base;
-                    }
-                }
-                for (int cc = 0; cc < 6; ++cc) {
-                    const int64_t d = m->dof[I * 6 + cc];
-                    if (d < nrows) std::memcpy(colval + B.rowptr[d], cols.data(), cols.size() * sizeof(int64_t));
-                }
-            }
-        });
+    if (colval && B.nnz) {
+        // written on the device and copied out in windows of positions, so
+        // that the scratch stays within PATTERN_WINDOW entries (less where
+        // the device has no room for that)
+        fs_ctx *c = m->ctx;
+        DevBuf w;
+        int64_t win = std::min(B.nnz, PATTERN_WINDOW);
+        while ((s = dalloc(c, w, (size_t)win * 8)) == FS_ERR_NOMEM && win > 65536) win = (win + 1) / 2;
+        if (s) return s;
+        c->err.clear();
+        for (int64_t w0 = 0; w0 < B.nnz; w0 += win) {
+            const int64_t w1 = std::min(B.nnz, w0 + win);
+            FS_HIP(c, fs::launch_pattern_cols(plan_of(B), m->node_dof.as<int64_t>(), index_base, w0, w1,
+                                              w.as<int64_t>(), c->stream));
+            if ((s = d2h(c, colval + w0, w.p, (size_t)(w1 - w0) * 8))) return s;
+        }
     }
     return FS_OK;
 }

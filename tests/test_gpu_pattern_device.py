@@ -1,0 +1,63 @@
+"""Patterns made on the device and results copied out in pinned chunks, at the
+sizes where the copy changes its form: one chunk, several, more chunks than
+slots, and more columns than one window.  The columns are compared with the
+structural union built with scipy (equal), the values with their transpose
+(bitwise: both triangles come from one sum)."""
+import numpy as np
+import pytest
+
+from test_gpu_pattern import _reference
+from flexshell import _lib, femm as FM
+from flexshell.material import MatDeforElastIso
+
+pytestmark = pytest.mark.gpu
+
+
+class _Dofs:
+    def __init__(self, dofnums, nfree):
+        self.dofnums, self.nfreedofs, self.nalldofs = dofnums, nfree, dofnums.size
+
+
+def _plate(nen, nx, ny, seed):
+    """Flat plate, its nodes shuffled, one edge simply supported: free dofs
+    numbered first in node order, then the fixed ones."""
+    X, Y = np.meshgrid(np.linspace(0, 2.0, nx + 1), np.linspace(0, 1.0, ny + 1), indexing="ij")
+    N = X.size
+    new = np.random.default_rng(seed).permutation(N)
+    xyz = np.zeros((N, 3))
+    xyz[new, 0], xyz[new, 1] = X.ravel(), Y.ravel()
+    i, j = np.meshgrid(np.arange(nx), np.arange(ny), indexing="ij")
+    a = (i * (ny + 1) + j).ravel()
+    b, c, d = a + ny + 1, a + ny + 2, a + 1
+    conn = np.stack([a, b, c, d], 1) if nen == 4 else np.vstack([np.stack([a, b, c], 1), np.stack([a, c, d], 1)])
+    fixed = np.zeros((N, 6), dtype=bool)
+    fixed[new[: ny + 1], :3] = True
+    dofs = np.empty((N, 6), dtype=np.int64)
+    nf = int((~fixed).sum())
+    dofs[~fixed] = np.arange(nf)
+    dofs[fixed] = np.arange(nf, 6 * N)
+    return xyz, new[conn], _Dofs(dofs, nf)
+
+
+# entries of the block: 30 thousand to 10 million (0.25 to 80 MB of columns)
+@pytest.mark.parametrize("nen, nx, ny, ff", [(4, 9, 9, False), (3, 30, 20, True), (4, 60, 41, False),
+                                             (3, 150, 120, True), (3, 210, 190, False)])
+def test_pattern_and_values_by_size(ctx, nen, nx, ny, ff):
+    print(f"[gpu] pattern by size {nen} {nx}x{ny} ff={ff}", flush=True)
+    xyz, conn, d = _plate(nen, nx, ny, nx)
+    cls = FM.FEMMShellT3FF if nen == 3 else FM.FEMMShellQ4RS
+    f = cls(conn, MatDeforElastIso(210e9, 0.3, 7850.0), thickness=0.01, ctx=ctx)
+    f.associategeometry(xyz)
+    nf, na = d.nfreedofs, d.nalldofs
+    asm = FM.SysmatAssemblerFFBlock(nf) if ff else FM.SysmatAssemblerSparseCSRSymm()
+    K = f.stiffness(asm, xyz, None, None, d)
+    P = _reference(conn, d.dofnums, nf if ff else na)
+    assert K.shape == P.shape
+    assert np.array_equal(K.indptr, P.indptr) and np.array_equal(K.indices, P.indices)
+    KT = K.T.tocsr()
+    KT.sort_indices()
+    assert np.array_equal(KT.data, K.data)
+    assert np.all(K.diagonal() > 0.0)
+    nr, rp, cv = f._model.pattern(_lib.FS_BLOCK_FF)
+    Pf = _reference(conn, d.dofnums, nf)
+    assert np.array_equal(rp, Pf.indptr) and np.array_equal(cv, Pf.indices)
