@@ -161,6 +161,46 @@ struct ScatterPlan {
     const int32_t *pair_slot;     // 2 * npairs: kI, kJ
 };
 
+// Longest neighbour list that the planner's kernels order (plan_runs_kernel).
+constexpr int PLAN_HUB = 256;
+
+// Totals of a block's row structure, found while it is planned.
+struct PlanTotals {
+    unsigned long long bad;  // lowest 2 I + kind whose dofs are not consecutive (kind 0: free, 1: fixed)
+    int64_t nnz;
+    int32_t max_any, max_free;  // longest row of a node; of a node with free dofs
+};
+
+// Planning of a block on the device (launch_plan_rows, launch_plan_pairs):
+// ScatterPlan's arrays and the records of the row products are its results.
+struct PlanArgs {
+    int64_t N, E, nrows, nfree, nnb, npairs;
+    int nen;
+    const int64_t *dof;                 // N x 6
+    const int32_t *conn;                // nen planes of E
+    const int32_t *ne_ptr, *ne_list;    // node -> elements, ascending
+    const int32_t *nbr_ptr, *nbr;       // node -> neighbours, ascending
+    PlanTotals *tot;
+    int64_t *sums;                      // scan_tiles(longest scan) + 1
+    int8_t *code;                       // N x 6
+    int64_t *first;                     // N x 2: first free, first fixed dof
+    int32_t *count;                     // free dofs | fixed dofs << 4
+    int32_t *off;                       // 2 nnb
+    int32_t *rowlen;                    // N
+    int32_t *rowptr;                    // nrows + 1
+    int32_t *rowstart;                  // N x 6
+    int4 *node_rec;                     // N
+    int32_t *diag, *base;               // N, N + 1
+    int32_t *nbr_pair;                  // nnb
+    int32_t *pair_node, *pair_slot;     // 2 npairs
+    int32_t *contrib_ptr, *contrib;     // npairs + 1, E nen (nen + 1) / 2
+    // free-free block only (else null)
+    int32_t *isfree;                    // N + 1
+    int4 *rowrec, *noderec;
+    int32_t *nodeinfo;
+    int2 *slotrec;
+};
+
 // Parameters of one stress-resultant launch (inspectintegpoints): one thread
 // per (listed element, integration point).
 //   g_mat  homogeneous: per group 16 doubles -- Dps 9 (row-major), 5/6 Dt 4,

@@ -39,6 +39,9 @@ hipError_t launch_element_blocks(const ElemParams &p, const double *x, const dou
 int element_variants(int nen);
 void element_variant_shape(int nen, int variant, int *ne, int *wg);
 hipError_t launch_scatter(const ScatterPlan &sp, const double *Kb, double *vals, hipStream_t st);
+int64_t scan_tiles(int64_t n);
+hipError_t launch_plan_rows(const PlanArgs &a, hipStream_t st);
+hipError_t launch_plan_pairs(const PlanArgs &a, hipStream_t st);
 hipError_t launch_pattern_cols(const ScatterPlan &sp, const int64_t *node_dof, int base, int64_t w0, int64_t w1,
                                int64_t *col, hipStream_t st);
 int fused_tile_elems(int nen);
@@ -283,15 +286,15 @@ struct Block {
     int64_t nrows = 0;
     int64_t nnz = 0;
     int64_t nnodes = 0;
-    std::vector<int64_t> rowptr;   // nrows + 1
     // scatter plan (device)
     int64_t npairs = 0;
     // running maximum over the pairs, in pair order, of the last element
     // contributing to a pair: the pairs [0, k) with pair_emax[k-1] < e are
     // complete once the elements [0, e) are (host)
     std::vector<int32_t> pair_emax;
-    DevBuf nbr_ptr, nbr_node, nbr_pair, nbr_off, node_code, node_rowstart, contrib_ptr, contrib, pair_node,
-        pair_slot;
+    int64_t nnb = 0, ncontrib = 0;  // neighbour slots, contributions
+    DevBuf rowptr, nbr_ptr, nbr_node, nbr_pair, nbr_off, node_code, node_rowstart, node_rec, contrib_ptr, contrib,
+        pair_node, pair_slot;
     // device values (CSR order) and, for the free-free block, the run records
     // of the row products of the time loop (fs::RunRows)
     DevBuf rowrec, slotrec, kval, mdiag;
@@ -302,29 +305,28 @@ struct Block {
     bool k_ready = false, m_ready = false;
     uint64_t vgen = 0;  // raised before each launch that writes kval
     PatchStore patch;
-    // host copies for the fused-assembly planner: neighbour slot -> (pair <<
+    // host copies for the fused-assembly planner (host_plan): neighbour slot -> (pair <<
     // 1 | side), pair nodes and slots, contributions per pair (counts)
-    std::vector<int32_t> h_nb_pair, h_pnode, h_pslot, h_cptr;
+    std::unique_ptr<int32_t[]> h_nb_pair, h_pnode, h_pslot, h_cptr;
     // per node {first free row's CSR position, first fixed row's (-1), row
     // length, 4-bit comp codes}; per neighbour slot the free / fixed run offsets
-    std::vector<int32_t> h_node_rec, h_nb_off;
+    std::unique_ptr<int32_t[]> h_node_rec, h_nb_off;
     TileStore tiles;
     void reset() {
         built = k_ready = m_ready = false;
-        h_nb_pair.clear();
-        h_pnode.clear();
-        h_pslot.clear();
-        h_cptr.clear();
-        h_node_rec.clear();
-        h_nb_off.clear();
+        h_nb_pair.reset();
+        h_pnode.reset();
+        h_pslot.reset();
+        h_cptr.reset();
+        h_node_rec.reset();
+        h_nb_off.reset();
         tiles.reset();
         patch.reset();
-        nrows = nnz = npairs = nrownodes = 0;
+        nrows = nnz = npairs = nrownodes = nnb = ncontrib = 0;
         max_rowlen = 0;
-        rowptr.clear();
         pair_emax.clear();
-        for (DevBuf *b : {&nbr_ptr, &nbr_node, &nbr_pair, &nbr_off, &node_code, &node_rowstart, &contrib_ptr,
-                          &contrib, &pair_node, &pair_slot, &rowrec, &slotrec, &kval, &mdiag, &noderec, &nodeinfo})
+        for (DevBuf *b : {&rowptr, &nbr_ptr, &nbr_node, &nbr_pair, &nbr_off, &node_code, &node_rowstart, &node_rec,
+                          &contrib_ptr, &contrib, &pair_node, &pair_slot, &rowrec, &slotrec, &kval, &mdiag, &noderec, &nodeinfo})
             b->release();
     }
 };
@@ -654,291 +656,182 @@ void cm2rm(int n, const double *cm, double *rm) {
         for (int j = 0; j < n; ++j) rm[i * n + j] = cm[j * n + i];
 }
 
+// Pattern, scatter plan and records of the row products of a block, planned on
+// the device from the node lists and the dof numbers (fs::PlanArgs); the
+// host reads the totals between the two parts, and copies of the plan only where
+// a host planner asks for them (host_plan).
 int build_block(fs_model *m, int which) {
     fs_ctx *c = m->ctx;
     Block &B = m->blk[which];
     if (B.built) return FS_OK;
     if (!m->dofs_ready) return fail(c, FS_ERR_STATE, "pattern: equation numbers not set (fs_model_set_dofs)");
-    const int64_t N = m->N;
-    const int64_t nrows = which == FS_BLOCK_FF ? m->nfree : m->nall;
-    const int64_t nfree = m->nfree;
-    // per-node codes: offset of each comp within the node's free / fixed run
-    std::vector<int8_t> code(N * 6, -1);
-    std::vector<int8_t> nfr(N, 0), nfx(N, 0);
-    std::vector<int64_t> minfr(N, INT64_MAX), minfx(N, INT64_MAX);
-    // lowest node (2 I + 0: free, 2 I + 1: fixed) whose dofs are not consecutive
-    std::atomic<int64_t> bad{INT64_MAX};
-    auto flag = [&](int64_t v) {
-        int64_t cur = bad.load();
-        while (v < cur && !bad.compare_exchange_weak(cur, v)) {
-        }
-    };
-    parallel_chunks(N, [&](int64_t I0, int64_t I1) {
-        for (int64_t I = I0; I < I1; ++I) {
-            int64_t fr[6], fx[6];
-            int a = 0, b = 0;
-            for (int cc = 0; cc < 6; ++cc) {
-                const int64_t d = m->dof[I * 6 + cc];
-                if (d >= nrows) continue;
-                if (d < nfree)
-                    fr[a++] = d;
-                else
-                    fx[b++] = d;
-            }
-            std::sort(fr, fr + a);
-            std::sort(fx, fx + b);
-            if (a && fr[a - 1] - fr[0] + 1 != a) {
-                flag(2 * I);
-                continue;
-            }
-            if (b && fx[b - 1] - fx[0] + 1 != b) {
-                flag(2 * I + 1);
-                continue;
-            }
-            for (int cc = 0; cc < 6; ++cc) {
-                const int64_t d = m->dof[I * 6 + cc];
-                if (d >= nrows) continue;
-                if (d < nfree)
-                    code[I * 6 + cc] = (int8_t)(d - fr[0]);
-                else
-                    code[I * 6 + cc] = (int8_t)(8 + (d - fx[0]));
-            }
-            nfr[I] = (int8_t)a;
-            nfx[I] = (int8_t)b;
-            if (a) minfr[I] = fr[0];
-            if (b) minfx[I] = fx[0];
-        }
-    });
-    if (bad.load() != INT64_MAX)
-        return fail(c, FS_ERR_UNSUPPORTED, "node %lld: %s dofs are not consecutive numbers",
-                    (long long)(bad.load() / 2), bad.load() % 2 ? "fixed" : "free");
-    // per node: sorted column list = runs of the neighbours ordered by first dof
-    // (runs are contiguous integer ranges, so sorting runs sorts the columns)
-    const size_t nnb = m->nbr_list.size();
-    std::vector<int32_t> rowlen(N, 0);
-    std::vector<int32_t> nb_offfree(nnb, -1), nb_offfix(nnb, -1);
-    parallel_chunks(N, [&](int64_t I0, int64_t I1) {
-        std::vector<std::pair<int64_t, int64_t>> runs;  // (first dof, nbr slot*2 + kind)
-        for (int64_t I = I0; I < I1; ++I) {
-            runs.clear();
-            for (int k = m->nbr_ptr[I]; k < m->nbr_ptr[I + 1]; ++k) {
-                const int J = m->nbr_list[k];
-                if (nfr[J]) runs.push_back({minfr[J], (int64_t)k * 2 + 0});
-                if (nfx[J]) runs.push_back({minfx[J], (int64_t)k * 2 + 1});
-            }
-            std::sort(runs.begin(), runs.end());
-            int32_t pos = 0;
-            for (auto &r : runs) {
-                const int64_t k = r.second / 2;
-                const int J = m->nbr_list[k];
-                if (r.second % 2 == 0) {
-                    nb_offfree[k] = pos;
-                    pos += nfr[J];
-                } else {
-                    nb_offfix[k] = pos;
-                    pos += nfx[J];
-                }
-            }
-            rowlen[I] = pos;
-        }
-    });
-    // row owners
-    std::vector<int64_t> owner(nrows, -1);
-    for (int64_t I = 0; I < N; ++I)
-        for (int cc = 0; cc < 6; ++cc) {
-            const int64_t d = m->dof[I * 6 + cc];
-            if (d < nrows) owner[d] = I;
-        }
-    B.rowptr.assign(nrows + 1, 0);
-    for (int64_t d = 0; d < nrows; ++d) {
-        if (owner[d] < 0) return fail(c, FS_ERR_ARG, "dof %lld is not used by any node", (long long)d);
-        B.rowptr[d + 1] = B.rowptr[d] + rowlen[owner[d]];
-    }
-    const int64_t nnz = B.rowptr[nrows];
-    if (nnz >= (int64_t(1) << 31))
-        return fail(c, FS_ERR_UNSUPPORTED, "block with %lld stored entries exceeds 32-bit positions", (long long)nnz);
-    // upper node pairs: the neighbours J >= I of each node, in order
-    std::vector<int64_t> pair_base(N + 1, 0);
-    parallel_chunks(N, [&](int64_t I0, int64_t I1) {
-        for (int64_t I = I0; I < I1; ++I) {
-            int cnt = 0;
-            for (int k = m->nbr_ptr[I]; k < m->nbr_ptr[I + 1]; ++k)
-                if (m->nbr_list[k] >= I) ++cnt;
-            pair_base[I + 1] = cnt;
-        }
-    });
-    for (int64_t I = 0; I < N; ++I) pair_base[I + 1] += pair_base[I];
-    const int64_t npairs = pair_base[N];
-    if (npairs >= (int64_t(1) << 27)) return fail(c, FS_ERR_UNSUPPORTED, "too many node pairs (%lld)", (long long)npairs);
-    auto slot_of = [&](int64_t I, int64_t J) -> int {
-        const int32_t *b0 = m->nbr_list.data() + m->nbr_ptr[I];
-        const int32_t *e0 = m->nbr_list.data() + m->nbr_ptr[I + 1];
-        return (int)(std::lower_bound(b0, e0, (int32_t)J) - m->nbr_list.data());
-    };
-    // slot of each node in its own list: the upper pairs of I are its slots
-    // from diag[I] on, numbered from pair_base[I]
-    std::vector<int32_t> diag(N);
-    parallel_chunks(N, [&](int64_t I0, int64_t I1) {
-        for (int64_t I = I0; I < I1; ++I) diag[I] = slot_of(I, I);
-    });
-    // neighbour tables: pair, side, run offsets; node row starts (each node
-    // writes its own slots, its own upper pairs and its own rows)
-    std::vector<int32_t> nb_pair(nnb), nb_off(2 * nnb), rowstart(N * 6, -1);
-    std::vector<int32_t> pnode(2 * npairs), pslot(2 * npairs);
-    parallel_chunks(N, [&](int64_t I0, int64_t I1) {
-        for (int64_t I = I0; I < I1; ++I) {
-            for (int k = m->nbr_ptr[I]; k < m->nbr_ptr[I + 1]; ++k) {
-                const int J = m->nbr_list[k];
-                const int64_t p = I <= J ? pair_base[I] + (k - diag[I]) : pair_base[J] + (slot_of(J, I) - diag[J]);
-                nb_pair[k] = (int32_t)((p << 1) | (I > J ? 1 : 0));
-                nb_off[2 * k] = nb_offfree[k];
-                nb_off[2 * k + 1] = nb_offfix[k];
-                if (I <= J) {
-                    pnode[2 * p] = (int32_t)I;
-                    pnode[2 * p + 1] = J;
-                    pslot[2 * p] = k;
-                    pslot[2 * p + 1] = slot_of(J, I);
-                }
-            }
-            for (int cc = 0; cc < 6; ++cc) {
-                const int64_t d = m->dof[I * 6 + cc];
-                if (d < nrows) rowstart[I * 6 + cc] = (int32_t)B.rowptr[d];
-            }
-        }
-    });
-    // contributions, element order within each pair
-    const int nen = m->nen;
-    const int nblk = nen * (nen + 1) / 2;
-    if ((int64_t)m->E * nblk >= (int64_t(1) << 30))
-        return fail(c, FS_ERR_UNSUPPORTED, "too many element blocks (%lld)", (long long)(m->E * nblk));
-    // The contributions of the upper pair (I, J) are the elements incident to
-    // both nodes (an intersection of the two ascending incidence lists, so in
-    // element order), each with the local block (a <= b) that holds the pair
-    // and whether the block's row node is J (transposed).  Two passes over
-    // the pairs: counts, then the lists.
-    auto pair_contribs = [&](int64_t p, int32_t *outl) -> int {
-        const int I = pnode[2 * p], J = pnode[2 * p + 1];
-        int ki = m->ne_ptr[I], kj = m->ne_ptr[J], cnt = 0;
-        const int ei = m->ne_ptr[I + 1], ej = m->ne_ptr[J + 1];
-        while (ki < ei && kj < ej) {
-            const int32_t e1 = m->ne_list[ki], e2 = m->ne_list[kj];
-            if (e1 < e2) {
-                ++ki;
-            } else if (e2 < e1) {
-                ++kj;
-            } else {
-                if (outl) {
-                    const int32_t *ce = m->conn.data() + (int64_t)e1 * nen;
-                    int a = 0, b = 0;
-                    for (int q = 0; q < nen; ++q) {
-                        if (ce[q] == I) a = q;
-                        if (ce[q] == J) b = q;
-                    }
-                    const int lo = std::min(a, b), hi = std::max(a, b);
-                    const int bl = lo * nen - lo * (lo - 1) / 2 + (hi - lo);  // upper pairs in row order
-                    const int tr = ce[lo] > ce[hi] ? 1 : 0;
-                    outl[cnt] = (int32_t)((((int64_t)e1 * nblk + bl) << 1) | tr);
-                }
-                ++cnt;
-                ++ki;
-                ++kj;
-            }
-        }
-        return cnt;
-    };
-    std::vector<int32_t> cptr(npairs + 1, 0);
-    parallel_chunks(npairs, [&](int64_t p0, int64_t p1) {
-        for (int64_t p = p0; p < p1; ++p) cptr[p + 1] = pair_contribs(p, nullptr);
-    });
-    for (int64_t p = 0; p < npairs; ++p) cptr[p + 1] += cptr[p];
-    std::vector<int32_t> clist(cptr[npairs]);
-    B.pair_emax.assign(npairs, -1);
-    parallel_chunks(npairs, [&](int64_t p0, int64_t p1) {
-        for (int64_t p = p0; p < p1; ++p) {
-            const int n = pair_contribs(p, clist.data() + cptr[p]);
-            if (n) B.pair_emax[p] = (clist[cptr[p] + n - 1] >> 1) / nblk;  // last (largest) element
-        }
-    });
-    for (int64_t p = 1; p < npairs; ++p) B.pair_emax[p] = std::max(B.pair_emax[p], B.pair_emax[p - 1]);
-    // run records of the free-free block (fs::RunRows): every row of node I
-    // is the runs of I's neighbours in slot order, each run the neighbour's
-    // free dofs (consecutive columns starting at its first free dof)
-    std::vector<int32_t> rrec, srec, nrec, ninfo;
-    if (which == FS_BLOCK_FF) {
-        // node records: the nodes with free dofs, in node order
-        for (int64_t I = 0; I < N; ++I)
-            if (nfr[I]) {
-                nrec.push_back((int32_t)B.rowptr[minfr[I]]);
-                nrec.push_back((int32_t)minfr[I]);
-                nrec.push_back(m->nbr_ptr[I]);
-                nrec.push_back(m->nbr_ptr[I + 1]);
-                ninfo.push_back((rowlen[I] << 3) | nfr[I]);
-                B.max_rowlen = std::max(B.max_rowlen, rowlen[I]);
-            }
-        rrec.assign(4 * nrows, 0);
-        parallel_chunks(nrows, [&](int64_t d0, int64_t d1) {
-            for (int64_t d = d0; d < d1; ++d) {
-                const int64_t I = owner[d];
-                rrec[4 * d + 0] = (int32_t)B.rowptr[d];
-                rrec[4 * d + 1] = m->nbr_ptr[I];
-                rrec[4 * d + 2] = m->nbr_ptr[I + 1];
-            }
-        });
-        for (int64_t I = 0; I < N; ++I)
-            if (rowlen[I] >= (1 << 27)) return fail(c, FS_ERR_UNSUPPORTED, "row of more than 2^27 entries");
-        srec.assign(2 * nnb, 0);
-        parallel_chunks((int64_t)nnb, [&](int64_t k0, int64_t k1) {
-            for (int64_t k = k0; k < k1; ++k) {
-                const int J = m->nbr_list[k];
-                const int nf = nfr[J];
-                if (nf == 0) continue;  // no free dofs: an empty run
-                srec[2 * k] = (nb_offfree[k] << 4) | nf;
-                srec[2 * k + 1] = (int32_t)minfr[J];
-            }
-        });
-    }
-    // upload
+    const int64_t N = m->N, E = m->E;
+    const bool ff = which == FS_BLOCK_FF;
+    const int nblk = m->nen * (m->nen + 1) / 2;
+    fs::PlanArgs a{};
+    a.N = N;
+    a.E = E;
+    a.nen = m->nen;
+    a.nrows = ff ? m->nfree : m->nall;
+    a.nfree = m->nfree;
+    a.nnb = (int64_t)m->nbr_list.size();
+    // every node in an element is its own neighbour, and neighbours are mutual
+    int64_t used = 0;
+    for (int64_t I = 0; I < N; ++I) used += m->nbr_ptr[I + 1] > m->nbr_ptr[I];
+    a.npairs = (a.nnb + used) / 2;
+    DevBuf tot, sums, first, count, rowlen, diag, base, isfree;
+    fs::PlanTotals t{UINT64_MAX, 0, 0, 0};
+    const int64_t longest = std::max({a.nrows, N, a.npairs});
     int s;
-    if ((s = upload(c, B.nbr_ptr, m->nbr_ptr.data(), m->nbr_ptr.size()))) return s;
-    if ((s = upload(c, B.nbr_node, m->nbr_list.data(), m->nbr_list.size()))) return s;
-    if ((s = upload(c, B.nbr_pair, nb_pair.data(), nb_pair.size()))) return s;
-    if ((s = upload(c, B.nbr_off, nb_off.data(), nb_off.size()))) return s;
-    if ((s = upload(c, B.node_code, code.data(), code.size()))) return s;
-    if ((s = upload(c, B.node_rowstart, rowstart.data(), rowstart.size()))) return s;
-    if ((s = upload(c, B.contrib_ptr, cptr.data(), cptr.size()))) return s;
-    if ((s = upload(c, B.contrib, clist.data(), clist.size()))) return s;
-    if ((s = upload(c, B.pair_node, pnode.data(), pnode.size()))) return s;
-    if ((s = upload(c, B.pair_slot, pslot.data(), pslot.size()))) return s;
-    if (which == FS_BLOCK_FF) {
-        if ((s = upload(c, B.rowrec, rrec.data(), rrec.size()))) return s;
-        if ((s = upload(c, B.slotrec, srec.data(), srec.size()))) return s;
-        if ((s = upload(c, B.noderec, nrec.data(), nrec.size()))) return s;
-        if ((s = upload(c, B.nodeinfo, ninfo.data(), ninfo.size()))) return s;
-        B.nrownodes = (int64_t)ninfo.size();
-    }
-    if ((s = dalloc(c, B.kval, (size_t)nnz * sizeof(double)))) return s;
-    if ((s = dalloc(c, B.mdiag, (size_t)nrows * sizeof(double)))) return s;
-    FS_HIP(c, hipStreamSynchronize(c->stream));
-    B.h_node_rec.assign(4 * N, -1);
+    if ((s = dalloc(c, tot, sizeof t)) || (s = dalloc(c, sums, (fs::scan_tiles(longest) + 1) * 8)) ||
+        (s = dalloc(c, first, 2 * N * 8)) || (s = dalloc(c, count, N * 4)) || (s = dalloc(c, rowlen, N * 4)) ||
+        (s = upload(c, B.nbr_ptr, m->nbr_ptr.data(), m->nbr_ptr.size())) ||
+        (s = upload(c, B.nbr_node, m->nbr_list.data(), m->nbr_list.size())) ||
+        (s = dalloc(c, B.node_code, N * 6)) || (s = dalloc(c, B.nbr_off, 2 * a.nnb * 4)) ||
+        (s = dalloc(c, B.rowptr, (a.nrows + 1) * 4)))
+        return s;
+    a.dof = m->node_dof.as<int64_t>();
+    a.conn = m->dconn.as<int32_t>();
+    a.ne_ptr = m->dne_ptr.as<int32_t>();
+    a.ne_list = m->dne_list.as<int32_t>();
+    a.nbr_ptr = B.nbr_ptr.as<int32_t>();
+    a.nbr = B.nbr_node.as<int32_t>();
+    a.tot = tot.as<fs::PlanTotals>();
+    a.sums = sums.as<int64_t>();
+    a.code = B.node_code.as<int8_t>();
+    a.first = first.as<int64_t>();
+    a.count = count.as<int32_t>();
+    a.off = B.nbr_off.as<int32_t>();
+    a.rowlen = rowlen.as<int32_t>();
+    a.rowptr = B.rowptr.as<int32_t>();
+    // the rows of nodes with long lists, which would take a lane of the kernel
+    // the square of the length
+    std::vector<std::vector<int32_t>> hubs;  // row length, then offsets
     for (int64_t I = 0; I < N; ++I) {
-        int32_t codes = 0;
-        for (int cc = 0; cc < 6; ++cc) codes |= (code[I * 6 + cc] < 0 ? 15 : (int)code[I * 6 + cc]) << (4 * cc);
-        B.h_node_rec[4 * I] = nfr[I] ? (int32_t)B.rowptr[minfr[I]] : -1;
-        B.h_node_rec[4 * I + 1] = nfx[I] ? (int32_t)B.rowptr[minfx[I]] : -1;
-        B.h_node_rec[4 * I + 2] = rowlen[I];
-        B.h_node_rec[4 * I + 3] = codes;
+        const int k0 = m->nbr_ptr[I], n = m->nbr_ptr[I + 1] - k0;
+        if (n <= fs::PLAN_HUB) continue;
+        hubs.emplace_back(1 + 2 * (size_t)n, -1);
+        std::vector<int32_t> &h = hubs.back();
+        std::vector<std::pair<int64_t, int>> runs;  // first dof, 2 slot + kind
+        for (int k = 0; k < n; ++k) {
+            int64_t lo[2] = {INT64_MAX, INT64_MAX};
+            for (int cc = 0; cc < 6; ++cc) {
+                const int64_t d = m->dof[(int64_t)m->nbr_list[k0 + k] * 6 + cc];
+                if (d < a.nrows) lo[d >= a.nfree] = std::min(lo[d >= a.nfree], d);
+            }
+            for (int q = 0; q < 2; ++q)
+                if (lo[q] != INT64_MAX) runs.push_back({lo[q], 2 * k + q});
+        }
+        std::sort(runs.begin(), runs.end());
+        int32_t pos = 0;
+        for (const auto &run : runs) {
+            h[1 + run.second] = pos;
+            const int64_t J = m->nbr_list[k0 + run.second / 2];
+            for (int cc = 0; cc < 6; ++cc) {
+                const int64_t d = m->dof[J * 6 + cc];
+                pos += d < a.nrows && (d >= a.nfree) == (run.second % 2 == 1);
+            }
+        }
+        h[0] = pos;
+        t.max_any = std::max(t.max_any, pos);
+        for (int cc = 0; cc < 6; ++cc)
+            if (m->dof[I * 6 + cc] < a.nfree) t.max_free = std::max(t.max_free, pos);
+        FS_HIP(c, hipMemcpyAsync(a.rowlen + I, &h[0], 4, hipMemcpyHostToDevice, c->stream));
+        FS_HIP(c, hipMemcpyAsync(a.off + 2 * (int64_t)k0, &h[1], 8 * (size_t)n, hipMemcpyHostToDevice, c->stream));
     }
-    B.h_nb_off = std::move(nb_off);
-    B.h_nb_pair = std::move(nb_pair);
-    B.h_pnode = std::move(pnode);
-    B.h_pslot = std::move(pslot);
-    B.h_cptr = std::move(cptr);
-    B.npairs = npairs;
+    FS_HIP(c, hipMemcpyAsync(tot.p, &t, sizeof t, hipMemcpyHostToDevice, c->stream));
+    FS_HIP(c, fs::launch_plan_rows(a, c->stream));
+    if ((s = d2h(c, &t, tot.p, sizeof t))) return s;
+    if (t.bad != UINT64_MAX)
+        return fail(c, FS_ERR_UNSUPPORTED, "node %lld: %s dofs are not consecutive numbers", (long long)(t.bad / 2),
+                    t.bad % 2 ? "fixed" : "free");
+    if (t.nnz >= (int64_t(1) << 31))
+        return fail(c, FS_ERR_UNSUPPORTED, "block with %lld stored entries exceeds 32-bit positions", (long long)t.nnz);
+    if (a.npairs >= (int64_t(1) << 27))
+        return fail(c, FS_ERR_UNSUPPORTED, "too many node pairs (%lld)", (long long)a.npairs);
+    if (E * nblk >= (int64_t(1) << 30))
+        return fail(c, FS_ERR_UNSUPPORTED, "too many element blocks (%lld)", (long long)(E * nblk));
+    if (ff && t.max_any >= (1 << 27)) return fail(c, FS_ERR_UNSUPPORTED, "row of more than 2^27 entries");
+    if ((s = dalloc(c, B.node_rowstart, N * 6 * 4)) || (s = dalloc(c, B.node_rec, N * 16)) ||
+        (s = dalloc(c, diag, N * 4)) || (s = dalloc(c, base, (N + 1) * 4)) || (s = dalloc(c, B.nbr_pair, a.nnb * 4)) ||
+        (s = dalloc(c, B.pair_node, 2 * a.npairs * 4)) || (s = dalloc(c, B.pair_slot, 2 * a.npairs * 4)) ||
+        (s = dalloc(c, B.contrib_ptr, (a.npairs + 1) * 4)) || (s = dalloc(c, B.contrib, E * nblk * 4)))
+        return s;
+    a.rowstart = B.node_rowstart.as<int32_t>();
+    a.node_rec = B.node_rec.as<int4>();
+    a.diag = diag.as<int32_t>();
+    a.base = base.as<int32_t>();
+    a.nbr_pair = B.nbr_pair.as<int32_t>();
+    a.pair_node = B.pair_node.as<int32_t>();
+    a.pair_slot = B.pair_slot.as<int32_t>();
+    a.contrib_ptr = B.contrib_ptr.as<int32_t>();
+    a.contrib = B.contrib.as<int32_t>();
+    int32_t nodes = 0;
+    if (ff) {
+        if ((s = dalloc(c, isfree, (N + 1) * 4)) || (s = dalloc(c, B.rowrec, a.nrows * 16)) ||
+            (s = dalloc(c, B.slotrec, a.nnb * 8)) || (s = dalloc(c, B.noderec, N * 16)) ||
+            (s = dalloc(c, B.nodeinfo, N * 4)))
+            return s;
+        a.isfree = isfree.as<int32_t>();
+        a.rowrec = B.rowrec.as<int4>();
+        a.slotrec = B.slotrec.as<int2>();
+        a.noderec = B.noderec.as<int4>();
+        a.nodeinfo = B.nodeinfo.as<int32_t>();
+    }
+    if ((s = dalloc(c, B.kval, (size_t)t.nnz * sizeof(double)))) return s;
+    if ((s = dalloc(c, B.mdiag, (size_t)a.nrows * sizeof(double)))) return s;
+    FS_HIP(c, fs::launch_plan_pairs(a, c->stream));
+    if (ff && (s = d2h(c, &nodes, isfree.as<int32_t>() + N, 4))) return s;
+    FS_HIP(c, hipStreamSynchronize(c->stream));
+    B.nrownodes = nodes;
+    B.max_rowlen = ff ? t.max_free : 0;
+    B.nnb = a.nnb;
+    B.ncontrib = E * nblk;
+    B.npairs = a.npairs;
     B.nnodes = N;
-    B.nrows = nrows;
-    B.nnz = nnz;
+    B.nrows = a.nrows;
+    B.nnz = t.nnz;
     B.built = true;
     B.k_ready = B.m_ready = false;
+    return FS_OK;
+}
+
+// A device array of a block's plan, copied to the host once; not zeroed first,
+// so that the threads of the copy touch its pages.
+template <class T>
+int host_copy(fs_ctx *c, HostArray<T> &v, const DevBuf &b, int64_t n) {
+    if (v) return FS_OK;
+    v = host_array<T>(n);
+    const int s = d2h(c, v.get(), b.p, n * sizeof(T));
+    if (s) v.reset();
+    return s;
+}
+
+// Host copies of the plan for the planner of the fused assembly.
+int host_plan(fs_ctx *c, Block &B) {
+    int s;
+    if ((s = host_copy(c, B.h_nb_pair, B.nbr_pair, B.nnb)) || (s = host_copy(c, B.h_pnode, B.pair_node, 2 * B.npairs)) ||
+        (s = host_copy(c, B.h_pslot, B.pair_slot, 2 * B.npairs)) ||
+        (s = host_copy(c, B.h_cptr, B.contrib_ptr, B.npairs + 1)) ||
+        (s = host_copy(c, B.h_node_rec, B.node_rec, 4 * B.nnodes)) || (s = host_copy(c, B.h_nb_off, B.nbr_off, 2 * B.nnb)))
+        return s;
+    return FS_OK;
+}
+
+// pair_emax, for the pipelined assembly.
+int pair_order(fs_model *m, Block &B) {
+    if ((int64_t)B.pair_emax.size() == B.npairs) return FS_OK;
+    const int nblk = m->nen * (m->nen + 1) / 2;
+    HostArray<int32_t> list;
+    int s;
+    if ((s = host_copy(m->ctx, B.h_cptr, B.contrib_ptr, B.npairs + 1)) ||
+        (s = host_copy(m->ctx, list, B.contrib, B.ncontrib)))
+        return s;
+    B.pair_emax.assign(B.npairs, -1);
+    for (int64_t p = 0; p < B.npairs; ++p) {
+        if (B.h_cptr[p + 1] > B.h_cptr[p]) B.pair_emax[p] = (list[B.h_cptr[p + 1] - 1] >> 1) / nblk;  // its last element
+        if (p) B.pair_emax[p] = std::max(B.pair_emax[p], B.pair_emax[p - 1]);
+    }
     return FS_OK;
 }
 
@@ -1043,7 +936,14 @@ int build_patches(fs_model *m) {
     const int64_t N = m->N;
     constexpr int PN = fs::PATCH_NODES;
     if (N >= (int64_t(1) << 27)) return FS_OK;
-    auto active = [&](int64_t I) { return B.h_node_rec[4 * I] >= 0; };  // node with free dofs
+    std::vector<uint8_t> act(N);
+    parallel_chunks(N, [&](int64_t I0, int64_t I1) {
+        for (int64_t I = I0; I < I1; ++I) {
+            act[I] = 0;
+            for (int cc = 0; cc < 6; ++cc) act[I] |= m->dof[I * 6 + cc] < m->nfree;
+        }
+    });
+    auto active = [&](int64_t I) { return act[I] != 0; };  // node with free dofs
     auto degree = [&](int64_t I) { return m->nbr_ptr[I + 1] - m->nbr_ptr[I]; };
     // coordinates, copied while the components are found
     HostArray<double> xyz = host_array<double>(3 * N);
@@ -1274,6 +1174,8 @@ int build_tiles(fs_model *m, int which, int NE) {
     const int nblk = nen * (nen + 1) / 2;
     const int64_t E = m->E, N = m->N;
     if (NE > 32 || nblk > 16) return fail(c, FS_ERR_UNSUPPORTED, "fused assembly: tile of %d elements", NE);
+    int s;
+    if ((s = host_plan(c, B))) return s;
     // components: union-find over the nodes of each element
     std::vector<int32_t> par(N);
     for (int64_t i = 0; i < N; ++i) par[i] = (int32_t)i;
@@ -2305,10 +2207,13 @@ int fs_model_pattern_get(fs_model *m, int block, int64_t *rowptr, int64_t *colva
     int s = fs_model_pattern(m, block, nullptr, nullptr);
     if (s) return s;
     const Block &B = m->blk[block];
-    if (rowptr)
+    if (rowptr) {
+        HostArray<int32_t> rp;
+        if ((s = host_copy(m->ctx, rp, B.rowptr, B.nrows + 1))) return s;
         parallel_chunks(B.nrows + 1, [&](int64_t i0, int64_t i1) {
-            for (int64_t i = i0; i < i1; ++i) rowptr[i] = B.rowptr[i] + index_base;
+            for (int64_t i = i0; i < i1; ++i) rowptr[i] = (int64_t)rp[i] + index_base;
         });
+    }
     if (colval && B.nnz) {
         // written on the device and copied out in windows of positions, so
         // that the scratch stays within PATTERN_WINDOW entries (less where
@@ -2423,6 +2328,7 @@ int fs_model_stiffness(fs_model *m, const fs_shell_params *p, int block, double 
     }
     if (!c->stream2) FS_HIP(c, hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking));
     const bool piped = nranges > 1;
+    if (piped && (s = pair_order(m, B))) return s;
     hipEvent_t t0, t1, t2;
     FS_HIP(c, hipEventCreate(&t0));
     FS_HIP(c, hipEventCreate(&t1));

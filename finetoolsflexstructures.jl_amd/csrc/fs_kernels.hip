@@ -1425,6 +1425,327 @@ __global__ __launch_bounds__(SC_WG) void scatter_pair_kernel(ScatterPlan sp, con
     write_pair_row(sp, I, J, kI, kJ, r, sum, vals);
 }
 
+// ---------------------------------------------------------------------------
+// Pattern and scatter plan of a block
+//
+//   plan_codes_kernel   per node: runs of its free and fixed dofs (thread per node)
+//   plan_runs_kernel    per neighbour slot: offsets of its runs in the row
+//   plan_rowlen_kernel  per row: its length
+//   scan_*_kernel       exclusive prefix sum: row pointers, pair and list starts
+//   plan_rows_kernel    per node: its rows' starts and the records made of them
+//   plan_diag_kernel    per node: its own slot, upper neighbours
+//   plan_pairs_kernel   per upper pair: nodes, slots, contributions counted
+//   plan_contrib_kernel per upper pair: its contributions
+//   plan_slots_kernel   per neighbour slot: run records of the row products
+//
+// Lists are short (7 to 9 neighbours, 2 to 6 elements), so each lane walks its
+// own and all of it is bound by the latency of a few dependent loads.  A call
+// plans 263,000 nodes (512 x 512 Q4) in 0.87 ms, where 16 host threads and the
+// upload of their tables took 29 ms, 12,600 in 0.5 ms (3.5) and 1,089 in 0.15 ms
+// (0.33); half of the kernels' time is plan_runs_kernel (154 us, 33 us).
+// ---------------------------------------------------------------------------
+
+__global__ __launch_bounds__(256) void plan_codes_kernel(int64_t N, int64_t nrows, int64_t nfree,
+                                                         const int64_t *__restrict__ dof, int8_t *__restrict__ code,
+                                                         int64_t *__restrict__ first, int32_t *__restrict__ count,
+                                                         PlanTotals *__restrict__ tot) {
+    const int64_t I = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (I >= N) return;
+    int64_t lo[2] = {INT64_MAX, INT64_MAX}, hi[2] = {-1, -1};
+    int n[2] = {0, 0};
+    int64_t d[6];
+    for (int c = 0; c < 6; ++c) {
+        d[c] = dof[I * 6 + c];
+        if (d[c] >= nrows) continue;
+        const int k = d[c] < nfree ? 0 : 1;
+        lo[k] = min(lo[k], d[c]);
+        hi[k] = max(hi[k], d[c]);
+        ++n[k];
+    }
+    // the dofs of a run are distinct: consecutive if their span is their count
+    for (int k = 1; k >= 0; --k)
+        if (n[k] && hi[k] - lo[k] + 1 != n[k]) atomicMin(&tot->bad, (unsigned long long)(2 * I + k));
+    for (int c = 0; c < 6; ++c)
+        code[I * 6 + c] = d[c] >= nrows ? -1 : (int8_t)(d[c] < nfree ? d[c] - lo[0] : 8 + d[c] - lo[1]);
+    first[2 * I] = lo[0];
+    first[2 * I + 1] = lo[1];
+    count[I] = n[0] | n[1] << 4;
+}
+
+// Eight lanes a node.  The runs are contiguous ranges of dofs, so a row's
+// sorted columns are its runs in the order of their first dof: the offset of a
+// run is the sum of the lengths of those before it.  That is a square of the
+// list's length: the host sorts the lists of more than PLAN_HUB nodes.
+__global__ __launch_bounds__(256) void plan_runs_kernel(int64_t N, const int32_t *__restrict__ nbr_ptr,
+                                                        const int32_t *__restrict__ nbr,
+                                                        const int64_t *__restrict__ first,
+                                                        const int32_t *__restrict__ count, int32_t *__restrict__ off,
+                                                        int32_t *__restrict__ rowlen, PlanTotals *__restrict__ tot) {
+    const int64_t I = (int64_t)blockIdx.x * 32 + threadIdx.x / 8;
+    if (I >= N) return;
+    const int k0 = nbr_ptr[I], k1 = nbr_ptr[I + 1];
+    if (k1 - k0 > PLAN_HUB) return;
+    for (int k = k0 + threadIdx.x % 8; k < k1; k += 8) {
+        const int J = nbr[k], n = count[J];
+        const int64_t f = first[2 * (int64_t)J], x = first[2 * (int64_t)J + 1];
+        int of = 0, ox = 0;
+        for (int q = k0; q < k1; ++q) {
+            const int64_t L = nbr[q];
+            const int m = count[L];
+            const int64_t g = first[2 * L], y = first[2 * L + 1];
+            of += (g < f ? m & 15 : 0) + (y < f ? m >> 4 : 0);
+            ox += (g < x ? m & 15 : 0) + (y < x ? m >> 4 : 0);
+        }
+        off[2 * (int64_t)k] = n & 15 ? of : -1;
+        off[2 * (int64_t)k + 1] = n >> 4 ? ox : -1;
+    }
+    if (threadIdx.x % 8) return;
+    int len = 0;
+    for (int q = k0; q < k1; ++q) {
+        const int m = count[nbr[q]];
+        len += (m & 15) + (m >> 4);
+    }
+    rowlen[I] = len;
+    // most nodes raise neither maximum: look before the atomic
+    if (len > *(volatile int *)&tot->max_any) atomicMax(&tot->max_any, len);
+    if ((count[I] & 15) && len > *(volatile int *)&tot->max_free) atomicMax(&tot->max_free, len);
+}
+
+__global__ __launch_bounds__(256) void plan_rowlen_kernel(int64_t N, int64_t nrows, const int64_t *__restrict__ dof,
+                                                          const int32_t *__restrict__ rowlen,
+                                                          int32_t *__restrict__ len) {
+    const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (q >= 6 * N) return;
+    const int64_t d = dof[q];
+    if (d < nrows) len[d] = rowlen[q / 6];
+}
+
+// Exclusive prefix sum in place: tiles of 2048 (eight values a thread), then the
+// tiles' sums in one workgroup, then their addition.  v[n] gets the total; the
+// sums of tiles, and the total in tot, have 64 bits.
+constexpr int SCAN_TILE = 2048;
+
+__global__ __launch_bounds__(256) void scan_tile_kernel(int64_t n, int32_t *__restrict__ v,
+                                                        int64_t *__restrict__ sums) {
+    __shared__ int64_t part[256];
+    const int t = threadIdx.x;
+    const int64_t i0 = (int64_t)blockIdx.x * SCAN_TILE + t * 8;
+    int32_t x[8];
+    int64_t s = 0;
+    for (int k = 0; k < 8; ++k) {
+        x[k] = i0 + k < n ? v[i0 + k] : 0;
+        s += x[k];
+    }
+    part[t] = s;
+    __syncthreads();
+    for (int w = 1; w < 256; w <<= 1) {
+        const int64_t a = t >= w ? part[t - w] : 0;
+        __syncthreads();
+        part[t] += a;
+        __syncthreads();
+    }
+    int64_t run = part[t] - s;
+    for (int k = 0; k < 8; ++k) {
+        if (i0 + k < n) v[i0 + k] = (int32_t)run;
+        run += x[k];
+    }
+    if (t == 255) sums[blockIdx.x] = part[255];
+}
+
+__global__ __launch_bounds__(1024) void scan_sums_kernel(int64_t n, int64_t *__restrict__ sums,
+                                                         int64_t *__restrict__ tot) {
+    __shared__ int64_t part[1024];
+    const int t = threadIdx.x;
+    int64_t base = 0;
+    for (int64_t i0 = 0; i0 < n; i0 += 1024) {
+        const int64_t x = i0 + t < n ? sums[i0 + t] : 0;
+        part[t] = x;
+        __syncthreads();
+        for (int w = 1; w < 1024; w <<= 1) {
+            const int64_t a = t >= w ? part[t - w] : 0;
+            __syncthreads();
+            part[t] += a;
+            __syncthreads();
+        }
+        if (i0 + t < n) sums[i0 + t] = base + part[t] - x;
+        base += part[1023];
+        __syncthreads();
+    }
+    if (t == 0) {
+        sums[n] = base;
+        if (tot) *tot = base;
+    }
+}
+
+__global__ __launch_bounds__(256) void scan_add_kernel(int64_t n, int32_t *__restrict__ v,
+                                                       const int64_t *__restrict__ sums, int64_t ntiles) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n)
+        v[i] += (int32_t)sums[i / SCAN_TILE];
+    else if (i == n)
+        v[n] = (int32_t)sums[ntiles];
+}
+
+// Starts of a node's rows, its record (starts of the first free and the first
+// fixed row, row length, codes), and for the free-free block the run records of
+// its rows (RunRows); isfree counts the nodes with free dofs before the scan.
+__global__ __launch_bounds__(256) void plan_rows_kernel(int64_t N, int64_t nrows, const int64_t *__restrict__ dof,
+                                                        const int8_t *__restrict__ code,
+                                                        const int64_t *__restrict__ first,
+                                                        const int32_t *__restrict__ count,
+                                                        const int32_t *__restrict__ rowlen,
+                                                        const int32_t *__restrict__ rowptr,
+                                                        const int32_t *__restrict__ nbr_ptr,
+                                                        int32_t *__restrict__ rowstart, int4 *__restrict__ node_rec,
+                                                        int4 *__restrict__ rowrec, int32_t *__restrict__ isfree) {
+    const int64_t I = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (I >= N) return;
+    const int k0 = nbr_ptr[I], k1 = nbr_ptr[I + 1], n = count[I];
+    int codes = 0;
+    for (int c = 0; c < 6; ++c) {
+        const int64_t d = dof[I * 6 + c];
+        const int rs = d < nrows ? rowptr[d] : -1;
+        rowstart[I * 6 + c] = rs;
+        if (rowrec && d < nrows) rowrec[d] = make_int4(rs, k0, k1, 0);
+        codes |= (code[I * 6 + c] & 15) << (4 * c);
+    }
+    node_rec[I] = make_int4(n & 15 ? rowptr[first[2 * I]] : -1, n >> 4 ? rowptr[first[2 * I + 1]] : -1, rowlen[I], codes);
+    if (isfree) isfree[I] = n & 15 ? 1 : 0;
+}
+
+// Node records of the free-free block (NodeRows): the nodes with free dofs in
+// order, isfree scanned.
+__global__ __launch_bounds__(256) void plan_nodes_kernel(int64_t N, const int64_t *__restrict__ first,
+                                                         const int32_t *__restrict__ count,
+                                                         const int4 *__restrict__ node_rec,
+                                                         const int32_t *__restrict__ nbr_ptr,
+                                                         const int32_t *__restrict__ isfree, int4 *__restrict__ noderec,
+                                                         int32_t *__restrict__ nodeinfo) {
+    const int64_t I = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (I >= N || !(count[I] & 15)) return;
+    const int4 r = node_rec[I];
+    const int q = isfree[I];
+    noderec[q] = make_int4(r.x, (int)first[2 * I], nbr_ptr[I], nbr_ptr[I + 1]);
+    nodeinfo[q] = r.z << 3 | (count[I] & 15);
+}
+
+__device__ __forceinline__ int slot_lower_bound(const int32_t *__restrict__ nbr, int lo, int hi, int J) {
+    while (lo < hi) {
+        const int mid = lo + (hi - lo) / 2;
+        if (nbr[mid] < J)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
+__global__ __launch_bounds__(256) void plan_diag_kernel(int64_t N, const int32_t *__restrict__ nbr_ptr,
+                                                        const int32_t *__restrict__ nbr, int32_t *__restrict__ diag,
+                                                        int32_t *__restrict__ upper) {
+    const int64_t I = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (I >= N) return;
+    const int k1 = nbr_ptr[I + 1];
+    const int k = slot_lower_bound(nbr, nbr_ptr[I], k1, (int)I);
+    diag[I] = k;
+    upper[I] = k1 - k;
+}
+
+// The contributions of the upper pair (I, J) are the elements incident to both
+// nodes, in element order: the intersection of two ascending lists, or, where
+// one is long (a hub), the elements of the shorter that hold the other node.
+template <class F>
+__device__ __forceinline__ int pair_elements(int nen, int64_t E, const int32_t *__restrict__ conn,
+                                             const int32_t *__restrict__ ne_ptr, const int32_t *__restrict__ ne_list,
+                                             int I, int J, F f) {
+    int i = ne_ptr[I], j = ne_ptr[J], n = 0;
+    const int ie = ne_ptr[I + 1], je = ne_ptr[J + 1];
+    if (max(ie - i, je - j) > 64) {
+        const bool swap = je - j < ie - i;
+        const int v = swap ? I : J, q1 = swap ? je : ie;
+        for (int q = swap ? j : i; q < q1; ++q) {
+            const int e = ne_list[q];
+            bool in = false;
+            for (int a = 0; a < nen; ++a) in |= conn[(int64_t)a * E + e] == v;
+            if (in) f(n++, e);
+        }
+        return n;
+    }
+    while (i < ie && j < je) {
+        const int a = ne_list[i], b = ne_list[j];
+        if (a == b) f(n++, a);
+        i += a <= b;
+        j += b <= a;
+    }
+    return n;
+}
+
+// Eight lanes a node; base is upper's prefix sum: the pairs (I, J >= I) are numbered
+// from base[I] in the order of I's list.
+__global__ __launch_bounds__(256) void plan_pairs_kernel(int64_t N, int nen, int64_t E,
+                                                         const int32_t *__restrict__ conn, const int32_t *__restrict__ nbr_ptr,
+                                                         const int32_t *__restrict__ nbr,
+                                                         const int32_t *__restrict__ diag,
+                                                         const int32_t *__restrict__ base,
+                                                         const int32_t *__restrict__ ne_ptr,
+                                                         const int32_t *__restrict__ ne_list,
+                                                         int32_t *__restrict__ nbr_pair, int32_t *__restrict__ pair_node,
+                                                         int32_t *__restrict__ pair_slot, int32_t *__restrict__ ncontrib) {
+    const int64_t I = (int64_t)blockIdx.x * 32 + threadIdx.x / 8;
+    if (I >= N) return;
+    const int k1 = nbr_ptr[I + 1], kd = diag[I];
+    for (int k = kd + threadIdx.x % 8; k < k1; k += 8) {
+        const int J = nbr[k];
+        const int64_t p = (int64_t)base[I] + (k - kd);
+        const int kj = J == I ? k : slot_lower_bound(nbr, nbr_ptr[J], diag[J], (int)I);
+        pair_node[2 * p] = (int)I;
+        pair_node[2 * p + 1] = J;
+        pair_slot[2 * p] = k;
+        pair_slot[2 * p + 1] = kj;
+        nbr_pair[k] = (int)(p << 1);
+        if (J != I) nbr_pair[kj] = (int)(p << 1) | 1;
+        ncontrib[p] = pair_elements(nen, E, conn, ne_ptr, ne_list, (int)I, J, [](int, int) {});
+    }
+}
+
+// Local block of the contribution: the upper pairs of an element's nodes in row
+// order, and whether the block's row node is the pair's J (transposed).
+__global__ __launch_bounds__(256) void plan_contrib_kernel(int64_t npairs, int nen, int64_t E,
+                                                           const int32_t *__restrict__ conn,
+                                                           const int32_t *__restrict__ pair_node,
+                                                           const int32_t *__restrict__ ne_ptr,
+                                                           const int32_t *__restrict__ ne_list,
+                                                           const int32_t *__restrict__ contrib_ptr,
+                                                           int32_t *__restrict__ contrib) {
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (p >= npairs) return;
+    const int I = pair_node[2 * p], J = pair_node[2 * p + 1];
+    const int nblk = nen * (nen + 1) / 2;
+    int32_t *out = contrib + contrib_ptr[p];
+    pair_elements(nen, E, conn, ne_ptr, ne_list, I, J, [&](int n, int e) {
+        int a = 0, b = 0;
+        for (int q = 0; q < nen; ++q) {
+            const int v = conn[(int64_t)q * E + e];
+            if (v == I) a = q;
+            if (v == J) b = q;
+        }
+        const int lo = min(a, b), hi = max(a, b);
+        const int bl = lo * nen - lo * (lo - 1) / 2 + (hi - lo);
+        out[n] = (int32_t)((((int64_t)e * nblk + bl) << 1) | (a > b ? 1 : 0));
+    });
+}
+
+__global__ __launch_bounds__(256) void plan_slots_kernel(int64_t nnb, const int32_t *__restrict__ nbr,
+                                                         const int64_t *__restrict__ first,
+                                                         const int32_t *__restrict__ count,
+                                                         const int32_t *__restrict__ off, int2 *__restrict__ slotrec) {
+    const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (k >= nnb) return;
+    const int64_t J = nbr[k];
+    const int nf = count[J] & 15;  // none: an empty run
+    slotrec[k] = nf ? make_int2(off[2 * k] << 4 | nf, (int)first[2 * J]) : make_int2(0, 0);
+}
+
 constexpr int PCOL_WG = 256;
 // Column numbers of a block's CSR positions [w0, w1), into col[pos - w0].  All
 // rows of a node hold the same columns, its neighbours' runs at their offsets
@@ -3804,6 +4125,57 @@ hipError_t launch_scatter(const ScatterPlan &sp, const double *Kb, double *vals,
     if (threads == 0) return hipSuccess;
     hipLaunchKernelGGL(scatter_pair_kernel, dim3((unsigned)((threads + SC_WG - 1) / SC_WG)), dim3(SC_WG), 0, st, sp, Kb,
                        vals);
+    return hipGetLastError();
+}
+
+namespace {
+unsigned blocks_of(int64_t n, int per) { return (unsigned)((n + per - 1) / per); }
+
+// Exclusive prefix sum of v[0, n) in place, the total in v[n]; sums: scan_tiles(n) + 1 values.
+void launch_scan(int64_t n, int32_t *v, int64_t *sums, int64_t *tot, hipStream_t st) {
+    const int64_t nt = (n + SCAN_TILE - 1) / SCAN_TILE;
+    if (nt) hipLaunchKernelGGL(scan_tile_kernel, dim3((unsigned)nt), dim3(256), 0, st, n, v, sums);
+    hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(1024), 0, st, nt, sums, tot);
+    hipLaunchKernelGGL(scan_add_kernel, dim3(blocks_of(n + 1, 256)), dim3(256), 0, st, n, v, sums, nt);
+}
+}  // namespace
+
+int64_t scan_tiles(int64_t n) { return (n + SCAN_TILE - 1) / SCAN_TILE; }
+
+// Row structure: codes, runs and row pointers (rowptr: nrows + 1), and the totals.
+hipError_t launch_plan_rows(const PlanArgs &a, hipStream_t st) {
+    const dim3 wg(256);
+    hipLaunchKernelGGL(plan_codes_kernel, dim3(blocks_of(a.N, 256)), wg, 0, st, a.N, a.nrows, a.nfree, a.dof, a.code,
+                       a.first, a.count, a.tot);
+    hipLaunchKernelGGL(plan_runs_kernel, dim3(blocks_of(a.N, 32)), wg, 0, st, a.N, a.nbr_ptr, a.nbr, a.first, a.count,
+                       a.off, a.rowlen, a.tot);
+    hipLaunchKernelGGL(plan_rowlen_kernel, dim3(blocks_of(6 * a.N, 256)), wg, 0, st, a.N, a.nrows, a.dof, a.rowlen,
+                       a.rowptr);
+    launch_scan(a.nrows, a.rowptr, a.sums, &a.tot->nnz, st);
+    return hipGetLastError();
+}
+
+// The rest of the plan, once the totals are known to fit.
+hipError_t launch_plan_pairs(const PlanArgs &a, hipStream_t st) {
+    const dim3 wg(256), nodes(blocks_of(a.N, 256));
+    hipLaunchKernelGGL(plan_rows_kernel, nodes, wg, 0, st, a.N, a.nrows, a.dof, a.code, a.first, a.count, a.rowlen,
+                       a.rowptr, a.nbr_ptr, a.rowstart, a.node_rec, a.rowrec, a.isfree);
+    if (a.isfree) {
+        launch_scan(a.N, a.isfree, a.sums, nullptr, st);
+        hipLaunchKernelGGL(plan_nodes_kernel, nodes, wg, 0, st, a.N, a.first, a.count, a.node_rec, a.nbr_ptr, a.isfree,
+                           a.noderec, a.nodeinfo);
+        if (a.nnb)
+            hipLaunchKernelGGL(plan_slots_kernel, dim3(blocks_of(a.nnb, 256)), wg, 0, st, a.nnb, a.nbr, a.first,
+                               a.count, a.off, a.slotrec);
+    }
+    hipLaunchKernelGGL(plan_diag_kernel, nodes, wg, 0, st, a.N, a.nbr_ptr, a.nbr, a.diag, a.base);
+    launch_scan(a.N, a.base, a.sums, nullptr, st);
+    hipLaunchKernelGGL(plan_pairs_kernel, dim3(blocks_of(a.N, 32)), wg, 0, st, a.N, a.nen, a.E, a.conn, a.nbr_ptr, a.nbr, a.diag,
+                       a.base, a.ne_ptr, a.ne_list, a.nbr_pair, a.pair_node, a.pair_slot, a.contrib_ptr);
+    launch_scan(a.npairs, a.contrib_ptr, a.sums, nullptr, st);
+    if (a.npairs)
+        hipLaunchKernelGGL(plan_contrib_kernel, dim3(blocks_of(a.npairs, 256)), wg, 0, st, a.npairs, a.nen, a.E, a.conn,
+                           a.pair_node, a.ne_ptr, a.ne_list, a.contrib_ptr, a.contrib);
     return hipGetLastError();
 }
 

@@ -40,10 +40,11 @@ def footprint_bytes(nen, nelem, nnodes, nrows, kind):
     nnz = nrows * per_row
     mesh = nnodes * (24 + 24 + 1 + 48 + 4 + 6 + 24 + 3 * 4 * 8) + nelem * nen * 12
     blocks = nelem * nblk * (36 * 8 + 4)
-    csr = nnz * 12 + nrows * 16
+    csr = nnz * 12 + nrows * 20 + nnodes * 120
+    cols = 0 if kind == EXPLICIT else min(nnz * 8, 64 << 20)  # the window the columns are written to
     vec = nrows * 8 * (11 if kind == EXPLICIT else 1)
     patch = nnz * 6 if kind == EXPLICIT else 0  # 0.67 of the values, entry tables
-    return int(1.25 * (mesh + blocks + csr + vec + patch)) + (4 << 20)
+    return int(1.25 * (mesh + blocks + csr + cols + vec + patch)) + (4 << 20)
 
 
 class Request:

@@ -5,12 +5,28 @@ structural union built with scipy (equal), the values with their transpose
 (bitwise: both triangles come from one sum)."""
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
-from test_gpu_pattern import _reference
+import test_gpu_cd_forms as CF
 from flexshell import _lib, femm as FM
 from flexshell.material import MatDeforElastIso
 
 pytestmark = pytest.mark.gpu
+
+
+def _reference(conn, dofnums, nrows):
+    """Union of the element dof pairs below nrows (counts in 32 bits: a hub may
+    have a multiple of 256 elements)."""
+    E, nen = conn.shape
+    inc = sp.csr_matrix((np.ones(E * nen, dtype=np.int32), (np.repeat(np.arange(E), nen), conn.ravel())),
+                        shape=(E, dofnums.shape[0]))
+    adj = (inc.T @ inc).tocoo()
+    r = np.repeat(dofnums[adj.row], 6, axis=1)
+    c = np.tile(dofnums[adj.col], (1, 6))
+    keep = (r < nrows) & (c < nrows)
+    pat = sp.csr_matrix((np.ones(int(keep.sum()), dtype=np.int8), (r[keep], c[keep])), shape=(nrows, nrows))
+    pat.sort_indices()
+    return pat
 
 
 class _Dofs:
@@ -61,3 +77,31 @@ def test_pattern_and_values_by_size(ctx, nen, nx, ny, ff):
     nr, rp, cv = f._model.pattern(_lib.FS_BLOCK_FF)
     Pf = _reference(conn, d.dofnums, nf)
     assert np.array_equal(rp, Pf.indptr) and np.array_equal(cv, Pf.indices)
+
+
+# spokes: element lists of a hub around 64 (the two ways to intersect them), its
+# neighbour list around 256 (ordered by the kernel or by the host), and far past both
+@pytest.mark.parametrize("spokes", [64, 65, 255, 256, 700])
+@pytest.mark.parametrize("mode", [0, 1])
+def test_hub(ctx, spokes, mode):
+    print(f"[gpu] hub of {spokes} mode {mode}", flush=True)
+    nen, xyz, conn, d = CF._fan_t3(spokes)
+    ctx.set_assembly(mode)
+    try:
+        f = FM.FEMMShellT3FF(conn, MatDeforElastIso(210e9, 0.3, 7850.0), thickness=0.01, ctx=ctx)
+        f.associategeometry(xyz)
+        Ke = f.element_matrices(xyz, d)
+        for asm, n in ((FM.SysmatAssemblerFFBlock(d.nfreedofs), d.nfreedofs),
+                       (FM.SysmatAssemblerSparseCSRSymm(), d.nalldofs)):
+            K = f.stiffness(asm, xyz, None, None, d)
+            P = _reference(conn, d.dofnums, n)
+            assert np.array_equal(K.indptr, P.indptr) and np.array_equal(K.indices, P.indices)
+            q = d.dofnums[conn].reshape(len(conn), 18)
+            r, c = np.repeat(q, 18, axis=1).ravel(), np.tile(q, (1, 18)).ravel()
+            keep = (r < n) & (c < n)
+            S, A = (sp.coo_matrix((v.ravel()[keep], (r[keep], c[keep])), shape=(n, n)).toarray()
+                    for v in (Ke, np.abs(Ke)))
+            # each sum of at most `spokes` terms is within spokes * eps of the sum of magnitudes
+            assert np.all(np.abs(K.toarray() - S) <= 2 * spokes * np.finfo(float).eps * A)
+    finally:
+        ctx.set_assembly(1)
