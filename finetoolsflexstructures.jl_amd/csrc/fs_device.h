@@ -161,6 +161,9 @@ struct ScatterPlan {
     const int32_t *pair_slot;     // 2 * npairs: kI, kJ
 };
 
+// Longest neighbour list that node_neighbours_kernel makes.
+constexpr int NBR_MAX = 32;
+
 // Longest neighbour list that the planner's kernels order (plan_runs_kernel).
 constexpr int PLAN_HUB = 256;
 

@@ -40,6 +40,8 @@ int element_variants(int nen);
 void element_variant_shape(int nen, int variant, int *ne, int *wg);
 hipError_t launch_scatter(const ScatterPlan &sp, const double *Kb, double *vals, hipStream_t st);
 int64_t scan_tiles(int64_t n);
+hipError_t launch_neighbours(bool fill, int64_t N, int nen, int64_t E, const int32_t *conn, const int32_t *ne_ptr,
+                             const int32_t *ne_list, int32_t *nbr_ptr, int32_t *nbr, int64_t *sums, hipStream_t st);
 hipError_t launch_plan_rows(const PlanArgs &a, hipStream_t st);
 hipError_t launch_plan_pairs(const PlanArgs &a, hipStream_t st);
 hipError_t launch_pattern_cols(const ScatterPlan &sp, const int64_t *node_dof, int base, int64_t w0, int64_t w1,
@@ -293,7 +295,8 @@ struct Block {
     // complete once the elements [0, e) are (host)
     std::vector<int32_t> pair_emax;
     int64_t nnb = 0, ncontrib = 0;  // neighbour slots, contributions
-    DevBuf rowptr, nbr_ptr, nbr_node, nbr_pair, nbr_off, node_code, node_rowstart, node_rec, contrib_ptr, contrib,
+    const int32_t *nbr_ptr = nullptr, *nbr_node = nullptr;  // the model's lists (device)
+    DevBuf rowptr, nbr_pair, nbr_off, node_code, node_rowstart, node_rec, contrib_ptr, contrib,
         pair_node, pair_slot;
     // device values (CSR order) and, for the free-free block, the run records
     // of the row products of the time loop (fs::RunRows)
@@ -325,7 +328,7 @@ struct Block {
         nrows = nnz = npairs = nrownodes = nnb = ncontrib = 0;
         max_rowlen = 0;
         pair_emax.clear();
-        for (DevBuf *b : {&rowptr, &nbr_ptr, &nbr_node, &nbr_pair, &nbr_off, &node_code, &node_rowstart, &node_rec,
+        for (DevBuf *b : {&rowptr, &nbr_pair, &nbr_off, &node_code, &node_rowstart, &node_rec,
                           &contrib_ptr, &contrib, &pair_node, &pair_slot, &rowrec, &slotrec, &kval, &mdiag, &noderec, &nodeinfo})
             b->release();
     }
@@ -377,8 +380,12 @@ struct fs_model {
     int64_t N = 0, E = 0;
     std::vector<int32_t> conn;       // E x nen row-major, 0-based (host)
     std::vector<int32_t> ne_ptr, ne_list;  // node -> elements (ascending)
-    std::vector<int32_t> nbr_ptr, nbr_list;  // node -> neighbour nodes (sorted)
-    DevBuf x, y, z, dconn, dne_ptr, dne_list, nx, ny, nz, valid, node_dof, Kb, status;
+    // node -> neighbour nodes, itself among them (sorted): on the device, and on
+    // the host once a host planner has asked for them (host_lists)
+    int64_t nnb = 0;
+    std::unique_ptr<int32_t[]> nbr_ptr, nbr_list;
+    DevBuf x, y, z, dconn, dne_ptr, dne_list, dnbr_ptr, dnbr_list, nx, ny, nz, valid, node_dof, Kb, status;
+    bool hubs = false;  // a node has more elements than node_neighbours_kernel takes
     bool normals_ready = false;
     bool dofs_ready = false;
     std::vector<int64_t> dof;  // N x 6 row-major, 0-based
@@ -656,6 +663,85 @@ void cm2rm(int n, const double *cm, double *rm) {
         for (int j = 0; j < n; ++j) rm[i * n + j] = cm[j * n + i];
 }
 
+// A device array of a plan, copied to the host once; not zeroed first,
+// so that the threads of the copy touch its pages.
+template <class T>
+int host_copy(fs_ctx *c, HostArray<T> &v, const DevBuf &b, int64_t n) {
+    if (v) return FS_OK;
+    v = host_array<T>(n);
+    const int s = d2h(c, v.get(), b.p, n * sizeof(T));
+    if (s) v.reset();
+    return s;
+}
+
+// Host copies of the neighbour lists.
+int host_lists(fs_model *m) {
+    const int s = host_copy(m->ctx, m->nbr_ptr, m->dnbr_ptr, m->N + 1);
+    return s ? s : host_copy(m->ctx, m->nbr_list, m->dnbr_list, m->nnb);
+}
+
+// Node -> neighbour lists (sorted, including the node itself); a node in no
+// element has none: its rows stay empty, as in the COO assembly.  Made by a kernel
+// unless a node has more elements than NBR_MAX neighbours can come from; then on
+// the host, in two passes over the nodes (sizes, then lists).
+int make_neighbours(fs_model *m) {
+    fs_ctx *c = m->ctx;
+    const int nen = m->nen;
+    const int64_t N = m->N;
+    int s;
+    int32_t most = 0, nnb = 0;
+    for (int64_t n = 0; n < N; ++n) most = std::max(most, m->ne_ptr[n + 1] - m->ne_ptr[n]);
+    m->hubs = (int64_t)most * (nen - 1) + 1 > fs::NBR_MAX;
+    if (!m->hubs) {
+        DevBuf sums;
+        if ((s = dalloc(c, m->dnbr_ptr, (N + 1) * 4)) || (s = dalloc(c, sums, (fs::scan_tiles(N) + 1) * 8))) return s;
+        auto launch = [&](bool fill) {
+            return fs::launch_neighbours(fill, N, nen, m->E, m->dconn.as<int32_t>(), m->dne_ptr.as<int32_t>(),
+                                         m->dne_list.as<int32_t>(), m->dnbr_ptr.as<int32_t>(),
+                                         m->dnbr_list.as<int32_t>(), sums.as<int64_t>(), c->stream);
+        };
+        FS_HIP(c, launch(false));
+        if ((s = d2h(c, &nnb, m->dnbr_ptr.as<int32_t>() + N, 4)) || (s = dalloc(c, m->dnbr_list, (size_t)nnb * 4)))
+            return s;
+        m->nnb = nnb;
+        FS_HIP(c, launch(true));
+        FS_HIP(c, hipStreamSynchronize(c->stream));
+        return FS_OK;
+    }
+    m->nbr_ptr = host_array<int32_t>(N + 1);
+    auto neighbours = [&](int64_t n, std::vector<int32_t> &tmp) {
+        tmp.clear();
+        for (int k = m->ne_ptr[n]; k < m->ne_ptr[n + 1]; ++k) {
+            const int e = m->ne_list[k];
+            for (int a = 0; a < nen; ++a) tmp.push_back(m->conn[(int64_t)e * nen + a]);
+        }
+        std::sort(tmp.begin(), tmp.end());
+        tmp.erase(std::unique(tmp.begin(), tmp.end()), tmp.end());
+    };
+    m->nbr_ptr[0] = 0;
+    parallel_chunks(N, [&](int64_t n0, int64_t n1) {
+        std::vector<int32_t> tmp;
+        for (int64_t n = n0; n < n1; ++n) {
+            neighbours(n, tmp);
+            m->nbr_ptr[n + 1] = (int32_t)tmp.size();
+        }
+    });
+    for (int64_t n = 0; n < N; ++n) m->nbr_ptr[n + 1] += m->nbr_ptr[n];
+    m->nnb = m->nbr_ptr[N];
+    m->nbr_list = host_array<int32_t>(m->nnb);
+    parallel_chunks(N, [&](int64_t n0, int64_t n1) {
+        std::vector<int32_t> tmp;
+        for (int64_t n = n0; n < n1; ++n) {
+            neighbours(n, tmp);
+            std::copy(tmp.begin(), tmp.end(), m->nbr_list.get() + m->nbr_ptr[n]);
+        }
+    });
+    if ((s = upload(c, m->dnbr_ptr, m->nbr_ptr.get(), N + 1)) || (s = upload(c, m->dnbr_list, m->nbr_list.get(), m->nnb)))
+        return s;
+    FS_HIP(c, hipStreamSynchronize(c->stream));
+    return FS_OK;
+}
+
 // Pattern, scatter plan and records of the row products of a block, planned on
 // the device from the node lists and the dof numbers (fs::PlanArgs); the
 // host reads the totals between the two parts, and copies of the plan only where
@@ -674,10 +760,10 @@ int build_block(fs_model *m, int which) {
     a.nen = m->nen;
     a.nrows = ff ? m->nfree : m->nall;
     a.nfree = m->nfree;
-    a.nnb = (int64_t)m->nbr_list.size();
+    a.nnb = m->nnb;
     // every node in an element is its own neighbour, and neighbours are mutual
     int64_t used = 0;
-    for (int64_t I = 0; I < N; ++I) used += m->nbr_ptr[I + 1] > m->nbr_ptr[I];
+    for (int64_t I = 0; I < N; ++I) used += m->ne_ptr[I + 1] > m->ne_ptr[I];
     a.npairs = (a.nnb + used) / 2;
     DevBuf tot, sums, first, count, rowlen, diag, base, isfree;
     fs::PlanTotals t{UINT64_MAX, 0, 0, 0};
@@ -685,8 +771,6 @@ int build_block(fs_model *m, int which) {
     int s;
     if ((s = dalloc(c, tot, sizeof t)) || (s = dalloc(c, sums, (fs::scan_tiles(longest) + 1) * 8)) ||
         (s = dalloc(c, first, 2 * N * 8)) || (s = dalloc(c, count, N * 4)) || (s = dalloc(c, rowlen, N * 4)) ||
-        (s = upload(c, B.nbr_ptr, m->nbr_ptr.data(), m->nbr_ptr.size())) ||
-        (s = upload(c, B.nbr_node, m->nbr_list.data(), m->nbr_list.size())) ||
         (s = dalloc(c, B.node_code, N * 6)) || (s = dalloc(c, B.nbr_off, 2 * a.nnb * 4)) ||
         (s = dalloc(c, B.rowptr, (a.nrows + 1) * 4)))
         return s;
@@ -694,8 +778,8 @@ int build_block(fs_model *m, int which) {
     a.conn = m->dconn.as<int32_t>();
     a.ne_ptr = m->dne_ptr.as<int32_t>();
     a.ne_list = m->dne_list.as<int32_t>();
-    a.nbr_ptr = B.nbr_ptr.as<int32_t>();
-    a.nbr = B.nbr_node.as<int32_t>();
+    a.nbr_ptr = B.nbr_ptr = m->dnbr_ptr.as<int32_t>();
+    a.nbr = B.nbr_node = m->dnbr_list.as<int32_t>();
     a.tot = tot.as<fs::PlanTotals>();
     a.sums = sums.as<int64_t>();
     a.code = B.node_code.as<int8_t>();
@@ -707,7 +791,7 @@ int build_block(fs_model *m, int which) {
     // the rows of nodes with long lists, which would take a lane of the kernel
     // the square of the length
     std::vector<std::vector<int32_t>> hubs;  // row length, then offsets
-    for (int64_t I = 0; I < N; ++I) {
+    for (int64_t I = 0; I < (m->hubs ? N : 0); ++I) {
         const int k0 = m->nbr_ptr[I], n = m->nbr_ptr[I + 1] - k0;
         if (n <= fs::PLAN_HUB) continue;
         hubs.emplace_back(1 + 2 * (size_t)n, -1);
@@ -796,17 +880,6 @@ int build_block(fs_model *m, int which) {
     return FS_OK;
 }
 
-// A device array of a block's plan, copied to the host once; not zeroed first,
-// so that the threads of the copy touch its pages.
-template <class T>
-int host_copy(fs_ctx *c, HostArray<T> &v, const DevBuf &b, int64_t n) {
-    if (v) return FS_OK;
-    v = host_array<T>(n);
-    const int s = d2h(c, v.get(), b.p, n * sizeof(T));
-    if (s) v.reset();
-    return s;
-}
-
 // Host copies of the plan for the planner of the fused assembly.
 int host_plan(fs_ctx *c, Block &B) {
     int s;
@@ -863,8 +936,8 @@ int node_pj(const fs_ctx *c, const Block &B) {
 fs::ScatterPlan plan_of(const Block &B) {
     fs::ScatterPlan sp;
     sp.nnodes = B.nnodes;
-    sp.nbr_ptr = B.nbr_ptr.as<int32_t>();
-    sp.nbr_node = B.nbr_node.as<int32_t>();
+    sp.nbr_ptr = B.nbr_ptr;
+    sp.nbr_node = B.nbr_node;
     sp.nbr_pair = B.nbr_pair.as<int32_t>();
     sp.nbr_off = B.nbr_off.as<int32_t>();
     sp.node_code = B.node_code.as<int8_t>();
@@ -936,6 +1009,7 @@ int build_patches(fs_model *m) {
     const int64_t N = m->N;
     constexpr int PN = fs::PATCH_NODES;
     if (N >= (int64_t(1) << 27)) return FS_OK;
+    if (const int e = host_lists(m)) return e;
     std::vector<uint8_t> act(N);
     parallel_chunks(N, [&](int64_t I0, int64_t I1) {
         for (int64_t I = I0; I < I1; ++I) {
@@ -1099,7 +1173,7 @@ int build_patches(fs_model *m) {
     // the lists on the device
     int s;
     DevBuf dorder, dstart, dslot, dtot;
-    const int32_t *nbp = B.nbr_ptr.as<int32_t>(), *nbn = B.nbr_node.as<int32_t>();
+    const int32_t *nbp = B.nbr_ptr, *nbn = B.nbr_node;
     if ((s = upload(c, dorder, order.get(), npt)) || (s = upload(c, dstart, pstart.data(), pstart.size())) ||
         (s = dalloc(c, dslot, N * 4)) || (s = dalloc(c, dtot, 32)) || (s = dalloc(c, P.dpnode, (size_t)np * PN * 4)) ||
         (s = dalloc(c, P.rec, (size_t)np * 16)) || (s = dalloc(c, P.nptr, (size_t)np * (PN + 1) * 2)))
@@ -1175,7 +1249,7 @@ int build_tiles(fs_model *m, int which, int NE) {
     const int64_t E = m->E, N = m->N;
     if (NE > 32 || nblk > 16) return fail(c, FS_ERR_UNSUPPORTED, "fused assembly: tile of %d elements", NE);
     int s;
-    if ((s = host_plan(c, B))) return s;
+    if ((s = host_plan(c, B)) || (s = host_lists(m))) return s;
     // components: union-find over the nodes of each element
     std::vector<int32_t> par(N);
     for (int64_t i = 0; i < N; ++i) par[i] = (int32_t)i;
@@ -1305,9 +1379,9 @@ int build_tiles(fs_model *m, int which, int NE) {
     }
     // pair entries per tile
     auto slot_of = [&](int64_t I, int64_t J) -> int32_t {
-        const int32_t *b0 = m->nbr_list.data() + m->nbr_ptr[I];
-        const int32_t *e0 = m->nbr_list.data() + m->nbr_ptr[I + 1];
-        return (int32_t)(std::lower_bound(b0, e0, (int32_t)J) - m->nbr_list.data());
+        const int32_t *b0 = m->nbr_list.get() + m->nbr_ptr[I];
+        const int32_t *e0 = m->nbr_list.get() + m->nbr_ptr[I + 1];
+        return (int32_t)(std::lower_bound(b0, e0, (int32_t)J) - m->nbr_list.get());
     };
     struct Ent {
         int32_t p;
@@ -1634,6 +1708,7 @@ int build_mixed(fs_model *m, bool shear_fp32) {
     const int K = 6 * nen;
     const int nsr = shear_fp32 ? 0 : nen == 3 ? (m->last_ep.formulation == FS_SHEAR_AVERAGE_K ? 6 : 2) : 8;
     const int64_t N = m->N, E = m->E, nrows = 6 * N;
+    if (const int e = host_lists(m)) return e;
     // slices of 10 nodes (60 rows): slot count = largest neighbour count of the slice's nodes
     (void)nrows;
     const int64_t ns = (N + 9) / 10;
@@ -1703,8 +1778,8 @@ fs::MixedOp mixed_op(const fs_model *m) {
     op.goff = m->mixed.goff.as<int64_t>();
     op.kmb = m->mixed.kmb.as<float2>();
     op.kml = m->mixed.kml.as<short2>();
-    op.nbr_ptr = B.nbr_ptr.as<int32_t>();
-    op.nbr_node = B.nbr_node.as<int32_t>();
+    op.nbr_ptr = B.nbr_ptr;
+    op.nbr_node = B.nbr_node;
     op.dr = m->mixed.dr.as<double>();
     op.ne_ptr = m->dne_ptr.as<int32_t>();
     op.ne_pack = m->mixed.ne_pack.as<int32_t>();
@@ -1925,35 +2000,6 @@ int fs_model_create(fs_ctx *ctx, int nen, int64_t nnodes, const double *xyz, int
         for (int64_t e = 0; e < nelem; ++e)
             for (int a = 0; a < nen; ++a) m->ne_list[fill[m->conn[e * nen + a]]++] = (int32_t)e;
     }
-    // node -> neighbour lists (sorted, including the node itself); a node in
-    // no element has no neighbours: its rows stay empty, as in the COO
-    // assembly.  Two passes over the nodes (sizes, then lists).
-    m->nbr_ptr.assign(nnodes + 1, 0);
-    auto neighbours = [&](int64_t n, std::vector<int32_t> &tmp) {
-        tmp.clear();
-        for (int k = m->ne_ptr[n]; k < m->ne_ptr[n + 1]; ++k) {
-            const int e = m->ne_list[k];
-            for (int a = 0; a < nen; ++a) tmp.push_back(m->conn[(int64_t)e * nen + a]);
-        }
-        std::sort(tmp.begin(), tmp.end());
-        tmp.erase(std::unique(tmp.begin(), tmp.end()), tmp.end());
-    };
-    parallel_chunks(nnodes, [&](int64_t n0, int64_t n1) {
-        std::vector<int32_t> tmp;
-        for (int64_t n = n0; n < n1; ++n) {
-            neighbours(n, tmp);
-            m->nbr_ptr[n + 1] = (int32_t)tmp.size();
-        }
-    });
-    for (int64_t n = 0; n < nnodes; ++n) m->nbr_ptr[n + 1] += m->nbr_ptr[n];
-    m->nbr_list.resize(m->nbr_ptr[nnodes]);
-    parallel_chunks(nnodes, [&](int64_t n0, int64_t n1) {
-        std::vector<int32_t> tmp;
-        for (int64_t n = n0; n < n1; ++n) {
-            neighbours(n, tmp);
-            std::copy(tmp.begin(), tmp.end(), m->nbr_list.begin() + m->nbr_ptr[n]);
-        }
-    });
     // device geometry (SoA) and connectivity planes
     int s;
     std::vector<int32_t> planes((size_t)nelem * nen);
@@ -1967,7 +2013,7 @@ int fs_model_create(fs_ctx *ctx, int nen, int64_t nnodes, const double *xyz, int
         (s = upload(ctx, m->dne_list, m->ne_list.data(), m->ne_list.size())) ||
         (s = dalloc(ctx, m->nx, nnodes * 8)) || (s = dalloc(ctx, m->ny, nnodes * 8)) ||
         (s = dalloc(ctx, m->nz, nnodes * 8)) || (s = dalloc(ctx, m->valid, nnodes)) ||
-        (s = dalloc(ctx, m->status, sizeof(int)))) {
+        (s = dalloc(ctx, m->status, sizeof(int))) || (s = make_neighbours(m))) {
         delete m;
         return s;
     }
@@ -3144,7 +3190,7 @@ int fs_model_mixed_info(const fs_model *m, int64_t *info) {
     const MixedStore &X = m->mixed;
     info[0] = X.built ? X.kmb_pairs : 0;
     info[1] = X.built ? X.nsr : 0;
-    info[2] = (int64_t)m->nbr_list.size();
+    info[2] = m->nnb;
     info[3] = X.built ? X.nslices : 0;
     return FS_OK;
 }

@@ -1445,6 +1445,43 @@ __global__ __launch_bounds__(SC_WG) void scatter_pair_kernel(ScatterPlan sp, con
 // (0.33); half of the kernels' time is plan_runs_kernel (154 us, 33 us).
 // ---------------------------------------------------------------------------
 
+// Neighbours of a node: the nodes of its elements, itself among them, ascending.
+// A lane keeps its node's list sorted in LDS (NBR_MAX entries, a column a lane,
+// so without bank conflicts); run once for the lengths, and, they summed up, once
+// for the lists.  12,600 nodes take 0.03 ms, 0.78 ms on one host thread (creation
+// of the model 1.0 -> 0.35 ms).
+template <bool FILL>
+__global__ __launch_bounds__(64) void node_neighbours_kernel(int64_t N, int nen, int64_t E,
+                                                             const int32_t *__restrict__ conn,
+                                                             const int32_t *__restrict__ ne_ptr,
+                                                             const int32_t *__restrict__ ne_list,
+                                                             int32_t *__restrict__ nbr_ptr, int32_t *__restrict__ nbr) {
+    __shared__ int32_t list[NBR_MAX][64];
+    const int t = threadIdx.x;
+    const int64_t I = (int64_t)blockIdx.x * 64 + t;
+    if (I >= N) return;
+    int n = 0;
+    const int k1 = ne_ptr[I + 1];
+    for (int k = ne_ptr[I]; k < k1; ++k) {
+        const int e = ne_list[k];
+        for (int a = 0; a < nen; ++a) {
+            const int J = conn[(int64_t)a * E + e];
+            int at = n;
+            while (at > 0 && list[at - 1][t] > J) --at;
+            if ((at > 0 && list[at - 1][t] == J) || n == NBR_MAX) continue;
+            for (int q = n; q > at; --q) list[q][t] = list[q - 1][t];
+            list[at][t] = J;
+            ++n;
+        }
+    }
+    if (FILL) {
+        int32_t *out = nbr + nbr_ptr[I];
+        for (int q = 0; q < n; ++q) out[q] = list[q][t];
+    } else {
+        nbr_ptr[I] = n;
+    }
+}
+
 __global__ __launch_bounds__(256) void plan_codes_kernel(int64_t N, int64_t nrows, int64_t nfree,
                                                          const int64_t *__restrict__ dof, int8_t *__restrict__ code,
                                                          int64_t *__restrict__ first, int32_t *__restrict__ count,
@@ -4141,6 +4178,20 @@ void launch_scan(int64_t n, int32_t *v, int64_t *sums, int64_t *tot, hipStream_t
 }  // namespace
 
 int64_t scan_tiles(int64_t n) { return (n + SCAN_TILE - 1) / SCAN_TILE; }
+
+// Lengths of the neighbour lists, summed up into nbr_ptr (N + 1), then the lists.
+hipError_t launch_neighbours(bool fill, int64_t N, int nen, int64_t E, const int32_t *conn, const int32_t *ne_ptr,
+                             const int32_t *ne_list, int32_t *nbr_ptr, int32_t *nbr, int64_t *sums, hipStream_t st) {
+    const dim3 grid(blocks_of(N, 64)), wg(64);
+    if (fill) {
+        hipLaunchKernelGGL(node_neighbours_kernel<true>, grid, wg, 0, st, N, nen, E, conn, ne_ptr, ne_list, nbr_ptr, nbr);
+    } else {
+        hipLaunchKernelGGL(node_neighbours_kernel<false>, grid, wg, 0, st, N, nen, E, conn, ne_ptr, ne_list, nbr_ptr,
+                           nbr);
+        launch_scan(N, nbr_ptr, sums, nullptr, st);
+    }
+    return hipGetLastError();
+}
 
 // Row structure: codes, runs and row pointers (rowptr: nrows + 1), and the totals.
 hipError_t launch_plan_rows(const PlanArgs &a, hipStream_t st) {

@@ -79,16 +79,36 @@ def test_pattern_and_values_by_size(ctx, nen, nx, ny, ff):
     assert np.array_equal(rp, Pf.indptr) and np.array_equal(cv, Pf.indices)
 
 
-# spokes: element lists of a hub around 64 (the two ways to intersect them), its
-# neighbour list around 256 (ordered by the kernel or by the host), and far past both
-@pytest.mark.parametrize("spokes", [64, 65, 255, 256, 700])
+def _fan_q4(m):
+    """m quadrilaterals around node 0, the outer nodes fixed."""
+    ang = np.pi * np.arange(2 * m) / m
+    r = np.where(np.arange(2 * m) % 2 == 0, 0.6, 1.0)
+    xyz = np.vstack([[0.0, 0.0, 0.0], np.column_stack([r * np.cos(ang), r * np.sin(ang), 0.02 * np.cos(3 * ang)])])
+    i = np.arange(m)
+    conn = np.stack([0 * i, 1 + 2 * i, 2 + 2 * i, 1 + (2 * i + 2) % (2 * m)], 1)
+    N = len(xyz)
+    fixed = np.zeros((N, 6), dtype=bool)
+    fixed[2::2] = True
+    dofs = np.empty((N, 6), dtype=np.int64)
+    nf = int((~fixed).sum())
+    dofs[~fixed], dofs[fixed] = np.arange(nf), np.arange(nf, 6 * N)
+    return 4, xyz, conn, _Dofs(dofs, nf)
+
+
+# A hub's elements, where the planning changes its form: 15 | 16 triangles and 10 |
+# 11 quadrilaterals (neighbour lists by the kernel or the host), 64 | 65 elements (two
+# ways to intersect their lists), 255 | 256 spokes (the hub's list ordered by the
+# kernel or the host), and far past all of these.
+@pytest.mark.parametrize("nen, spokes", [(3, 15), (3, 16), (4, 10), (4, 11), (3, 64), (3, 65), (3, 255), (3, 256),
+                                         (3, 700)])
 @pytest.mark.parametrize("mode", [0, 1])
-def test_hub(ctx, spokes, mode):
-    print(f"[gpu] hub of {spokes} mode {mode}", flush=True)
-    nen, xyz, conn, d = CF._fan_t3(spokes)
+def test_hub(ctx, nen, spokes, mode):
+    print(f"[gpu] hub of {spokes} nen {nen} mode {mode}", flush=True)
+    nen, xyz, conn, d = CF._fan_t3(spokes) if nen == 3 else _fan_q4(spokes)
+    cls = FM.FEMMShellT3FF if nen == 3 else FM.FEMMShellQ4RS
     ctx.set_assembly(mode)
     try:
-        f = FM.FEMMShellT3FF(conn, MatDeforElastIso(210e9, 0.3, 7850.0), thickness=0.01, ctx=ctx)
+        f = cls(conn, MatDeforElastIso(210e9, 0.3, 7850.0), thickness=0.01, ctx=ctx)
         f.associategeometry(xyz)
         Ke = f.element_matrices(xyz, d)
         for asm, n in ((FM.SysmatAssemblerFFBlock(d.nfreedofs), d.nfreedofs),
@@ -96,8 +116,8 @@ def test_hub(ctx, spokes, mode):
             K = f.stiffness(asm, xyz, None, None, d)
             P = _reference(conn, d.dofnums, n)
             assert np.array_equal(K.indptr, P.indptr) and np.array_equal(K.indices, P.indices)
-            q = d.dofnums[conn].reshape(len(conn), 18)
-            r, c = np.repeat(q, 18, axis=1).ravel(), np.tile(q, (1, 18)).ravel()
+            q = d.dofnums[conn].reshape(len(conn), 6 * nen)
+            r, c = np.repeat(q, 6 * nen, axis=1).ravel(), np.tile(q, (1, 6 * nen)).ravel()
             keep = (r < n) & (c < n)
             S, A = (sp.coo_matrix((v.ravel()[keep], (r[keep], c[keep])), shape=(n, n)).toarray()
                     for v in (Ke, np.abs(Ke)))
