@@ -44,6 +44,7 @@ hipError_t launch_neighbours(bool fill, int64_t N, int nen, int64_t E, const int
                              const int32_t *ne_list, int32_t *nbr_ptr, int32_t *nbr, int64_t *sums, hipStream_t st);
 hipError_t launch_plan_rows(const PlanArgs &a, hipStream_t st);
 hipError_t launch_plan_pairs(const PlanArgs &a, hipStream_t st);
+hipError_t launch_pattern_rows(int64_t n, const int32_t *rowptr, int base, int64_t *out, hipStream_t st);
 hipError_t launch_pattern_cols(const ScatterPlan &sp, const int64_t *node_dof, int base, int64_t w0, int64_t w1,
                                int64_t *col, hipStream_t st);
 int fused_tile_elems(int nen);
@@ -2245,7 +2246,7 @@ int fs_model_pattern(fs_model *m, int block, int64_t *nrows, int64_t *nnz) {
     return FS_OK;
 }
 
-// Column entries that fs_model_pattern_get holds on the device at a time (64 MB).
+// Pattern entries that fs_model_pattern_get holds on the device at a time (64 MB).
 static constexpr int64_t PATTERN_WINDOW = int64_t(1) << 23;
 
 int fs_model_pattern_get(fs_model *m, int block, int64_t *rowptr, int64_t *colval, int index_base) {
@@ -2253,29 +2254,25 @@ int fs_model_pattern_get(fs_model *m, int block, int64_t *rowptr, int64_t *colva
     int s = fs_model_pattern(m, block, nullptr, nullptr);
     if (s) return s;
     const Block &B = m->blk[block];
-    if (rowptr) {
-        HostArray<int32_t> rp;
-        if ((s = host_copy(m->ctx, rp, B.rowptr, B.nrows + 1))) return s;
-        parallel_chunks(B.nrows + 1, [&](int64_t i0, int64_t i1) {
-            for (int64_t i = i0; i < i1; ++i) rowptr[i] = (int64_t)rp[i] + index_base;
-        });
+    // written on the device as the caller takes them, and copied out in windows, so
+    // that the scratch stays within PATTERN_WINDOW entries (less where the device
+    // has no room for that)
+    fs_ctx *c = m->ctx;
+    DevBuf w;
+    int64_t win = std::min(std::max(B.nnz, B.nrows + 1), PATTERN_WINDOW);
+    while ((s = dalloc(c, w, (size_t)win * 8)) == FS_ERR_NOMEM && win > 65536) win = (win + 1) / 2;
+    if (s) return s;
+    c->err.clear();
+    for (int64_t i0 = 0; rowptr && i0 <= B.nrows; i0 += win) {
+        const int64_t n = std::min(B.nrows + 1 - i0, win);
+        FS_HIP(c, fs::launch_pattern_rows(n, B.rowptr.as<int32_t>() + i0, index_base, w.as<int64_t>(), c->stream));
+        if ((s = d2h(c, rowptr + i0, w.p, (size_t)n * 8))) return s;
     }
-    if (colval && B.nnz) {
-        // written on the device and copied out in windows of positions, so
-        // that the scratch stays within PATTERN_WINDOW entries (less where
-        // the device has no room for that)
-        fs_ctx *c = m->ctx;
-        DevBuf w;
-        int64_t win = std::min(B.nnz, PATTERN_WINDOW);
-        while ((s = dalloc(c, w, (size_t)win * 8)) == FS_ERR_NOMEM && win > 65536) win = (win + 1) / 2;
-        if (s) return s;
-        c->err.clear();
-        for (int64_t w0 = 0; w0 < B.nnz; w0 += win) {
-            const int64_t w1 = std::min(B.nnz, w0 + win);
-            FS_HIP(c, fs::launch_pattern_cols(plan_of(B), m->node_dof.as<int64_t>(), index_base, w0, w1,
-                                              w.as<int64_t>(), c->stream));
-            if ((s = d2h(c, colval + w0, w.p, (size_t)(w1 - w0) * 8))) return s;
-        }
+    for (int64_t w0 = 0; colval && w0 < B.nnz; w0 += win) {
+        const int64_t w1 = std::min(B.nnz, w0 + win);
+        FS_HIP(c, fs::launch_pattern_cols(plan_of(B), m->node_dof.as<int64_t>(), index_base, w0, w1, w.as<int64_t>(),
+                                          c->stream));
+        if ((s = d2h(c, colval + w0, w.p, (size_t)(w1 - w0) * 8))) return s;
     }
     return FS_OK;
 }

@@ -1772,6 +1772,13 @@ __global__ __launch_bounds__(256) void plan_contrib_kernel(int64_t npairs, int n
     });
 }
 
+// Row pointers [i0, i0 + n) as the caller takes them.
+__global__ __launch_bounds__(256) void pattern_rows_kernel(int64_t n, const int32_t *__restrict__ rowptr, int base,
+                                                           int64_t *__restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) out[i] = (int64_t)rowptr[i] + base;
+}
+
 __global__ __launch_bounds__(256) void plan_slots_kernel(int64_t nnb, const int32_t *__restrict__ nbr,
                                                          const int64_t *__restrict__ first,
                                                          const int32_t *__restrict__ count,
@@ -4227,6 +4234,11 @@ hipError_t launch_plan_pairs(const PlanArgs &a, hipStream_t st) {
     if (a.npairs)
         hipLaunchKernelGGL(plan_contrib_kernel, dim3(blocks_of(a.npairs, 256)), wg, 0, st, a.npairs, a.nen, a.E, a.conn,
                            a.pair_node, a.ne_ptr, a.ne_list, a.contrib_ptr, a.contrib);
+    return hipGetLastError();
+}
+
+hipError_t launch_pattern_rows(int64_t n, const int32_t *rowptr, int base, int64_t *out, hipStream_t st) {
+    hipLaunchKernelGGL(pattern_rows_kernel, dim3(blocks_of(n, 256)), dim3(256), 0, st, n, rowptr, base, out);
     return hipGetLastError();
 }
 

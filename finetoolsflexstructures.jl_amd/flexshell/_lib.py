@@ -300,15 +300,15 @@ class Model:
         nr, nz = C.c_int64(), C.c_int64()
         self.ctx.check(self.ctx.lib.fs_model_pattern(self.h, int(block), C.byref(nr), C.byref(nz)),
                        "fs_model_pattern")
-        rp = np.zeros(nr.value + 1, dtype=np.int64)
-        cv = np.zeros(nz.value, dtype=np.int64)
+        rp = np.empty(nr.value + 1, dtype=np.int64)  # written in full below
+        cv = np.empty(nz.value, dtype=np.int64)
         self.ctx.check(self.ctx.lib.fs_model_pattern_get(self.h, int(block), ptr(rp, C.c_int64),
                                                          ptr(cv, C.c_int64), 0), "fs_model_pattern_get")
         return nr.value, rp, cv
 
     def stiffness(self, params, block, nnz=None):
         """CSR values of the block; nnz None keeps them on the device only."""
-        out = None if nnz is None else np.zeros(nnz)
+        out = None if nnz is None else np.empty(nnz)  # written in full, or the call raises
         self.ctx.check(self.ctx.lib.fs_model_stiffness(self.h, C.byref(params), int(block), ptr(out)),
                        "fs_model_stiffness")
         return out
