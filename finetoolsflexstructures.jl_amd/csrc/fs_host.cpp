@@ -44,6 +44,8 @@ hipError_t launch_neighbours(bool fill, int64_t N, int nen, int64_t E, const int
                              const int32_t *ne_list, int32_t *nbr_ptr, int32_t *nbr, int64_t *sums, hipStream_t st);
 hipError_t launch_plan_rows(const PlanArgs &a, hipStream_t st);
 hipError_t launch_plan_pairs(const PlanArgs &a, hipStream_t st);
+hipError_t launch_tile_place(int64_t n, const int32_t *pairs, const ScatterPlan &sp, const int4 *node_rec, int4 *rec,
+                             hipStream_t st);
 hipError_t launch_pattern_rows(int64_t n, const int32_t *rowptr, int base, int64_t *out, hipStream_t st);
 hipError_t launch_pattern_cols(const ScatterPlan &sp, const int64_t *node_dof, int base, int64_t w0, int64_t w1,
                                int64_t *col, hipStream_t st);
@@ -309,21 +311,18 @@ struct Block {
     bool k_ready = false, m_ready = false;
     uint64_t vgen = 0;  // raised before each launch that writes kval
     PatchStore patch;
-    // host copies for the fused-assembly planner (host_plan): neighbour slot -> (pair <<
-    // 1 | side), pair nodes and slots, contributions per pair (counts)
-    std::unique_ptr<int32_t[]> h_nb_pair, h_pnode, h_pslot, h_cptr;
-    // per node {first free row's CSR position, first fixed row's (-1), row
-    // length, 4-bit comp codes}; per neighbour slot the free / fixed run offsets
-    std::unique_ptr<int32_t[]> h_node_rec, h_nb_off;
+    // host copies for the planner of the fused assembly (host_plan): neighbour
+    // slot -> (pair << 1 | side), pair nodes, starts of the pairs' contributions;
+    // per node {first free row's CSR position, first fixed row's (-1), row length,
+    // 4-bit comp codes}
+    std::unique_ptr<int32_t[]> h_nb_pair, h_pnode, h_cptr, h_node_rec;
     TileStore tiles;
     void reset() {
         built = k_ready = m_ready = false;
         h_nb_pair.reset();
         h_pnode.reset();
-        h_pslot.reset();
         h_cptr.reset();
         h_node_rec.reset();
-        h_nb_off.reset();
         tiles.reset();
         patch.reset();
         nrows = nnz = npairs = nrownodes = nnb = ncontrib = 0;
@@ -885,9 +884,8 @@ int build_block(fs_model *m, int which) {
 int host_plan(fs_ctx *c, Block &B) {
     int s;
     if ((s = host_copy(c, B.h_nb_pair, B.nbr_pair, B.nnb)) || (s = host_copy(c, B.h_pnode, B.pair_node, 2 * B.npairs)) ||
-        (s = host_copy(c, B.h_pslot, B.pair_slot, 2 * B.npairs)) ||
         (s = host_copy(c, B.h_cptr, B.contrib_ptr, B.npairs + 1)) ||
-        (s = host_copy(c, B.h_node_rec, B.node_rec, 4 * B.nnodes)) || (s = host_copy(c, B.h_nb_off, B.nbr_off, 2 * B.nnb)))
+        (s = host_copy(c, B.h_node_rec, B.node_rec, 4 * B.nnodes)))
         return s;
     return FS_OK;
 }
@@ -1452,22 +1450,9 @@ int build_tiles(fs_model *m, int which, int NE) {
     std::vector<int32_t> tp_ptr(ntiles + 1, 0);
     for (int64_t t = 0; t < ntiles; ++t) tp_ptr[t + 1] = tp_ptr[t] + (int32_t)tent[t].size();
     const int64_t nent = tp_ptr[ntiles];
-    // placement record of upper pair pp (fs::TilePlan trec)
-    auto place = [&](int64_t pp, int32_t *rec) {
-        const int64_t I = B.h_pnode[2 * pp], J = B.h_pnode[2 * pp + 1];
-        const int64_t kI = B.h_pslot[2 * pp], kJ = B.h_pslot[2 * pp + 1];
-        for (int k = 0; k < 4; ++k) {
-            rec[k] = B.h_node_rec[4 * I + k];
-            rec[4 + k] = B.h_node_rec[4 * J + k];
-        }
-        if (I == J) rec[3] |= 1 << 30;
-        rec[8] = B.h_nb_off[2 * kI];
-        rec[9] = B.h_nb_off[2 * kI + 1];
-        rec[10] = B.h_nb_off[2 * kJ];
-        rec[11] = B.h_nb_off[2 * kJ + 1];
-    };
-    std::vector<int32_t> trec(12 * nent), tslot(nent);
-    std::vector<uint64_t> tcw(nent);
+    // the pair of each entry; the placement records are made from them on the device
+    HostArray<int32_t> tpair = host_array<int32_t>(nent), tslot = host_array<int32_t>(nent);
+    HostArray<uint64_t> tcw = host_array<uint64_t>(nent);
     // partial slots: the slots of one boundary pair are consecutive (its
     // tiles in tile order), so the finalize reads each pair's partials as one
     // stretch
@@ -1475,12 +1460,11 @@ int build_tiles(fs_model *m, int which, int NE) {
     for (int64_t t = 0; t < ntiles; ++t)
         for (const Ent &en : tent[t])
             if (en.boundary) pcount[en.p + 1]++;
-    std::vector<int32_t> bidx(B.npairs, -1), brec, bp_ptr(1, 0);
+    std::vector<int32_t> bidx(B.npairs, -1), bpair, bp_ptr(1, 0);
     for (int64_t pp = 0; pp < B.npairs; ++pp)
         if (pcount[pp + 1]) {
             bidx[pp] = (int32_t)(bp_ptr.size() - 1);
-            brec.resize(brec.size() + 12);
-            place(pp, &brec[brec.size() - 12]);
+            bpair.push_back((int32_t)pp);
             bp_ptr.push_back(bp_ptr.back() + pcount[pp + 1]);
         }
     const int64_t nbnd = (int64_t)bp_ptr.size() - 1;
@@ -1490,23 +1474,28 @@ int build_tiles(fs_model *m, int which, int NE) {
         for (size_t i = 0; i < tent[t].size(); ++i) {
             const Ent &en = tent[t][i];
             const int64_t q = tp_ptr[t] + (int64_t)i;
-            place(en.p, &trec[12 * q]);
+            tpair[q] = en.p;
             tcw[q] = en.cw;
             tslot[q] = en.boundary ? bfill[bidx[en.p]]++ : -1;
         }
     int st;
+    DevBuf dtpair, dbpair;
     // the tiles' own connectivity (node a of tile element le at (t NE + le) nen + a)
     std::vector<int32_t> tconn(telem.size() * nen);
     for (size_t i = 0; i < telem.size(); ++i)
         for (int a = 0; a < nen; ++a) tconn[i * nen + a] = m->conn[(size_t)telem[i] * nen + a];
     if ((st = upload(c, T.tile_elem, telem.data(), telem.size())) || (st = upload(c, T.tile_conn, tconn.data(), tconn.size())) ||
         (st = upload(c, T.tp_ptr, tp_ptr.data(), tp_ptr.size())) ||
-        (st = upload(c, T.trec, trec.data(), trec.size())) || (st = upload(c, T.tcontrib, tcw.data(), tcw.size())) ||
-        (st = upload(c, T.tslot, tslot.data(), tslot.size())) ||
-        (st = upload(c, T.brec, brec.data(), brec.size())) ||
+        (st = upload(c, dtpair, tpair.get(), nent)) || (st = upload(c, dbpair, bpair.data(), bpair.size())) ||
+        (st = dalloc(c, T.trec, 48 * nent)) || (st = upload(c, T.tcontrib, tcw.get(), nent)) ||
+        (st = upload(c, T.tslot, tslot.get(), nent)) || (st = dalloc(c, T.brec, 48 * nbnd)) ||
         (st = upload(c, T.bp_ptr, bp_ptr.data(), bp_ptr.size())) ||
         (st = dalloc(c, T.partial, (size_t)std::max<int64_t>(nslots, 1) * 36 * 8)))
         return st;
+    const fs::ScatterPlan sp = plan_of(B);
+    for (const bool bnd : {false, true})
+        FS_HIP(c, fs::launch_tile_place(bnd ? nbnd : nent, (bnd ? dbpair : dtpair).as<int32_t>(), sp,
+                                        B.node_rec.as<int4>(), (bnd ? T.brec : T.trec).as<int4>(), c->stream));
     FS_HIP(c, hipStreamSynchronize(c->stream));
     T.ne = NE;
     T.ntiles = ntiles;

@@ -1772,6 +1772,28 @@ __global__ __launch_bounds__(256) void plan_contrib_kernel(int64_t npairs, int n
     });
 }
 
+// Placement records (TilePlan trec, brec) of the listed upper pairs: the node
+// records of I and J (bit 30 of the first's codes: I == J) and the run offsets of
+// the pair's two slots.  48 bytes an entry that neither the host writes nor PCIe
+// carries: the 1.9 million entries of the 512 x 512 Q4 mesh and its boundary pairs take
+// 50 us (a new model's first assembly there 155 -> 112 ms).
+__global__ __launch_bounds__(256) void tile_place_kernel(int64_t n, const int32_t *__restrict__ pairs,
+                                                         const int2 *__restrict__ pair_node,
+                                                         const int2 *__restrict__ pair_slot,
+                                                         const int4 *__restrict__ node_rec,
+                                                         const int2 *__restrict__ nbr_off, int4 *__restrict__ rec) {
+    const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (q >= n) return;
+    const int64_t p = pairs[q];
+    const int2 nodes = pair_node[p], slots = pair_slot[p];
+    int4 a = node_rec[nodes.x];
+    if (nodes.x == nodes.y) a.w |= 1 << 30;
+    const int2 oi = nbr_off[slots.x], oj = nbr_off[slots.y];
+    rec[3 * q] = a;
+    rec[3 * q + 1] = node_rec[nodes.y];
+    rec[3 * q + 2] = make_int4(oi.x, oi.y, oj.x, oj.y);
+}
+
 // Row pointers [i0, i0 + n) as the caller takes them.
 __global__ __launch_bounds__(256) void pattern_rows_kernel(int64_t n, const int32_t *__restrict__ rowptr, int base,
                                                            int64_t *__restrict__ out) {
@@ -4234,6 +4256,15 @@ hipError_t launch_plan_pairs(const PlanArgs &a, hipStream_t st) {
     if (a.npairs)
         hipLaunchKernelGGL(plan_contrib_kernel, dim3(blocks_of(a.npairs, 256)), wg, 0, st, a.npairs, a.nen, a.E, a.conn,
                            a.pair_node, a.ne_ptr, a.ne_list, a.contrib_ptr, a.contrib);
+    return hipGetLastError();
+}
+
+hipError_t launch_tile_place(int64_t n, const int32_t *pairs, const ScatterPlan &sp, const int4 *node_rec, int4 *rec,
+                             hipStream_t st) {
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(tile_place_kernel, dim3(blocks_of(n, 256)), dim3(256), 0, st, n, pairs,
+                       reinterpret_cast<const int2 *>(sp.pair_node), reinterpret_cast<const int2 *>(sp.pair_slot),
+                       node_rec, reinterpret_cast<const int2 *>(sp.nbr_off), rec);
     return hipGetLastError();
 }
 
