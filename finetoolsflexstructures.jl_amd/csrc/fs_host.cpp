@@ -1015,7 +1015,7 @@ int build_patches(fs_model *m) {
             act[I] = 0;
             for (int cc = 0; cc < 6; ++cc) act[I] |= m->dof[I * 6 + cc] < m->nfree;
         }
-    });
+    }, 262144);
     auto active = [&](int64_t I) { return act[I] != 0; };  // node with free dofs
     auto degree = [&](int64_t I) { return m->nbr_ptr[I + 1] - m->nbr_ptr[I]; };
     // coordinates, copied while the components are found
