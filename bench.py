@@ -40,6 +40,19 @@ def cd_step_bytes(n, nnz, nnb, nnodes):
     return nnz * 8 + nnodes * 20 + nnb * 8 + n * 72
 
 
+PATCH_MIN_STEPS = 100  # loops of at least this many steps run on the patch form of K
+
+
+def patch_step_bytes(n, nnb, nnodes, block=36 * 8, fmag_frac=0.0):
+    """Algorithmic bytes of one CD step on the patch form: the block of each
+    pair of distinct neighbours once (nnb neighbour slots, the node itself
+    among them; 36 FP64 values, or FP32 values with int16 residuals: 216 B), the
+    upper triangle of each node's own block, and per dof U, the half-step
+    velocity and invM read and the first two written; Fmag on the fraction
+    fmag_frac of the steps that carry load."""
+    return (nnb - nnodes) // 2 * block + nnodes * 21 * 8 + n * (40 + 8 * fmag_frac)
+
+
 def resultant_bytes(E, N, nen, npts):
     """Algorithmic HBM bytes of one stress-resultant launch over all elements:
     connectivity 4 nen E, per node coordinates 24 + normal and flag 25 + the
@@ -371,11 +384,15 @@ def bench_mixed(nsteps, nx=1024, ny=512):
     for name in ("mixed", "mixed_f32"):
         out[f"{name}_over_fp64"] = out[f"{name}_dof_steps_per_s"] / out["fp64_dof_steps_per_s"]
         kmb_pairs, nsr, nnb, _ = info[name]
-        b_mx = mixed_step_bytes(N, E, 3, kmb_pairs, nsr, nnb, float(np.mean(g[1:] != 0)))
+        frac = float(np.mean(g[1:] != 0))
+        patch = nsteps >= PATCH_MIN_STEPS
+        b_mx = (patch_step_bytes(nf, nnb, N, 36 * 8 if name == "mixed" else 36 * 6, frac) if patch
+                else mixed_step_bytes(N, E, 3, kmb_pairs, nsr, nnb, frac))
         ach = b_mx / (runs[name]["ms"] / nsteps / 1e3) / 1e9
         out[f"roofline_{name}"] = {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                    "frac": ach / HBM_PEAK_GBS,
-                                   "kernel": f"cd_mixed_step_kernel<3, {nsr}>",
+                                   "kernel": ("cd_patch_step_kernel" if patch
+                                              else f"cd_mixed_step_kernel<3, {nsr}>"),
                                    "algorithmic_bytes": b_mx, "bytes_per_dof": b_mx / nf}
     f._model.close()
     return out
@@ -655,7 +672,9 @@ def main():
           f"locations)", file=sys.stderr, flush=True)
 
     b_asm = assembly_bytes(E, N, 4, nnz)
-    b_cd = cd_step_bytes(nf, nnz, model.mixed_info()[2], N)
+    cd_patch = ncd >= PATCH_MIN_STEPS
+    nnb = model.mixed_info()[2]
+    b_cd = patch_step_bytes(nf, nnb, N) if cd_patch else cd_step_bytes(nf, nnz, nnb, N)
     ach = b_asm / (dev_ms / 1e3) / 1e9
     ach_cd = b_cd / (cd_ms / ncd / 1e3) / 1e9
     # HBM bytes per assembly (fused element kernel + finalize) from the
@@ -695,7 +714,8 @@ def main():
         "dof_steps_per_s": dof_steps,
         "cd_us_per_step": cd_ms / ncd * 1e3,
         "roofline_cd": {"bound": "hbm", "achieved": ach_cd, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                        "frac": ach_cd / HBM_PEAK_GBS, "kernel": "cd_node_step_kernel (8 lanes per node)",
+                        "frac": ach_cd / HBM_PEAK_GBS, "kernel": ("cd_patch_step_kernel" if cd_patch
+                                                              else "cd_node_step_kernel (8 lanes per node)"),
                         "algorithmic_bytes": b_cd},
         "roofline_elem": (None if elem_flops is None else
                           {"bound": "fp64-valu", "achieved": elem_flops / elem_s / 1e12, "peak": FP64_PEAK_TFS,

@@ -61,6 +61,9 @@ extern "C" {
                                rounding grows with the element size over the
                                thickness, so it suits meshes with elements of
                                a few thicknesses or less */
+/* In loops of 100 steps or more both precisions run on patches of the symmetric
+   operator: FS_PREC_MIXED adds its parts up into FP64 blocks once, FS_PREC_MIXED_F32
+   keeps FP32 values with their residuals off the diagonal. */
 
 typedef struct fs_ctx fs_ctx;
 typedef struct fs_model fs_model;
@@ -468,8 +471,8 @@ int fs_ctx_set_cd_lanes(fs_ctx *ctx, int lanes_per_node, int positions_per_lane)
  * negative: always step by step. */
 int fs_ctx_set_cd_loop(fs_ctx *ctx, int64_t polls);
 
-/* Storage of the mixed-precision operator built by the last FS_PREC_MIXED /
- * FS_PREC_MIXED_F32 loop (no counterpart in the reference, whose loop runs on
+/* Storage of the mixed-precision operator in slices, built by the last
+ * FS_PREC_MIXED / FS_PREC_MIXED_F32 loop (no counterpart in the reference, whose loop runs on
  * the FP64 CSR matrix only): info[0] FP32 value pairs of the slices
  * (membrane + bending, plus shear for FS_PREC_MIXED_F32), info[1] FP64 shear
  * factor rows per element (0 for FS_PREC_MIXED_F32), info[2] entries of the
