@@ -100,7 +100,8 @@ hipError_t launch_cd_node_step(int nl, int pj, const NodeRows &nrw, const int2 *
                                const double *Cd, const double *Fmag, double gstep, double dt, int damped,
                                const int32_t *probe_slot, double *probe_dst, const int32_t *row_group,
                                const double *group_dt, const double *gtab, hipStream_t st);
-hipError_t launch_patch_count(int64_t np, const int32_t *order, const int32_t *pstart, const int32_t *nbr_ptr,
+hipError_t launch_patch_cut(int64_t nsegs, int most, const int4 *segs, const float4 *src, float4 *dst, hipStream_t st);
+hipError_t launch_patch_count(int64_t np, const float4 *points, const int32_t *pstart, const int32_t *nbr_ptr,
                               const int32_t *nbr_node, int32_t *pnode, int32_t *slot, int4 *rec, uint16_t *nptr,
                               int64_t *tot, hipStream_t st);
 hipError_t launch_patch_fill(int64_t np, const int32_t *nbr_ptr, const int32_t *nbr_node, const int32_t *pnode,
@@ -1065,7 +1066,7 @@ int build_patches(fs_model *m) {
         return q;
     };
     std::atomic<int64_t> roots{0};
-    std::atomic<bool> hub{false};
+    std::atomic<bool> hub{false}, wide{false};
     constexpr int64_t CH = 8192;  // nodes counted together
     const int64_t nch = (N + CH - 1) / CH;
     std::vector<int64_t> at(nch + 1, 0);
@@ -1076,6 +1077,7 @@ int build_patches(fs_model *m) {
                 nr += find((int32_t)I) == I;
                 at[k + 1] += active(I);
                 if (active(I) && degree(I) > PATCH_MAX_SLOTS) hub = true;
+                if (active(I) && degree(I) * PN > PATCH_MAX_SLOTS) wide = true;
             }
         roots += nr;
     }, 16);
@@ -1110,7 +1112,35 @@ int build_patches(fs_model *m) {
             if (active(I)) pt[fill[cid[I]]++] = point(I, cfirst[cid[I]]);
     }
     const int64_t nc = (int64_t)cptr.size() - 1;
+    // Where no patch of PN nodes can have too many slots, the sizes of the cuts are
+    // known beforehand and kernels make them, a launch a level; else the host cuts
+    // (a patch with too many slots is cut again).  The host also cuts small meshes:
+    // a loop's first call takes 0.46 ms that way and 0.50 with the launches on 56
+    // nodes, 0.81 and 0.77 on 2,928, 4.2 and 2.8 on 26,000, 16.7 and 12.5 on 131,000.
+    // Both make the same patches.
+    if (npt >= INT32_MAX) return FS_OK;
+    const bool kernel_cuts = !wide && npt >= 2048;
+    std::vector<std::vector<int4>> levels;
     std::vector<uint8_t> head(npt + 1, 0);  // 1 where a patch begins
+    if (kernel_cuts) {
+        std::vector<int4> segs;
+        for (int64_t k = 0; k < nc; ++k)
+            if (cptr[k + 1] > cptr[k]) segs.push_back({(int)cptr[k], (int)(cptr[k + 1] - cptr[k]), 0, 0});
+        for (bool cut = true; cut;) {
+            cut = false;
+            std::vector<int4> next;
+            for (int4 &q : segs) {
+                const int64_t k = (q.y + PN - 1) / PN;
+                q.z = (int)((int64_t)q.y * (k / 2) / k);  // 0: a patch
+                if (q.z) next.push_back({q.x, q.z, 0, 0});
+                next.push_back({q.x + q.z, q.y - q.z, 0, 0});
+                cut |= q.z != 0;
+            }
+            if (cut) levels.push_back(std::move(segs));
+            segs = std::move(next);
+        }
+        for (const int4 &q : segs) head[q.x] = 1;
+    }
     std::function<void(int64_t, int64_t)> bisect = [&](int64_t b, int64_t n) {
         Pt *q = pt.get() + b;
         int64_t k = (n + PN - 1) / PN;
@@ -1145,7 +1175,7 @@ int build_patches(fs_model *m) {
             bisect(b + n1, n - n1);
         }
     };
-    parallel_chunks(nc, [&](int64_t k0, int64_t k1) {
+    parallel_chunks(kernel_cuts ? 0 : nc, [&](int64_t k0, int64_t k1) {
         for (int64_t k = k0; k < k1; ++k)
             if (cptr[k + 1] > cptr[k]) bisect(cptr[k], cptr[k + 1] - cptr[k]);
     }, 16);
@@ -1154,9 +1184,7 @@ int build_patches(fs_model *m) {
         if (head[i]) pstart.push_back((int32_t)i);
     const int64_t np = (int64_t)pstart.size();
     pstart.push_back((int32_t)npt);
-    if (np * PN >= (int64_t(1) << 26) || npt >= INT32_MAX) return FS_OK;  // slots are 26-bit numbers
-    HostArray<int32_t> order = host_array<int32_t>(npt);
-    for (int64_t i = 0; i < npt; ++i) order[i] = pt[i].id;
+    if (np * PN >= (int64_t(1) << 26)) return FS_OK;  // slots are 26-bit numbers
     // sets of consecutive components for the one-launch loop (a component begins
     // a patch, and is a set of its own unless it fits the current one)
     P.sets.assign(1, 0);
@@ -1171,14 +1199,27 @@ int build_patches(fs_model *m) {
     for (size_t k = 0; k + 1 < P.sets.size(); ++k) P.largest_set = std::max(P.largest_set, P.sets[k + 1] - P.sets[k]);
     // the lists on the device
     int s;
-    DevBuf dorder, dstart, dslot, dtot;
+    DevBuf dpt[2], dsegs, dstart, dslot, dtot;
     const int32_t *nbp = B.nbr_ptr, *nbn = B.nbr_node;
-    if ((s = upload(c, dorder, order.get(), npt)) || (s = upload(c, dstart, pstart.data(), pstart.size())) ||
+    if ((s = upload(c, dpt[0], pt.get(), npt)) || (s = upload(c, dstart, pstart.data(), pstart.size())) ||
         (s = dalloc(c, dslot, N * 4)) || (s = dalloc(c, dtot, 32)) || (s = dalloc(c, P.dpnode, (size_t)np * PN * 4)) ||
         (s = dalloc(c, P.rec, (size_t)np * 16)) || (s = dalloc(c, P.nptr, (size_t)np * (PN + 1) * 2)))
         return s;
+    std::vector<int4> all;
+    for (const std::vector<int4> &l : levels) all.insert(all.end(), l.begin(), l.end());
+    if (!all.empty() && ((s = upload(c, dsegs, all.data(), all.size())) || (s = dalloc(c, dpt[1], npt * sizeof(Pt)))))
+        return s;
+    int at0 = 0, cur = 0;
+    for (const std::vector<int4> &l : levels) {
+        int most = 0;
+        for (const int4 &q : l) most = std::max(most, q.y);
+        FS_HIP(c, fs::launch_patch_cut((int64_t)l.size(), most, dsegs.as<int4>() + at0, dpt[cur].as<float4>(),
+                                       dpt[1 - cur].as<float4>(), c->stream));
+        at0 += (int)l.size();
+        cur = 1 - cur;
+    }
     FS_HIP(c, hipMemsetAsync(dslot.p, 0xff, N * 4, c->stream));
-    FS_HIP(c, fs::launch_patch_count(np, dorder.as<int32_t>(), dstart.as<int32_t>(), nbp, nbn, P.dpnode.as<int32_t>(),
+    FS_HIP(c, fs::launch_patch_count(np, dpt[cur].as<float4>(), dstart.as<int32_t>(), nbp, nbn, P.dpnode.as<int32_t>(),
                                      dslot.as<int32_t>(), P.rec.as<int4>(), P.nptr.as<uint16_t>(),
                                      dtot.as<int64_t>(), c->stream));
     int64_t tot[4];
@@ -1203,10 +1244,11 @@ int build_patches(fs_model *m) {
 }
 
 // Steps from which a loop takes the patch form.  Its plan costs a model's first
-// such loop once about 60 ns per node (0.4 ms for 6,076 nodes, 2.7 for 36,381; 12 ms
-// for the 1024 x 512 plate's 525,825 on 16 threads), and a step then saves 0.2 to 0.5
-// ns per node: from 100 to 200 steps on the first loop has paid for it, from 100
-// on the second.
+// such loop once.  A first loop of 100 steps takes, row form against patch form with
+// its plan, 0.67 | 0.74 ms (1,271 nodes), 0.99 | 1.06 (6,076), 1.47 | 1.27 (12,221),
+// 3.7 | 3.3 (36,381), 6.2 | 4.6 (51,657), and a later one 0.65 | 0.43, 0.81 | 0.43,
+// 1.21 | 0.57, 2.9 | 1.6, 4.9 | 2.3: at 100 steps the first loop breaks even on the
+// small meshes, below that it would lose.
 constexpr int64_t PATCH_MIN_STEPS = 100;
 
 // 3 x 21-bit Morton code of a point scaled into [0, 1)^3.

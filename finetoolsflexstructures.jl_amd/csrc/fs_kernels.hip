@@ -2969,14 +2969,136 @@ __device__ __forceinline__ double mx_value(float hi, short lo) { return (double)
 // with 16 threads, the same lists took 1.3 ms of a plan of 3.2 ms for 12,221
 // nodes, and as much again to create the threads.)
 
+// Order of a point along an axis, ties by node: finite coordinates as unsigned
+// numbers (both zeros alike), the node below them.
+__device__ __forceinline__ uint64_t cut_key(const float4 &q, int ax) {
+    const float x = ax == 0 ? q.x : ax == 1 ? q.y : q.z;
+    const uint32_t u = x == 0.f ? 0u : __float_as_uint(x);
+    return (uint64_t)(u & 0x80000000u ? ~u : u | 0x80000000u) << 32 | (uint32_t)__float_as_int(q.w);
+}
+
+// One level of the recursive bisection: segment {first, n, n1} of src goes to dst
+// with its n1 least points along its longest extent first (n1 = 0: as it is).  The
+// n1-th key is found digit by digit, eight bits of 64 a pass, ending where its
+// digit holds one point; the order within the two parts is left open, as later cuts
+// and patch_rank_kernel go by keys and numbers alone.  A workgroup a segment: the
+// first levels, with few, are bound by one CU's loads and LDS atomics (131,000
+// nodes: 400 us for the first level, half of it for the next, 9 to 30 us for the
+// last seven); all twelve take 0.9 ms where the host took 5 to 6.
+template <int WG>
+__global__ __launch_bounds__(WG) void patch_cut_kernel(const int4 *__restrict__ segs, const float4 *__restrict__ src,
+                                                       float4 *__restrict__ dst) {
+    __shared__ float lo[3][WG / 64], hi[3][WG / 64];
+    __shared__ int hist[256];
+    __shared__ int pick[3];  // digit, its count, points before it
+    __shared__ int left, right;
+    const int4 seg = segs[blockIdx.x];
+    const int t = threadIdx.x, n = seg.y, n1 = seg.z;
+    src += seg.x;
+    dst += seg.x;
+    if (n1 == 0) {
+        for (int i = t; i < n; i += WG) dst[i] = src[i];
+        return;
+    }
+    float a[3] = {INFINITY, INFINITY, INFINITY}, b[3] = {-INFINITY, -INFINITY, -INFINITY};
+    for (int i = t; i < n; i += WG) {
+        const float4 q = src[i];
+        a[0] = fminf(a[0], q.x);
+        a[1] = fminf(a[1], q.y);
+        a[2] = fminf(a[2], q.z);
+        b[0] = fmaxf(b[0], q.x);
+        b[1] = fmaxf(b[1], q.y);
+        b[2] = fmaxf(b[2], q.z);
+    }
+    for (int d = 0; d < 3; ++d) {
+        for (int w = 32; w; w >>= 1) {
+            a[d] = fminf(a[d], __shfl_xor(a[d], w));
+            b[d] = fmaxf(b[d], __shfl_xor(b[d], w));
+        }
+        if (t % 64 == 0) {
+            lo[d][t / 64] = a[d];
+            hi[d][t / 64] = b[d];
+        }
+    }
+    if (t == 0) left = right = 0;
+    __syncthreads();
+    float ext[3];
+    for (int d = 0; d < 3; ++d) {
+        float x = lo[d][0], y = hi[d][0];
+        for (int w = 1; w < WG / 64; ++w) {
+            x = fminf(x, lo[d][w]);
+            y = fmaxf(y, hi[d][w]);
+        }
+        ext[d] = y - x;
+    }
+    int ax = 0;
+    for (int d = 1; d < 3; ++d)
+        if (ext[d] > ext[ax]) ax = d;
+    // the key of rank n1: prefix and shift, with `rank` points of the prefix before it
+    uint64_t prefix = 0;
+    int shift = 64, rank = n1;
+    while (shift > 0) {
+        const int s0 = shift - 8;
+        for (int i = t; i < 256; i += WG) hist[i] = 0;
+        __syncthreads();
+        for (int i = t; i < n; i += WG) {
+            const uint64_t k = cut_key(src[i], ax);
+            if (shift == 64 || k >> shift == prefix) atomicAdd(&hist[(k >> s0) & 255], 1);
+        }
+        __syncthreads();
+        if (t < 64) {  // the digit whose points contain the rank
+            int c[4], s = 0;
+            for (int i = 0; i < 4; ++i) s += c[i] = hist[4 * t + i];
+            int upto = s;
+            for (int w = 1; w < 64; w <<= 1) {
+                const int v = __shfl_up(upto, w);
+                if (t >= w) upto += v;
+            }
+            int before = upto - s;
+            for (int i = 0; i < 4; ++i) {
+                if (rank >= before && rank < before + c[i]) {
+                    pick[0] = 4 * t + i;
+                    pick[1] = c[i];
+                    pick[2] = before;
+                }
+                before += c[i];
+            }
+        }
+        __syncthreads();
+        prefix = prefix << 8 | (uint32_t)pick[0];
+        rank -= pick[2];
+        shift = s0;
+        const bool one = pick[1] == 1;
+        __syncthreads();
+        if (one) break;
+    }
+    for (int i0 = 0; i0 < n; i0 += WG) {
+        const int i = i0 + t;
+        const bool in = i < n;
+        float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (in) q = src[i];
+        const bool l = in && cut_key(q, ax) >> shift < prefix, rr = in && !l;
+        const uint64_t ml = __ballot(l), mr = __ballot(rr), below = ((uint64_t)1 << (t % 64)) - 1;
+        int bl = 0, br = 0;
+        if (t % 64 == 0) {
+            bl = atomicAdd(&left, __popcll(ml));
+            br = atomicAdd(&right, __popcll(mr));
+        }
+        bl = __shfl(bl, 0);
+        br = __shfl(br, 0);
+        if (l) dst[bl + __popcll(ml & below)] = q;
+        if (rr) dst[n1 + br + __popcll(mr & below)] = q;
+    }
+}
+
 // Nodes of a patch by their numbers: pnode and slot.
-__global__ __launch_bounds__(64) void patch_rank_kernel(const int32_t *__restrict__ order,
+__global__ __launch_bounds__(64) void patch_rank_kernel(const float4 *__restrict__ points,
                                                         const int32_t *__restrict__ pstart,
                                                         int32_t *__restrict__ pnode, int32_t *__restrict__ slot) {
     __shared__ int32_t id[PATCH_NODES];
     const int p = blockIdx.x, t = threadIdx.x;
     const int b = pstart[p], n = pstart[p + 1] - b;
-    if (t < n) id[t] = order[b + t];
+    if (t < n) id[t] = __float_as_int(points[b + t].w);
     __syncthreads();
     if (t >= PATCH_NODES) return;
     if (t < n) {
@@ -4613,11 +4735,21 @@ hipError_t launch_coo_reduce(int64_t nnz, const int64_t *cptr, const int64_t *cl
     return hipGetLastError();
 }
 
-hipError_t launch_patch_count(int64_t np, const int32_t *order, const int32_t *pstart, const int32_t *nbr_ptr,
+// most: points of the largest segment
+hipError_t launch_patch_cut(int64_t nsegs, int most, const int4 *segs, const float4 *src, float4 *dst, hipStream_t st) {
+    const dim3 grid((unsigned)nsegs);
+    if (most > 4096)
+        hipLaunchKernelGGL(patch_cut_kernel<1024>, grid, dim3(1024), 0, st, segs, src, dst);
+    else
+        hipLaunchKernelGGL(patch_cut_kernel<256>, grid, dim3(256), 0, st, segs, src, dst);
+    return hipGetLastError();
+}
+
+hipError_t launch_patch_count(int64_t np, const float4 *points, const int32_t *pstart, const int32_t *nbr_ptr,
                               const int32_t *nbr_node, int32_t *pnode, int32_t *slot, int4 *rec, uint16_t *nptr,
                               int64_t *tot, hipStream_t st) {
     const dim3 grid((unsigned)np);
-    hipLaunchKernelGGL(patch_rank_kernel, grid, dim3(64), 0, st, order, pstart, pnode, slot);
+    hipLaunchKernelGGL(patch_rank_kernel, grid, dim3(64), 0, st, points, pstart, pnode, slot);
     hipLaunchKernelGGL(patch_count_kernel, grid, dim3(64), 0, st, nbr_ptr, nbr_node, pnode, slot, rec, nptr);
     hipLaunchKernelGGL(patch_scan_kernel, dim3(1), dim3(1024), 0, st, (int)np, rec, tot);
     return hipGetLastError();
