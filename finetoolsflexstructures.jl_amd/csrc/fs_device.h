@@ -1,4 +1,4 @@
-// fs_device.h -- data layouts shared by the host planner and the gfx950 kernels.
+// fs_device.h -- data layouts shared by the host runtime and the gfx950 kernels.
 //
 // Device-resident model layout (all structure-of-arrays, coalesced by element
 // or node index):

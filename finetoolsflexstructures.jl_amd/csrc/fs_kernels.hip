@@ -2964,9 +2964,9 @@ __device__ __forceinline__ double mx_value(float hi, short lo) { return (double)
 // second, 22.8, 22.7, 22.0, 25.7, 23.9 on the batch, where large patches leave
 // a half-empty last round of workgroups.
 
-// Plan of the patch form, from the nodes of each patch (the host's cuts): four
-// small kernels, a workgroup per patch, the scan one workgroup.  (On the host,
-// with 16 threads, the same lists took 1.3 ms of a plan of 3.2 ms for 12,221
+// Plan of the patch form: the cuts of larger meshes (patch_cut_kernel), then four
+// small kernels from the nodes of each patch, a workgroup per patch, the scan one
+// workgroup.  (On the host, with 16 threads, the lists took 1.3 ms for 12,221
 // nodes, and as much again to create the threads.)
 
 // Order of a point along an axis, ties by node: finite coordinates as unsigned
