@@ -3391,9 +3391,12 @@ __global__ __launch_bounds__(256) void patch_build_kernel(PatchOp op, PatchSourc
         double *dg = op.dg + ((int64_t)p * PATCH_NODES + li) * PATCH_TRI + r * (11 - r) / 2;
         double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         if (I >= 0) {
+            // a node is in its own list, unless it is in no element: then its list is empty
+            // and its block zero
+            const int k1 = src.sp.nbr_ptr[I + 1];
             int k = src.sp.nbr_ptr[I];
-            while (src.sp.nbr_node[k] != I) ++k;  // a node is in its own list
-            patch_block_row<KIND>(src, I, k, r, v);
+            while (k < k1 && src.sp.nbr_node[k] != I) ++k;
+            if (k < k1) patch_block_row<KIND>(src, I, k, r, v);
         }
         for (int c = r; c < 6; ++c) dg[c] = v[c];
     }
