@@ -79,9 +79,9 @@ hipError_t launch_cd_mass(int64_t nv, int64_t n, const int64_t *map, const doubl
                           const int32_t *row_group, const double *group_dt, const double *group_cdamp, double *Cd,
                           double *invMC, hipStream_t st);
 hipError_t launch_cd_place(int64_t nv, int64_t n, const int64_t *map, const double *src, double *dst, hipStream_t st);
-hipError_t launch_cd_place(int64_t nv, int64_t n, const int64_t *map, const int32_t *src, int32_t *dst, hipStream_t st);
-hipError_t launch_cd_probe(int64_t nv, const int64_t *map, int nprobes, const int64_t *plist, int32_t *slot,
+hipError_t launch_cd_place(int64_t nv, int64_t n, const int64_t *map, const int32_t *src, int32_t *dst, int32_t rest,
                            hipStream_t st);
+hipError_t launch_cd_probe(int64_t n, int nprobes, const int64_t *plist, int32_t *probe, hipStream_t st);
 hipError_t launch_cd_collect(int64_t nv, int64_t n, const int64_t *map, const double *src, double *dst,
                              hipStream_t st);
 hipError_t launch_cd_init(int64_t n, double dt, double g0, const double *invMC, const double *Fmag, const double *U0,
@@ -2691,7 +2691,6 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
     DevBuf &dV = sc.dV, &dA = sc.dA, &dF = sc.dF, &dInv = sc.dInv, &dC = sc.dC, &dSlot = sc.dSlot,
            &dProbe = sc.dProbe, &dRG = sc.dRG, &dGdt = sc.dGdt, &dG = sc.dG;
     const int64_t nrec = p->nsteps / stride + 1;
-    std::vector<int64_t> probe_list;  // read by a copy that the loop does not wait for
     // the caller's vectors into the state buffers; placed positions are filled
     // on the device from the free-dof order (through dA, which is free until
     // the loop starts)
@@ -2713,23 +2712,18 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
                 return e;
             FS_HIP(c, hipMemcpyAsync(placed ? dA.p : dRG.p, p->row_group, n * 4, hipMemcpyHostToDevice, c->stream));
             if (placed)
-                FS_HIP(c, fs::launch_cd_place(nv, n, map, dA.as<int32_t>(), dRG.as<int32_t>(), c->stream));
+                FS_HIP(c, fs::launch_cd_place(nv, n, map, dA.as<int32_t>(), dRG.as<int32_t>(), 0, c->stream));
         }
         FS_HIP(c, fs::launch_cd_mass(nv, n, map, B.mdiag.as<double>(), p->dt_mass > 0.0 ? p->dt_mass : p->dt, p->cdamp,
                                      batch ? dRG.as<int32_t>() : nullptr, dGdt.as<double>(), sc.dGcd.as<double>(),
                                      dC.as<double>(), dInv.as<double>(), c->stream));
         if (nprobes > 0) {
-            // the probes sorted by dof (of two probes of one dof the later one
-            // counts): dofs, then their slots, in one buffer
-            std::map<int64_t, int64_t> by_dof;
-            for (int k = 0; k < nprobes; ++k) by_dof[probe_dofs[k]] = k;
-            for (const auto &kv : by_dof) probe_list.push_back(kv.first);
-            for (const auto &kv : by_dof) probe_list.push_back(kv.second);
-            if ((e = ensure(c, dSlot, nv * 4)) || (e = put(c, sc.dPlist, probe_list.data(), probe_list.size())) ||
+            if ((e = ensure(c, dSlot, nv * 4)) || (e = put(c, sc.dPlist, probe_dofs, nprobes)) ||
                 (e = ensure(c, dProbe, (size_t)nrec * nprobes * 8)))
                 return e;
-            FS_HIP(c, fs::launch_cd_probe(nv, map, (int)by_dof.size(), sc.dPlist.as<int64_t>(), dSlot.as<int32_t>(),
-                                          c->stream));
+            int32_t *probe = placed ? dA.as<int32_t>() : dSlot.as<int32_t>();
+            FS_HIP(c, fs::launch_cd_probe(n, nprobes, sc.dPlist.as<int64_t>(), probe, c->stream));
+            if (placed) FS_HIP(c, fs::launch_cd_place(nv, n, map, probe, dSlot.as<int32_t>(), -1, c->stream));
             for (int k = 0; k < nprobes; ++k) probe_out[k] = U0[probe_dofs[k]];  // peek(0, U0)
         }
         return FS_OK;
@@ -2892,7 +2886,6 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
         // on this context any more
         c->loop_gave_up = true;
         loop = false;
-        probe_list.clear();
         if ((s = set_up())) {
             sc.drop_graph();
             return s;

@@ -2637,7 +2637,7 @@ __global__ __launch_bounds__(256) void cd_init_kernel(int64_t n, double dt, doub
 //                    (plate_expl_examples.jl:68-71, with the dt from before
 //                    the adjustment), per model in a batch
 //   cd_place_kernel  dst[q] = src[map[q]]
-//   cd_probe_kernel  the probe slot of each position
+//   cd_probe_kernel  the probe of each free dof
 //   cd_collect_kernel  dst[map[q]] = src[q]
 // HBM-bound streams.  Computing C and invMC from the resident mass, and
 // placing the vectors here, took the call of the 1024 x 512 plate (3.1 M
@@ -2667,32 +2667,29 @@ __global__ __launch_bounds__(256) void cd_mass_kernel(int64_t nv, int64_t n, con
     invMC[q] = iq;
 }
 
+// Positions of fixed dofs get `rest`.
 template <class T>
 __global__ __launch_bounds__(256) void cd_place_kernel(int64_t nv, int64_t n, const int64_t *__restrict__ map,
-                                                       const T *__restrict__ src, T *__restrict__ dst) {
+                                                       const T *__restrict__ src, T *__restrict__ dst, T rest) {
     const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= nv) return;
     const int64_t d = map[q];
-    dst[q] = d < n ? src[d] : T(0);
+    dst[q] = d < n ? src[d] : rest;
 }
 
-// slot[q] = plist[nprobes + k] where map[q] is the dof plist[k] (the probes,
-// sorted by dof, then their slots), -1 at the other positions.
-__global__ __launch_bounds__(256) void cd_probe_kernel(int64_t nv, const int64_t *__restrict__ map, int nprobes,
-                                                       const int64_t *__restrict__ plist,
-                                                       int32_t *__restrict__ slot) {
-    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= nv) return;
-    const int64_t d = map ? map[q] : q;
-    int lo = 0, hi = nprobes;  // first probe dof not below d
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (plist[mid] < d)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    slot[q] = lo < nprobes && plist[lo] == d ? (int32_t)plist[nprobes + lo] : -1;
+__global__ __launch_bounds__(256) void cd_probe_clear_kernel(int64_t n, int32_t *__restrict__ probe) {
+    const int64_t d = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (d < n) probe[d] = -1;
+}
+
+// probe[plist[k]] = k, of several probes of a dof the last.  A pass over the dofs
+// and one over the probes, whatever their number: the call of a 20-step loop that
+// records all 723,303 dofs of a 400 x 300 Q4 mesh takes 4.5 ms, where it took 109
+// with the probes sorted in a tree on the host (2.6 without probes, either way).
+__global__ __launch_bounds__(256) void cd_probe_kernel(int nprobes, const int64_t *__restrict__ plist,
+                                                       int32_t *__restrict__ probe) {
+    const int k = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (k < nprobes) atomicMax(&probe[plist[k]], k);
 }
 
 __global__ __launch_bounds__(256) void cd_collect_kernel(int64_t nv, int64_t n, const int64_t *__restrict__ map,
@@ -4510,23 +4507,23 @@ hipError_t launch_cd_mass(int64_t nv, int64_t n, const int64_t *map, const doubl
 hipError_t launch_cd_place(int64_t nv, int64_t n, const int64_t *map, const double *src, double *dst, hipStream_t st) {
     if (nv == 0) return hipSuccess;
     hipLaunchKernelGGL(cd_place_kernel<double>, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, st, nv, n, map, src,
-                       dst);
+                       dst, 0.0);
     return hipGetLastError();
 }
 
-hipError_t launch_cd_place(int64_t nv, int64_t n, const int64_t *map, const int32_t *src, int32_t *dst,
+hipError_t launch_cd_place(int64_t nv, int64_t n, const int64_t *map, const int32_t *src, int32_t *dst, int32_t rest,
                            hipStream_t st) {
     if (nv == 0) return hipSuccess;
     hipLaunchKernelGGL(cd_place_kernel<int32_t>, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, st, nv, n, map, src,
-                       dst);
+                       dst, rest);
     return hipGetLastError();
 }
 
-hipError_t launch_cd_probe(int64_t nv, const int64_t *map, int nprobes, const int64_t *plist, int32_t *slot,
-                           hipStream_t st) {
-    if (nv == 0) return hipSuccess;
-    hipLaunchKernelGGL(cd_probe_kernel, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, st, nv, map, nprobes, plist,
-                       slot);
+// probe: the probe of each of the n free dofs, -1 where there is none
+hipError_t launch_cd_probe(int64_t n, int nprobes, const int64_t *plist, int32_t *probe, hipStream_t st) {
+    if (n == 0 || nprobes == 0) return hipSuccess;
+    hipLaunchKernelGGL(cd_probe_clear_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, n, probe);
+    hipLaunchKernelGGL(cd_probe_kernel, dim3((unsigned)((nprobes + 255) / 256)), dim3(256), 0, st, nprobes, plist, probe);
     return hipGetLastError();
 }
 
