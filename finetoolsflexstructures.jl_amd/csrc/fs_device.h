@@ -254,7 +254,8 @@ struct NodeRows {
 };
 
 // Symmetric form of the free-free stiffness for the time loop, by patches: up
-// to PATCH_NODES nodes that lie together, all of one connected component.
+// to PATCH_NODES nodes that lie together, of one connected component or of several
+// small ones that are whole in the patch.
 // Node slot s = p PATCH_NODES + li holds local node li of patch p, and the
 // state vectors of the loop are in slot order, position q = 6 s + c (unused
 // slots and fixed dofs carry zeros).  A block K_IJ (6 x 6, zero rows and
