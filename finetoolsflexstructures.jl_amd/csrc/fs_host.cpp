@@ -2124,15 +2124,19 @@ int fs_model_set_dofs(fs_model *m, const int64_t *dofnums, int64_t nalldofs, int
         }
     if ((int64_t)N * 6 != nalldofs) return fail(c, FS_ERR_ARG, "nalldofs must equal 6 * nnodes");
     FS_HIP(c, hipSetDevice(c->device));
-    m->dof.swap(dof);
-    m->nall = nalldofs;
-    m->nfree = nfreedofs;
+    // the planner's kernels read the device copy: from here on no numbers, until
+    // the new ones are there (in the buffer of the old, which have as many)
+    int s = ensure(c, m->node_dof, dof.size() * 8);
+    if (s) return s;
+    m->dofs_ready = false;
     m->blk[0].reset();
     m->blk[1].reset();
     m->mixed.reset();
-    int s = upload(c, m->node_dof, m->dof.data(), m->dof.size());
-    if (s) return s;
+    FS_HIP(c, hipMemcpyAsync(m->node_dof.p, dof.data(), dof.size() * 8, hipMemcpyHostToDevice, c->stream));
     FS_HIP(c, hipStreamSynchronize(c->stream));
+    m->dof.swap(dof);
+    m->nall = nalldofs;
+    m->nfree = nfreedofs;
     m->dofs_ready = true;
     return FS_OK;
 }
@@ -2161,8 +2165,14 @@ int fs_model_number_dofs(fs_model *m, const uint8_t *is_fixed, const int64_t *pe
     int s;
     if ((s = upload(c, dfix, perm ? pf.data() : is_fixed, (size_t)n)) ||
         (s = dalloc(c, dtile, fs::number_dofs_tiles(n) * 8 + 8)) || (s = dalloc(c, dtot, 8)) ||
-        (s = dalloc(c, m->node_dof, (size_t)n * 8)))
+        (s = ensure(c, m->node_dof, (size_t)n * 8)))
         return s;
+    // the planner's kernels read the device copy: from here on no numbers, until
+    // the new ones are there
+    m->dofs_ready = false;
+    m->blk[0].reset();
+    m->blk[1].reset();
+    m->mixed.reset();
     FS_HIP(c, hipMemsetAsync(dtot.p, 0, 8, c->stream));
     FS_HIP(c, fs::launch_number_dofs(n, dfix.as<uint8_t>(), dtile.as<int64_t>(), dtot.as<int64_t>(),
                                      m->node_dof.as<int64_t>(), c->stream));
@@ -2177,16 +2187,13 @@ int fs_model_number_dofs(fs_model *m, const uint8_t *is_fixed, const int64_t *pe
         for (int64_t k = 0; k < N; ++k)
             for (int cc = 0; cc < 6; ++cc) byn[perm[k] * 6 + cc] = dof[k * 6 + cc];
         dof.swap(byn);
-        if ((s = upload(c, m->node_dof, dof.data(), dof.size()))) return s;
+        FS_HIP(c, hipMemcpyAsync(m->node_dof.p, dof.data(), (size_t)n * 8, hipMemcpyHostToDevice, c->stream));
         FS_HIP(c, hipStreamSynchronize(c->stream));
     }
     // the host copy feeds the pattern planner
     m->dof.swap(dof);
     m->nall = n;
     m->nfree = nfree;
-    m->blk[0].reset();
-    m->blk[1].reset();
-    m->mixed.reset();
     m->dofs_ready = true;
     if (dofnums_out)
         for (int64_t I = 0; I < m->N; ++I)

@@ -200,6 +200,7 @@ class _ShellFEMM:
     def _ensure_dofs(self, dchi):
         key = self._dofs_key
         if key is None or key[:2] != (dchi.nalldofs, dchi.nfreedofs) or not _same_bits(dchi.dofnums, key[2]):
+            self._dofs_key = None  # a call that fails leaves the model without numbers
             self._model.set_dofs(dchi.dofnums, dchi.nalldofs, dchi.nfreedofs)
             self._dofs_key = (dchi.nalldofs, dchi.nfreedofs, dchi.dofnums.copy())
             self._patterns = {}

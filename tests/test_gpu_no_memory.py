@@ -1,0 +1,91 @@
+"""Calls that find no device memory.  A small library loaded before the HIP runtime
+takes hipMalloc's place in a process of its own and refuses requests of given
+sizes, as a full device does."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SHIM = """
+#define _GNU_SOURCE
+#include <dlfcn.h>
+#include <stddef.h>
+static size_t lo = 1, hi = 0;
+static long refused = 0;
+void refuse(size_t a, size_t b) { lo = a; hi = b; refused = 0; }
+long refusals(void) { return refused; }
+int hipMalloc(void **p, size_t n) {
+    static int (*real)(void **, size_t);
+    if (n >= lo && n <= hi) { ++refused; *p = 0; return 2; }  /* hipErrorOutOfMemory */
+    if (!real) real = (int (*)(void **, size_t))dlsym(dlopen("libamdhip64.so.7", RTLD_NOW), "hipMalloc");
+    return real(p, n);
+}
+"""
+
+HEAD = """
+import ctypes as C, sys
+shim = C.CDLL(sys.argv[1], C.RTLD_GLOBAL)
+shim.refuse.argtypes = [C.c_size_t, C.c_size_t]
+shim.refusals.restype = C.c_long
+sys.path[:0] = [sys.argv[2], sys.argv[2] + "/finetoolsflexstructures.jl_amd"]
+import numpy as np
+from flexshell import _lib, explicit, fe, femm as FM
+from flexshell.material import MatDeforElastIso
+ctx = _lib.Context(0)
+NONE, ALL = (1, 0), (0, 2 ** 63)
+def refuse(r): shim.refuse(*r)
+"""
+
+
+def _run(tmp_path, script):
+    c, so = tmp_path / "shim.c", tmp_path / "libshim.so"
+    c.write_text(SHIM)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-o", str(so), str(c), "-ldl"], check=True)
+    r = subprocess.run([sys.executable, "-u", "-c", HEAD + textwrap.dedent(script), str(so), ROOT],
+                       stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.strip().endswith("done"), r.stdout[-3000:]
+
+
+@pytest.mark.gpu
+def test_new_equation_numbers_need_no_memory(tmp_path):
+    """The numbers of a model that has some go into the buffer that it has, also
+    where the context keeps no more spare buffers (4 GiB of them here) and none is to
+    be had."""
+    print("[gpu] equation numbers without memory", flush=True)
+    _run(tmp_path, """
+        N = 2000000
+        big = _lib.Model(ctx, 3, np.random.default_rng(0).random((N, 3)), np.array([[0, 1, 2]]))
+        fixed = np.zeros((N, 6), dtype=np.uint8)
+        dn, nf = big.number_dofs(fixed)
+        ctx.set_assembly(0)
+        models = []
+        for _ in range(4):
+            xy, conn = fe.Q4block(1.0, 1.0, 512, 512)
+            xyz = fe.xyz3(xy)
+            d = fe.DofField(len(xyz)).numberdofs()
+            f = FM.make(conn, MatDeforElastIso(70e9, 0.33, 2700.0), thickness=0.02, ctx=ctx)
+            f.associategeometry(xyz)
+            f.stiffness(FM.SysmatAssemblerHIP(_lib.FS_BLOCK_FF), xyz, None, None, d)
+            models.append(f)
+        for f in models:
+            f._model.close()
+        # three nodes carry rows; the first pattern of the old numbers
+        nr, rp, cv = big.pattern(_lib.FS_BLOCK_ALL)
+        assert nr == 6 * N and len(cv) == 18 * 18
+        refuse((90 * 10 ** 6, 2 ** 63))
+        fixed[1] = 1
+        dn2, nf2 = big.number_dofs(fixed)
+        assert nf2 == nf - 6 and dn2[1].min() == nf2
+        big.set_dofs(dn[::-1], 6 * N, nf)
+        big.set_dofs(dn2, 6 * N, nf2)
+        assert shim.refusals() == 0
+        refuse(NONE)
+        nr, rp, cv = big.pattern(_lib.FS_BLOCK_FF)
+        assert nr == nf2 and len(cv) == 12 * 12
+        big.close()
+        print("done")
+    """)
