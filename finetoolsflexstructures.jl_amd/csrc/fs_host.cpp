@@ -395,6 +395,7 @@ struct fs_model {
     // group data for the last stiffness/mass call
     DevBuf g_Labd, g_Lh, g_csys, g_t, g_group, g_inertia, m_group, g_homog, g_rho_t;
     double timing[7] = {0, 0, 0, 0, 0, 0, 0};
+    int32_t cd_form = -1;  // FS_CD_* of the last loop
     // parameters of the last element-stiffness launch (device pointers into
     // the group buffers above) and their generation
     fs::ElemParams last_ep{};
@@ -2924,10 +2925,11 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
         FS_HIP(c, hipEventRecord(e1, c->stream));
         FS_HIP(c, hipStreamSynchronize(c->stream));
     }
+    bool restarted = false;
     if (loop && __atomic_load_n(c->loop_stop, __ATOMIC_SEQ_CST) != 0) {
         // a wait ran out: from the start again, step by step, and no such loop
         // on this context any more
-        c->loop_gave_up = true;
+        c->loop_gave_up = restarted = true;
         loop = false;
         if ((s = set_up())) {
             sc.drop_graph();
@@ -2937,6 +2939,7 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
         FS_HIP(c, hipEventRecord(e1, c->stream));
         FS_HIP(c, hipStreamSynchronize(c->stream));
     }
+    m->cd_form = restarted ? FS_CD_RESTARTED : loop ? FS_CD_ONE_LAUNCH : patch ? FS_CD_PATCHES : FS_CD_ROWS;
     float ms = 0.f;
     FS_HIP(c, hipEventElapsedTime(&ms, e0, e1));
     (void)hipEventDestroy(e0);
@@ -3256,6 +3259,12 @@ int fs_model_mixed_info(const fs_model *m, int64_t *info) {
     info[1] = X.built ? X.nsr : 0;
     info[2] = m->nnb;
     info[3] = X.built ? X.nslices : 0;
+    return FS_OK;
+}
+
+int fs_model_cd_form(const fs_model *m, int32_t *form) {
+    if (!m || !form) return FS_ERR_ARG;
+    *form = m->cd_form;
     return FS_OK;
 }
 

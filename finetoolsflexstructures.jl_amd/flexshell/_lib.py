@@ -19,6 +19,7 @@ FS_SHEAR_AVERAGE_K = 1
 FS_PREC_FP64 = 0
 FS_PREC_MIXED = 1
 FS_PREC_MIXED_F32 = 2
+FS_CD_ROWS, FS_CD_PATCHES, FS_CD_ONE_LAUNCH, FS_CD_RESTARTED = 0, 1, 2, 3
 FS_OCSYS_ISOPARAMETRIC = 0
 FS_OCSYS_MATRIX = 1
 FS_OCSYS_PER_POINT = 2
@@ -126,6 +127,7 @@ SIGNATURES = {
     "fs_ctx_set_assembly": (C.c_int, [C.c_void_p, C.c_int]),
     "fs_ctx_set_cd_lanes": (C.c_int, [C.c_void_p, C.c_int, C.c_int]),
     "fs_ctx_set_cd_loop": (C.c_int, [C.c_void_p, C.c_int64]),
+    "fs_model_cd_form": (C.c_int, [C.c_void_p, C.POINTER(C.c_int32)]),
     "fs_coo_create": (C.c_int, [C.c_void_p, C.c_int64, C.c_int64, C.c_int32, C.c_int32, C.c_int64, _i64p, _i64p,
                                 C.c_int, C.POINTER(C.c_void_p)]),
     "fs_coo_pattern": (C.c_int, [C.c_void_p, _i64p]),
@@ -385,6 +387,12 @@ class Model:
     def timing(self, which):
         v = C.c_double()
         self.ctx.check(self.ctx.lib.fs_model_last_timing(self.h, int(which), C.byref(v)), "fs_model_last_timing")
+        return v.value
+
+    def cd_form(self):
+        """Form of the last explicit loop (FS_CD_*; -1 before the first)."""
+        v = C.c_int32()
+        self.ctx.check(self.ctx.lib.fs_model_cd_form(self.h, C.byref(v)), "fs_model_cd_form")
         return v.value
 
     def mixed_info(self):

@@ -410,6 +410,15 @@ void fs_coo_destroy(fs_coo *h);
  * graph: same sizes, scalars, load factors and buffers as the graph's). */
 int fs_model_last_timing(const fs_model *m, int which, double *ms);
 
+/* Form that the last fs_model_explicit took (-1: none yet).  With
+ * FS_CD_RESTARTED the context has left the one-launch form until the next
+ * fs_ctx_set_cd_loop. */
+#define FS_CD_ROWS 0      /* row products, or the slices of the mixed precisions */
+#define FS_CD_PATCHES 1   /* patches, step by step */
+#define FS_CD_ONE_LAUNCH 2 /* patches, the whole loop in one launch */
+#define FS_CD_RESTARTED 3 /* the same, a wait ran out: again, step by step */
+int fs_model_cd_form(const fs_model *m, int32_t *form);
+
 /* Element-kernel launch shape chosen by the autotuner for a family (FS_T3 /
  * FS_Q4) and shear formulation on this context (no counterpart in the
  * reference, which has no GPU launch shapes): shape[0] = variant index (-1
