@@ -2885,6 +2885,8 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
         key_add(key, B.slotrec.p);
         key_add(key, sc.dPub.p);
         key_add(key, sc.dForced.p);
+        if (loop)  // the bounds of its launches
+            for (const int32_t b : P.sets) key_add(key, b);
         if (patch) key_add(key, pop);
         else if (mixed) key_add(key, op);
         else if (c->cd_lanes > 0) key_add(key, noderows_of(B));
