@@ -7,8 +7,6 @@
 // normals and the time loop runs in the kernels of fs_kernels.hip.
 #include <hip/hip_runtime.h>
 
-#include <sched.h>
-
 #include <algorithm>
 #include <array>
 #include <atomic>
@@ -24,13 +22,13 @@
 #include <cstring>
 #include <new>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <type_traits>
 #include <vector>
 
 #include "../../include/flexshell.h"
 #include "fs_device.h"
+#include "fs_threads.h"
 
 namespace fs {
 hipError_t launch_element_blocks(const ElemParams &p, const double *x, const double *y, const double *z,
@@ -418,22 +416,6 @@ struct fs_coo {
 
 namespace {
 
-// Host threads for the parallel loops: the CPUs this process may run on,
-// capped by OMP_NUM_THREADS when that is set.
-int64_t host_threads() {
-    static const int64_t nt = [] {
-        int64_t n = std::max<int64_t>(1, std::thread::hardware_concurrency());
-        cpu_set_t set;
-        if (sched_getaffinity(0, sizeof set, &set) == 0) n = std::max(1, CPU_COUNT(&set));
-        if (const char *e = std::getenv("OMP_NUM_THREADS")) {
-            const long v = std::strtol(e, nullptr, 10);
-            if (v > 0) n = std::min<int64_t>(n, v);
-        }
-        return n;
-    }();
-    return nt;
-}
-
 // Host array whose elements are not initialised: for large arrays that
 // threads fill, so that one thread does not touch all their pages first.
 template <class T>
@@ -441,22 +423,6 @@ using HostArray = std::unique_ptr<T[]>;
 template <class T>
 HostArray<T> host_array(int64_t n) {
     return HostArray<T>(new T[(size_t)std::max<int64_t>(n, 1)]);
-}
-
-// Runs fn(begin, end) over [0, n) in up to host_threads() chunks of at
-// least `grain` iterations on threads of their own; for host loops whose
-// iterations write disjoint data.
-template <class F>
-void parallel_chunks(int64_t n, F fn, int64_t grain = 65536) {
-    const int64_t nt = std::max<int64_t>(1, std::min<int64_t>(host_threads(), n / grain));
-    if (nt <= 1) {
-        fn((int64_t)0, n);
-        return;
-    }
-    std::vector<std::thread> th;
-    th.reserve(nt);
-    for (int64_t t = 0; t < nt; ++t) th.emplace_back(fn, n * t / nt, n * (t + 1) / nt);
-    for (auto &x : th) x.join();
 }
 
 // Records the message of a failing call and waits for the work the call
@@ -639,16 +605,13 @@ int d2h(fs_ctx *c, void *dst, const void *src, size_t bytes) {
             if (i + ns < n) enqueue(i + ns);
         }
     };
-    std::thread th[STAGE_THREADS - 1];
-    const size_t nt = std::min({(size_t)host_threads(), (size_t)STAGE_THREADS, bytes / (2 * MB) + 1});
-    try {
-        for (size_t t = 0; t + 1 < nt; ++t) th[t] = std::thread(work);
-    } catch (const std::system_error &) {
-        // no more threads to be had: those there, and this one, do the copy
+    {
+        const size_t nt = std::min({(size_t)fs::host_threads(), (size_t)STAGE_THREADS, bytes / (2 * MB) + 1});
+        fs::Threads th;
+        for (size_t t = 1; t < nt && th.start(work); ++t) {
+        }
+        work();
     }
-    work();
-    for (auto &t : th)
-        if (t.joinable()) t.join();
     FS_HIP(c, (hipError_t)err.load());
     return FS_OK;
 }
@@ -733,7 +696,7 @@ int make_neighbours(fs_model *m) {
         tmp.erase(std::unique(tmp.begin(), tmp.end()), tmp.end());
     };
     m->nbr_ptr[0] = 0;
-    parallel_chunks(N, [&](int64_t n0, int64_t n1) {
+    fs::parallel_chunks(N, [&](int64_t n0, int64_t n1) {
         std::vector<int32_t> tmp;
         for (int64_t n = n0; n < n1; ++n) {
             neighbours(n, tmp);
@@ -743,7 +706,7 @@ int make_neighbours(fs_model *m) {
     for (int64_t n = 0; n < N; ++n) m->nbr_ptr[n + 1] += m->nbr_ptr[n];
     m->nnb = m->nbr_ptr[N];
     m->nbr_list = host_array<int32_t>(m->nnb);
-    parallel_chunks(N, [&](int64_t n0, int64_t n1) {
+    fs::parallel_chunks(N, [&](int64_t n0, int64_t n1) {
         std::vector<int32_t> tmp;
         for (int64_t n = n0; n < n1; ++n) {
             neighbours(n, tmp);
@@ -1024,7 +987,7 @@ int build_patches(fs_model *m) {
     if (N >= (int64_t(1) << 27)) return FS_OK;
     if (const int e = host_lists(m)) return e;
     std::vector<uint8_t> act(N);
-    parallel_chunks(N, [&](int64_t I0, int64_t I1) {
+    fs::parallel_chunks(N, [&](int64_t I0, int64_t I1) {
         for (int64_t I = I0; I < I1; ++I) {
             act[I] = 0;
             for (int cc = 0; cc < 6; ++cc) act[I] |= m->dof[I * 6 + cc] < m->nfree;
@@ -1049,7 +1012,7 @@ int build_patches(fs_model *m) {
             x = g;
         }
     };
-    parallel_chunks(N, [&](int64_t I0, int64_t I1) {
+    fs::parallel_chunks(N, [&](int64_t I0, int64_t I1) {
         for (int64_t I = I0; I < I1; ++I)
             for (int k = m->nbr_ptr[I]; k < m->nbr_ptr[I + 1] && m->nbr_list[k] < I; ++k) {
                 int32_t a = (int32_t)I, b = m->nbr_list[k];
@@ -1083,7 +1046,7 @@ int build_patches(fs_model *m) {
     constexpr int64_t CH = 8192;  // nodes counted together
     const int64_t nch = (N + CH - 1) / CH;
     std::vector<int64_t> at(nch + 1, 0);
-    parallel_chunks(nch, [&](int64_t k0, int64_t k1) {
+    fs::parallel_chunks(nch, [&](int64_t k0, int64_t k1) {
         int64_t nr = 0;
         for (int64_t k = k0; k < k1; ++k)
             for (int64_t I = k * CH; I < std::min(N, (k + 1) * CH); ++I) {
@@ -1101,7 +1064,7 @@ int build_patches(fs_model *m) {
     std::vector<int64_t> cptr(2, 0);
     if (roots == 1) {
         cptr[1] = npt;
-        parallel_chunks(nch, [&](int64_t k0, int64_t k1) {
+        fs::parallel_chunks(nch, [&](int64_t k0, int64_t k1) {
             int64_t to = at[k0];
             for (int64_t I = k0 * CH; I < std::min(N, k1 * CH); ++I)
                 if (active(I)) pt[to++] = point(I, 0);
@@ -1204,15 +1167,13 @@ int build_patches(fs_model *m) {
             return u.x[ax] != v.x[ax] ? u.x[ax] < v.x[ax] : u.id < v.id;
         });
         if (n > 65536) {  // creating a thread can take as long as cutting 50,000 nodes (3 ms)
-            std::thread th(bisect, b + n1, n - n1);
-            bisect(b, n1);
-            th.join();
+            fs::run_shares(2, [&](int64_t t) { t ? bisect(b + n1, n - n1) : bisect(b, n1); });
         } else {
             bisect(b, n1);
             bisect(b + n1, n - n1);
         }
     };
-    parallel_chunks(kernel_cuts ? 0 : nc, [&](int64_t k0, int64_t k1) {
+    fs::parallel_chunks(kernel_cuts ? 0 : nc, [&](int64_t k0, int64_t k1) {
         for (int64_t k = k0; k < k1; ++k)
             if (cptr[k + 1] > cptr[k]) bisect(cptr[k], cptr[k + 1] - cptr[k]);
     }, 16);
@@ -1376,7 +1337,7 @@ int build_tiles(fs_model *m, int which, int NE) {
         }
     }
     std::vector<uint64_t> key(E);
-    parallel_chunks(E, [&](int64_t e0, int64_t e1) {
+    fs::parallel_chunks(E, [&](int64_t e0, int64_t e1) {
         for (int64_t e = e0; e < e1; ++e) {
             const int g = comp[e];
             double ext = 0.0;
@@ -1430,9 +1391,7 @@ int build_tiles(fs_model *m, int which, int NE) {
                 return cu != cv ? cu < cv : u < v;
             });
             if (n > (int64_t(1) << 16)) {
-                std::thread th(bisect, b + n1, n - n1);
-                bisect(b, n1);
-                th.join();
+                fs::run_shares(2, [&](int64_t t) { t ? bisect(b + n1, n - n1) : bisect(b, n1); });
             } else {
                 bisect(b, n1);
                 bisect(b + n1, n - n1);
@@ -1468,7 +1427,7 @@ int build_tiles(fs_model *m, int which, int NE) {
     };
     std::vector<std::vector<Ent>> tent(ntiles);
     std::atomic<int> bad{0};
-    parallel_chunks(ntiles, [&](int64_t t0, int64_t t1) {
+    fs::parallel_chunks(ntiles, [&](int64_t t0, int64_t t1) {
         std::vector<std::array<int32_t, 4>> tup;  // (pair, element, code, 0)
         for (int64_t t = t0; t < t1; ++t) {
             tup.clear();
@@ -2072,7 +2031,7 @@ int fs_model_create(fs_ctx *ctx, int nen, int64_t nnodes, const double *xyz, int
     // device geometry (SoA) and connectivity planes
     int s;
     std::vector<int32_t> planes((size_t)nelem * nen);
-    parallel_chunks(nelem, [&](int64_t e0, int64_t e1) {
+    fs::parallel_chunks(nelem, [&](int64_t e0, int64_t e1) {
         for (int64_t e = e0; e < e1; ++e)
             for (int a = 0; a < nen; ++a) planes[(size_t)a * nelem + e] = m->conn[e * nen + a];
     });
@@ -3134,31 +3093,28 @@ int fs_coo_create(fs_ctx *ctx, int64_t nrows, int64_t ncols, int32_t kr, int32_t
     // row receives its entries in stream order.
     std::vector<int64_t> cnt(nrows + 1, 0);
     auto rowpass = [&](std::vector<int64_t> *fill, int64_t *bcol, int64_t *bpos) {
-        const int64_t nt = std::max<int64_t>(1, std::min<int64_t>(host_threads(), nrows / 4096 + 1));
-        std::vector<std::thread> th;
-        for (int64_t t = 0; t < nt; ++t)
-            th.emplace_back([&, t] {
-                const int64_t r0 = nrows * t / nt, r1 = nrows * (t + 1) / nt;
-                for (int64_t m = 0; m < nmat; ++m) {
-                    const int64_t *dr = dofnums_row + m * kr, *dc = dofnums_col + m * kc;
-                    for (int j = 0; j < kc; ++j) {
-                        const int64_t c = dc[j] - index_base;
-                        if (c >= ncols) continue;
-                        for (int i = 0; i < kr; ++i) {
-                            const int64_t r = dr[i] - index_base;
-                            if (r < r0 || r >= r1) continue;
-                            if (!fill) {
-                                cnt[r + 1]++;
-                            } else {
-                                const int64_t q = (*fill)[r]++;
-                                bcol[q] = c;
-                                bpos[q] = m * ke + (int64_t)j * kr + i;
-                            }
+        const int64_t nt = std::max<int64_t>(1, std::min<int64_t>(fs::host_threads(), nrows / 4096 + 1));
+        fs::run_shares(nt, [&](int64_t t) {
+            const int64_t r0 = nrows * t / nt, r1 = nrows * (t + 1) / nt;
+            for (int64_t m = 0; m < nmat; ++m) {
+                const int64_t *dr = dofnums_row + m * kr, *dc = dofnums_col + m * kc;
+                for (int j = 0; j < kc; ++j) {
+                    const int64_t c = dc[j] - index_base;
+                    if (c >= ncols) continue;
+                    for (int i = 0; i < kr; ++i) {
+                        const int64_t r = dr[i] - index_base;
+                        if (r < r0 || r >= r1) continue;
+                        if (!fill) {
+                            cnt[r + 1]++;
+                        } else {
+                            const int64_t q = (*fill)[r]++;
+                            bcol[q] = c;
+                            bpos[q] = m * ke + (int64_t)j * kr + i;
                         }
                     }
                 }
-            });
-        for (auto &x : th) x.join();
+            }
+        });
     };
     rowpass(nullptr, nullptr, nullptr);
     for (int64_t r = 0; r < nrows; ++r) cnt[r + 1] += cnt[r];
@@ -3168,7 +3124,7 @@ int fs_coo_create(fs_ctx *ctx, int64_t nrows, int64_t ncols, int32_t kr, int32_t
     // per row: a stable sort by column keeps stream order among duplicates;
     // each run of equal columns is one stored entry (zeros retained)
     std::vector<int64_t> rlen(nrows, 0), perm(M);
-    parallel_chunks(nrows, [&](int64_t r0, int64_t r1) {
+    fs::parallel_chunks(nrows, [&](int64_t r0, int64_t r1) {
         for (int64_t r = r0; r < r1; ++r) {
             const int64_t b = cnt[r], e = cnt[r + 1];
             for (int64_t q = b; q < e; ++q) perm[q] = q;
@@ -3185,7 +3141,7 @@ int fs_coo_create(fs_ctx *ctx, int64_t nrows, int64_t ncols, int32_t kr, int32_t
     h->nnz = nnz;
     h->colval.resize(nnz);
     std::vector<int64_t> cptr(nnz + 1), clist(M);
-    parallel_chunks(nrows, [&](int64_t r0, int64_t r1) {
+    fs::parallel_chunks(nrows, [&](int64_t r0, int64_t r1) {
         for (int64_t r = r0; r < r1; ++r) {
             int64_t s = h->rowptr[r] - 1;
             for (int64_t q = cnt[r]; q < cnt[r + 1]; ++q) {
@@ -3223,7 +3179,7 @@ int fs_coo_pattern(const fs_coo *h, int64_t *nnz) {
 int fs_coo_pattern_get(const fs_coo *h, int64_t *rowptr, int64_t *colval, int index_base) {
     if (!h || !rowptr || !colval) return FS_ERR_ARG;
     for (int64_t r = 0; r <= h->nrows; ++r) rowptr[r] = h->rowptr[r] + index_base;
-    parallel_chunks(h->nnz, [&](int64_t a, int64_t b) {
+    fs::parallel_chunks(h->nnz, [&](int64_t a, int64_t b) {
         for (int64_t q = a; q < b; ++q) colval[q] = h->colval[q] + index_base;
     });
     return FS_OK;
