@@ -7,9 +7,14 @@
 // normals and the time loop runs in the kernels of fs_kernels.hip.
 #include <hip/hip_runtime.h>
 
+#include <fcntl.h>
+#include <sys/file.h>
+#include <sys/stat.h>
+
 #include <algorithm>
 #include <array>
 #include <atomic>
+#include <cerrno>
 #include <chrono>
 #include <cmath>
 #include <cstdlib>
@@ -1819,37 +1824,66 @@ fs::MixedOp mixed_op(const fs_model *m) {
 // one another, so all loops in flight have to fit the device together.  A loop
 // takes as many places as it has patches and gives them back when it has
 // ended; there are two per CU, of the three and more workgroups that a CU holds.
+// They are counted within a process, and one process at a time has them: it holds a
+// lock on a file of the device's (by its PCI address, in /dev/shm) while loops of
+// its own are in flight (two system calls), and the kernel gives the lock back when
+// a process ends.  Where no such file is to be had the count stands alone, and loops of
+// two processes that do not fit together end by their bounded waits.
 class LoopPlaces {
   public:
     ~LoopPlaces() {
         if (n_ == 0) return;
         std::lock_guard<std::mutex> lk(mu());
-        used(dev_) -= n_;
+        Device &d = device(dev_);
+        d.used -= n_;
+        if (d.used == 0 && d.lock >= 0) (void)flock(d.lock, LOCK_UN);
     }
     bool take(int dev, int64_t n) {
-        static std::array<int64_t, 64> cus{};
-        if (dev < 0 || dev >= 64) return false;
+        if (dev < 0 || dev >= 64 || n <= 0) return false;
         std::lock_guard<std::mutex> lk(mu());
-        if (cus[dev] == 0) {
+        Device &d = device(dev);
+        if (d.cus == 0) {
             int v = 0;
             if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return false;
-            cus[dev] = v;
+            d.lock = open_lock(dev);
+            d.cus = v;
         }
-        if (used(dev) + n > 2 * cus[dev]) return false;
-        used(dev) += n;
+        if (d.used + n > 2 * d.cus) return false;
+        if (d.used == 0 && d.lock >= 0 && flock(d.lock, LOCK_EX | LOCK_NB) != 0 && errno == EWOULDBLOCK) return false;
+        d.used += n;
         dev_ = dev;
         n_ = n;
         return true;
     }
 
   private:
+    struct Device {
+        int64_t cus = 0, used = 0;
+        int lock = -1;
+    };
     static std::mutex &mu() {
         static std::mutex m;
         return m;
     }
-    static int64_t &used(int dev) {
-        static std::array<int64_t, 64> u{};
-        return u[dev];
+    static Device &device(int dev) {
+        static std::array<Device, 64> d;
+        return d[dev];
+    }
+    // read-only, so that it works for a file of another user too
+    static int open_lock(int dev) {
+        char bus[64] = "";
+        if (hipDeviceGetPCIBusId(bus, sizeof bus, dev) != hipSuccess) {
+            (void)hipGetLastError();
+            return -1;
+        }
+        const std::string path = std::string("/dev/shm/flexshell-loops-") + bus;
+        const int flags = O_RDONLY | O_CLOEXEC | O_NOFOLLOW;
+        int fd = open(path.c_str(), flags);
+        if (fd < 0) {
+            fd = open(path.c_str(), flags | O_CREAT, 0644);
+            if (fd >= 0) (void)fchmod(fd, 0644);  // whatever the umask
+        }
+        return fd;
     }
     int dev_ = 0;
     int64_t n_ = 0;

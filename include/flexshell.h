@@ -473,8 +473,9 @@ int fs_ctx_set_cd_lanes(fs_ctx *ctx, int lanes_per_node, int positions_per_lane)
 
 /* Explicit loops of 100 steps or more on small meshes (no counterpart in the
  * reference) run in one launch whose workgroups wait for one another's
- * displacements, where there is room for all of them on the device, else
- * step by step with bitwise the same results.  polls: the longest wait of a
+ * displacements, where there is room for all of them on the device and no
+ * other process has such loops in flight there, else step by step with bitwise
+ * the same results.  polls: the longest wait of a
  * lane in polls (at most 2^21, about two seconds; 0 = that default), after
  * which the call starts again step by step, as do later calls on the context;
  * negative: always step by step. */
