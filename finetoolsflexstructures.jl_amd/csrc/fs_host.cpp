@@ -376,6 +376,11 @@ struct StepCache {
         key.clear();
     }
     ~StepCache() { drop_graph(); }
+    void release() {
+        for (DevBuf *b : {&dPub, &dForced, &dU[0], &dU[1], &dV, &dA, &dF, &dInv, &dC, &dSlot, &dProbe, &dRG, &dGdt, &dGcd,
+                          &dG, &dPlist})
+            b->release();
+    }
 };
 
 struct fs_model {
@@ -2711,16 +2716,21 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
     // in one launch where the mesh is small enough and there is room
     bool loop = false;
     if (patch && p->nsteps < INT32_MAX && (s = patch_loops(m, p->precision, &loop))) return s;
-    const bool loop_form = loop;
+    bool loop_form = loop;
     LoopPlaces places;
     if (loop) loop = places.take(c->device, P.largest_set);
     // State vectors: the free dofs themselves (row products), node-major dof
     // positions 6 i + c (mixed path), or the patches' slot positions; fixed
     // dofs stay zero in the last two.
-    const bool placed = mixed || patch;
-    const int64_t nv = patch ? P.npatch * fs::PATCH_WG : mixed ? 6 * m->N : n;
-    // dof at each position
-    const int64_t *map = patch ? P.map.as<int64_t>() : mixed ? m->node_dof.as<int64_t>() : nullptr;
+    bool placed = false;
+    int64_t nv = 0;
+    const int64_t *map = nullptr;  // dof at each position
+    auto lay_out = [&] {
+        placed = mixed || patch;
+        nv = patch ? P.npatch * fs::PATCH_WG : mixed ? 6 * m->N : n;
+        map = patch ? P.map.as<int64_t>() : mixed ? m->node_dof.as<int64_t>() : nullptr;
+    };
+    lay_out();
     bool damped = false;
     for (int gi = 0; gi < ng; ++gi) damped |= (batch ? p->group_cdamp[gi] : p->cdamp) != 0.0;
     StepCache &sc = m->step;
@@ -2769,9 +2779,28 @@ int fs_model_explicit(fs_model *m, const fs_cd_params *p, const double *U0, cons
     std::vector<uint8_t> forced(p->nsteps + 1, 0);
     for (int64_t step = 0; step <= p->nsteps; ++step)
         for (int gi = 0; gi < ng && !forced[step]; ++gi) forced[step] = g[step * ng + gi] != 0.0;
-    if ((s = set_up()) ||
-        (loop && ((s = ensure(c, sc.dPub, nv * 32)) || (s = put(c, sc.dForced, forced.data(), forced.size())) ||
-                  (!batch && (s = put(c, dG, g, (size_t)p->nsteps + 1)))))) {
+    s = set_up();
+    if (s == FS_ERR_NOMEM && patch) {
+        // no memory for the slots of the patches (up to twice the dofs): the other
+        // forms, for this block
+        sc.drop_graph();
+        sc.release();
+        P.reset();
+        P.planned = true;
+        patch = loop = loop_form = false;
+        lay_out();
+        c->err.clear();
+        s = set_up();
+    }
+    if (s == FS_OK && loop &&
+        ((s = ensure(c, sc.dPub, nv * 32)) || (s = put(c, sc.dForced, forced.data(), forced.size())) ||
+         (!batch && (s = put(c, dG, g, (size_t)p->nsteps + 1)))) &&
+        s == FS_ERR_NOMEM) {
+        loop = false;  // step by step
+        c->err.clear();
+        s = FS_OK;
+    }
+    if (s) {
         sc.drop_graph();
         return s;
     }
