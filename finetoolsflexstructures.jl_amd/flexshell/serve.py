@@ -30,11 +30,13 @@ from . import _lib, explicit, femm as FM
 ASSEMBLY, MODAL, EXPLICIT = "assembly", "modal", "explicit"
 
 
-def footprint_bytes(nen, nelem, nnodes, nrows, kind):
+def footprint_bytes(nen, nelem, nnodes, nrows, kind, precision=_lib.FS_PREC_FP64):
     """Upper estimate of the device bytes a request holds while it runs: mesh
     and adjacency, normals, dof map, element blocks, the CSR pattern, values
     and scatter tables of one block, the lumped mass and, for explicit jobs,
-    the step vectors and power-iteration vectors."""
+    the step vectors (whole patches of 42 nodes), power-iteration vectors and the
+    patches' blocks, in the mixed precisions beside the operator that these are made
+    from: element blocks, slices, and shear rows for FS_PREC_MIXED."""
     nblk = nen * (nen + 1) // 2
     per_row = 6 * (9 if nen == 4 else 7)  # structured stencil (neighbour nodes incl. self) x 6
     nnz = nrows * per_row
@@ -42,9 +44,16 @@ def footprint_bytes(nen, nelem, nnodes, nrows, kind):
     blocks = nelem * nblk * (36 * 8 + 4)
     csr = nnz * 12 + nrows * 20 + nnodes * 120
     cols = 0 if kind == EXPLICIT else min(nnz * 8, 64 << 20)  # the window the columns are written to
-    vec = nrows * 8 * (11 if kind == EXPLICIT else 1)
-    patch = nnz * 6 if kind == EXPLICIT else 0  # 0.67 of the values, entry tables
-    return int(1.25 * (mesh + blocks + csr + cols + vec + patch)) + (4 << 20)
+    vec = nrows * 8
+    patch = mixed = 0
+    if kind == EXPLICIT:
+        vec = max(nrows, 6 * 42 * -(-nnodes // 42)) * 8 * 11
+        patch = nnz * 6  # 0.67 of the values, entry tables
+        if precision != _lib.FS_PREC_FP64:
+            mixed = blocks + nnz * 6
+        if precision == _lib.FS_PREC_MIXED:
+            mixed += nelem * (6 if nen == 3 else 8) * 6 * nen * 8
+    return int(1.25 * (mesh + blocks + csr + cols + vec + patch + mixed)) + (4 << 20)
 
 
 class Request:
@@ -72,7 +81,8 @@ class Request:
         d = m["dchi"]
         nrows = d.nalldofs if kind == ASSEMBLY else d.nfreedofs
         self.nelem = int(m["conn"].shape[0])
-        self.footprint = footprint_bytes(int(m["conn"].shape[1]), self.nelem, int(m["xyz"].shape[0]), nrows, kind)
+        self.footprint = footprint_bytes(int(m["conn"].shape[1]), self.nelem, int(m["xyz"].shape[0]), nrows, kind,
+                                         self.precision)
 
     @property
     def latency(self):
