@@ -10,7 +10,10 @@ central-difference step) processes all models in one launch; the step loop
 is captured in a hipGraph.  Each model keeps its own material, time step,
 damping and load history, and its results are bitwise identical to running
 it alone: per element and per CSR row the arithmetic and its order do not
-depend on the other models in the batch.
+depend on the other models in the batch.  (A node of more than 1,024
+neighbours is the exception: loops of 100 steps or more then take the row
+products for the whole batch, and the other models' results equal those
+alone up to the order of addition.)
 """
 import ctypes as C
 

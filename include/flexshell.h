@@ -468,7 +468,10 @@ int fs_ctx_set_assembly(fs_ctx *ctx, int mode);
  * reproducible and gives a model bitwise the same result alone and in a
  * batch.  Default 8 lanes per node, positions chosen; with that setting,
  * explicit loops of 100 steps or more run on a symmetric copy of K cut into
- * node patches (each block read once per patch), which the model keeps. */
+ * node patches (each block read once per patch), which the model keeps.  They
+ * take the row products instead where a node has more than 1024 neighbours or
+ * there is no memory for the patches: a batch with such a node for all of its
+ * models, which then equal themselves alone up to the order of addition. */
 int fs_ctx_set_cd_lanes(fs_ctx *ctx, int lanes_per_node, int positions_per_lane);
 
 /* Explicit loops of 100 steps or more on small meshes (no counterpart in the

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 import test_gpu_patch_step as PS
-from flexshell import _lib, explicit, fe, femm as FM
+from flexshell import _lib, batch as FB, explicit, fe, femm as FM
 from flexshell.material import MatDeforElastIso
 
 pytestmark = pytest.mark.gpu
@@ -103,3 +103,25 @@ def test_loops_at_the_same_time(ctx):
     assert all(run() == ONE for _, run in jobs)  # none has left the form
     for f, _ in jobs:
         f._model.close()
+
+
+def test_batch_with_a_hub_past_a_patch(ctx):
+    """The row products for the whole batch: a model beside the hub equals itself alone
+    (on patches) up to the order of addition, 1e-12 relative as between the forms."""
+    print("[gpu] batch with a hub", flush=True)
+    models = [dict(xyz=xyz, conn=conn, dchi=d, material=MatDeforElastIso(70e9, 0.33, 2700.0), t=0.02)
+              for _, xyz, conn, d in (PS._grid(3, 17, 13), PS._fan(1100))]
+    b = FB.ShellBatch(models, ctx=ctx)
+    b.assemble_device()
+    b.mass()
+    V0, z = np.random.default_rng(6).normal(0, 1e-3, b.nfree), np.zeros(b.nfree)
+    r = b.explicit([1e-8] * 2, [0.0] * 2, z, V0, z, np.zeros((121, 2)), 120, use_graph=False)
+    assert b.model.cd_form() == ROWS
+    m, sl = models[0], b.model_slice(0)
+    f, run = _femm(ctx, (3, m["xyz"], m["conn"], m["dchi"]))
+    a = explicit.run(f._model, 0.0, z[sl], V0[sl], 1e-8, 120, z[sl], np.zeros(121))
+    assert f._model.cd_form() == ONE
+    for key in ("U", "V"):
+        assert np.linalg.norm(a[key] - r[key][sl]) <= 1e-12 * np.linalg.norm(a[key]), key
+    f._model.close()
+    b.close()
