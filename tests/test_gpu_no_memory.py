@@ -1,6 +1,6 @@
 """Calls that find no device memory.  A small library loaded before the HIP runtime
 takes hipMalloc's place in a process of its own and refuses requests of given
-sizes, as a full device does."""
+sizes, as a full device does.  (It counts the bytes of hipHostMalloc too.)"""
 import os
 import subprocess
 import sys
@@ -23,6 +23,14 @@ int hipMalloc(void **p, size_t n) {
     if (n >= lo && n <= hi && first-- <= 0) { ++refused; *p = 0; return 2; }  /* hipErrorOutOfMemory */
     if (!real) real = (int (*)(void **, size_t))dlsym(dlopen("libamdhip64.so.7", RTLD_NOW), "hipMalloc");
     return real(p, n);
+}
+static size_t host_bytes = 0;
+size_t pinned(void) { return host_bytes; }
+int hipHostMalloc(void **p, size_t n, unsigned flags) {
+    static int (*real)(void **, size_t, unsigned);
+    if (!real) real = (int (*)(void **, size_t, unsigned))dlsym(dlopen("libamdhip64.so.7", RTLD_NOW), "hipHostMalloc");
+    host_bytes += n;
+    return real(p, n, flags);
 }
 """
 
